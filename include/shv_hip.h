@@ -79,6 +79,24 @@ int shv_download(shv_ctx *ctx, void *dst_host, const void *src_dev, size_t bytes
 int shv_upload_async(shv_ctx *ctx, void *dst_dev, const void *src_host, size_t bytes);
 int shv_copy(shv_ctx *ctx, void *dst_dev, const void *src_dev, size_t bytes);  /* async, in order */
 int shv_zero(shv_ctx *ctx, void *dst_dev, size_t bytes);                       /* Buffer.Zero*, async */
+/* 32-bit words from host memory to several places in one launch (a pass's positions, planes, tables and ids): they
+ * travel in the launch's own arguments, src may be reused at once, nothing waits.  async, in order. */
+typedef struct shv_words {
+    void *dst;
+    const int32_t *src;
+    int32_t n;
+} shv_words;
+int shv_upload_words(shv_ctx *ctx, const shv_words *words, int n);
+/* Many copies of the device's memory in one launch (a sequence's carried state is a few pieces a layer): every span's
+ * bytes from src to dst, zeros where src is NULL.  Addresses and lengths are multiples of 4 (of 16 to run at
+ * full width); no span's dst may overlap
+ * another span.  async, in order. */
+typedef struct shv_span {
+    void *dst;
+    const void *src;
+    uint64_t bytes;
+} shv_span;
+int shv_copy_spans(shv_ctx *ctx, const shv_span *spans, int n);
 /* Pinned host memory the device can address: staging for transfers, and somewhere an op can leave a
  * small result (the arg-max's best) that the host reads after the submit's wait without a download. */
 int shv_host_alloc(shv_ctx *ctx, size_t bytes, void **hptr);
@@ -419,7 +437,7 @@ typedef struct {
     void *kcache;
     void *vcache;
     float *partial;
-    float *out;
+    float *out;  /* NULL: the rows' cells are written and nothing is attended */
     const int32_t *pos;
     const int32_t *slot;
     int32_t n_seq, seq_len;

@@ -37,6 +37,49 @@ __global__ __launch_bounds__(256) void dequant_q4k_kernel(const uint8_t *w, floa
         }
 }
 
+// Up to kSpans copies (or fills with zeros) a launch, the list in the kernel's arguments.  Bound by HBM: the 12 states
+// and 36 ring rows of a 16-layer sequence, 27 MB, take 12 us where 48 hipMemcpyAsync took 1.3 ms from pageable memory.
+// grid (kSpanBlocks, spans): a span's blocks walk it in steps of the whole span, 64 bytes a thread and step.
+constexpr int kSpans = 128, kSpanBlocks = 32;
+struct SpanList {
+    shv_span s[kSpans];
+};
+__global__ __launch_bounds__(256) void copy_spans_kernel(SpanList list) {
+    const shv_span sp = list.s[blockIdx.y];
+    if (((reinterpret_cast<uintptr_t>(sp.dst) | reinterpret_cast<uintptr_t>(sp.src) | sp.bytes) & 15) != 0) {
+        const size_t nw = sp.bytes / 4;
+        for (size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x; i < nw; i += kSpanBlocks * 256)
+            static_cast<uint32_t *>(sp.dst)[i] = sp.src ? static_cast<const uint32_t *>(sp.src)[i] : 0;
+        return;
+    }
+    const size_t n = sp.bytes / 16, step = static_cast<size_t>(kSpanBlocks) * 1024;
+    uint4 *dst = static_cast<uint4 *>(sp.dst);
+    const uint4 *src = static_cast<const uint4 *>(sp.src);
+    for (size_t i0 = static_cast<size_t>(blockIdx.x) * 1024 + threadIdx.x; i0 < n; i0 += step) {
+        uint4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[u] = src && i0 + u * 256 < n ? src[i0 + u * 256] : make_uint4(0, 0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (i0 + u * 256 < n) dst[i0 + u * 256] = v[u];
+    }
+}
+
+// Words that travel in the launch's arguments: the control words of a pass cost one launch (4 us of host time, 2 on the
+// device), where a copy from pinned memory each cost as much and a copy engine's hand-over on the device.
+constexpr int kWordSpans = 32, kWords = 640;
+struct WordList {
+    int32_t *dst[kWordSpans];
+    uint16_t end[kWordSpans];  // the words of span i are end[i-1] .. end[i]-1
+    int32_t w[kWords];
+};
+__global__ __launch_bounds__(256) void upload_words_kernel(WordList list, int spans) {
+    for (int s = 0; s < spans; s++) {
+        const int from = s > 0 ? list.end[s - 1] : 0, to = list.end[s];
+        for (int i = from + static_cast<int>(threadIdx.x); i < to; i += 256) list.dst[s][i - from] = list.w[i];
+    }
+}
+
 __device__ __forceinline__ uint64_t splitmix64(uint64_t x) {
     x += 0x9E3779B97F4A7C15ull;
     x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
@@ -269,5 +312,43 @@ int shv_launch_argmax_static(shv_ctx *ctx, const shv_argmax_args *a) {
 int shv_launch_advance(shv_ctx *ctx, const shv_advance_args *a) {
     SHV_REQUIRE(a->pos && a->n_seq >= 1, "advance: NULL pos or n_seq %d", a->n_seq);
     SHV_LAUNCH(ctx, advance_kernel, dim3((a->n_seq + 63) / 64), dim3(64), 0, *a);
+    return SHV_OK;
+}
+
+int shv_launch_copy_spans(shv_ctx *ctx, const shv_span *spans, int n) {
+    for (int i = 0; i < n; i++) {
+        SHV_REQUIRE(spans[i].dst && ((reinterpret_cast<uintptr_t>(spans[i].dst) | reinterpret_cast<uintptr_t>(spans[i].src) | spans[i].bytes) & 3) == 0,
+                    "copy_spans: span %d is not whole words at word addresses", i);
+    }
+    for (int i0 = 0; i0 < n; i0 += kSpans) {
+        SpanList list{};
+        const int m = n - i0 < kSpans ? n - i0 : kSpans;
+        for (int i = 0; i < m; i++) list.s[i] = spans[i0 + i];
+        SHV_LAUNCH(ctx, copy_spans_kernel, dim3(kSpanBlocks, m), dim3(256), 0, list);
+    }
+    return SHV_OK;
+}
+
+int shv_launch_upload_words(shv_ctx *ctx, const shv_words *words, int n) {
+    for (int i = 0; i < n; i++)
+        SHV_REQUIRE(words[i].n >= 0 && (words[i].n == 0 || (words[i].dst && words[i].src && (reinterpret_cast<uintptr_t>(words[i].dst) & 3) == 0)),
+                    "upload_words: span %d: bad argument", i);
+    WordList list;
+    int spans = 0, used = 0;
+    for (int i = 0; i < n; i++) {
+        for (int at = 0; at < words[i].n;) {
+            const int m = words[i].n - at < kWords - used ? words[i].n - at : kWords - used;
+            list.dst[spans] = static_cast<int32_t *>(words[i].dst) + at;
+            for (int k = 0; k < m; k++) list.w[used + k] = words[i].src[at + k];
+            at += m;
+            used += m;
+            list.end[spans++] = static_cast<uint16_t>(used);
+            if (spans == kWordSpans || used == kWords) {
+                SHV_LAUNCH(ctx, upload_words_kernel, dim3(1), dim3(256), 0, list, spans);
+                spans = used = 0;
+            }
+        }
+    }
+    if (spans > 0) SHV_LAUNCH(ctx, upload_words_kernel, dim3(1), dim3(256), 0, list, spans);
     return SHV_OK;
 }

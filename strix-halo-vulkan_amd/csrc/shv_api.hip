@@ -271,6 +271,18 @@ int shv_zero(shv_ctx *ctx, void *dst, size_t bytes) {
     return SHV_OK;
 }
 
+int shv_upload_words(shv_ctx *ctx, const shv_words *words, int n) {
+    SHV_REQUIRE(ctx && (words || n == 0) && n >= 0, "shv_upload_words: bad argument");
+    SHV_REQUIRE(!ctx->capturing, "shv_upload_words: not valid while recording");
+    return shv_launch_upload_words(ctx, words, n);
+}
+
+int shv_copy_spans(shv_ctx *ctx, const shv_span *spans, int n) {
+    SHV_REQUIRE(ctx && (spans || n == 0) && n >= 0, "shv_copy_spans: bad argument");
+    SHV_REQUIRE(!ctx->capturing, "shv_copy_spans: not valid while recording");
+    return shv_launch_copy_spans(ctx, spans, n);
+}
+
 int shv_dispatch_multi(shv_ctx *ctx, const shv_op *ops, int n_ops, int iters, uint64_t *total_ns,
                        uint64_t *per_op_ns) {
     SHV_REQUIRE(ctx && ops, "shv_dispatch_multi: NULL argument");

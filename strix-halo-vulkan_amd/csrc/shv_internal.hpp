@@ -184,5 +184,7 @@ int shv_launch_router_fold(shv_ctx *ctx, const shv_router_fold_args *a);
 int shv_launch_qsa_index(shv_ctx *ctx, const shv_qsa_index_args *a);
 bool shv_dn_chunk_covers(const shv_dn_step_args &a);
 int shv_launch_dn_chunk(shv_ctx *ctx, const shv_dn_step_args &a);
+int shv_launch_copy_spans(shv_ctx *ctx, const shv_span *spans, int n);
+int shv_launch_upload_words(shv_ctx *ctx, const shv_words *words, int n);
 int shv_static_scratch_bind(shv_ctx *ctx);  // at shv_init, with ctx->device current
 int shv_launch_argmax_static(shv_ctx *ctx, const shv_argmax_args *a);

@@ -150,6 +150,14 @@ class RingRowsArgs(C.Structure):
                 ("count", C.c_int32)]
 
 
+class Span(C.Structure):
+    _fields_ = [("dst", C.c_void_p), ("src", C.c_void_p), ("bytes", C.c_uint64)]
+
+
+class Words(C.Structure):
+    _fields_ = [("dst", C.c_void_p), ("src", C.c_void_p), ("n", C.c_int32)]
+
+
 class Op(C.Structure):
     _fields_ = [("kind", C.c_uint32), ("flags", C.c_uint32), ("args", C.c_uint8 * 248)]
 
@@ -166,7 +174,7 @@ def make_op(kind, args, flags=0):
 # every symbol include/shv_hip.h declares; the CPU test suite checks the library exports them all
 SYMBOLS = [
     "shv_last_error", "shv_device_count", "shv_init", "shv_destroy", "shv_device_props", "shv_sync",
-    "shv_submits", "shv_alloc", "shv_free", "shv_upload", "shv_upload_async", "shv_download", "shv_copy", "shv_zero",
+    "shv_submits", "shv_alloc", "shv_free", "shv_upload", "shv_upload_async", "shv_download", "shv_copy", "shv_zero", "shv_copy_spans", "shv_upload_words",
     "shv_host_alloc", "shv_host_free", "shv_enqueue", "shv_dispatch_multi", "shv_prerecord",
     "shv_prerecorded_submit", "shv_prerecorded_launch", "shv_stamp", "shv_stamp_elapsed", "shv_prerecorded_count",
     "shv_prerecorded_destroy", "shv_gemv_q4k", "shv_dequant_q4k", "shv_dequant", "shv_gemv", "shv_quantize_q4k",
@@ -202,6 +210,8 @@ def load():
     L.shv_download.argtypes = [vp, vp, vp, C.c_size_t]
     L.shv_copy.argtypes = [vp, vp, vp, C.c_size_t]
     L.shv_zero.argtypes = [vp, vp, C.c_size_t]
+    L.shv_copy_spans.argtypes = [vp, C.POINTER(Span), C.c_int]
+    L.shv_upload_words.argtypes = [vp, C.POINTER(Words), C.c_int]
     L.shv_host_alloc.argtypes = [vp, C.c_size_t, vpp]
     L.shv_host_free.argtypes = [vp, vp]
     L.shv_enqueue.argtypes = [vp, C.c_uint32, vp, C.c_size_t]

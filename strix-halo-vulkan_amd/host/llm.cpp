@@ -18,19 +18,34 @@ static uint64_t q4k_bytes(int64_t rows, int64_t cols) { return rows * (cols / SH
 
 // ------------------------------------------------------------------------------- Device -------
 
-Device::Device(int index) { check(shv_init(index, &ctx_), "NewDevice"); }
+Device::Device(int index) : index_(index) {
+    shv_ctx *c = nullptr;
+    check(shv_init(index, &c), "NewDevice");
+    ctx_ = std::shared_ptr<shv_ctx>(c, shv_destroy);
+}
 
 Device::~Device() {
     if (!ctx_) return;
-    shv_sync(ctx_);
-    for (void *p : owned_) shv_free(ctx_, p);
-    for (void *p : host_owned_) shv_host_free(ctx_, p);
-    shv_destroy(ctx_);
+    shv_sync(ctx());
+    for (void *p : owned_) shv_free(ctx(), p);
+    for (void *p : host_owned_) shv_host_free(ctx(), p);
+}
+
+std::vector<float> DeviceBlock::Read() const {
+    std::vector<float> v(bytes / 4);
+    check(shv_download(ctx_.get(), v.data(), ptr, bytes), "DeviceBlock.Read");
+    return v;
+}
+
+std::shared_ptr<DeviceBlock> Device::block(size_t bytes) {
+    void *p = nullptr;
+    if (shv_alloc(ctx(), bytes, &p) != SHV_OK) return nullptr;
+    return std::make_shared<DeviceBlock>(ctx_, index_, p, bytes);
 }
 
 void *Device::host_alloc(size_t bytes) {
     void *p = nullptr;
-    check(shv_host_alloc(ctx_, bytes, &p), "host_alloc");
+    check(shv_host_alloc(ctx(), bytes, &p), "host_alloc");
     std::memset(p, 0, bytes);
     host_owned_.push_back(p);
     return p;
@@ -38,7 +53,7 @@ void *Device::host_alloc(size_t bytes) {
 
 void *Device::alloc(size_t bytes) {
     void *p = nullptr;
-    check(shv_alloc(ctx_, bytes < 256 ? 256 : bytes, &p), "alloc");
+    check(shv_alloc(ctx(), bytes < 256 ? 256 : bytes, &p), "alloc");
     owned_.push_back(p);
     allocated_ += bytes;
     return p;
@@ -48,7 +63,7 @@ void Device::release(void *p, size_t bytes) {
     auto it = std::find(owned_.begin(), owned_.end(), p);
     if (it == owned_.end()) throw Error("llm: release of memory this device did not hand out");
     sync();
-    check(shv_free(ctx_, p), "free");
+    check(shv_free(ctx(), p), "free");
     owned_.erase(it);
     allocated_ -= bytes;
 }
@@ -61,14 +76,16 @@ void *Device::alloc_zero(size_t bytes) {
 
 // small transfers (a pass's control words and ids) do not wait for the device; everything here runs on this
 // device's one stream, which orders them
-void Device::upload(void *dst, const void *src, size_t bytes) { check(shv_upload_async(ctx_, dst, src, bytes), "upload"); }
-void Device::download(void *dst, const void *src, size_t bytes) { check(shv_download(ctx_, dst, src, bytes), "download"); }
-void Device::zero(void *dst, size_t bytes) { check(shv_zero(ctx_, dst, bytes), "zero"); }
-void Device::sync() { check(shv_sync(ctx_), "sync"); }
+void Device::upload(void *dst, const void *src, size_t bytes) { check(shv_upload_async(ctx(), dst, src, bytes), "upload"); }
+void Device::download(void *dst, const void *src, size_t bytes) { check(shv_download(ctx(), dst, src, bytes), "download"); }
+void Device::zero(void *dst, size_t bytes) { check(shv_zero(ctx(), dst, bytes), "zero"); }
+void Device::words(const shv_words *w, int n) { check(shv_upload_words(ctx(), w, n), "words"); }
+void Device::copy(const std::vector<shv_span> &spans) { check(shv_copy_spans(ctx(), spans.data(), static_cast<int>(spans.size())), "copy"); }
+void Device::sync() { check(shv_sync(ctx()), "sync"); }
 
 void Device::run(const std::vector<shv_op> &ops) {
     uint64_t ns = 0;
-    check(shv_dispatch_multi(ctx_, ops.data(), static_cast<int>(ops.size()), 1, &ns, nullptr), "dispatch");
+    check(shv_dispatch_multi(ctx(), ops.data(), static_cast<int>(ops.size()), 1, &ns, nullptr), "dispatch");
 }
 
 // -------------------------------------------------------------------------------- Model -------
@@ -760,11 +777,13 @@ void DeltaNetGPU::ResetSlot(int slot) {
     if (slot < 0 || slot >= slots_) throw Error("llm: DeltaNetGPU.ResetSlot: slot " + std::to_string(slot) + " of " + std::to_string(slots_));
     const size_t ring_floats = static_cast<size_t>(ring_slots_) * c_.DNFusedRows();
     const size_t st_floats = static_cast<size_t>(planes_) * c_.SSMHeadV * c_.SSMHeadDim * c_.SSMHeadDim;
+    std::vector<shv_span> zeros;
     for (int l = 0; l < c_.NLayer; l++) {
         if (!state_[l]) continue;
-        dev_.zero(ring_[l] + slot * ring_floats, ring_floats * 4);
-        dev_.zero(state_[l] + slot * st_floats, st_floats * 4);
+        zeros.push_back({ring_[l] + slot * ring_floats, nullptr, ring_floats * 4});
+        zeros.push_back({state_[l] + slot * st_floats, nullptr, st_floats * 4});
     }
+    dev_.copy(zeros);
 }
 
 std::vector<shv_op> DeltaNetGPU::Dispatches(int l, const float *in, float *out, int nTok, std::vector<std::string> *labels) const {
@@ -930,6 +949,34 @@ void DeltaNetGPU::RestoreCarried(const float *src, int slot, int plane, int past
         for (int j = 3; j >= 1; j--, src += row)
             if (past - j >= 0) dev_.upload(ring_[l] + (static_cast<size_t>(slot) * ring_slots_ + (past - j) % ring_slots_) * row, src, row * 4);
     }
+}
+
+void DeltaNetGPU::SaveCarriedOnDevice(float *dst, int slot, int plane, int past) const {
+    if (slot < 0 || slot >= slots_ || plane < 0 || plane >= planes_) throw Error("llm: DeltaNetGPU.SaveCarried: no such slot or plane");
+    const size_t n = static_cast<size_t>(c_.SSMHeadV) * c_.SSMHeadDim * c_.SSMHeadDim, row = c_.DNFusedRows();
+    std::vector<shv_span> spans;
+    for (int l = 0; l < c_.NLayer; l++) {
+        if (!state_[l]) continue;
+        spans.push_back({dst, state_[l] + (static_cast<size_t>(slot) * planes_ + plane) * n, n * 4});
+        dst += n;
+        for (int j = 3; j >= 1; j--, dst += row)  // positions past-3, past-2, past-1; zero before the start
+            spans.push_back({dst, past - j < 0 ? nullptr : ring_[l] + (static_cast<size_t>(slot) * ring_slots_ + (past - j) % ring_slots_) * row, row * 4});
+    }
+    dev_.copy(spans);
+}
+
+void DeltaNetGPU::RestoreCarriedOnDevice(const float *src, int slot, int plane, int past) {
+    if (slot < 0 || slot >= slots_ || plane < 0 || plane >= planes_) throw Error("llm: DeltaNetGPU.RestoreCarried: no such slot or plane");
+    const size_t n = static_cast<size_t>(c_.SSMHeadV) * c_.SSMHeadDim * c_.SSMHeadDim, row = c_.DNFusedRows();
+    std::vector<shv_span> spans;
+    for (int l = 0; l < c_.NLayer; l++) {
+        if (!state_[l]) continue;
+        spans.push_back({state_[l] + (static_cast<size_t>(slot) * planes_ + plane) * n, src, n * 4});
+        src += n;
+        for (int j = 3; j >= 1; j--, src += row)
+            if (past - j >= 0) spans.push_back({ring_[l] + (static_cast<size_t>(slot) * ring_slots_ + (past - j) % ring_slots_) * row, src, row * 4});
+    }
+    dev_.copy(spans);
 }
 
 std::vector<float> DeltaNetGPU::Result() const { return read_back<float>(dev_, attn_, static_cast<size_t>(n_tok_) * c_.VWidth()); }
@@ -1809,21 +1856,39 @@ void Graph::Checkpoint(struct Checkpoint &c) {
     c.past = q.past;
     c.ids.resize(q.past);
     dev_.download(c.ids.data(), ids_ + slot_ * ids_stride_, static_cast<size_t>(q.past) * 4);
-    c.dn.resize(dn_->CarriedLen());
-    dn_->SaveCarried(c.dn.data(), slot_, q.plane, q.past);
+    const size_t carried = dn_->CarriedLen() * 4;
 }
 
+    if (!c.on_device || c.on_device->device != dev_.index() || c.on_device->bytes != carried) {
+        c.on_device = nullptr;
+        if (carried > 0) c.on_device = dev_.block(carried);
+    }
+    if (c.on_device) {
+        c.dn.clear();
+        dn_->SaveCarriedOnDevice(static_cast<float *>(c.on_device->ptr), slot_, q.plane, q.past);
+    } else {
+        c.dn.resize(dn_->CarriedLen());
+        dn_->SaveCarried(c.dn.data(), slot_, q.plane, q.past);
+    }
+    // last, since it waits: the checkpoint is whole when this returns
 void Graph::Restore(const struct Checkpoint &c) {
     Seq &q = seq_[slot_];
     if (spec_armed_) throw Error("llm: a speculative pass is in flight; commit or rewind it first");
-    bool same = c.past > 0 && c.past <= q.past && static_cast<int>(c.ids.size()) == c.past && c.dn.size() == dn_->CarriedLen();
+    bool same = c.past > 0 && c.past <= q.past && static_cast<int>(c.ids.size()) == c.past && (c.on_device ? c.on_device->bytes / 4 : c.dn.size()) == dn_->CarriedLen();
     if (same) {
         std::vector<int32_t> have(c.past);
         dev_.download(have.data(), ids_ + slot_ * ids_stride_, static_cast<size_t>(c.past) * 4);
         same = have == c.ids;
     }
     if (!same) throw Error("llm: this slot no longer holds the checkpoint's tokens");
-    dn_->RestoreCarried(c.dn.data(), slot_, q.plane, c.past);
+    if (c.on_device && c.on_device->device == dev_.index()) {
+        dn_->RestoreCarriedOnDevice(static_cast<const float *>(c.on_device->ptr), slot_, q.plane, c.past);
+    } else if (c.on_device) {  // taken on another GPU
+        const auto carried = c.on_device->Read();
+        dn_->RestoreCarried(carried.data(), slot_, q.plane, c.past);
+    } else {
+        dn_->RestoreCarried(c.dn.data(), slot_, q.plane, c.past);
+    }
     q.past = c.past;
     put_pos();
 }
@@ -1900,6 +1965,90 @@ Pass &MTPHead::draft_pass(int n, bool head, int k, int32_t *ring) {
     const std::vector<int> key{slot_, n, head ? 1 : 0, ring ? 1 + k : 0};
     auto it = passes_.find(key);
     if (it != passes_.end() && it->second.ring != ring) {
+// What every pass of this block begins with: the tokens' embeddings and eh_proj over them and h.
+std::vector<shv_op> MTPHead::input_ops(int n, int32_t *ring, std::vector<std::string> *labels) const {
+    const int E = c_.NEmbd;
+    std::vector<shv_op> ops;
+    shv_embed_args e{};
+    e.table = m_.Tensor("token_embd.weight").ptr;
+    e.type = static_cast<int32_t>(m_.Tensor("token_embd.weight").ggml);
+    e.ids = ring ? ring : ids_;
+    e.pos = ring ? pos_ + slot_ : nullptr;
+    e.x = e_;
+    e.n_tok = n;
+    e.n_embd = E;
+    e.vocab = c_.VocabSize;
+    e.x_stride = E;
+    ops.push_back(make_op(SHV_OP_EMBED, e));
+    if (labels) labels->push_back("embed");
+    shv_gemv_q4k_args g{};
+    g.w = m_.Tensor(Model::Blk(layer_, "nextn.eh_proj")).ptr;
+    g.x = e_;
+    g.z = h_;
+    g.y = x_;
+    g.gamma = static_cast<const float *>(m_.Tensor(Model::Blk(layer_, "nextn.ehnorm_fused")).ptr);
+    g.n = E;
+    g.k = 2 * E;
+    g.n_tok = n;
+    g.prologue = SHV_PRO_RMSNORM_PAIR;
+    g.eps = c_.RMSEps;
+    g.x_stride = g.z_stride = g.y_stride = E;
+    ops.push_back(make_op(SHV_OP_GEMV_Q4K, g));
+    if (labels) labels->push_back("mtp.eh_proj");
+    return ops;
+}
+
+PassRows MTPHead::rows_of(int n) const {
+    PassRows r;
+    r.pos = pos_ + slot_;
+    r.slot = slot_ix_ + slot_;
+    r.host_slot = slot_;
+    r.seq_len = n;
+    return r;
+}
+
+Pass &MTPHead::cell_pass(int n) {
+    const std::vector<int> key{slot_, n, 2, 0};
+    auto it = passes_.find(key);
+    if (it == passes_.end()) {
+        Pass p;
+        p.ops = input_ops(n, nullptr, &p.labels);
+        auto a = attn_->Dispatches(layer_, x_, x_, rows_of(n), &p.labels);
+        shv_attn_decode_args cells{};
+        std::memcpy(&cells, a[1].args, sizeof cells);
+        cells.out = nullptr;  // the rows' cells, nothing attended
+        p.ops.push_back(a[0]);
+        p.ops.push_back(make_op(SHV_OP_ATTN_DECODE, cells));
+        it = passes_.emplace(key, std::move(p)).first;
+    }
+    return it->second;
+}
+
+void MTPHead::check_rows(const std::vector<int32_t> &ids, int pos) const {
+    const int n = static_cast<int>(ids.size());
+    if (pos < 0 || pos > pasts_[slot_]) throw Error("llm: MTPHead.Rows: position " + std::to_string(pos) + " leaves a gap after the draft cache's " + std::to_string(pasts_[slot_]) + " cells");
+    if (pos + n + 1 > n_kv_) throw Error("llm: MTPHead.Rows: " + std::to_string(pos + n) + " cells do not fit " + std::to_string(n_kv_));
+    for (int32_t id : ids)
+        if (id < 0 || id >= c_.VocabSize) throw Error("llm: token " + std::to_string(id) + " is outside the vocabulary");
+}
+
+void MTPHead::WriteCells(const float *hs, const std::vector<int32_t> &ids, int pos) {
+    const int n = static_cast<int>(ids.size());
+    if (!hs || n < 1) throw Error("llm: MTPHead.WriteCells: no rows");
+    check_rows(ids, pos);
+    for (int a = 0; a < n; a += cell_rows_) {
+        const int k = std::min(cell_rows_, n - a);
+        Pass &pass = cell_pass(k);
+        const int32_t p32 = pos + a;
+        check(shv_copy(dev_.ctx(), h_, hs + static_cast<size_t>(a) * c_.NEmbd, static_cast<size_t>(k) * c_.NEmbd * 4), "draft input");
+        dev_.words({{ids_, ids.data() + a, k}, {pos_ + slot_, &p32, 1}});
+        if (!pass.rec) check(shv_prerecord(dev_.ctx(), pass.ops.data(), static_cast<int>(pass.ops.size()), &pass.rec), "draft cells");
+        check(shv_prerecorded_launch(dev_.ctx(), pass.rec), "draft cells");
+        Steps++;
+    }
+    pasts_[slot_] = pos + n;
+}
+
         if (it->second.rec) shv_prerecorded_destroy(dev_.ctx(), it->second.rec);
         passes_.erase(it);
         it = passes_.end();

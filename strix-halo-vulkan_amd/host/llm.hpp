@@ -27,6 +27,22 @@ struct Error : std::runtime_error {
     using std::runtime_error::runtime_error;
 };
 
+// A device allocation that may outlive the Device it came from: it holds the context itself.
+class DeviceBlock {
+public:
+    DeviceBlock(std::shared_ptr<shv_ctx> ctx, int device, void *p, size_t bytes) : device(device), ptr(p), bytes(bytes), ctx_(std::move(ctx)) {}
+    ~DeviceBlock() { shv_free(ctx_.get(), ptr); }
+    DeviceBlock(const DeviceBlock &) = delete;
+    DeviceBlock &operator=(const DeviceBlock &) = delete;
+    std::vector<float> Read() const;
+    const int device;
+    void *const ptr;
+    const size_t bytes;
+
+private:
+    std::shared_ptr<shv_ctx> ctx_;
+};
+
 // vk.Device (vk/engine.go:266-311): owns the context; every block borrows it.
 class Device {
 public:
@@ -34,7 +50,9 @@ public:
     ~Device();
     Device(const Device &) = delete;
     Device &operator=(const Device &) = delete;
-    shv_ctx *ctx() const { return ctx_; }
+    shv_ctx *ctx() const { return ctx_.get(); }
+    int index() const { return index_; }
+    std::shared_ptr<DeviceBlock> block(size_t bytes);  // nullptr where the device has no room
     void *alloc(size_t bytes);  // tracked; released with the device
     void *alloc_zero(size_t bytes);
     void release(void *p, size_t bytes);  // an alloc() handed back early; bytes as asked for
@@ -42,12 +60,16 @@ public:
     void upload(void *dst, const void *src, size_t bytes);
     void download(void *dst, const void *src, size_t bytes);
     void zero(void *dst, size_t bytes);
+    void words(const std::vector<shv_words> &w) { words(w.data(), static_cast<int>(w.size())); }  // shv_upload_words: in order, does not wait
+    void words(const shv_words *w, int n);
+    void copy(const std::vector<shv_span> &spans);  // shv_copy_spans: in order, does not wait
     void sync();
     void run(const std::vector<shv_op> &ops);  // dispatch and block
     size_t allocated() const { return allocated_; }
 
 private:
-    shv_ctx *ctx_ = nullptr;
+    std::shared_ptr<shv_ctx> ctx_;
+    int index_ = 0;
     std::vector<void *> owned_, host_owned_;
     size_t allocated_ = 0;
 };
@@ -283,6 +305,9 @@ public:
     size_t CarriedLen() const;
     void SaveCarried(float *dst, int slot, int plane, int past) const;
     void RestoreCarried(const float *src, int slot, int plane, int past);
+    // the same from and to device memory of CarriedLen() floats, one launch, without waiting
+    void SaveCarriedOnDevice(float *dst, int slot, int plane, int past) const;
+    void RestoreCarriedOnDevice(const float *src, int slot, int plane, int past);
     std::vector<float> Result() const;  // [T][hv*d] attention output before the gated norm
     std::vector<float> Out() const;     // [T][NEmbd]
     float *InPort() const { return in_; }
@@ -411,6 +436,7 @@ struct Checkpoint {
     std::vector<int32_t> ids;
     std::vector<float> dn;
 };
+    std::shared_ptr<DeviceBlock> on_device;
 
 // llm.Graph (llm/graph.go:184-289, NewGraph :609): the whole model as recorded op sequences, one
 // per (slot, row count, kind of pass), recorded the first time each is needed.
