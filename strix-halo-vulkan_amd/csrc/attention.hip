@@ -969,7 +969,7 @@ int launch_rows(shv_ctx *ctx, const shv_attn_decode_args &a, int row0, int n_gro
 
 int shv_launch_attn_decode(shv_ctx *ctx, const shv_attn_decode_args *pa) {
     const shv_attn_decode_args &a = *pa;
-    SHV_REQUIRE(a.qkv && a.q_norm && a.k_norm && a.rope && a.kcache && a.vcache && a.partial && a.out, "attn_decode: NULL argument");
+    SHV_REQUIRE(a.qkv && a.q_norm && a.k_norm && a.rope && a.kcache && a.vcache && a.partial, "attn_decode: NULL argument");
     SHV_REQUIRE(a.head_dim == kD, "attn_decode: head_dim %d; built for %d", a.head_dim, kD);
     SHV_REQUIRE(a.n_head_kv >= 1 && a.n_head == a.n_head_kv * kRep, "attn_decode: %d query heads over %d KV heads; built for %d per KV head",
                 a.n_head, a.n_head_kv, kRep);
@@ -985,6 +985,11 @@ int shv_launch_attn_decode(shv_ctx *ctx, const shv_attn_decode_args *pa) {
     SHV_REQUIRE(shv_aligned16(a.qkv) && shv_aligned16(a.kcache) && shv_aligned16(a.vcache) && shv_aligned16(a.q_norm) &&
                     shv_aligned16(a.k_norm) && shv_aligned16(a.out) && shv_aligned16(a.partial) && a.qkv_stride % 4 == 0,
                 "attn_decode: qkv, caches, norms, partial and out must be 16-byte aligned");
+    if (!a.out) {
+        SHV_REQUIRE(a.seq_len <= 65535, "attn_decode: %d rows", a.seq_len);
+        SHV_LAUNCH(ctx, attn_append_kernel, dim3(a.n_head_kv, a.seq_len, a.n_seq), dim3(kBlock), 0, a);
+        return SHV_OK;
+    }
     // The rows of a sequence go two at a time: both see one pass over the cache.  One or two rows
     // write their own cells on the way; more rows have all their cells written first and then go
     // through as pairs of one launch (a last pair of one row repeats it and drops the copy).

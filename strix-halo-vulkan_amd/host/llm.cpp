@@ -1322,7 +1322,7 @@ Graph::Graph(Device &dev, const Model &m, const GraphOpts &opts) : dev_(dev), m_
     x_ = static_cast<float *>(dev.alloc(static_cast<size_t>(rows_max_) * c_.NEmbd * 4));
     ids_stride_ = static_cast<size_t>(o_.NKV) + 2;
     ids_ = static_cast<int32_t *>(dev.alloc_zero(ids_stride_ * o_.Slots * 4));
-    const size_t S = o_.Slots, R = rows_max_;
+    const size_t S = o_.Slots, R = kBatchRows;
     ctl_ = static_cast<int32_t *>(dev.alloc_zero((3 * S + 3 * R) * 4));
     pos_ = ctl_;
     plane_ = ctl_ + S;
@@ -1517,19 +1517,21 @@ int Graph::Dispatches() { return static_cast<int>(pass(slot_, 1, head_ ? kSample
 
 // The host is the authority on where each sequence stands between calls; the recorded passes
 // move the device copy themselves while they replay.
-void Graph::put_pos() {
+void Graph::put_words(std::vector<shv_words> w) {
     std::vector<int32_t> v(2 * o_.Slots);
     for (int s = 0; s < o_.Slots; s++) {
         v[s] = seq_[s].past;
         v[o_.Slots + s] = seq_[s].plane;
     }
-    dev_.upload(ctl_, v.data(), v.size() * 4);
+    w.push_back({ctl_, v.data(), static_cast<int32_t>(v.size())});
+    std::vector<int32_t> g;
     if (groups_ > 1) {
-        std::vector<int32_t> g(static_cast<size_t>(o_.Slots) * groups_);
+        g.resize(static_cast<size_t>(o_.Slots) * groups_);
         for (int s = 0; s < o_.Slots; s++)
             for (int j = 0; j < groups_; j++) g[static_cast<size_t>(s) * groups_ + j] = seq_[s].past + j * block_rows_;
-        dev_.upload(grp_pos_, g.data(), g.size() * 4);
+        w.push_back({grp_pos_, g.data(), static_cast<int32_t>(g.size())});
     }
+    dev_.words(w);
 }
 
 void Graph::Reset() {
@@ -1555,6 +1557,12 @@ void Graph::Forward(const std::vector<int32_t> &ids, std::vector<float> *logits,
     Extend(ids, logits, hidden);
 }
 
+void Graph::Extend(const std::vector<int32_t> &ids, std::vector<float> *logits, std::vector<float> *hidden) {
+    if (logits) logits->resize(c_.VocabSize);
+    if (hidden) hidden->resize(c_.NEmbd);
+    Extend(ids, logits ? logits->data() : nullptr, hidden ? hidden->data() : nullptr);
+}
+
 // The rows go through in chunks of MaxTokens; every chunk but the last is headless, the last one
 // samples.  res_all, when given, receives every row's residual.
 void Graph::extend(const std::vector<int32_t> &ids, float *res_all) {
@@ -1564,8 +1572,7 @@ void Graph::extend(const std::vector<int32_t> &ids, float *res_all) {
     if (spec_armed_) throw Error("llm: a speculative pass is in flight; commit or rewind it first");
     if (q.past + n + 1 > o_.NKV) throw Error("llm: Graph.Extend: " + std::to_string(q.past + n) + " tokens do not fit " + std::to_string(o_.NKV) + " cells");
     check_ids(ids);
-    dev_.upload(ids_ + slot_ * ids_stride_ + q.past, ids.data(), static_cast<size_t>(n) * 4);
-    put_pos();
+    put_words({id_words(q.past, ids)});
     const int M = o_.MaxTokens;
     const int last = n % M == 0 ? M : n % M;
     const int full = (n - last) / M;
@@ -1590,16 +1597,12 @@ void Graph::extend(const std::vector<int32_t> &ids, float *res_all) {
 
 int Graph::StepRows() const { return head_ ? std::min(head_->MaxRows(), o_.Slots) : 0; }
 
-void Graph::Extend(const std::vector<int32_t> &ids, std::vector<float> *logits, std::vector<float> *hidden) {
+void Graph::Extend(const std::vector<int32_t> &ids, float *logits, float *hidden) {
     if (logits && !head_) throw Error("llm: Graph.Extend: the graph was staged without a head");
     extend(ids, nullptr);
-    if (logits) {
-        logits->resize(c_.VocabSize);
-        dev_.download(logits->data(), head_->LogitsPort(), static_cast<size_t>(c_.VocabSize) * 4);
-    }
+    if (logits) dev_.download(logits, head_->LogitsPort(), static_cast<size_t>(c_.VocabSize) * 4);
     if (hidden) {
-        hidden->resize(c_.NEmbd);
-        dev_.download(hidden->data(), x_ + static_cast<size_t>(last_rows_ - 1) * c_.NEmbd, static_cast<size_t>(c_.NEmbd) * 4);
+        dev_.download(hidden, x_ + static_cast<size_t>(last_rows_ - 1) * c_.NEmbd, static_cast<size_t>(c_.NEmbd) * 4);
     }
 }
 
@@ -1642,8 +1645,7 @@ void Graph::ExtendRows(const std::vector<int32_t> &ids, std::vector<float> *logi
     if (q.past + n + 1 > o_.NKV) throw Error("llm: Graph.ExtendRows: " + std::to_string(q.past + n) + " tokens do not fit " + std::to_string(o_.NKV) + " cells");
     check_ids(ids);
     Pass &p = pass(slot_, n, kRows, spec_);
-    dev_.upload(ids_ + slot_ * ids_stride_ + q.past, ids.data(), static_cast<size_t>(n) * 4);
-    put_pos();
+    put_words({id_words(q.past, ids)});
     submit(p, 1, "rows");
     Stats.Runs++;
     if (spec_) {
@@ -1666,7 +1668,7 @@ void Graph::ExtendRows(const std::vector<int32_t> &ids, std::vector<float> *logi
 void Graph::StageIds(int at, const std::vector<int32_t> &ids) {
     if (at < 0 || at + static_cast<int>(ids.size()) > o_.NKV) throw Error("llm: Graph.StageIds: positions " + std::to_string(at) + ".. do not fit " + std::to_string(o_.NKV) + " cells");
     check_ids(ids);
-    dev_.upload(ids_ + slot_ * ids_stride_ + at, ids.data(), ids.size() * 4);
+    dev_.words({id_words(at, ids)});
 }
 
 void Graph::ExtendRowsStaged(int n) {
@@ -1689,6 +1691,13 @@ void Graph::ExtendRowsStaged(int n) {
 }
 
 void Graph::DecodeRows(const std::vector<int> &slots, const std::vector<int32_t> &ids, std::vector<float> *logits) {
+    DecodeRows(slots, ids, static_cast<float *>(nullptr));
+    if (!logits) return;
+    logits->resize(ids.size() * c_.VocabSize);
+    dev_.download(logits->data(), head_->LogitsPort(), logits->size() * 4);
+}
+
+void Graph::DecodeRows(const std::vector<int> &slots, const std::vector<int32_t> &ids, float *logits) {
     const int n = static_cast<int>(slots.size());
     if (n == 0 || n != static_cast<int>(ids.size())) throw Error("llm: " + std::to_string(n) + " slots and " + std::to_string(ids.size()) + " tokens");
     if (!head_) throw Error("llm: this graph was staged without a head");
@@ -1696,7 +1705,7 @@ void Graph::DecodeRows(const std::vector<int> &slots, const std::vector<int32_t>
     if (spec_) throw Error("llm: a speculating graph cannot batch sequences");
     check_ids(ids);
     // checkBatch (llm/batch.go:45-63): a slot out of range or named twice, a position past the cache
-    std::vector<int32_t> rows(3 * static_cast<size_t>(rows_max_), 0);
+    std::vector<int32_t> rows(3 * kBatchRows, 0);
     std::vector<bool> seen(o_.Slots, false);
     for (int r = 0; r < n; r++) {
         const int s = slots[r];
@@ -1705,22 +1714,18 @@ void Graph::DecodeRows(const std::vector<int> &slots, const std::vector<int32_t>
         seen[s] = true;
         if (seq_[s].past + 2 > o_.NKV) throw Error("llm: a token at position " + std::to_string(seq_[s].past) + " of a " + std::to_string(o_.NKV) + "-cell context");
         rows[r] = seq_[s].past;
-        rows[rows_max_ + r] = s;
-        rows[2 * rows_max_ + r] = ids[r];
+        rows[kBatchRows + r] = s;
+        rows[2 * kBatchRows + r] = ids[r];
     }
     Pass &p = pass(-1, n, kBatch, false);
-    put_pos();
-    dev_.upload(row_pos_, rows.data(), rows.size() * 4);
-    for (int r = 0; r < n; r++) dev_.upload(ids_ + slots[r] * ids_stride_ + seq_[slots[r]].past, &ids[r], 4);
+    std::vector<shv_words> w{{row_pos_, rows.data(), static_cast<int32_t>(rows.size())}};
+    for (int r = 0; r < n; r++) w.push_back({ids_ + slots[r] * ids_stride_ + seq_[slots[r]].past, &ids[r], 1});
+    put_words(std::move(w));
     submit(p, 1, "batched rows");
     Stats.Runs++;
-    for (int r = 0; r < n; r++) seq_[slots[r]].past++;
-    put_pos();
+    for (int r = 0; r < n; r++) seq_[slots[r]].past++;  // every later pass brings the positions with it
     last_rows_ = n;
-    if (logits) {
-        logits->resize(static_cast<size_t>(n) * c_.VocabSize);
-        dev_.download(logits->data(), head_->LogitsPort(), logits->size() * 4);
-    }
+    if (logits) dev_.download(logits, head_->LogitsPort(), static_cast<size_t>(n) * c_.VocabSize * 4);
 }
 
 std::vector<int32_t> Graph::Argmaxes() const {
@@ -1853,12 +1858,9 @@ void Graph::Checkpoint(struct Checkpoint &c) {
     const Seq &q = seq_[slot_];
     if (spec_armed_) throw Error("llm: a speculative pass is in flight; commit or rewind it first");
     if (q.past == 0) throw Error("llm: nothing to checkpoint at position 0");
+    const size_t carried = dn_->CarriedLen() * 4;
     c.past = q.past;
     c.ids.resize(q.past);
-    dev_.download(c.ids.data(), ids_ + slot_ * ids_stride_, static_cast<size_t>(q.past) * 4);
-    const size_t carried = dn_->CarriedLen() * 4;
-}
-
     if (!c.on_device || c.on_device->device != dev_.index() || c.on_device->bytes != carried) {
         c.on_device = nullptr;
         if (carried > 0) c.on_device = dev_.block(carried);
@@ -1871,6 +1873,9 @@ void Graph::Checkpoint(struct Checkpoint &c) {
         dn_->SaveCarried(c.dn.data(), slot_, q.plane, q.past);
     }
     // last, since it waits: the checkpoint is whole when this returns
+    dev_.download(c.ids.data(), ids_ + slot_ * ids_stride_, static_cast<size_t>(q.past) * 4);
+}
+
 void Graph::Restore(const struct Checkpoint &c) {
     Seq &q = seq_[slot_];
     if (spec_armed_) throw Error("llm: a speculative pass is in flight; commit or rewind it first");
@@ -1902,8 +1907,7 @@ std::vector<Stage> Graph::ProfileChunk(const std::vector<int32_t> &ids) {
     if (spec_armed_) throw Error("llm: a speculative pass is in flight; commit or rewind it first");
     if (q.past + n + 1 > o_.NKV) throw Error("llm: Graph.ProfileChunk: " + std::to_string(q.past + n) + " tokens do not fit " + std::to_string(o_.NKV) + " cells");
     check_ids(ids);
-    dev_.upload(ids_ + slot_ * ids_stride_ + q.past, ids.data(), static_cast<size_t>(n) * 4);
-    put_pos();
+    put_words({id_words(q.past, ids)});
     Pass &p = pass(slot_, n, kPrefill, false);
     std::vector<uint64_t> per(p.ops.size());
     uint64_t total = 0;
@@ -1920,7 +1924,8 @@ MTPHead::MTPHead(Device &dev, const Model &m, HeadGPU &head, int maxTok, int nKV
     if (maxTok < 1 || maxTok > 64) throw Error("llm: MTPHead: " + std::to_string(maxTok) + " rows a call; 1..64");
     if (slots < 1) throw Error("llm: MTPHead: no slots");
     pasts_.assign(slots, 0);
-    const size_t T = maxTok, E = c_.NEmbd;
+    cell_rows_ = std::max(maxTok, std::min(kBlockRows, nKV));
+    const size_t T = cell_rows_, E = c_.NEmbd;
     x_ = static_cast<float *>(dev.alloc(T * E * 4));
     h_ = static_cast<float *>(dev.alloc(T * E * 4));
     e_ = static_cast<float *>(dev.alloc(T * E * 4));
@@ -1934,7 +1939,7 @@ MTPHead::MTPHead(Device &dev, const Model &m, HeadGPU &head, int maxTok, int nKV
     std::vector<int32_t> ix(S);
     for (size_t i = 0; i < S; i++) ix[i] = static_cast<int32_t>(i);
     dev.upload(slot_ix_, ix.data(), S * 4);
-    attn_ = new AttnGPU(dev, m, maxTok, nKV, slots, pos_, layer_);
+    attn_ = new AttnGPU(dev, m, cell_rows_, nKV, slots, pos_, layer_);
     moe_ = new MoEGPU(dev, m, maxTok);
 }
 
@@ -1960,11 +1965,6 @@ void MTPHead::SetVocab(int k) {
     vocab_ = k;
 }
 
-Pass &MTPHead::draft_pass(int n, bool head, int k, int32_t *ring) {
-    // ring: the tokens come from the trunk's id ring at this head's position word, and the arg-max goes back there
-    const std::vector<int> key{slot_, n, head ? 1 : 0, ring ? 1 + k : 0};
-    auto it = passes_.find(key);
-    if (it != passes_.end() && it->second.ring != ring) {
 // What every pass of this block begins with: the tokens' embeddings and eh_proj over them and h.
 std::vector<shv_op> MTPHead::input_ops(int n, int32_t *ring, std::vector<std::string> *labels) const {
     const int E = c_.NEmbd;
@@ -2049,6 +2049,11 @@ void MTPHead::WriteCells(const float *hs, const std::vector<int32_t> &ids, int p
     pasts_[slot_] = pos + n;
 }
 
+Pass &MTPHead::draft_pass(int n, bool head, int k, int32_t *ring) {
+    // ring: the tokens come from the trunk's id ring at this head's position word, and the arg-max goes back there
+    const std::vector<int> key{slot_, n, head ? 1 : 0, ring ? 1 + k : 0};
+    auto it = passes_.find(key);
+    if (it != passes_.end() && it->second.ring != ring) {
         if (it->second.rec) shv_prerecorded_destroy(dev_.ctx(), it->second.rec);
         passes_.erase(it);
         it = passes_.end();
@@ -2056,45 +2061,15 @@ void MTPHead::WriteCells(const float *hs, const std::vector<int32_t> &ids, int p
     if (it == passes_.end()) {
         Pass p;
         p.ring = ring;
-        const int E = c_.NEmbd;
-        shv_embed_args e{};
-        e.table = m_.Tensor("token_embd.weight").ptr;
-        e.type = static_cast<int32_t>(m_.Tensor("token_embd.weight").ggml);
-        e.ids = ring ? ring : ids_;
-        e.pos = ring ? pos_ + slot_ : nullptr;
-        e.x = e_;
-        e.n_tok = n;
-        e.n_embd = E;
-        e.vocab = c_.VocabSize;
-        e.x_stride = E;
-        p.ops.push_back(make_op(SHV_OP_EMBED, e));
-        p.labels.push_back("embed");
-        shv_gemv_q4k_args g{};
-        g.w = m_.Tensor(Model::Blk(layer_, "nextn.eh_proj")).ptr;
-        g.x = e_;
-        g.z = h_;
-        g.y = x_;
-        g.gamma = static_cast<const float *>(m_.Tensor(Model::Blk(layer_, "nextn.ehnorm_fused")).ptr);
-        g.n = E;
-        g.k = 2 * E;
-        g.n_tok = n;
-        g.prologue = SHV_PRO_RMSNORM_PAIR;
-        g.eps = c_.RMSEps;
-        g.x_stride = g.z_stride = g.y_stride = E;
-        p.ops.push_back(make_op(SHV_OP_GEMV_Q4K, g));
-        p.labels.push_back("mtp.eh_proj");
-        PassRows r;
-        r.pos = pos_ + slot_;
-        r.slot = slot_ix_ + slot_;
-        r.host_slot = slot_;
-        r.seq_len = n;
+        p.ops = input_ops(n, ring, &p.labels);
+        const PassRows r = rows_of(n);
         auto a = attn_->Dispatches(layer_, x_, x_, r, &p.labels);
         p.ops.insert(p.ops.end(), a.begin(), a.end());
         auto f = moe_->Dispatches(layer_, x_, x_, n, &p.labels);
         p.ops.insert(p.ops.end(), f.begin(), f.end());
         if (head) {
             const int cols = vocab_ > 0 ? vocab_ : c_.VocabSize;
-            auto h = head_.DispatchesTo(x_ + static_cast<size_t>(n - 1) * E, 1,
+            auto h = head_.DispatchesTo(x_ + static_cast<size_t>(n - 1) * c_.NEmbd, 1,
                                         static_cast<const float *>(m_.Tensor(Model::Blk(layer_, "nextn.shared_head_norm")).ptr), logits_, cols, &p.labels);
             p.ops.insert(p.ops.end(), h.begin(), h.end());
             shv_argmax_args am{};
@@ -2126,7 +2101,7 @@ void MTPHead::RowsChained(const float *hs, int n, int pos, int k, int32_t *ring)
     check(shv_copy(dev_.ctx(), h_, hs, static_cast<size_t>(n) * c_.NEmbd * 4), "draft input");
     if (pos >= 0) {
         const int32_t p32 = pos;
-        dev_.upload(pos_ + slot_, &p32, 4);
+        dev_.words({{pos_ + slot_, &p32, 1}});
     }
     if (!pass.rec) check(shv_prerecord(dev_.ctx(), pass.ops.data(), static_cast<int>(pass.ops.size()), &pass.rec), "draft");
     check(shv_prerecorded_launch(dev_.ctx(), pass.rec), "draft");
@@ -2137,16 +2112,12 @@ void MTPHead::RowsChained(const float *hs, int n, int pos, int k, int32_t *ring)
 int32_t MTPHead::Rows(const float *hs, const std::vector<int32_t> &ids, int pos, bool head) {
     const int n = static_cast<int>(ids.size());
     if (!hs || n < 1 || n > max_tok_) throw Error("llm: MTPHead.Rows: " + std::to_string(n) + " rows, staged for " + std::to_string(max_tok_));
-    if (pos < 0 || pos > pasts_[slot_]) throw Error("llm: MTPHead.Rows: position " + std::to_string(pos) + " leaves a gap after the draft cache's " + std::to_string(pasts_[slot_]) + " cells");
-    if (pos + n + 1 > n_kv_) throw Error("llm: MTPHead.Rows: " + std::to_string(pos + n) + " cells do not fit " + std::to_string(n_kv_));
-    for (int32_t id : ids)
-        if (id < 0 || id >= c_.VocabSize) throw Error("llm: token " + std::to_string(id) + " is outside the vocabulary");
+    check_rows(ids, pos);
     Pass &pass = draft_pass(n, head, 0, nullptr);
     // the block's input h may be this block's own output rows: it is copied aside first
     check(shv_copy(dev_.ctx(), h_, hs, static_cast<size_t>(n) * c_.NEmbd * 4), "draft input");
-    dev_.upload(ids_, ids.data(), static_cast<size_t>(n) * 4);
     const int32_t p32 = pos;
-    dev_.upload(pos_ + slot_, &p32, 4);
+    dev_.words({{ids_, ids.data(), n}, {pos_ + slot_, &p32, 1}});
     GPUNanos += submit_pass(dev_, pass, 1, "draft");
     Steps++;
     pasts_[slot_] = pos + n;
@@ -2210,12 +2181,8 @@ void Speculator::Prime(const std::vector<int32_t> &ids, int at, const float *res
         d_.Reset();
         g_.Dev().zero(h_, E * 4);
     }
-    d_.Rows(h_, {ids[0]}, at, false);
-    const int M = d_.MaxRows();
-    for (int a = 1; a < n; a += M) {
-        const int k = std::min(M, n - a);
-        d_.Rows(res + static_cast<size_t>(a - 1) * E, std::vector<int32_t>(ids.begin() + a, ids.begin() + a + k), at + a, false);
-    }
+    d_.WriteCells(h_, {ids[0]}, at);
+    if (n > 1) d_.WriteCells(res, std::vector<int32_t>(ids.begin() + 1, ids.end()), at + 1);
     check(shv_copy(g_.Dev().ctx(), h_, res + static_cast<size_t>(n - 1) * E, E * 4), "seed");
     seeded_ = true;
     pend_ = -1;
@@ -2237,11 +2204,7 @@ void Speculator::settle_owed() {
     if (n == 0) return;
     const size_t E = g_.GetModel().config().NEmbd;
     use_slot();
-    const int at = past() - n, M = d_.MaxRows();
-    for (int p0 = 0; p0 < n; p0 += M) {
-        const int k = std::min(M, n - p0);
-        d_.Rows(h_ + static_cast<size_t>(p0) * E, std::vector<int32_t>(owe_x_.begin() + p0, owe_x_.begin() + p0 + k), at + p0, false);
-    }
+    d_.WriteCells(h_, owe_x_, past() - n);
     check(shv_copy(g_.Dev().ctx(), h_, h_ + static_cast<size_t>(n) * E, E * 4), "seed");
     owe_x_.clear();
 }
@@ -2291,12 +2254,8 @@ int32_t Speculator::Start(const std::vector<int32_t> &prompt) {
     // residual at p-1 and the token at p; cell 0 has nothing behind it and takes a zero residual.
     d_.Reset();
     g_.Dev().zero(h_, E * 4);
-    d_.Rows(h_, {prompt[0]}, 0, false);
-    const int M = d_.MaxRows();
-    for (int a = 1; a < T; a += M) {
-        const int n = std::min(M, T - a);
-        d_.Rows(res + static_cast<size_t>(a - 1) * E, std::vector<int32_t>(prompt.begin() + a, prompt.begin() + a + n), a, false);
-    }
+    d_.WriteCells(h_, {prompt[0]}, 0);
+    if (T > 1) d_.WriteCells(res, std::vector<int32_t>(prompt.begin() + 1, prompt.end()), 1);
     // the trunk's residual after the last prompt row seeds the first round
     check(shv_copy(g_.Dev().ctx(), h_, res + static_cast<size_t>(T - 1) * E, E * 4), "seed");
     owe_x_.clear();

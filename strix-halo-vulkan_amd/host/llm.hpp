@@ -429,14 +429,16 @@ struct Pass {
     int32_t *ring = nullptr;  // a draft pass that reads its tokens from the trunk's id ring: which ring
 };
 
-// llm.Checkpoint (llm/graph.go:902-1003): a sequence's position, tokens and DeltaNet carry, in host
-// memory; the KV cells need no copy, the ones past the checkpoint are simply written again.
+// llm.Checkpoint (llm/graph.go:902-1003): a sequence's position, tokens and DeltaNet carry; the KV
+// cells need no copy, the ones past the checkpoint are simply written again.  The carry (77 MB at 48
+// layers) stays in device memory, where saving and restoring it is one launch; in host memory, as the
+// reference keeps it, only when the device has no room.
 struct Checkpoint {
     int past = 0;
     std::vector<int32_t> ids;
+    std::shared_ptr<DeviceBlock> on_device;
     std::vector<float> dn;
 };
-    std::shared_ptr<DeviceBlock> on_device;
 
 // llm.Graph (llm/graph.go:184-289, NewGraph :609): the whole model as recorded op sequences, one
 // per (slot, row count, kind of pass), recorded the first time each is needed.
@@ -448,6 +450,8 @@ public:
     void Forward(const std::vector<int32_t> &ids, std::vector<float> *logits, std::vector<float> *hidden);
     // Extend appends ids to the sequence and returns the LAST row's logits (llm/graph.go:1709).
     void Extend(const std::vector<int32_t> &ids, std::vector<float> *logits, std::vector<float> *hidden);
+    // the same into the caller's own memory ([VocabSize], [NEmbd]; either may be nullptr)
+    void Extend(const std::vector<int32_t> &ids, float *logits, float *hidden);
     // ForwardResidual is Forward that also keeps the residual of EVERY prompt row on the device,
     // [T][NEmbd], which is what primes the draft head (llm/graph.go:1441-1450).
     const float *ForwardResidual(const std::vector<int32_t> &ids, std::vector<float> *logits);
@@ -461,6 +465,7 @@ public:
     void ExtendRows(const std::vector<int32_t> &ids, std::vector<float> *logits, std::vector<float> *res);
     // DecodeRows advances n sequences by one token each in one pass (llm/graph.go:1527-1666).
     void DecodeRows(const std::vector<int> &slots, const std::vector<int32_t> &ids, std::vector<float> *logits);
+    void DecodeRows(const std::vector<int> &slots, const std::vector<int32_t> &ids, float *logits);  // [n][VocabSize] or nullptr
     // The same pass over ids that are on the device already: StageIds puts tokens at positions at.. of the live
     // slot's id ring without waiting for the device, IdsPort() is that ring for an op that names a token itself
     // (a draft head's arg-max), ExtendRowsStaged runs the n rows at positions past.. that the ring then holds.
@@ -518,13 +523,16 @@ public:
 
 private:
     enum Kind { kPrefill = 0, kSample = 1, kRows = 2, kBatch = 3 };
+    static constexpr int kBatchRows = 16;  // the row tables' length: a batched pass carries at most 14 (HeadRows)
     struct Seq {
         int past = 0;
         int plane = 0;
     };
     Pass &pass(int slot, int rows, Kind kind, bool spec);
     uint64_t submit(Pass &p, int iters, const char *what);
-    void put_pos();
+    void put_pos() { put_words({}); }
+    void put_words(std::vector<shv_words> w);  // these and every sequence's position and plane
+    shv_words id_words(int at, const std::vector<int32_t> &ids) const { return {IdsPort() + at, ids.data(), static_cast<int32_t>(ids.size())}; }
     void check_ids(const std::vector<int32_t> &ids) const;
     void extend(const std::vector<int32_t> &ids, float *res_all);
     Device &dev_;
@@ -571,6 +579,12 @@ public:
     // the reference's host-side signature: hs from host memory, logits and residual copied back
     void RowsHost(const std::vector<float> &hs, const std::vector<int32_t> &ids, int pos, bool head,
                   std::vector<float> *logits, std::vector<float> *res);
+    // Rows for a caller that wants nothing but the cells it leaves in the draft's cache (priming over a prompt, owed
+    // rows): this block is the draft's only one, so what its cache holds depends on its key and value projection
+    // alone, and the attention, its output projection and the experts are not run.  Up to CellRows() rows a pass
+    // whatever the head was staged for, more in several; returns without waiting for the device.
+    void WriteCells(const float *hs, const std::vector<int32_t> &ids, int pos);
+    int CellRows() const { return cell_rows_; }
     // Rows for a caller that does not wait (a greedy round): the n tokens are read from `ring` (the trunk's id ring
     // of the sequence) at positions pos..pos+n-1, the head's arg-max is stored as the token at pos+n there, kept
     // for DraftAt(k) and moves this head's position word on, so that the call for draft k+1 (n = 1, pos < 0: the
@@ -594,13 +608,17 @@ private:
     const Model &m_;
     Config c_;
     HeadGPU &head_;
-    int max_tok_, n_kv_, layer_, slot_ = 0, vocab_ = 0;
+    int max_tok_, n_kv_, layer_, cell_rows_, slot_ = 0, vocab_ = 0;
     std::vector<int> pasts_;
     AttnGPU *attn_ = nullptr;
     MoEGPU *moe_ = nullptr;
     float *x_, *h_, *e_, *logits_;
     int32_t *ctl_, *pos_, *slot_ix_, *ids_, *best_;
     std::map<std::vector<int>, Pass> passes_;
+    void check_rows(const std::vector<int32_t> &ids, int pos) const;
+    std::vector<shv_op> input_ops(int n, int32_t *ring, std::vector<std::string> *labels) const;
+    PassRows rows_of(int n) const;
+    Pass &cell_pass(int n);
     Pass &draft_pass(int n, bool head, int k, int32_t *ring);
 };
 

@@ -221,10 +221,7 @@ int shvllm_extend(shvllm *h, const int32_t *ids, int n, float *logits, float *hi
     return guard([&] {
         if (!ids || n < 1) throw llm::Error("llm: shvllm_extend: no tokens");
         std::vector<int32_t> v(ids, ids + n);
-        std::vector<float> lg, hd;
-        graph_of(h).Extend(v, logits ? &lg : nullptr, hidden ? &hd : nullptr);
-        if (logits) std::memcpy(logits, lg.data(), lg.size() * 4);
-        if (hidden) std::memcpy(hidden, hd.data(), hd.size() * 4);
+        graph_of(h).Extend(v, logits, hidden);
     });
 }
 
@@ -298,10 +295,8 @@ int shvllm_extend_rows(shvllm *h, const int32_t *ids, int n, float *logits, floa
 int shvllm_decode_rows(shvllm *h, const int32_t *slots, const int32_t *ids, int n, float *logits, int32_t *best) {
     return guard([&] {
         if (!ids || !slots || n < 1) throw llm::Error("llm: shvllm_decode_rows: no rows");
-        std::vector<float> lg;
         const bool single = n == 1;
-        graph_of(h).DecodeRows(std::vector<int>(slots, slots + n), std::vector<int32_t>(ids, ids + n), logits ? &lg : nullptr);
-        if (logits) std::memcpy(logits, lg.data(), lg.size() * 4);
+        graph_of(h).DecodeRows(std::vector<int>(slots, slots + n), std::vector<int32_t>(ids, ids + n), logits);
         if (best) {
             auto b = graph_of(h).Argmaxes();
             std::memcpy(best, b.data(), (single ? 1 : b.size()) * 4);
