@@ -18,16 +18,14 @@
 //   moe_combine_kernel        out[t] = residual[t] + sum over slots of weights[t][s]*pairs[t][s],
 //                             slots in order
 // The shared expert is an expert every token lists: its blocks take 48 tokens each.
-#include "shv_device.hpp"
+#include "moe_staged.hpp"
 #include "shv_internal.hpp"
 
 namespace {
 
 using namespace shv;
+using namespace shv_moe;
 
-typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-typedef float float4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kWaves = 8;       // 256 registers a lane: the streams, the accumulators of four row tiles and the operands fit without spilling
 constexpr int kThreads = kWaves * 64;
@@ -142,9 +140,16 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int32_t *topk, in
 // counts (an expert's total, and what the blocks before it hold of it), forms the starts, and places its own pairs
 // behind those of the blocks before it; block 0 also writes the starts and the experts' launch order.
 constexpr int kGroupBlocks = 16;
-__global__ __launch_bounds__(1024) void moe_group_count_kernel(const int32_t *topk, int n_pairs, int chunk, int n_expert, int32_t *counts) {
+// Blocks past the counting ones, when the launch has them, stage the rows x [rows][k] for the list kernels meanwhile.
+__global__ __launch_bounds__(1024) void moe_group_count_kernel(const int32_t *topk, int n_pairs, int chunk, int n_expert, int32_t *counts, const float *x, int rows, int k,
+                                                               char *staged) {
     __shared__ int32_t s_cnt[kMaxExperts];
     const int tid = threadIdx.x;
+    if (blockIdx.x >= kGroupBlocks) {
+        const int quad = (blockIdx.x - kGroupBlocks) * 1024 + tid, t = quad / (k / 4), c = (quad % (k / 4)) * 4;
+        if (t < rows) stage_list_quad(*reinterpret_cast<const float4 *>(x + static_cast<size_t>(t) * k + c), t, c, k, rows, staged);
+        return;
+    }
     for (int e = tid; e < n_expert; e += 1024) s_cnt[e] = 0;
     __syncthreads();
     const int lo = blockIdx.x * chunk, hi = lo + chunk < n_pairs ? lo + chunk : n_pairs;
@@ -439,21 +444,6 @@ __device__ __forceinline__ void rows_times_tiles(const char *const (&rp)[kTiles]
 // this one is multiplied.  Wave w asks for sub-block w of the slab: its two parts for every token
 // tile.  The sub-blocks' sums of x come from the operands (slab_times_tiles with SXS 0).
 // tok_s: the listed rows' numbers in the staged array.
-// The masks and exponents of the two nibble positions a weight is read from.
-struct NibbleMasks {
-    uint32_t m0, m4;  // bits 0..3, 4..7 of both halves
-    uint32_t o0, o4;  // the halves 1024, 64
-};
-__device__ __forceinline__ NibbleMasks nibble_masks() {
-    NibbleMasks c;
-    c.m0 = 0x000F000Fu, c.m4 = 0x00F000F0u;
-    c.o0 = 0x64006400u, c.o4 = 0x54005400u;
-    // opaque to the optimiser: a mask in a scalar register and an exponent in a vector one make (q & m) | o one instruction
-    asm volatile("" : "+s"(c.m0), "+s"(c.m4));
-    asm volatile("" : "+v"(c.o0), "+v"(c.o4));
-    return c;
-}
-
 typedef const __attribute__((address_space(1))) void *global_ptr_t;
 typedef __attribute__((address_space(3))) void *lds_ptr_t;
 constexpr int kStWaves = kWaves;                 // waves of a block of the staged kernels: two such blocks share a compute unit, one's waits under the other's work
@@ -462,15 +452,9 @@ constexpr int kStSubs = kStWaves;             // sub-blocks of a staged slab: on
 constexpr int kStQuarter = 1024 / (32 * kStSubs);  // slabs in the 1024 columns one min-term product covers
 constexpr int kStSlab = 32 * kStSubs;
 constexpr int kStFrags = kStSubs * 2 * kTT * kFrag;
-constexpr int kStSubBytes = 128;              // a row's sub-block: 2 parts x 4 column blocks x 16 bytes
 constexpr int kStSumFrags = kTT * 2 * kFrag;   // the sums of a quarter of the columns (four super-blocks): [token tile][part]
 constexpr int kStMinHdrs = kStWaves * kTiles * kFrag;   // every lane's row header of its super-block of the quarter, a wave's own
 constexpr size_t kStagedLds = 2 * static_cast<size_t>(kStFrags) + 2 * kStSumFrags + kStMinHdrs + 2 * kTok * 4;
-
-// After the rows, every row's sums of x over its sub-blocks, as operands too: [row][super-block]
-// x 32 bytes, the eight sums' binary16 values and then what those leave.
-__host__ __device__ constexpr size_t staged_sums_offset(int rows, int k) { return static_cast<size_t>(rows) * (k / 32) * 128; }
-__host__ __device__ constexpr size_t staged_bytes(int rows, int k) { return staged_sums_offset(rows, k) + static_cast<size_t>(rows) * (k / 256) * 32; }
 
 // grid: (k / 1024, rows), 256 threads, a quad of columns each.
 __global__ __launch_bounds__(256) void moe_stage_kernel(const float *x, int x_stride, int k, int rows, char *staged) {
@@ -635,7 +619,6 @@ __device__ __forceinline__ void staged_slab_times_tiles(const char *const (&rp)[
 #pragma unroll
             for (int r = 0; r < R; r++) {
                 const uint32_t q0 = (u & 1) ? q[r].z : q[r].x, q1 = (u & 1) ? q[r].w : q[r].y;
-                typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
                 // A nibble in the low bits of a half's mantissa reads, under the right exponent, as
                 // C + n: bits 0..3 under 1024's, bits 4..7 under 64's (the odd bytes' nibbles take
                 // one shift down there).  One fused multiply-add then makes (C + n) * sc - C * sc =
@@ -778,10 +761,6 @@ struct Staging {
     }
 };
 constexpr size_t kGroupedLds = static_cast<size_t>(kSlabSubs) * 2 * kTT * kFrag + static_cast<size_t>(kSlabSubs) * kTok * 4 + kTok * sizeof(float *) + kTok * 4;
-
-// Where the grouped down projection finds a pair's act row when it comes as operands: the row's
-// own 4 * ffn bytes of act in the staged layout, and its sub-blocks' sums in the library's scratch.
-__host__ __device__ constexpr size_t packed_sums_bytes(long long pairs, int ffn) { return static_cast<size_t>(pairs) * (ffn / 256) * 32; }
 
 // One pass of a block of the gate/up kernel over up to 16 NTT of its tokens: the products, SwiGLU, act out
 // (as floats, or, packed, as the operands the grouped down projection stages from).
@@ -985,16 +964,18 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(shv_moe_down_args a) {
 // The per-expert lists of a pass: one block for short passes of few experts, kGroupBlocks in two launches from 2048
 // pairs or 128 experts on (ranking the experts by length is E^2 comparisons, a block's share of them a sixteenth)
 // (their counts meet in the library's scratch, which nothing else on the stream is using between the two).
-int launch_group(shv_ctx *ctx, const int32_t *topk, int n_tok, int n_used, int n_expert, int32_t *group) {
+// x: rows of k floats to stage for the list kernels in the first launch.
+int launch_group(shv_ctx *ctx, const int32_t *topk, int n_tok, int n_used, int n_expert, int32_t *group, const float *x = nullptr, int k = 0) {
     const int n_pairs = n_tok * n_used;
-    if ((n_pairs < 2048 && n_expert < 128) || !ctx->gemm_part || ctx->moe_group_one_block) {
+    if (!x && ((n_pairs < 2048 && n_expert < 128) || !ctx->gemm_part || ctx->moe_group_one_block)) {
         SHV_LAUNCH(ctx, moe_group_kernel, dim3(1), dim3(1024), 0, topk, n_tok, n_used, n_expert, group);
         return SHV_OK;
     }
     static_assert(static_cast<size_t>(kGroupBlocks) * kMaxExperts * 4 <= static_cast<size_t>(shv_ctx::kGemmPartBytes), "the blocks' counts fit the scratch");
     int32_t *counts = reinterpret_cast<int32_t *>(ctx->gemm_part);
     const int chunk = (n_pairs + kGroupBlocks - 1) / kGroupBlocks;
-    SHV_LAUNCH(ctx, moe_group_count_kernel, dim3(kGroupBlocks), dim3(1024), 0, topk, n_pairs, chunk, n_expert, counts);
+    const int stage_blocks = x ? static_cast<int>((static_cast<long long>(n_tok) * (k / 4) + 1023) / 1024) : 0;
+    SHV_LAUNCH(ctx, moe_group_count_kernel, dim3(kGroupBlocks + stage_blocks), dim3(1024), 0, topk, n_pairs, chunk, n_expert, counts, x, n_tok, k, ctx->gemm_stage);
     SHV_LAUNCH(ctx, moe_group_place_kernel, dim3(kGroupBlocks), dim3(1024), 0, topk, n_pairs, chunk, n_used, n_expert, counts, group);
     return SHV_OK;
 }
@@ -1006,7 +987,7 @@ int raise_lds(Kern kern, size_t lds) {
 }
 
 bool shapes_covered(const shv_ctx *ctx, int n_tok, int n_embd, int ffn, int n_used, int n_expert) {
-    return n_tok >= ctx->moe_group_min && n_embd == 2048 && ffn == 512 && n_expert >= 1 && n_expert <= kMaxExperts && n_used >= 1 &&
+    return n_tok >= ctx->moe_group_min && (n_tok >= 128 || ctx->moe_group_forced || shv_moe_list_tokens(n_tok, n_used, n_expert) > 0) && n_embd == 2048 && ffn == 512 && n_expert >= 1 && n_expert <= kMaxExperts && n_used >= 1 &&
            static_cast<long long>(n_tok) * (n_used + 1) < (1ll << 30) / 2048;
 }
 
@@ -1029,6 +1010,12 @@ int shv_launch_moe_up_grouped(shv_ctx *ctx, const shv_moe_up_args &a) {
     // refused before anything is enqueued: an error return leaves no half pass on the stream
     SHV_REQUIRE(!a.act_packed || (ctx->gemm_part && packed_sums_bytes(static_cast<long long>(a.n_tok) * (a.n_used + 1), a.ffn) <= static_cast<size_t>(shv_ctx::kGemmPartBytes)),
                 "moe_up: %d rows are too many for act_packed", a.n_tok);
+    if (shv_moe_list_tokens(a.n_tok, a.n_used, a.n_expert) > 0) {
+        // short lists: streamed, wave by wave
+        if (const int rc = launch_group(ctx, a.topk, a.n_tok, a.n_used, a.n_expert, a.group, a.xn, a.n_embd); rc != SHV_OK) return rc;
+        ctx->moe_stamp = {a.topk, a.group, a.act, a.n_tok, a.n_used, true, a.act_packed != 0};
+        return shv_launch_moe_up_lists(ctx, a);
+    }
     if (const int rc = launch_group(ctx, a.topk, a.n_tok, a.n_used, a.n_expert, a.group); rc != SHV_OK) return rc;
     SHV_LAUNCH(ctx, moe_stage_kernel, dim3((a.n_embd + 1023) / 1024, a.n_tok), dim3(256), 0, a.xn, a.n_embd, a.n_embd, a.n_tok, ctx->gemm_stage);
     constexpr size_t lds = kStagedLds;
@@ -1057,7 +1044,9 @@ int shv_launch_moe_down_grouped(shv_ctx *ctx, const shv_moe_down_args &a) {
         if (const int rc = launch_group(ctx, a.topk, a.n_tok, a.n_used, a.n_expert, const_cast<int32_t *>(a.group)); rc != SHV_OK) return rc;
     }
     const int parts = a.n_embd / 512, tiles = (a.n_tok + kTok - 1) / kTok;
-    if (a.act_packed) {
+    if (a.act_packed && shv_moe_list_tokens(a.n_tok, a.n_used, a.n_expert) > 0) {
+        if (const int rc = shv_launch_moe_down_lists(ctx, a); rc != SHV_OK) return rc;
+    } else if (a.act_packed) {
         constexpr size_t lds = kStagedLds;
         static const int raised = raise_lds(&moe_down_staged_kernel<512>, lds);
         if (raised != SHV_OK) return raised;

@@ -1,0 +1,96 @@
+// What the expert kernels of long passes share: rows of activations as matrix-core operands, a row's own bytes together.
+//
+// A row of k columns is [sub-block of 32][part hi, lo][block of 8 columns] x 16 bytes, 128 bytes a sub-block, the eight
+// columns of a block in slot order [0, 2, 1, 3, 4, 6, 5, 7] (the order a payload dword's nibbles come out of the masks).
+// After all rows come their sums over the sub-blocks, as operands too: [row][super-block] x 32 bytes, the eight sums'
+// binary16 values and then what those leave.
+#pragma once
+#include "shv_device.hpp"
+
+namespace shv_moe {
+
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef float float4_t __attribute__((ext_vector_type(4)));
+
+constexpr int kStSubBytes = 128;  // a row's sub-block: 2 parts x 4 column blocks x 16 bytes
+
+__host__ __device__ constexpr size_t staged_sums_offset(int rows, int k) { return static_cast<size_t>(rows) * (k / 32) * 128; }
+__host__ __device__ constexpr size_t staged_bytes(int rows, int k) { return staged_sums_offset(rows, k) + static_cast<size_t>(rows) * (k / 256) * 32; }
+// Where the grouped down projection finds a pair's act row when it comes as operands: the row's
+// own 4 * ffn bytes of act in the staged layout, and its sub-blocks' sums in the library's scratch.
+__host__ __device__ constexpr size_t packed_sums_bytes(long long pairs, int ffn) { return static_cast<size_t>(pairs) * (ffn / 256) * 32; }
+
+// Where the high part of columns 32 sub + 8 c .. + 7 lies in a row staged for the list kernels; its low part is 64 bytes on.
+// [super-block][low / high nibbles' sub-blocks][c][part][group]: what the lanes of one operand take of a token is a line.
+__host__ __device__ constexpr int list_block(int sub, int c) { return (sub >> 3) * 1024 + (sub & 1) * 512 + c * 128 + ((sub >> 1) & 3) * 16; }
+
+// Four columns c .. c + 3 of row t for the list kernels, and (the lane of a sub-block's first columns) the sub-block's sum;
+// the eight lanes of a sub-block are neighbours and all here.
+__device__ __forceinline__ void stage_list_quad(const float4 v, int t, int c, int k, int rows, char *staged) {
+    const float o[4] = {v.x, v.z, v.y, v.w};
+    half4_t h, l;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const _Float16 hi = static_cast<_Float16>(o[j]);
+        h[j] = hi;
+        l[j] = static_cast<_Float16>(o[j] - static_cast<float>(hi));
+    }
+    char *e = staged + static_cast<size_t>(t) * (k / 32) * kStSubBytes + list_block(c >> 5, (c & 31) >> 3) + ((c & 7) >> 2) * 8;
+    *reinterpret_cast<half4_t *>(e) = h;
+    *reinterpret_cast<half4_t *>(e + 64) = l;
+    const float sum = shv::sum8_all((v.x + v.y) + (v.z + v.w));
+    if ((c & 31) == 0) {
+        const _Float16 hi = static_cast<_Float16>(sum);
+        _Float16 *sp = reinterpret_cast<_Float16 *>(staged + staged_sums_offset(rows, k) + (static_cast<size_t>(t) * (k / 256) + (c >> 8)) * 32) + ((c >> 5) & 7);
+        sp[0] = hi;
+        sp[8] = static_cast<_Float16>(sum - static_cast<float>(hi));
+    }
+}
+
+// The masks and exponents of the two nibble positions a weight is read from.
+struct NibbleMasks {
+    uint32_t m0, m4;  // bits 0..3, 4..7 of both halves
+    uint32_t o0, o4;  // the halves 1024, 64
+};
+__device__ __forceinline__ NibbleMasks nibble_masks() {
+    NibbleMasks c;
+    c.m0 = 0x000F000Fu, c.m4 = 0x00F000F0u;
+    c.o0 = 0x64006400u, c.o4 = 0x54005400u;
+    // opaque to the optimiser: a mask in a scalar register and an exponent in a vector one make (q & m) | o one instruction
+    asm volatile("" : "+s"(c.m0), "+s"(c.m4));
+    asm volatile("" : "+v"(c.o0), "+v"(c.o4));
+    return c;
+}
+
+// Eight weights of two payload dwords as n * sc: HI false the low nibbles, true the high ones.  A nibble in the low bits
+// of a half's mantissa reads, under the right exponent, as C + n: bits 0..3 under 1024's, bits 4..7 under 64's (the odd
+// bytes' nibbles take one shift down there).  One fused multiply-add then makes (C + n) * sc - C * sc = n * sc: a whole
+// number up to 15 * 63, exact in binary16, as are C * sc.
+template <bool HI>
+__device__ __forceinline__ half8_t weights8(uint32_t q0, uint32_t q1, uint32_t sc, const NibbleMasks &nc) {
+    const _Float16 s1 = static_cast<_Float16>(static_cast<float>(sc));
+    const half2_t s2 = {s1, s1};
+    half2_t w[4], c[4];
+    if constexpr (!HI) {
+        w[0] = __builtin_bit_cast(half2_t, (q0 & nc.m0) | nc.o0); w[1] = __builtin_bit_cast(half2_t, ((q0 >> 4) & nc.m4) | nc.o4);
+        w[2] = __builtin_bit_cast(half2_t, (q1 & nc.m0) | nc.o0); w[3] = __builtin_bit_cast(half2_t, ((q1 >> 4) & nc.m4) | nc.o4);
+        c[0] = c[2] = s2 * static_cast<half2_t>(static_cast<_Float16>(-1024.f));
+        c[1] = c[3] = s2 * static_cast<half2_t>(static_cast<_Float16>(-64.f));
+    } else {
+        w[0] = __builtin_bit_cast(half2_t, (q0 & nc.m4) | nc.o4); w[1] = __builtin_bit_cast(half2_t, ((q0 >> 8) & nc.m4) | nc.o4);
+        w[2] = __builtin_bit_cast(half2_t, (q1 & nc.m4) | nc.o4); w[3] = __builtin_bit_cast(half2_t, ((q1 >> 8) & nc.m4) | nc.o4);
+        c[0] = c[1] = c[2] = c[3] = s2 * static_cast<half2_t>(static_cast<_Float16>(-64.f));
+    }
+    half8_t b;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const half2_t p = __builtin_elementwise_fma(w[i], s2, c[i]);
+        b[2 * i] = p[0];
+        b[2 * i + 1] = p[1];
+    }
+    return b;
+}
+
+}  // namespace shv_moe

@@ -55,7 +55,10 @@ int shv_init(int device, shv_ctx **out) {
     if (const char *e = std::getenv("SHV_ATTN_APPEND")) ctx->attn_append_launch = std::strcmp(e, "launch") == 0;
     if (const char *e = std::getenv("SHV_MOE_GROUP_MIN")) {
         const int v = std::atoi(e);
-        if (v >= 1) ctx->moe_group_min = v;
+        if (v >= 1) {
+            ctx->moe_group_min = v;
+            ctx->moe_group_forced = true;
+        }
     }
     if (const char *e = std::getenv("SHV_DN_RECS")) ctx->dn_chunk_no_recs = std::atoi(e) == 0;
     if (const char *e = std::getenv("SHV_MOE_GROUP_BLOCKS")) ctx->moe_group_one_block = std::atoi(e) == 1;

@@ -37,7 +37,10 @@ struct shv_ctx {
     bool mrows_four_waves = false;  // SHV_MROWS_WAVES=4: five to eight rows stay on blocks of four waves
     // SHV_ATTN_APPEND=launch: passes of three and four rows write their new cells in a launch of their own, as longer ones do
     bool attn_append_launch = false;
-    int moe_group_min = 128;  // rows from which a MoE pass with a workspace is grouped by expert on the matrix cores (SHV_MOE_GROUP_MIN)
+    // Rows from which a MoE pass with a workspace is grouped by expert on the matrix cores: 128, fewer where the lists are
+    // worth streaming (shv_moe_list_tokens); SHV_MOE_GROUP_MIN names another number
+    int moe_group_min = 32;
+    bool moe_group_forced = false;
     bool dn_chunk_no_recs = false;  // SHV_DN_RECS=0: the chunked delta rule forms every chunk's state-independent part inside the walk, whatever the workspace holds
     bool moe_group_one_block = false;  // SHV_MOE_GROUP_BLOCKS=1: the per-expert lists of a long pass by one block in one launch
     int moe_tall_min = 16;  // tokens from which the MoE kernels' blocks make several passes over their staged rows (SHV_MOE_TALL_MIN)
@@ -168,6 +171,10 @@ bool shv_moe_up_grouped_covers(const shv_ctx *ctx, const shv_moe_up_args &a);
 int shv_launch_moe_up_grouped(shv_ctx *ctx, const shv_moe_up_args &a);
 bool shv_moe_down_grouped_covers(const shv_ctx *ctx, const shv_moe_down_args &a);
 int shv_launch_moe_down_grouped(shv_ctx *ctx, const shv_moe_down_args &a);
+// ... and passes whose lists are short, streamed (moe_lists.hip): tokens a wave takes at a time, 0 where the lists are long
+int shv_moe_list_tokens(int n_tok, int n_used, int n_expert);
+int shv_launch_moe_up_lists(shv_ctx *ctx, const shv_moe_up_args &a);
+int shv_launch_moe_down_lists(shv_ctx *ctx, const shv_moe_down_args &a);
 int shv_launch_dn_step(shv_ctx *ctx, const shv_dn_step_args *a);
 int shv_launch_attn_decode(shv_ctx *ctx, const shv_attn_decode_args *a);
 // expert banks in other types than Q4_K: slots [slot0, slot0 + slots) of the up projection; slots
