@@ -1,0 +1,278 @@
+// Q4_K projections of 9 to some hundreds of activation rows: y[t] = W pro(x[t]) (+ residual[t]).
+//
+// A block takes 16 R weight rows and all their columns, a wave 256 or 512 of the columns: it reads its weights once, forms
+// n * sc of them in registers and keeps them there while the pass's tiles of 16 activation rows go by.  A tile's fragments
+// come straight from L2, where a launch before this one left them in operand order (a fragment is one contiguous kilobyte,
+// three are asked for ahead of the one in use); the waves' partial tiles meet in LDS behind one barrier a tile.  No slab is
+// staged, no column part is left for another launch to join.
+//   products   v_mfma_f32_16x16x32_f16, activations x weights: a lane holds one weight row (its scales, its d); the
+//              activations as two binary16 parts, the weights as the whole numbers n * sc, exact in binary16, one
+//              accumulator a super-block
+//   min term   per super-block one v_mfma_f32_16x16x16_f16 a part of the sub-blocks' sums with the rows' mins
+// Up to 64 rows the weights' way through memory and the two launches bound it; from there the fragments' way from L2: 128 KB
+// a tile and block of 64 weight rows go at 31 bytes a clock and compute unit (1.7 us a tile), whatever their number in
+// flight, where the products alone would take half of that.  More rows a block would need more registers than there are:
+// 64 rows of 2048 columns, formed, are 256 of a compute unit's 512 KB, and forming them again for each tile costs what it saves.
+// us, with the staging launch, against the launches of 16, of 64 rows and their joins before (n x k, rows):
+//   12352 x 2048   9: 20.3 -> 11.8   16: 24.6 -> 11.2   64: 29.9 -> 17.9   150: 69.1 -> 31   255: 49.0 -> 44   512: 90 -> 76
+//    2048 x 4096   9: 16.0 -> 10.9   16: 16.5 -> 10.7   64: 22.3 -> 13.3   150: 51.5 -> 22.7   255: 59.7 -> 26   512: 65 -> 40
+#include <atomic>
+#include "gemm_rows.hpp"
+#include "moe_staged.hpp"
+
+namespace {
+
+using namespace shv;
+using namespace shv_gemm;
+using namespace shv_moe;
+
+// The staged activations of a pass: fragments [tile of 16 rows][super-block][v][part] of 1 KB, v = nibble half * 4 + block of
+// 8 columns: lane (row n, group kb) holds columns 64 kb + 32 half + 8 block .. + 7 of the super-block, in the order a
+// payload dword's nibbles come; then the sub-blocks' sums [tile][super-block][part] of 256 bytes: lane (n, kb) those of
+// sub-blocks 2 kb, 2 kb + 1; then where each row's outputs go (a ring's row takes divisions and two loads to find).
+constexpr int kMidFrag = 1024, kMidSb = 16 * kMidFrag, kMidSums = 2 * 256;
+__host__ __device__ constexpr size_t mid_sums_offset(int tiles, int k) { return static_cast<size_t>(tiles) * (k / 256) * kMidSb; }
+__host__ __device__ constexpr size_t mid_rows_offset(int tiles, int k) { return mid_sums_offset(tiles, k) + static_cast<size_t>(tiles) * (k / 256) * kMidSums; }
+__host__ __device__ constexpr size_t mid_bytes(int tiles, int k) { return mid_rows_offset(tiles, k) + static_cast<size_t>(tiles) * 16 * sizeof(size_t); }
+
+// grid: (column parts, 4 quartets of rows of a tile, tiles), 256 threads: a wave takes one row's 64 quads of a super-block
+// at a time; rows past the pass's are written as zeros.
+__global__ __launch_bounds__(256) void gemm_mid_stage_kernel(shv_gemv_q4k_args a, char *staged, int tiles) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, K = a.k;
+    const int n = blockIdx.y * 4 + wave, t = blockIdx.z * 16 + n;
+    const bool on = t < a.n_tok;
+    if (blockIdx.x == 0 && lane == 0) reinterpret_cast<size_t *>(staged + mid_rows_offset(tiles, K))[t] = on ? out_offset(a, t) : 0;
+    float scale = 1.f;
+    if (a.prologue == SHV_PRO_RMSNORM && on) {
+        const float *x = a.x + static_cast<size_t>(t) * a.x_stride;
+        float ss = 0.f;
+        for (int q = lane; q < K / 4; q += 64) {
+            const float4 v = *reinterpret_cast<const float4 *>(x + 4 * q);
+            ss = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ss))));
+        }
+        scale = 1.f / sqrtf(wave_sum_all(ss) / static_cast<float>(K) + a.eps);
+    }
+    for (int sb = blockIdx.x; sb < K / 256; sb += gridDim.x) {
+        const int c = 4 * lane;  // within the super-block
+        float x[4] = {0.f, 0.f, 0.f, 0.f};
+        if (on) pro_quad(a, t, sb * 256 + c, scale, x);
+        const float sum = sum8_all((x[0] + x[1]) + (x[2] + x[3]));
+        const int sub = c >> 5, kb = sub >> 1, v = (sub & 1) * 4 + ((c & 31) >> 3);
+        const size_t at = static_cast<size_t>(blockIdx.z) * (K / 256) + sb;
+        if ((c & 31) == 0) {
+            const _Float16 hi = static_cast<_Float16>(sum);
+            _Float16 *sp = reinterpret_cast<_Float16 *>(staged + mid_sums_offset(tiles, K) + at * kMidSums + (kb * 16 + n) * 4) + (sub & 1);
+            sp[0] = hi;
+            sp[128] = static_cast<_Float16>(sum - static_cast<float>(hi));
+        }
+        const float o[4] = {x[0], x[2], x[1], x[3]};
+        half4_t h, l;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const _Float16 hi = static_cast<_Float16>(o[j]);
+            h[j] = hi;
+            l[j] = static_cast<_Float16>(o[j] - static_cast<float>(hi));
+        }
+        char *e = staged + at * kMidSb + v * (2 * kMidFrag) + (kb * 16 + n) * 16 + ((c & 7) >> 2) * 8;
+        *reinterpret_cast<half4_t *>(e) = h;
+        *reinterpret_cast<half4_t *>(e + kMidFrag) = l;
+    }
+}
+
+// A barrier behind which the waves' LDS writes are seen; fragments and stores in flight stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// grid: (groups of 16 R weight rows, chunks of the pass's tiles), W waves: wave w takes columns 256 S w .. of every tile.
+template <int R, int S, int W>
+__global__ __launch_bounds__(64 * W) void gemm_mid_kernel(shv_gemv_q4k_args a, const char *staged, int tiles, int per_chunk) {
+    extern __shared__ __align__(16) char smem[];
+    float *cpart = reinterpret_cast<float *>(smem);  // [2][W][R][64][4]
+    const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, kb = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr int SBS = S * W, ROWB = SBS * SHV_Q4K_BYTES;
+    const int row0 = blockIdx.x * (16 * R), tile0 = blockIdx.y * per_chunk;
+    const int tile_end = tile0 + per_chunk < tiles ? tile0 + per_chunk : tiles;
+    const NibbleMasks nc = nibble_masks();
+    // the wave's weights first: header and this lane's group of every super-block of every row
+    uint4 hdr[S][R], q[S][R][2];
+    const char *wbase = static_cast<const char *>(a.w) + static_cast<size_t>(row0) * ROWB + wave * (S * SHV_Q4K_BYTES);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int rr = row0 + 16 * r + n < a.n ? 16 * r + n : a.n - 1 - row0;
+        const char *p = wbase + static_cast<uint32_t>(rr) * ROWB;
+#pragma unroll
+        for (int s = 0; s < S; s++) {
+            hdr[s][r] = load_stream16(p + s * SHV_Q4K_BYTES);
+            q[s][r][0] = load_stream16(p + s * SHV_Q4K_BYTES + 16 + kb * 32);
+            q[s][r][1] = load_stream16(p + s * SHV_Q4K_BYTES + 32 + kb * 32);
+        }
+    }
+    const char *frag = staged + (static_cast<size_t>(tile0) * SBS + wave * S) * kMidSb + lane * 16;
+    const char *sums = staged + mid_sums_offset(tiles, a.k) + (static_cast<size_t>(tile0) * SBS + wave * S) * kMidSums + lane * 4;
+    constexpr int D = 4;  // fetches held; eight are no faster
+    auto ask = [&](const char *fp, int i, half8_t (&f)[2]) {
+#pragma unroll
+        for (int p = 0; p < 2; p++) f[p] = *reinterpret_cast<const half8_t *>(fp + (i * 2 + p) * kMidFrag);
+    };
+    half8_t f[D][2];
+    uint32_t sx[S][2];
+#pragma unroll
+    for (int i = 0; i < D - 1; i++) ask(frag, i, f[i]);
+#pragma unroll
+    for (int s = 0; s < S; s++)
+#pragma unroll
+        for (int p = 0; p < 2; p++) sx[s][p] = *reinterpret_cast<const uint32_t *>(sums + s * kMidSums + p * 256);
+    // n * sc of the wave's columns, held for every tile of the chunk
+    half8_t wt[S][R][8];
+    half4_t am[S][R];
+    float d[S][R], dmin[S][R];
+#pragma unroll
+    for (int s = 0; s < S; s++)
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            uint32_t sc, mn;
+            q4k_group_scale_min(hdr[s][r], kb, sc, mn);
+#pragma unroll
+            for (int v = 0; v < 8; v++) {
+                const uint4 &x = q[s][r][(v >> 1) & 1];
+                const uint32_t d0 = (v & 1) ? x.z : x.x, d1 = (v & 1) ? x.w : x.y;
+                wt[s][r][v] = v < 4 ? weights8<false>(d0, d1, sc & 0xFFu, nc) : weights8<true>(d0, d1, sc >> 8, nc);
+            }
+            am[s][r] = half4_t{static_cast<_Float16>(static_cast<float>(mn & 0xFFu)), static_cast<_Float16>(static_cast<float>(mn >> 8)),
+                               static_cast<_Float16>(0.f), static_cast<_Float16>(0.f)};
+            d[s][r] = f16_bits_to_f32(hdr[s][r].x);
+            dmin[s][r] = f16_bits_to_f32(hdr[s][r].x >> 16);
+        }
+    constexpr int PER = R * 256 >= 64 * W ? R * 256 / (64 * W) : 1;  // outputs a lane adds up over the waves
+    static_assert(PER == 1 || PER == 2 || PER == 4, "a lane's share of a tile");
+    const int o = tid * PER < R * 256 ? tid * PER : 0, row = row0 + 16 * (o >> 8) + ((o >> 2) & 15), t_in = 4 * (o >> 6 & 3) + (o & 3);
+    const bool mine = tid * PER < R * 256 && row < a.n;
+    const size_t *rows = reinterpret_cast<const size_t *>(staged + mid_rows_offset(tiles, a.k));
+    size_t to_at[PER];
+    float res[PER];
+    auto find = [&](int tile) {
+        const int t = tile * 16 + t_in;
+#pragma unroll
+        for (int j = 0; j < PER; j++) {
+            to_at[j] = rows[t + j];
+            res[j] = a.residual && mine ? a.residual[static_cast<size_t>(t + j < a.n_tok ? t + j : a.n_tok - 1) * a.y_stride + row] : 0.f;
+        }
+    };
+    int buf = 0;
+    for (int tile = tile0; tile < tile_end; tile++) {
+        const bool more = tile + 1 < tile_end;
+        const char *fnext = more ? frag + SBS * kMidSb : frag, *snext = more ? sums + SBS * kMidSums : sums;
+        find(tile);  // asked for here, needed at the tile's end
+        float4_t y[R];
+        uint32_t sn[S][2];
+#pragma unroll
+        for (int s = 0; s < S; s++) {
+            float4_t acc[R];
+#pragma unroll
+            for (int r = 0; r < R; r++) acc[r] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const int at = s * 8 + i, to = at + D - 1;
+                if (to < S * 8) ask(frag, to, f[to % D]);
+                else ask(fnext, to - S * 8, f[to % D]);
+                if (to == S * 8) {
+#pragma unroll
+                    for (int s2 = 0; s2 < S; s2++)
+#pragma unroll
+                        for (int p = 0; p < 2; p++) sn[s2][p] = *reinterpret_cast<const uint32_t *>(snext + s2 * kMidSums + p * 256);
+                }
+                __builtin_amdgcn_sched_barrier(0);  // the fragments stay ahead of their use
+#pragma unroll
+                for (int p = 0; p < 2; p++)
+#pragma unroll
+                    for (int r = 0; r < R; r++) acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f[at % D][p], wt[s][r][i], acc[r], 0, 0, 0);
+            }
+            // the super-block ends: its sums take the row's d, its mins the row's dmin
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                float4_t cm = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int p = 0; p < 2; p++) {
+                    const half2_t s2 = __builtin_bit_cast(half2_t, sx[s][p]);
+                    const half4_t bs = {s2[0], s2[1], static_cast<_Float16>(0.f), static_cast<_Float16>(0.f)};
+                    cm = __builtin_amdgcn_mfma_f32_16x16x16f16(bs, am[s][r], cm, 0, 0, 0);
+                }
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float m = -dmin[s][r] * cm[j];
+                    y[r][j] = s == 0 ? fmaf(d[s][r], acc[r][j], m) : fmaf(d[s][r], acc[r][j], y[r][j] + m);
+                }
+            }
+        }
+        frag = fnext; sums = snext;
+#pragma unroll
+        for (int s = 0; s < S; s++)
+#pragma unroll
+            for (int p = 0; p < 2; p++) sx[s][p] = sn[s][p];
+        // ---- the waves' columns meet: every lane adds up its share of the tile in wave order ----
+        float *cp = cpart + buf * (W * R * 256);
+#pragma unroll
+        for (int r = 0; r < R; r++) *reinterpret_cast<float4_t *>(cp + ((wave * R + r) * 64 + lane) * 4) = y[r];
+        lds_barrier();
+        if (mine) {
+#pragma unroll
+            for (int j = 0; j < PER; j++) {
+                float v = cp[o + j];
+#pragma unroll
+                for (int w = 1; w < W; w++) v += cp[w * (R * 256) + o + j];
+                if (tile * 16 + t_in + j < a.n_tok) a.y[to_at[j] + row] = v + res[j];  // C[activation row 4 kb + j][weight row n]
+            }
+        }
+        buf ^= 1;
+    }
+}
+
+template <int R, int S, int W>
+int launch(shv_ctx *ctx, const shv_gemv_q4k_args &a, int tiles) {
+    constexpr size_t lds = static_cast<size_t>(W) * R * 2048;
+    if (lds > 48 * 1024) {
+        static std::atomic<bool> raised{false};
+        if (!raised.load(std::memory_order_acquire)) {
+            SHV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_mid_kernel<R, S, W>), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+            raised.store(true, std::memory_order_release);
+        }
+    }
+    const int blocks = (a.n + 16 * R - 1) / (16 * R);
+    // the pass's tiles go to as many blocks as a chip of 256 compute units holds one each of: more would form the weights again
+    int chunks = 256 / blocks;
+    if (chunks < 1) chunks = 1;
+    if (chunks > tiles) chunks = tiles;
+    const int per = (tiles + chunks - 1) / chunks;
+    SHV_LAUNCH(ctx, (gemm_mid_kernel<R, S, W>), dim3(blocks, (tiles + per - 1) / per), dim3(64 * W), lds, a, static_cast<const char *>(ctx->gemm_stage), tiles, per);
+    return SHV_OK;
+}
+
+}  // namespace
+
+// From nine rows, where the kernels that form every weight once for up to eight of them end, to 512: past those the blocks
+// that share their activations through LDS have rows enough for every compute unit and read less from L2 (9216 x 2048 of
+// 1024 rows: 114 us there, 133 here; of 512: 75 there, 73 here).
+bool shv_gemm_mid_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a) {
+    if (!ctx->gemm_stage || (a.k != 2048 && a.k != 4096) || a.n_tok < 9 || a.n_tok > 512) return false;
+    if (a.prologue == SHV_PRO_GATED_NORM && 256 % a.head_dim != 0) return false;
+    return mid_bytes((a.n_tok + 15) / 16, a.k) <= static_cast<size_t>(shv_ctx::kGemmStageBytes);
+}
+
+int shv_launch_gemm_mid(shv_ctx *ctx, const shv_gemv_q4k_args &a) {
+    const int tiles = (a.n_tok + 15) / 16, sbs = a.k / 256;
+    // Only the RMSNorm prologue needs the whole row before a column of it: its blocks take column parts until they fill the
+    // chip, every one of them summing the whole row
+    int parts = sbs;
+    if (a.prologue == SHV_PRO_RMSNORM)
+        for (parts = 1; parts < sbs && parts * 4 * tiles < 512;) parts *= 2;
+    SHV_LAUNCH(ctx, gemm_mid_stage_kernel, dim3(parts, 4, tiles), dim3(256), 0, a, ctx->gemm_stage, tiles);
+    // 64 weight rows a block where the columns are 2048; of 4096, 32 fill the registers as well, and a single tile of
+    // activations is quicker over twice the blocks (10.7 against 12.1 us of 16 rows)
+    if (a.k == 2048) return launch<4, 1, 8>(ctx, a, tiles);
+    return tiles == 1 ? launch<1, 2, 8>(ctx, a, tiles) : launch<2, 2, 8>(ctx, a, tiles);
+}

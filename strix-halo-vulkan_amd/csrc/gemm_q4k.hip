@@ -21,11 +21,13 @@
 #include <algorithm>
 
 #include "shv_device.hpp"
+#include "gemm_rows.hpp"
 #include "shv_internal.hpp"
 
 namespace {
 
 using namespace shv;
+using namespace shv_gemm;
 
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
@@ -164,42 +166,6 @@ __device__ __forceinline__ void stage(const shv_gemv_q4k_args &a, int t0, int nt
             char *e = frags + (static_cast<size_t>((sub * 2 + chunk) * 2) * (4 * TT) + kb * TT + tl) * 8;
             *reinterpret_cast<half4_t *>(e) = h;
             *reinterpret_cast<half4_t *>(e + 4 * TT * 8) = l;
-        }
-    }
-}
-
-// pro(x) of the four columns c..c+3 of activation row t; `scale` is the row's RMSNorm factor.
-// Every lane of a wave calls it for the same row (the gated norm adds up across lanes).
-__device__ __forceinline__ void pro_quad(const shv_gemv_q4k_args &a, int t, int c, float scale, float (&x)[4]) {
-    const int sl = a.seq_len > 0 ? a.seq_len : a.n_tok;
-    const float4 v = *reinterpret_cast<const float4 *>(a.x + static_cast<size_t>(t) * a.x_stride + c);
-    x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
-    if (a.prologue == SHV_PRO_RMSNORM) {
-        const float4 g = *reinterpret_cast<const float4 *>(a.gamma + c);
-        x[0] *= scale * g.x; x[1] *= scale * g.y; x[2] *= scale * g.z; x[3] *= scale * g.w;
-    } else if (a.prologue == SHV_PRO_GATED_NORM || a.prologue == SHV_PRO_MUL_SIGMOID) {
-        const float *z = a.z + static_cast<size_t>(t) * a.z_stride;
-        if (a.z_ring) {
-            const int s = t / sl, k = t % sl;
-            const int p = a.pos ? a.pos[s] : 0;
-            const int slot = a.slot ? a.slot[s] : s;
-            z = a.z + (static_cast<size_t>(slot) * a.ring_slots + (p + k) % a.ring_slots) * a.ring_stride;
-        }
-        const int zi = a.prologue == SHV_PRO_MUL_SIGMOID && a.head_dim > 0 ? (c & ~(a.head_dim - 1)) * 2 + a.head_dim + (c & (a.head_dim - 1)) : c;
-        const float4 zq = *reinterpret_cast<const float4 *>(z + zi);
-        const float zz[4] = {zq.x, zq.y, zq.z, zq.w};
-        if (a.prologue == SHV_PRO_GATED_NORM) {
-            float ss = fmaf(x[0], x[0], fmaf(x[1], x[1], fmaf(x[2], x[2], x[3] * x[3])));
-            const int span = a.head_dim / 4;  // lanes a head spans: a power of two up to 64
-            for (int off = 1; off < span; off <<= 1) ss += __shfl_xor(ss, off, 64);
-            const float scale = 1.f / sqrtf(ss / static_cast<float>(a.head_dim) + a.eps);
-            const float4 g4 = *reinterpret_cast<const float4 *>(a.gamma + (c & (a.head_dim - 1)));
-            const float gg[4] = {g4.x, g4.y, g4.z, g4.w};
-#pragma unroll
-            for (int j = 0; j < 4; j++) x[j] = x[j] * scale * gg[j] * sigmoid_fast(zz[j]);
-        } else {
-#pragma unroll
-            for (int j = 0; j < 4; j++) x[j] *= sigmoid_fast(zz[j]);
         }
     }
 }
@@ -425,7 +391,6 @@ __global__ __launch_bounds__(NTHR) void gemm_q4k_kernel(shv_gemv_q4k_args a, int
 // holding columns 8 kb .. 8 kb + 7 of the sub-block in the order [0, 2, 1, 3, 4, 6, 5, 7]; a wave
 // stages whole sub-blocks (lane = token + 8 * quad of the sub-block), so its writes fill a
 // fragment's 512 bytes side by side.
-__device__ __forceinline__ size_t out_offset(const shv_gemv_q4k_args &a, int t);
 constexpr int kRowsTok = 8, kRowsWaves = 16, kRowsThreads = kRowsWaves * 64;
 constexpr int kRowsFrag = 4 * kRowsTok * 16;  // bytes of one (sub-block, part) fragment
 
@@ -692,18 +657,6 @@ constexpr int kWideSlab = kWideSlabA + 4 * kWideTok * 4;     // + the sub-blocks
 constexpr int kWideSumFrags = 4 * 2 * kWideFrag;
 __host__ __device__ constexpr size_t wide_sums_offset(int k) { return static_cast<size_t>(k / 128) * kWideSlab; }
 __host__ __device__ constexpr size_t wide_region(int k) { return wide_sums_offset(k) + static_cast<size_t>((k + 1023) / 1024) * kWideSumFrags; }
-
-// Where activation row t of the pass writes its outputs: the DeltaNet projection ring, or plain rows.
-__device__ __forceinline__ size_t out_offset(const shv_gemv_q4k_args &a, int t) {
-    if (a.ring_slots > 0 && !a.z_ring) {
-        const int sl = a.seq_len > 0 ? a.seq_len : a.n_tok;
-        const int s = t / sl, i = t % sl;
-        const int p = a.pos ? a.pos[s] : 0;
-        const int slot = a.slot ? a.slot[s] : s;
-        return (static_cast<size_t>(slot) * a.ring_slots + (p + i) % a.ring_slots) * a.ring_stride;
-    }
-    return static_cast<size_t>(t) * a.y_stride;
-}
 
 // The same for a pass of up to 64 rows a group, in the slab order gemm_wide_kernel streams.
 // grid: (parts of the k/256 column blocks, 16 quartets of rows, groups of 64 rows), 256 threads: a wave takes one row's 64
@@ -1496,6 +1449,7 @@ bool shv_gemm_q4k_covers(const shv_gemv_q4k_args &a) {
 
 int shv_launch_gemm_q4k(shv_ctx *ctx, const shv_gemv_q4k_args &a) {
     if (rows_kernel_covers(ctx, a)) return a.k == 2048 ? launch_rows_k<2048, 3>(ctx, a) : launch_rows_k<4096, 1>(ctx, a);
+    if (shv_gemm_mid_covers(ctx, a)) return shv_launch_gemm_mid(ctx, a);
     // the fragments of 16 rows of 4096 columns do not fit LDS: such a pass goes 8 rows at a time
     const int cap = a.k > 2048 ? 8 : 16;
     // more rows than one block keeps in LDS: groups of 64 stream their operands

@@ -155,6 +155,8 @@ int shv_launch_gemv_q4k(shv_ctx *ctx, const shv_gemv_q4k_args *a);
 bool shv_gemm_q4k_covers(const shv_gemv_q4k_args &a);
 bool shv_gemv_mrows_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a);
 int shv_launch_gemv_mrows(shv_ctx *ctx, const shv_gemv_q4k_args &a);
+bool shv_gemm_mid_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a);
+int shv_launch_gemm_mid(shv_ctx *ctx, const shv_gemv_q4k_args &a);
 int shv_launch_gemm_q4k(shv_ctx *ctx, const shv_gemv_q4k_args &a);
 bool shv_router_wide_covers(const shv_ctx *ctx, const shv_moe_router_args &a);
 int shv_launch_router_wide(shv_ctx *ctx, const shv_moe_router_args &a);

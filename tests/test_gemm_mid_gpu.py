@@ -1,0 +1,44 @@
+"""Projections of 9 to 512 rows keep a block's weights in registers while tiles of 16 activation rows go by (gemm_mid.hip).
+Here the ends of that range, ragged last tiles, several tiles a block and several blocks a tile range, weight rows that end
+inside a tile; each with a folded prologue, a residual updated in place or a ring to write, against a float64 product."""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+import shv
+
+pytestmark = pytest.mark.gpu
+A = shv.api
+
+
+@pytest.mark.parametrize("n,k,rows", [(48, 2048, 9), (12352, 2048, 17), (2048, 4096, 16), (2055, 4096, 33), (70, 2048, 512), (9216, 2048, 81),
+                                      (2048, 4096, 255), (17, 4096, 511), (12352, 2048, 150), (512, 2048, 513)])
+def test_rows_of_a_pass(n, k, rows):
+    rng = np.random.default_rng(n + k + rows)
+    ctx = A.Context(0)
+    try:
+        wq = O.quantize_q4k((rng.standard_normal((n, k)) * 0.02).astype(np.float32))
+        w64 = O.dequant_q4k(wq, k).astype(np.float64)
+        x = (rng.standard_normal((rows, k)) * rng.uniform(0.01, 30.0, size=(rows, 1))).astype(np.float32)
+        gamma = (1 + 0.1 * rng.standard_normal(k)).astype(np.float32)
+        x64 = x.astype(np.float64)
+        want = (x64 / np.sqrt((x64 * x64).mean(axis=1, keepdims=True) + 1e-6) * gamma) @ w64.T
+        # the norm folded in, the residual in place
+        res = rng.standard_normal((rows, n)).astype(np.float32)
+        dw, dx, dg, dy = ctx.upload(wq), ctx.upload(x), ctx.upload(gamma), ctx.upload(res)
+        ctx.gemv_q4k(dw, dx, dy, n, k, n_tok=rows, prologue=A.PRO_RMSNORM, gamma=dg, residual=dy)
+        got = dy.read(np.float32, rows * n).reshape(rows, n)
+        err = np.linalg.norm(got - (want + res), axis=1) / np.linalg.norm(want + res, axis=1)
+        assert err.max() <= 1e-5, (int(err.argmax()), float(err.max()))
+        # no prologue, written into a ring that wraps
+        slots, pos = rows + 3, np.array([rows - 2], np.int32)
+        ring = ctx.upload(np.full((slots, n), -7.0, np.float32))
+        ctx.gemv_q4k(dw, dx, ring, n, k, n_tok=rows, pos=ctx.upload(pos), seq_len=rows, ring_slots=slots, ring_stride=n)
+        got = ring.read(np.float32, slots * n).reshape(slots, n)
+        at = (pos[0] + np.arange(rows)) % slots
+        want = x64 @ w64.T
+        err = np.linalg.norm(got[at] - want, axis=1) / np.linalg.norm(want, axis=1)
+        assert err.max() <= 1e-5, (int(err.argmax()), float(err.max()))
+        assert (np.delete(got, at, axis=0) == -7.0).all()
+    finally:
+        ctx.destroy()
