@@ -37,7 +37,7 @@ __host__ __device__ constexpr size_t mid_bytes(int tiles, int k) { return mid_ro
 
 // grid: (column parts, 4 quartets of rows of a tile, tiles), 256 threads: a wave takes one row's 64 quads of a super-block
 // at a time; rows past the pass's are written as zeros.
-__global__ __launch_bounds__(256) void gemm_mid_stage_kernel(shv_gemv_q4k_args a, char *staged, int tiles) {
+__global__ __launch_bounds__(256) void gemm_mid_stage_kernel(shv_gemv_q4k_args a, char *staged, int tiles, float *x_out) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, K = a.k;
     const int n = blockIdx.y * 4 + wave, t = blockIdx.z * 16 + n;
     const bool on = t < a.n_tok;
@@ -56,6 +56,8 @@ __global__ __launch_bounds__(256) void gemm_mid_stage_kernel(shv_gemv_q4k_args a
         const int c = 4 * lane;  // within the super-block
         float x[4] = {0.f, 0.f, 0.f, 0.f};
         if (on) pro_quad(a, t, sb * 256 + c, scale, x);
+        // the transformed row itself, for a caller that also needs it as plain float32 (the router's xn)
+        if (x_out && on) *reinterpret_cast<float4 *>(x_out + static_cast<size_t>(t) * K + sb * 256 + c) = float4{x[0], x[1], x[2], x[3]};
         const float sum = sum8_all((x[0] + x[1]) + (x[2] + x[3]));
         const int sub = c >> 5, kb = sub >> 1, v = (sub & 1) * 4 + ((c & 31) >> 3);
         const size_t at = static_cast<size_t>(blockIdx.z) * (K / 256) + sb;
@@ -232,6 +234,86 @@ __global__ __launch_bounds__(64 * W) void gemm_mid_kernel(shv_gemv_q4k_args a, c
     }
 }
 
+// ------------------------------------------------------------ the router of a long pass -------
+// logits[t][e] = xn[t] . W[e] for float32 rows W (the router's experts and, as one more row, the shared expert's gate)
+// against the staged rows of a pass, in the same way: a block keeps 16 R router rows in registers.  A float32 weight enters
+// as two binary16 values (hi, and the remainder scaled by 2^11 so that it stays a normal number); x_hi*w_hi + x_lo*w_hi run
+// in one accumulator, x_hi*w_lo in a second one that carries the 2^11: about 22 bits of either operand, float32 sums.
+// A wave takes 256 columns, w, w + 8, ...: with more than 2048 columns its weights are read again for every tile.
+// Bound by the fragments' way from L2, as above, and below some 500 rows by the launches.  Slabs of 64 rows staged through LDS
+// took 46 us whatever the pass's height, 27 blocks of them at 150 rows: with its staging and the selection after it the router
+// went from 58 to 24 us a layer at 150 rows of 513 x 2048, from 60 to 31 at 512, from 76 to 62 at 2048.
+template <int R>
+__global__ __launch_bounds__(512) void router_rows_kernel(const float *W, const float *extra_row, int n_rows, int K, int n_tok, const char *staged, float *logits,
+                                                          int logits_stride, int tiles, int per_chunk) {
+    constexpr int NW = 8;
+    __shared__ __align__(16) float cpart[2][NW][R * 256];
+    const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, kb = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int sbs = K / 256, row0 = blockIdx.x * (16 * R), tile0 = blockIdx.y * per_chunk;
+    const int tile_end = tile0 + per_chunk < tiles ? tile0 + per_chunk : tiles;
+    half8_t wh[R][8], wl[R][8];
+    auto form = [&](int sb) {  // this lane's 64 columns of every row
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            // rows past the end read the last row (their results are dropped); row n_rows - 1 may live apart
+            const int rr = row0 + 16 * r + n < n_rows ? row0 + 16 * r + n : n_rows - 1;
+            const float *wp = ((extra_row && rr == n_rows - 1) ? extra_row : W + static_cast<size_t>(rr) * K) + sb * 256 + kb * 64;
+#pragma unroll
+            for (int v = 0; v < 8; v++) {
+                const float4 p = *reinterpret_cast<const float4 *>(wp + v * 8), q = *reinterpret_cast<const float4 *>(wp + v * 8 + 4);
+                // slot order of the eight columns, as the rows were staged: [0, 2, 1, 3, 4, 6, 5, 7]
+                const float o[8] = {p.x, p.z, p.y, p.w, q.x, q.z, q.y, q.w};
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const _Float16 hi = static_cast<_Float16>(o[j]);
+                    wh[r][v][j] = hi;
+                    wl[r][v][j] = static_cast<_Float16>((o[j] - static_cast<float>(hi)) * 2048.f);
+                }
+            }
+        }
+    };
+    if (wave < sbs) form(wave);
+    const int o = tid % (R * 256), out_row = row0 + 16 * (o >> 8) + ((o >> 2) & 15), t_in = 4 * (o >> 6 & 3) + (o & 3);
+    const bool mine = tid < R * 256 && out_row < n_rows;
+    int buf = 0;
+    for (int tile = tile0; tile < tile_end; tile++) {
+        float4_t ym[R], yl[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) ym[r] = yl[r] = float4_t{0.f, 0.f, 0.f, 0.f};
+        for (int sb = wave; sb < sbs; sb += NW) {
+            if (sbs > NW) form(sb);
+            const char *frag = staged + (static_cast<size_t>(tile) * sbs + sb) * kMidSb + lane * 16;
+            half8_t f[8][2];
+#pragma unroll
+            for (int v = 0; v < 8; v++)
+#pragma unroll
+                for (int p = 0; p < 2; p++) f[v][p] = *reinterpret_cast<const half8_t *>(frag + (v * 2 + p) * kMidFrag);
+#pragma unroll
+            for (int v = 0; v < 8; v++)
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    ym[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f[v][0], wh[r][v], ym[r], 0, 0, 0);
+                    ym[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f[v][1], wh[r][v], ym[r], 0, 0, 0);
+                    yl[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f[v][0], wl[r][v], yl[r], 0, 0, 0);
+                }
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) cpart[buf][wave][(r * 64 + lane) * 4 + j] = fmaf(yl[r][j], 1.f / 2048.f, ym[r][j]);
+        lds_barrier();
+        const int t = tile * 16 + t_in;
+        if (mine && t < n_tok) {
+            float v = cpart[buf][0][o];
+#pragma unroll
+            for (int w = 1; w < NW; w++) v += cpart[buf][w][o];
+            logits[static_cast<size_t>(t) * logits_stride + out_row] = v;
+        }
+        buf ^= 1;
+    }
+}
+
 template <int R, int S, int W>
 int launch(shv_ctx *ctx, const shv_gemv_q4k_args &a, int tiles) {
     constexpr size_t lds = static_cast<size_t>(W) * R * 2048;
@@ -252,27 +334,69 @@ int launch(shv_ctx *ctx, const shv_gemv_q4k_args &a, int tiles) {
     return SHV_OK;
 }
 
-}  // namespace
-
-// From nine rows, where the kernels that form every weight once for up to eight of them end, to 512: past those the blocks
-// that share their activations through LDS have rows enough for every compute unit and read less from L2 (9216 x 2048 of
-// 1024 rows: 114 us there, 133 here; of 512: 75 there, 73 here).
-bool shv_gemm_mid_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a) {
-    if (!ctx->gemm_stage || (a.k != 2048 && a.k != 4096) || a.n_tok < 9 || a.n_tok > 512) return false;
-    if (a.prologue == SHV_PRO_GATED_NORM && 256 % a.head_dim != 0) return false;
-    return mid_bytes((a.n_tok + 15) / 16, a.k) <= static_cast<size_t>(shv_ctx::kGemmStageBytes);
-}
-
-int shv_launch_gemm_mid(shv_ctx *ctx, const shv_gemv_q4k_args &a) {
-    const int tiles = (a.n_tok + 15) / 16, sbs = a.k / 256;
+int launch_stage(shv_ctx *ctx, const shv_gemv_q4k_args &a, int tiles, float *x_out) {
+    const int sbs = a.k / 256;
     // Only the RMSNorm prologue needs the whole row before a column of it: its blocks take column parts until they fill the
     // chip, every one of them summing the whole row
     int parts = sbs;
     if (a.prologue == SHV_PRO_RMSNORM)
         for (parts = 1; parts < sbs && parts * 4 * tiles < 512;) parts *= 2;
-    SHV_LAUNCH(ctx, gemm_mid_stage_kernel, dim3(parts, 4, tiles), dim3(256), 0, a, ctx->gemm_stage, tiles);
+    SHV_LAUNCH(ctx, gemm_mid_stage_kernel, dim3(parts, 4, tiles), dim3(256), 0, a, ctx->gemm_stage, tiles, x_out);
+    return SHV_OK;
+}
+
+}  // namespace
+
+// From nine rows, where the kernels that form every weight once for up to eight of them end, to 512, but for 17 to 64, which
+// keep the kernel of one 64-row group: a prompt of that height is one pass whose routing (a token's tenth expert or its
+// eleventh) every token decoded after it carries on, and the fewer roundings of these sums would decide some of it otherwise
+// for 12 us a layer, once a prompt.  Past 512 the blocks
+// that share their activations through LDS have rows enough for every compute unit and read less from L2 (9216 x 2048 of
+// 1024 rows: 114 us there, 133 here; of 512: 75 there, 73 here).
+bool shv_gemm_mid_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a) {
+    if (!ctx->gemm_stage || (a.k != 2048 && a.k != 4096) || a.n_tok < 9 || a.n_tok > 512) return false;
+    if (a.n_tok > 16 && a.n_tok <= 64) return false;
+    if (a.prologue == SHV_PRO_GATED_NORM && 256 % a.head_dim != 0) return false;
+    return mid_bytes((a.n_tok + 15) / 16, a.k) <= static_cast<size_t>(shv_ctx::kGemmStageBytes);
+}
+
+int shv_launch_gemm_mid(shv_ctx *ctx, const shv_gemv_q4k_args &a) {
+    const int tiles = (a.n_tok + 15) / 16;
+    const int rc = launch_stage(ctx, a, tiles, nullptr);
+    if (rc != SHV_OK) return rc;
     // 64 weight rows a block where the columns are 2048; of 4096, 32 fill the registers as well, and a single tile of
     // activations is quicker over twice the blocks (10.7 against 12.1 us of 16 rows)
     if (a.k == 2048) return launch<4, 1, 8>(ctx, a, tiles);
     return tiles == 1 ? launch<1, 2, 8>(ctx, a, tiles) : launch<2, 2, 8>(ctx, a, tiles);
+}
+
+// The router of a pass of many rows: xn = rmsnorm(h) * gamma staged (and written out as float32), then every token's
+// n_expert (+ 1, the shared expert's gate) logits on the matrix cores.
+bool shv_router_rows_covers(const shv_ctx *ctx, const shv_moe_router_args &a) {
+    if (!ctx->gemm_stage || a.n_tok < 128 || !a.gamma || !a.xn) return false;
+    if (a.n_embd % 256 != 0 || a.n_embd < 256 || a.h_stride % 4 != 0) return false;
+    if (!shv_aligned16(a.h) || !shv_aligned16(a.gamma) || !shv_aligned16(a.xn) || !shv_aligned16(a.router) || (a.shared_gate && !shv_aligned16(a.shared_gate))) return false;
+    return mid_bytes((a.n_tok + 15) / 16, a.n_embd) <= static_cast<size_t>(shv_ctx::kGemmStageBytes);
+}
+
+int shv_launch_router_rows(shv_ctx *ctx, const shv_moe_router_args &a) {
+    shv_gemv_q4k_args g{};
+    g.x = a.h;
+    g.gamma = a.gamma;
+    g.k = a.n_embd;
+    g.n_tok = a.n_tok;
+    g.prologue = SHV_PRO_RMSNORM;
+    g.eps = a.eps;
+    g.x_stride = a.h_stride;
+    const int tiles = (a.n_tok + 15) / 16, n_rows = a.n_expert + (a.shared_gate ? 1 : 0);
+    const int rc = launch_stage(ctx, g, tiles, a.xn);
+    if (rc != SHV_OK) return rc;
+    constexpr int R = 2;
+    const int blocks = (n_rows + 16 * R - 1) / (16 * R);
+    int chunks = 256 / blocks;
+    if (chunks < 1) chunks = 1;
+    const int per = (tiles + chunks - 1) / chunks;
+    SHV_LAUNCH(ctx, (router_rows_kernel<R>), dim3(blocks, (tiles + per - 1) / per), dim3(512), 0, a.router, a.shared_gate, n_rows, a.n_embd, a.n_tok,
+               static_cast<const char *>(ctx->gemm_stage), a.logits, a.n_expert + 1, tiles, per);
+    return SHV_OK;
 }

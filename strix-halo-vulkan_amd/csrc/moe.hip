@@ -923,8 +923,8 @@ int shv_launch_moe_router(shv_ctx *ctx, const shv_moe_router_args *pa) {
     SHV_REQUIRE(a.h_stride >= a.n_embd, "moe_router: h_stride %d < n_embd %d", a.h_stride, a.n_embd);
     SHV_REQUIRE(shv_aligned16(a.router) && shv_aligned16(a.shared_gate), "moe_router: router and shared_gate must be 16-byte aligned");
     // a pass of many rows: the logits on the matrix cores
-    if (shv_router_wide_covers(ctx, a)) {
-        const int rc = shv_launch_router_wide(ctx, a);
+    if (shv_router_rows_covers(ctx, a)) {
+        const int rc = shv_launch_router_rows(ctx, a);
         if (rc != SHV_OK) return rc;
         if (!a.defer_route) {
             if (a.n_expert > 64 && a.n_expert <= kRouteBlock) SHV_LAUNCH(ctx, moe_route_block_kernel, dim3(a.n_tok), dim3(kRouteBlock), 0, a);

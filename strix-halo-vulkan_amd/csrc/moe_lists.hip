@@ -345,10 +345,13 @@ __global__ __launch_bounds__(kListThreads, 2) void moe_down_list_kernel(shv_moe_
 //   64 (1.25)                      185 / 158 / 168      400 (7.8)       400 / 321 / 312
 //   150 (2.9)                      352 / 215 / 229      600 (11.7)      453 / 413 / 379
 //   200 (3.9)                      366 / 240 / 247      800 (15.6)      480 / 510 / 460      1000 (19.5)  494 / 608 / 542
-// Below the first line most experts a pass touches are touched once, and reading them row by row costs no list.
+// Below the first line most experts a pass touches are touched once, and reading them row by row costs no list.  Up to 64
+// rows the passes keep the other kernels' sums all the same: the choice between a token's tenth and eleventh expert can hang
+// on the last bits, a short prompt's choices are carried through every token decoded after it, and the 15 % at 64 rows are one
+// part in two hundred of a reply of a hundred tokens.
 int shv_moe_list_tokens(int n_tok, int n_used, int n_expert) {
     const long long pairs = static_cast<long long>(n_tok) * n_used;
-    if (n_tok < 32 || 4 * pairs < 3ll * n_expert || pairs > 15ll * n_expert) return 0;
+    if (n_tok <= 64 || 4 * pairs < 3ll * n_expert || pairs > 15ll * n_expert) return 0;
     return pairs <= 6ll * n_expert ? 8 : 16;
 }
 

@@ -39,7 +39,7 @@ struct shv_ctx {
     bool attn_append_launch = false;
     // Rows from which a MoE pass with a workspace is grouped by expert on the matrix cores: 128, fewer where the lists are
     // worth streaming (shv_moe_list_tokens); SHV_MOE_GROUP_MIN names another number
-    int moe_group_min = 32;
+    int moe_group_min = 65;
     bool moe_group_forced = false;
     bool dn_chunk_no_recs = false;  // SHV_DN_RECS=0: the chunked delta rule forms every chunk's state-independent part inside the walk, whatever the workspace holds
     bool moe_group_one_block = false;  // SHV_MOE_GROUP_BLOCKS=1: the per-expert lists of a long pass by one block in one launch
@@ -158,8 +158,8 @@ int shv_launch_gemv_mrows(shv_ctx *ctx, const shv_gemv_q4k_args &a);
 bool shv_gemm_mid_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a);
 int shv_launch_gemm_mid(shv_ctx *ctx, const shv_gemv_q4k_args &a);
 int shv_launch_gemm_q4k(shv_ctx *ctx, const shv_gemv_q4k_args &a);
-bool shv_router_wide_covers(const shv_ctx *ctx, const shv_moe_router_args &a);
-int shv_launch_router_wide(shv_ctx *ctx, const shv_moe_router_args &a);
+bool shv_router_rows_covers(const shv_ctx *ctx, const shv_moe_router_args &a);
+int shv_launch_router_rows(shv_ctx *ctx, const shv_moe_router_args &a);
 int shv_launch_dequant_q4k(shv_ctx *ctx, const shv_dequant_q4k_args *a);
 int shv_launch_dequant(shv_ctx *ctx, const shv_dequant_args *a);
 int shv_launch_gemv(shv_ctx *ctx, const shv_gemv_args *a);

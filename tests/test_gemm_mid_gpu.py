@@ -1,4 +1,4 @@
-"""Projections of 9 to 512 rows keep a block's weights in registers while tiles of 16 activation rows go by (gemm_mid.hip).
+"""Projections of 9 to 16 and of 65 to 512 rows keep a block's weights in registers while tiles of 16 activation rows go by (gemm_mid.hip).
 Here the ends of that range, ragged last tiles, several tiles a block and several blocks a tile range, weight rows that end
 inside a tile; each with a folded prologue, a residual updated in place or a ring to write, against a float64 product."""
 import numpy as np
@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 A = shv.api
 
 
-@pytest.mark.parametrize("n,k,rows", [(48, 2048, 9), (12352, 2048, 17), (2048, 4096, 16), (2055, 4096, 33), (70, 2048, 512), (9216, 2048, 81),
+@pytest.mark.parametrize("n,k,rows", [(48, 2048, 9), (12352, 2048, 65), (2048, 4096, 16), (2055, 4096, 80), (70, 2048, 512), (9216, 2048, 81),
                                       (2048, 4096, 255), (17, 4096, 511), (12352, 2048, 150), (512, 2048, 513)])
 def test_rows_of_a_pass(n, k, rows):
     rng = np.random.default_rng(n + k + rows)
@@ -40,5 +40,27 @@ def test_rows_of_a_pass(n, k, rows):
         err = np.linalg.norm(got[at] - want, axis=1) / np.linalg.norm(want, axis=1)
         assert err.max() <= 1e-5, (int(err.argmax()), float(err.max()))
         assert (np.delete(got, at, axis=0) == -7.0).all()
+    finally:
+        ctx.destroy()
+
+
+@pytest.mark.parametrize("rows,H,E", [(128, 256, 7), (129, 1024, 31), (145, 2304, 64), (2001, 512, 32)])
+def test_router_logits_of_a_long_pass(rows, H, E):
+    """Columns of one super-block, of fewer than the block's waves and of more; router rows (the experts and the shared
+    expert's gate) around a block's 32; whole and ragged tiles, one and several a block."""
+    rng = np.random.default_rng(rows + H + E)
+    ctx = A.Context(0)
+    try:
+        h = (rng.standard_normal((rows, H)) * 2).astype(np.float32)
+        gamma = (1 + 0.1 * rng.standard_normal(H)).astype(np.float32)
+        router, gate = (rng.standard_normal((E, H)) * 0.08).astype(np.float32), (rng.standard_normal(H) * 0.08).astype(np.float32)
+        xn, logits = ctx.alloc(rows * H * 4), ctx.alloc(rows * (E + 1) * 4)
+        args = A.MoeRouterArgs(ctx.upload(h).ptr, ctx.upload(gamma).ptr, ctx.upload(router).ptr, ctx.upload(gate).ptr, xn.ptr, logits.ptr,
+                               ctx.alloc(rows * 4 * 4).ptr, ctx.alloc(rows * 5 * 4).ptr, rows, H, E, 4, 1e-6, H, 0)
+        ctx.dispatch_multi([A.make_op(A.OP_MOE_ROUTER, args)])
+        h64 = h.astype(np.float64)
+        want = (h64 / np.sqrt((h64 * h64).mean(axis=1, keepdims=True) + 1e-6) * gamma) @ np.vstack([router, gate]).astype(np.float64).T
+        got = logits.read(np.float32, rows * (E + 1)).reshape(rows, E + 1)
+        assert np.abs(got - want).max() <= 1e-6 * np.abs(want).max() * 4
     finally:
         ctx.destroy()

@@ -63,10 +63,10 @@ def block(rig, topk, grouped, packed):
 
 # (lengths, used): eight tokens at a time up to six pairs an expert, sixteen up to fifteen, and on either side of the rule
 @pytest.mark.parametrize("lengths,used", [
-    ([0, 1, 2, 7, 8, 9, 3, 0] + [2] * 16 + [], 2),       # 62 pairs, 31 tokens: below the rule (32 tokens)
-    ([0, 1, 2, 7, 8, 9, 5, 0] + [2] * 16 + [], 2),       # 64 pairs, 32 tokens: the shortest
+    ([0, 1, 2, 7, 8, 9, 5, 0] + [2] * 16, 1),            # 64 tokens: below the rule
+    ([0, 1, 2, 7, 8, 9, 6, 0] + [2] * 16, 1),            # 65 tokens: the shortest
     ([16, 17, 33, 1, 0, 8, 9, 0] + [3] * 16, 2),         # lists of several passes of eight
-    ([6] * 24, 3),                                       # 144 pairs, exactly six an expert
+    ([6] * 24, 2),                                       # 144 pairs, exactly six an expert
     ([6] * 23 + [8], 2),                                 # one more: sixteen at a time
     ([0, 1, 8, 9, 15, 16, 17, 33, 34, 47] + [12] * 13 + [14], 2),
     ([15] * 24, 4),                                      # fifteen an expert, the last of these kernels' passes
