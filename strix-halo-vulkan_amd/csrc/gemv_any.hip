@@ -1,7 +1,7 @@
 // y = W x for a weight matrix in any tensor type the reference's loader accepts: the CPU path's
 // matvec over Tensor.DequantizeRow (llm/hc.go:255-264, gguf/dequant.go:119-124) for the tensors
 // of a checkpoint that are not Q4_K (a UD-Q4_K_XL file keeps dense projections in Q8_0 and some
-// banks in Q5_K / Q6_K).  HBM-bound like the Q4_K kernel, not yet tuned like it: a lane takes one
+// banks in Q5_K / Q6_K).  HBM-bound like the Q4_K kernel, not yet tuned like it (Q6_K and Q8_0 of 2048 columns go to gemv_q68.hip): a lane takes one
 // 32-element group of a row, dequantises it exactly as the format's CPU arm does and multiplies
 // it with its 32 activations from LDS; a wave owns a row at a time and adds the lanes up.
 #include "group_dot.hpp"
@@ -90,6 +90,7 @@ int shv_launch_gemv(shv_ctx *ctx, const shv_gemv_args *pa) {
     SHV_REQUIRE(shv_aligned16(a.w), "gemv: the weight matrix must be 16-byte aligned");
     const int blk = a.type == SHV_GGML_Q4_K || a.type == SHV_GGML_Q5_K || a.type == SHV_GGML_Q6_K ? 256 : 32;
     SHV_REQUIRE(row_bytes(a.type, a.k) > 0 && a.k % blk == 0, "gemv: rows of %d elements of ggml type %d (not a type the loader accepts, or not whole blocks)", a.k, a.type);
+    if (shv_gemv_q68_covers(a)) return shv_launch_gemv_q68(ctx, a);
     switch (a.type) {
         case SHV_GGML_F32: return launch_type<SHV_GGML_F32>(ctx, a);
         case SHV_GGML_F16: return launch_type<SHV_GGML_F16>(ctx, a);

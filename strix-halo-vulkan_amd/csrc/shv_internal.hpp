@@ -162,6 +162,8 @@ bool shv_router_rows_covers(const shv_ctx *ctx, const shv_moe_router_args &a);
 int shv_launch_router_rows(shv_ctx *ctx, const shv_moe_router_args &a);
 int shv_launch_dequant_q4k(shv_ctx *ctx, const shv_dequant_q4k_args *a);
 int shv_launch_dequant(shv_ctx *ctx, const shv_dequant_args *a);
+bool shv_gemv_q68_covers(const shv_gemv_args &a);
+int shv_launch_gemv_q68(shv_ctx *ctx, const shv_gemv_args &a);
 int shv_launch_gemv(shv_ctx *ctx, const shv_gemv_args *a);
 int shv_launch_quantize_q4k(shv_ctx *ctx, const shv_quantize_q4k_args *a);
 int shv_launch_fill_normal(shv_ctx *ctx, const shv_fill_normal_args *a);
