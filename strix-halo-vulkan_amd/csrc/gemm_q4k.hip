@@ -896,21 +896,23 @@ __global__ __launch_bounds__(NW * 64) void gemm_wide_kernel(shv_gemv_q4k_args a,
 // whole numbers n * sc (exact in binary16), one matrix accumulator runs over a super-block and takes
 // its d at the end, and the min term is the only per-sub-block vector work: half the vector
 // instructions per matrix instruction of the kernel above, and no branch inside a step.
-// grid: (row blocks of NW*R*16 rows) x groups; all four token tiles are multiplied whatever the
-// group holds (rows it does not have were staged as zeros).
-template <int NW, int R>
+// grid: (row blocks of NW*R*16 rows) x bundles of TG groups; all token tiles are multiplied whatever the
+// groups hold (rows they do not have were staged as zeros).
+template <int NW, int R, int TG>
 __global__ __launch_bounds__(NW * 64) void gemm_pass_kernel(shv_gemv_q4k_args a, const char *staged_all, int groups) {
     extern __shared__ __align__(16) char smem[];
-    char *sumf = smem + 2 * kWideSlab;   // the sums of the quarter of the columns in hand, as operands
-    size_t *yoffs = reinterpret_cast<size_t *>(sumf + kWideSumFrags);
+    char *sumf = smem + 2 * TG * kWideSlab;   // the sums of the quarter of the columns in hand, as operands
+    size_t *yoffs = reinterpret_cast<size_t *>(sumf + TG * kWideSumFrags);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int n = lane & 15, kb = lane >> 4;
     const int sbs = a.k / SHV_Q4K_BLOCK;
     const size_t row_bytes = static_cast<size_t>(sbs) * SHV_Q4K_BYTES;
-    const int grp = blockIdx.x % groups, xb = blockIdx.x / groups;
+    const int bundles = (groups + TG - 1) / TG, grp = blockIdx.x % bundles * TG, xb = blockIdx.x / bundles;
     const int t0 = grp * kWideTok;
-    const int nt = a.n_tok - t0 < kWideTok ? a.n_tok - t0 : kWideTok;
-    const char *staged = staged_all + static_cast<size_t>(grp) * wide_region(a.k);
+    const int nt = a.n_tok - t0 < TG * kWideTok ? a.n_tok - t0 : TG * kWideTok;
+    const char *staged[TG];
+#pragma unroll
+    for (int u = 0; u < TG; u++) staged[u] = staged_all + static_cast<size_t>(grp + u < groups ? grp + u : grp) * wide_region(a.k);  // past the last: one again, not stored
     const int row0 = (xb * NW + wave) * (R * kTileRows);
     const int steps = a.k / 128;
 
@@ -938,18 +940,26 @@ __global__ __launch_bounds__(NW * 64) void gemm_pass_kernel(shv_gemv_q4k_args a,
     constexpr int kPieces = kWideSlab / 1024;
     static_assert(kPieces * 1024 == kWideSlab, "whole pieces");
     auto ask_slab = [&](int s, char *buf) {
-        const char *src = staged + static_cast<size_t>(s) * kWideSlab + lane * 16;
-        for (int c = wave; c < kPieces; c += NW)
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(src + c * 1024), (__attribute__((address_space(3))) void *)(buf + c * 1024), 16, 0, 0);
+#pragma unroll
+        for (int u = 0; u < TG; u++) {
+            const char *src = staged[u] + static_cast<size_t>(s) * kWideSlab + lane * 16;
+            for (int c = wave; c < kPieces; c += NW)
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(src + c * 1024),
+                                                 (__attribute__((address_space(3))) void *)(buf + u * kWideSlab + c * 1024), 16, 0, 0);
+        }
     };
     // the min term of columns [1024 qt, 1024 qt + 1024): the tokens' sums (wave w asks for fragment w of eight) and this lane's
     // rows' headers of super-block 4 qt + kb, both a step ahead of their use
     static_assert(NW >= 8, "a fragment of sums a wave");
     uint4 hq[R];
     auto ask_quarter = [&](int qt) {
-        if (wave < 8)
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(staged + wide_sums_offset(a.k) + static_cast<size_t>(qt * 8 + wave) * kWideFrag + lane * 16),
-                                             (__attribute__((address_space(3))) void *)(sumf + wave * kWideFrag), 16, 0, 0);
+        if (wave < 8) {
+#pragma unroll
+            for (int u = 0; u < TG; u++)
+                __builtin_amdgcn_global_load_lds(
+                    (const __attribute__((address_space(1))) void *)(staged[u] + wide_sums_offset(a.k) + static_cast<size_t>(qt * 8 + wave) * kWideFrag + lane * 16),
+                    (__attribute__((address_space(3))) void *)(sumf + u * kWideSumFrags + wave * kWideFrag), 16, 0, 0);
+        }
         const int sb = 4 * qt + kb < sbs ? 4 * qt + kb : 0;
 #pragma unroll
         for (int r = 0; r < R; r++) hq[r] = *reinterpret_cast<const uint4 *>(rp[r] + static_cast<size_t>(sb) * SHV_Q4K_BYTES);
@@ -963,18 +973,18 @@ __global__ __launch_bounds__(NW * 64) void gemm_pass_kernel(shv_gemv_q4k_args a,
     uint32_t m0 = 0x000F000Fu, o0 = 0x64006400u;   // bits 0..3 of both halves under the exponent of 1024
     asm volatile("" : "+s"(m0));
     asm volatile("" : "+v"(o0));
-    float4_t y[R][4], acc[R][4];
+    float4_t y[R][4 * TG], acc[R][4 * TG];
 #pragma unroll
     for (int r = 0; r < R; r++)
 #pragma unroll
-        for (int tt = 0; tt < 4; tt++) y[r][tt] = acc[r][tt] = float4_t{0.f, 0.f, 0.f, 0.f};
+        for (int tt = 0; tt < 4 * TG; tt++) y[r][tt] = acc[r][tt] = float4_t{0.f, 0.f, 0.f, 0.f};
 
     for (int s = 0; s < steps; s++) {
         const int cur = s & 1;
         const bool more = s + 1 < steps;
         {
             const int sn = more ? s + 1 : s;
-            if (more) ask_slab(sn, smem + (cur ^ 1) * kWideSlab);   // the other buffer was read to its end before the barrier that ended the last step
+            if (more) ask_slab(sn, smem + (cur ^ 1) * (TG * kWideSlab));   // the other buffer was read to its end before the barrier that ended the last step
             if (more && (sn & 7) == 0) {
                 // the sums in LDS were read at this quarter's first step, steps ago; every wave is past that
                 ask_quarter(sn >> 3);
@@ -985,7 +995,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_pass_kernel(shv_gemv_q4k_args a,
                 for (int r = 0; r < R; r++) hdrn[r] = *reinterpret_cast<const uint4 *>(rp[r] + static_cast<size_t>(sn >> 1) * SHV_Q4K_BYTES);
             }
         }
-        const char *A = smem + cur * kWideSlab;
+        const char *A = smem + cur * (TG * kWideSlab);
         if ((s & 7) == 0) {
             // y -= sum over the quarter's sub-blocks of dmin * m * sum(x), as three matrix products a token tile:
             // -dmin * m has 17 significant bits and goes as two halves, the sums come as two halves too
@@ -1004,7 +1014,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_pass_kernel(shv_gemv_q4k_args a,
                     bl[j] = static_cast<_Float16>(p - static_cast<float>(hi));
                 }
 #pragma unroll
-                for (int tt = 0; tt < 4; tt++) {
+                for (int tt = 0; tt < 4 * TG; tt++) {
                     half8_t sh = *reinterpret_cast<const half8_t *>(sumf + (tt * 2) * kWideFrag + lane * 16);
                     half8_t sl = *reinterpret_cast<const half8_t *>(sumf + (tt * 2 + 1) * kWideFrag + lane * 16);
                     if (!on) sh = sl = static_cast<half8_t>(static_cast<_Float16>(0.f));   // a super-block past the row: nothing was staged there
@@ -1056,8 +1066,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_pass_kernel(shv_gemv_q4k_args a,
                     }
                 }
 #pragma unroll
-                for (int tt = 0; tt < 4; tt++) {
-                    const char *f = A + static_cast<size_t>((sub * 4 + tt) * 2) * kWideFrag + lane * 16;
+                for (int tt = 0; tt < 4 * TG; tt++) {
+                    const char *f = A + (tt >> 2) * kWideSlab + static_cast<size_t>((sub * 4 + (tt & 3)) * 2) * kWideFrag + lane * 16;
                     const half8_t xh = *reinterpret_cast<const half8_t *>(f);
                     const half8_t xl = *reinterpret_cast<const half8_t *>(f + kWideFrag);
 #pragma unroll
@@ -1074,7 +1084,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_pass_kernel(shv_gemv_q4k_args a,
             for (int r = 0; r < R; r++) {
                 const float dd = f16_bits_to_f32(hdr[r].x);
 #pragma unroll
-                for (int tt = 0; tt < 4; tt++) {
+                for (int tt = 0; tt < 4 * TG; tt++) {
 #pragma unroll
                     for (int j = 0; j < 4; j++) y[r][tt][j] = fmaf(dd, acc[r][tt][j], y[r][tt][j]);
                     acc[r][tt] = float4_t{0.f, 0.f, 0.f, 0.f};
@@ -1096,7 +1106,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_pass_kernel(shv_gemv_q4k_args a,
         const int row = row0 + r * kTileRows + n;
         if (row >= a.n) continue;
 #pragma unroll
-        for (int tt = 0; tt < 4; tt++) {
+        for (int tt = 0; tt < 4 * TG; tt++) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const int tok = tt * kTileRows + 4 * kb + j;
@@ -1259,18 +1269,18 @@ bool rows_kernel_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a) {
 
 // Every group of 64 rows of a long pass in one launch (the operands of all of them are in
 // ctx->gemm_stage): no split along the columns, the groups themselves fill the chip.
-template <int NW, int R>
+template <int NW, int R, int TG>
 int launch_wide_all(shv_ctx *ctx, const shv_gemv_q4k_args &a, int groups) {
     constexpr int kRows = NW * R * kTileRows;
     const int bx = (a.n + kRows - 1) / kRows;
-    const size_t lds = 2 * kWideSlab + kWideSumFrags + kWideTok * sizeof(size_t);
+    const size_t lds = TG * (2 * kWideSlab + kWideSumFrags + kWideTok * sizeof(size_t));
     static std::atomic<bool> raised{false};
     if (!raised.load(std::memory_order_acquire)) {
-        SHV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_pass_kernel<NW, R>), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+        SHV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_pass_kernel<NW, R, TG>), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
         raised.store(true, std::memory_order_release);
     }
     SHV_REQUIRE(static_cast<long long>(bx) * groups <= 0x7fffffffll, "gemm_q4k: %d row blocks of %d groups", bx, groups);
-    SHV_LAUNCH(ctx, (gemm_pass_kernel<NW, R>), dim3(bx * groups), dim3(NW * 64), lds, a, static_cast<const char *>(ctx->gemm_stage), groups);
+    SHV_LAUNCH(ctx, (gemm_pass_kernel<NW, R, TG>), dim3(bx * ((groups + TG - 1) / TG)), dim3(NW * 64), lds, a, static_cast<const char *>(ctx->gemm_stage), groups);
     return SHV_OK;
 }
 
@@ -1305,7 +1315,17 @@ int shv_launch_gemm_q4k(shv_ctx *ctx, const shv_gemv_q4k_args &a) {
         const int groups = (a.n_tok + kWideTok - 1) / kWideTok;
         SHV_REQUIRE(groups * wide_region(a.k) <= static_cast<size_t>(shv_ctx::kGemmStageBytes), "gemm_q4k: %d rows of %d columns do not fit the staging buffer", a.n_tok, a.k);
         SHV_LAUNCH(ctx, gemm_wide_stage_kernel, dim3(stage_parts(a, groups), kWideTok / 4, groups), dim3(256), 0, a, ctx->gemm_stage);
-        if (groups >= 4) return launch_wide_all<8, 1>(ctx, a, groups);
+        if (groups >= 4) {
+            // Blocks of 256 rows and two groups form each weight once for 128 activation rows: an eighth less work in all (9216 x
+            // 2048 of 4096 rows 403 -> 380 us, 2048 x 4096 203 -> 180), when their rounds of the chip, one a compute unit, leave
+            // no more of it idle than the rounds of the blocks of 128 rows and one group, two a unit, do (12352 x 2048 of 2048
+            // rows 278 so and 290 with two groups).
+            const int cus = ctx->prop.multiProcessorCount;
+            const auto filled = [](long long blocks, int slots) { return static_cast<double>(blocks) / static_cast<double>((blocks + slots - 1) / slots * slots); };
+            const int pairs = (groups + 1) / 2;
+            const double two = filled(static_cast<long long>((a.n + 255) / 256) * pairs, cus) * groups / (2 * pairs), one = filled(static_cast<long long>((a.n + 127) / 128) * groups, 2 * cus);
+            return 1.12 * two >= one ? launch_wide_all<16, 1, 2>(ctx, a, groups) : launch_wide_all<8, 1, 1>(ctx, a, groups);
+        }
         for (int g = 0; g < groups; g++) {
             const int t0 = g * kWideTok;
             const int nt = a.n_tok - t0 < kWideTok ? a.n_tok - t0 : kWideTok;

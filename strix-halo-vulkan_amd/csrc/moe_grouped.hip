@@ -456,6 +456,14 @@ constexpr int kStSumFrags = kTT * 2 * kFrag;   // the sums of a quarter of the c
 constexpr int kStMinHdrs = kStWaves * kTiles * kFrag;   // every lane's row header of its super-block of the quarter, a wave's own
 constexpr size_t kStagedLds = 2 * static_cast<size_t>(kStFrags) + 2 * kStSumFrags + kStMinHdrs + 2 * kTok * 4;
 
+// Where the eight columns of block blk of sub-block `sub` stand in a row's operands, part 0 (part 1: 64 on): [super-block]
+// [product][part][lane kb of the products] x 16 bytes, so that the four lanes of a row ask for 64 bytes in a line.  Product
+// pr * 4 + hi * 2 + half: pair pr of the super-block's groups, low or high nibbles, first or second eight of a lane's sixteen.
+__device__ __forceinline__ size_t group_block(int sub, int blk) {
+    const int product = ((sub >> 2) & 1) * 4 + (sub & 1) * 2 + (blk & 1), kb = ((sub >> 1) & 1) * 2 + (blk >> 1);
+    return static_cast<size_t>(sub >> 3) * (8 * kStSubBytes) + product * 128 + kb * 16;
+}
+
 // grid: (k / 1024, rows), 256 threads, a quad of columns each.
 __global__ __launch_bounds__(256) void moe_stage_kernel(const float *x, int x_stride, int k, int rows, char *staged) {
     const int t = blockIdx.y, c = (blockIdx.x * 256 + threadIdx.x) * 4;
@@ -469,7 +477,7 @@ __global__ __launch_bounds__(256) void moe_stage_kernel(const float *x, int x_st
         h[j] = hi;
         l[j] = static_cast<_Float16>(o[j] - static_cast<float>(hi));
     }
-    char *e = staged + (static_cast<size_t>(t) * (k / 32) + (c >> 5)) * kStSubBytes + ((c & 31) >> 3) * 16 + ((c & 7) >> 2) * 8;
+    char *e = staged + static_cast<size_t>(t) * (k / 32) * kStSubBytes + group_block(c >> 5, (c & 31) >> 3) + ((c & 7) >> 2) * 8;
     *reinterpret_cast<half4_t *>(e) = h;
     *reinterpret_cast<half4_t *>(e + 64) = l;
     // the sub-block's sum: eight neighbouring lanes (k is a multiple of 32, so they are all here)
@@ -485,21 +493,21 @@ __global__ __launch_bounds__(256) void moe_stage_kernel(const float *x, int x_st
     }
 }
 
+// Where lane (row n, piece kb) of the products finds its sixteen bytes of a fragment that ask_staged_slab has brought.
+__device__ __forceinline__ int frag_at(int lane) { return (lane & 15) * 64 + (((lane >> 4) ^ (lane >> 2)) & 3) * 16; }
+
 template <int K>
 __device__ __forceinline__ void ask_staged_slab(const char *staged, const int32_t *tok_s, int m, int n_tt, int sl, char *buf, int lane, int wave) {
-    // Wave w asks for product w of the slab's eight: pair w / 4 of its groups, the pair's low (0) or high (1) nibbles,
-    // the first or second eight of a lane's sixteen bytes.  Its lane (token, kb) stands where the weights' lane
-    // (row, kb) does: sub-block 2 (group of the lane) + nibble, columns 16 (kb & 1) + 8 (half) .. + 7 of it.
-    const int n = lane & 15, kb = lane >> 4;
-    const int pr = wave >> 2, hi = (wave >> 1) & 1, half = wave & 1;
-    const int sg = sl * kStSubs + 4 * pr + 2 * (kb >> 1) + hi;  // the sub-block this lane's eight columns lie in
-    const int cb = 2 * (kb & 1) + half;                          // and which eight of its 32
+    // Wave w asks for product w of the slab's eight.  Four neighbouring lanes ask for a row's four pieces, which lie in a
+    // line of 64 bytes and are one request; which of them asks for which is turned with the row, so that the products' lanes
+    // (row n, piece kb), reading at frag_at, find eight rows' pieces in different banks.
+    const int n = lane >> 2, kb = (lane & 3) ^ ((n >> 2) & 3);
 #pragma unroll
     for (int tt = 0; tt < kTT; tt++) {
         if (tt >= n_tt) break;
         const int i = 16 * tt + n;
         const int t = tok_s[i < m ? i : 0];  // a column past the list repeats the first row; nobody reads its products
-        const char *g = staged + (static_cast<size_t>(t) * (K / 32) + sg) * kStSubBytes + cb * 16;
+        const char *g = staged + (static_cast<size_t>(t) * (K / 32) + sl * kStSubs) * kStSubBytes + wave * 128 + kb * 16;
         char *f = buf + ((wave * 2) * kTT + tt) * kFrag;
         __builtin_amdgcn_global_load_lds((global_ptr_t)(g), (lds_ptr_t)(f), 16, 0, 0);
         __builtin_amdgcn_global_load_lds((global_ptr_t)(g + 64), (lds_ptr_t)(f + kTT * kFrag), 16, 0, 0);
@@ -583,7 +591,7 @@ __device__ __forceinline__ void staged_slab_times_tiles(const char *const (&rp)[
     // LDS addresses are 32 bits wide: kept as such, a fragment's place costs no 64-bit arithmetic
     typedef const __attribute__((address_space(3))) char *lds_bytes_t;
     typedef const __attribute__((address_space(3))) half8_t *lds_half8_t;
-    const lds_bytes_t fl = (lds_bytes_t)(frags) + lane * 16;
+    const lds_bytes_t fl = (lds_bytes_t)(frags) + frag_at(lane);
     half8_t nh = *(lds_half8_t)(fl), nl = *(lds_half8_t)(fl + kTT * kFrag);
 #pragma unroll 1
     for (int pi = 0; pi < NG / 2; pi++) {
@@ -799,12 +807,13 @@ __device__ __forceinline__ void up_pass(const shv_moe_up_args &a, const char *co
                 sum += __shfl_xor(sum, 8, 64);
                 if (i < m) {
                     const size_t pair = static_cast<size_t>(pair_s[i]);
-                    char *e = reinterpret_cast<char *>(a.act) + (pair * (a.ffn / 32) + sub) * kStSubBytes + (n >> 3) * 16 + slot * 2;
+                    char *e = reinterpret_cast<char *>(a.act) + pair * (a.ffn / 32) * kStSubBytes + slot * 2;
 #pragma unroll
                     for (int r = 0; r < 2; r++) {
                         const _Float16 hi = static_cast<_Float16>(v[r]);
-                        *reinterpret_cast<_Float16 *>(e + r * 32) = hi;
-                        *reinterpret_cast<_Float16 *>(e + r * 32 + 64) = static_cast<_Float16>(v[r] - static_cast<float>(hi));
+                        const size_t at = group_block(sub, 2 * r + (n >> 3));
+                        *reinterpret_cast<_Float16 *>(e + at) = hi;
+                        *reinterpret_cast<_Float16 *>(e + at + 64) = static_cast<_Float16>(v[r] - static_cast<float>(hi));
                     }
                     if (n == 0) {
                         const _Float16 hi = static_cast<_Float16>(sum);

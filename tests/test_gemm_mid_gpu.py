@@ -1,6 +1,6 @@
 """Projections of 9 to 16 and of 65 to 512 rows keep a block's weights in registers while tiles of 16 activation rows go by (gemm_mid.hip).
 Here the ends of that range, ragged last tiles, several tiles a block and several blocks a tile range, weight rows that end
-inside a tile; each with a folded prologue, a residual updated in place or a ring to write, against a float64 product."""
+inside a tile, and two passes past it, in blocks of one and of two groups of 64 rows; each with a folded prologue, a residual updated in place or a ring to write, against a float64 product."""
 import numpy as np
 import pytest
 
@@ -12,7 +12,7 @@ A = shv.api
 
 
 @pytest.mark.parametrize("n,k,rows", [(48, 2048, 9), (12352, 2048, 65), (2048, 4096, 16), (2055, 4096, 80), (70, 2048, 512), (9216, 2048, 81),
-                                      (2048, 4096, 255), (17, 4096, 511), (12352, 2048, 150), (512, 2048, 513)])
+                                      (2048, 4096, 255), (17, 4096, 511), (12352, 2048, 150), (512, 2048, 513), (200, 2048, 1050)])
 def test_rows_of_a_pass(n, k, rows):
     rng = np.random.default_rng(n + k + rows)
     ctx = A.Context(0)
