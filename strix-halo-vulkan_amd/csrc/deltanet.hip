@@ -171,6 +171,111 @@ __global__ __launch_bounds__(kBlock) void dn_step_kernel(shv_dn_step_args a) {
     }
 }
 
+// One row of each of the call's sequences (the decode step): the same arithmetic, laid out as one trip to memory.  The kernel
+// above, made for groups of rows, asks for a row's conv taps, ring values, gates and v channels behind one another and behind
+// branches, four trips in a row of the 4.75 us it takes for one row; here everything that the row's position does not name goes
+// out first, the ring's values behind the position, the state behind the plane, and nothing is waited for before all is asked for.
+template <int RW>
+__global__ __launch_bounds__(kBlock) void dn_step_one_kernel(shv_dn_step_args a) {
+    constexpr int kRowsPerBlock = 4 * RW, NS = RW / 2;
+    __shared__ __align__(16) float qs[kD];
+    __shared__ __align__(16) float ks[kD];
+    __shared__ float vs[kRowsPerBlock];
+    __shared__ float red[4];
+    __shared__ float gb[2];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int chunk = blockIdx.x, h = blockIdx.y, seq = blockIdx.z;
+    const int hk = h % a.n_head_k;
+    const int qk = a.n_head_k * kD, vw = a.n_head_v * kD;
+    const int alpha_off = 2 * qk + 2 * vw, beta_off = alpha_off + a.n_head_v;
+    const int rsub = lane >> 5, li = lane & 31;
+    const int jl = wave * RW + rsub;
+    const int j = chunk * kRowsPerBlock + jl;
+    const int ch = tid < kD ? hk * kD + tid : qk + hk * kD + (tid - kD);
+    const int vr = tid % kRowsPerBlock, vch = 2 * qk + h * kD + chunk * kRowsPerBlock + vr;
+    const float4 tp = *reinterpret_cast<const float4 *>(a.conv1d + static_cast<size_t>(ch) * 4);
+    const float4 tv = *reinterpret_cast<const float4 *>(a.conv1d + static_cast<size_t>(vch) * 4);
+    const float dt_bias = load_in_turn(a.dt_bias + h), decay = load_in_turn(a.a + h);
+    // (no branch around the two: any readable word in an absent one's place, so that both are on their way together)
+    const int32_t *any = reinterpret_cast<const int32_t *>(a.conv1d);
+    const int32_t slot_word = *(a.slot ? a.slot + seq : any), pos_word = *(a.pos ? a.pos + seq : any);
+    const int slot = a.slot ? slot_word : seq, p0 = a.pos ? pos_word : 0;
+    const int planes = a.n_planes > 1 ? a.n_planes : 1;
+    // one copy of the state is found without its number
+    int cur = 0;
+    if (a.plane && planes > 1) cur = static_cast<int>(static_cast<unsigned>(a.plane[slot]) % static_cast<unsigned>(planes));
+    const float *ring = a.ring + static_cast<size_t>(slot) * a.ring_slots * a.ring_stride;
+    float x[4], xv[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        // a row before the sequence's start is zero: any row of the ring is asked for in its place
+        const float *row = ring + static_cast<size_t>((p0 + i < 3 ? p0 : p0 + i - 3) % a.ring_slots) * a.ring_stride;
+        x[i] = row[ch];
+        xv[i] = row[vch];
+    }
+    const float *row = ring + static_cast<size_t>(p0 % a.ring_slots) * a.ring_stride;
+    const float alpha = load_in_turn(row + alpha_off + h), write = load_in_turn(row + beta_off + h);
+    const size_t plane_floats = static_cast<size_t>(a.n_head_v) * kD * kD;
+    float *sslot = a.state + static_cast<size_t>(slot) * planes * plane_floats + (static_cast<size_t>(h) * kD + j) * kD + li * 4;
+    float *srow = sslot + cur * plane_floats;
+    float4 s[NS];
+#pragma unroll
+    for (int u = 0; u < NS; u++) s[u] = *reinterpret_cast<const float4 *>(srow + static_cast<size_t>(2 * u) * kD);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        if (p0 + i < 3) x[i] = xv[i] = 0.f;
+
+    const float scale = 1.f / sqrtf(static_cast<float>(kD));
+    float c = 0.f;
+    c += x[0] * tp.x;
+    c += x[1] * tp.y;
+    c += x[2] * tp.z;
+    c += x[3] * tp.w;
+    const float act = c * sigmoid_exact(c);
+    const float ss = wave_sum_all(act * act);
+    if (lane == 0) red[wave] = ss;
+    if (tid < kRowsPerBlock) {
+        float cv = 0.f;
+        cv += xv[0] * tv.x;
+        cv += xv[1] * tv.y;
+        cv += xv[2] * tv.z;
+        cv += xv[3] * tv.w;
+        vs[vr] = cv * sigmoid_exact(cv);
+    } else if (tid == kBlock - 1) {
+        const float asp = softplus_ref(alpha + dt_bias);
+        gb[0] = expf(asp * decay);
+        gb[1] = sigmoid_exact(write);
+    }
+    __syncthreads();
+    {
+        const float ssq = tid < kD ? red[0] + red[1] : red[2] + red[3];
+        const float nrm = a.qk_norm_max ? 1.f / fmaxf(sqrtf(ssq), a.eps) : 1.f / sqrtf(ssq + a.eps);
+        if (tid < kD) qs[tid] = act * nrm; else ks[tid - kD] = act * nrm;
+    }
+    __syncthreads();
+    const float4 k4 = *reinterpret_cast<const float4 *>(&ks[li * 4]);
+    const float4 q4 = *reinterpret_cast<const float4 *>(&qs[li * 4]);
+    const float g = gb[0], beta = gb[1];
+#pragma unroll
+    for (int u = 0; u < NS; u++) {
+        float4 &su = s[u];
+        const float vj = vs[jl + 2 * u];
+        su.x *= g; su.y *= g; su.z *= g; su.w *= g;
+        const float dk = sum32_all(fmaf(su.x, k4.x, fmaf(su.y, k4.y, fmaf(su.z, k4.z, su.w * k4.w))));
+        const float delta = (vj - dk) * beta;
+        su.x = fmaf(delta, k4.x, su.x);
+        su.y = fmaf(delta, k4.y, su.y);
+        su.z = fmaf(delta, k4.z, su.z);
+        su.w = fmaf(delta, k4.w, su.w);
+        // a rewindable pass keeps every prefix: the state after its row goes to its own plane
+        float *to = a.spec ? sslot + ((cur + 1) % planes) * plane_floats : srow;
+        *reinterpret_cast<float4 *>(to + static_cast<size_t>(2 * u) * kD) = su;
+        const float oq = sum32_all(fmaf(su.x, q4.x, fmaf(su.y, q4.y, fmaf(su.z, q4.z, su.w * q4.w))));
+        if (li == 0) a.out[static_cast<size_t>(seq) * vw + static_cast<size_t>(h) * kD + j + 2 * u] = oq * scale;
+    }
+}
+
 // The same step for calls of many rows (prompt chunks), where the groups' preparation - not the
 // rule - is most of the time of the kernel above: here eight more waves prepare group g+1 into a
 // second set of LDS buffers while the four waves that hold the state walk group g, with one
@@ -317,6 +422,8 @@ int shv_launch_dn_step(shv_ctx *ctx, const shv_dn_step_args *pa) {
     dim3 grid(kD / kRowsPerBlock, a.n_head_v, a.n_seq);
     // more than one group of rows: preparation and rule overlap
     if (a.seq_len > kPrep) SHV_LAUNCH(ctx, dn_step_pipe_kernel, grid, dim3(kBlock + 64 * kPrepWaves), 0, a);
+    else if (a.seq_len == 1 && a.n_seq >= 4) SHV_LAUNCH(ctx, dn_step_one_kernel<4>, dim3(kD / 16, a.n_head_v, a.n_seq), dim3(kBlock), 0, a);
+    else if (a.seq_len == 1) SHV_LAUNCH(ctx, dn_step_one_kernel<2>, grid, dim3(kBlock), 0, a);
     else if (a.n_seq >= 4) SHV_LAUNCH(ctx, dn_step_kernel<4>, dim3(kD / 16, a.n_head_v, a.n_seq), dim3(kBlock), 0, a);
     else SHV_LAUNCH(ctx, dn_step_kernel<2>, grid, dim3(kBlock), 0, a);
     return SHV_OK;

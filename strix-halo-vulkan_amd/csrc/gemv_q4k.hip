@@ -325,11 +325,22 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_row_kernel(shv_gemv_q4k_args 
     // Loads return in the order they were asked for, so the input row goes first: it comes from
     // cache in a fraction of the weights' latency, and the staging below (and the block-wide wait)
     // is over by the time the first weights arrive, instead of queueing behind all of them.
-    int ring_row = 0;  // the ring slot of the row (its sequence's position and slot)
-    if (a.ring_slots > 0) {
-        const int p = a.pos ? a.pos[0] : 0;
-        const int slot = a.slot ? a.slot[0] : 0;
-        ring_row = slot * a.ring_slots + p % a.ring_slots;
+    // The ring slot of the row (its sequence's position and slot) is two trips to memory away: a gate in the ring needs it for a
+    // load of its own and has it asked for first, a row to be stored there asks for it behind the weights.
+    constexpr bool GATE = PRO == SHV_PRO_GATED_NORM;
+    int32_t rpos = 0, rslot = 0;
+    const auto ask_ring = [&] {
+        if (a.ring_slots > 0) {
+            if (a.pos) rpos = load_in_turn(a.pos);
+            if (a.slot) rslot = load_in_turn(a.slot);
+        }
+    };
+    const auto ring_row = [&] { return a.ring_slots > 0 ? __builtin_amdgcn_readfirstlane(rslot) * a.ring_slots + __builtin_amdgcn_readfirstlane(rpos) % a.ring_slots : 0; };
+    if constexpr (GATE) {
+        if (a.ring_slots > 0) {
+            if (a.pos) rpos = a.pos[0];
+            if (a.slot) rslot = a.slot[0];
+        }
     }
     float4 xv[NV], gv[NV], zv[NV];
 #pragma unroll
@@ -338,8 +349,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_row_kernel(shv_gemv_q4k_args 
         xv[j] = *reinterpret_cast<const float4 *>(a.x + c);
         if constexpr (PRO == SHV_PRO_RMSNORM) {
             gv[j] = *reinterpret_cast<const float4 *>(a.gamma + c);
-        } else if constexpr (PRO == SHV_PRO_GATED_NORM) {
-            const float *z = a.z_ring ? a.z + static_cast<size_t>(ring_row) * a.ring_stride : a.z;
+        } else if constexpr (GATE) {
+            const float *z = a.z_ring ? a.z + static_cast<size_t>(ring_row()) * a.ring_stride : a.z;
             zv[j] = *reinterpret_cast<const float4 *>(z + c);
             gv[j] = *reinterpret_cast<const float4 *>(a.gamma + (c & (a.head_dim - 1)));
         } else if constexpr (PRO == SHV_PRO_MUL_SIGMOID) {
@@ -368,6 +379,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_row_kernel(shv_gemv_q4k_args 
     float res[P];
 #pragma unroll
     for (int u = 0; u < P; u++) res[u] = (a.residual && row[u] >= 0 && group_sum_owner<LPR>(lane)) ? a.residual[row[u]] : 0.f;
+    if constexpr (!GATE) ask_ring();
     // the wave's quarter of its fold row, behind the weights
     float4 fw[FOLD ? FA + FB : 1];
     if constexpr (FOLD) {
@@ -424,7 +436,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_row_kernel(shv_gemv_q4k_args 
     float xr[64], xs_lo, xs_hi;
     load_x_slice_presummed(xs, xsum, gi, xr, xs_lo, xs_hi);
     float *y = a.y;
-    if (a.ring_slots > 0 && !a.z_ring) y += static_cast<size_t>(ring_row) * a.ring_stride;
+    if (a.ring_slots > 0 && !a.z_ring) y += static_cast<size_t>(ring_row()) * a.ring_stride;
     const NibbleConsts nc = nibble_consts();
     __shared__ float4 staged_sc[STAGED ? WAVES * P * 64 : 1];
     if constexpr (STAGED) {

@@ -442,7 +442,7 @@ __global__ __launch_bounds__(kRouteBlock) void moe_route_block_kernel(shv_moe_ro
 // the selected probabilities cannot engage with at most 512 experts (the largest probability is
 // at least 1/512).  Two different logits whose probabilities round to the same float would be
 // ordered by index in the reference and are ordered by logit here: a tie of the last bit.
-// sel_e [kMaxUsed] / sel_w [kMaxUsed + 1] receive experts, weights and the shared expert's gate;
+// sel_e [kMaxUsed] / sel_w [kMaxUsed + 1] receive experts, weights and the shared expert's gate (of `all`);
 // probs is the one-wave road's scratch.  On return every wave can read sel_e / sel_w (each has
 // written the same values there itself).
 constexpr int kCandMax = 64;
@@ -466,9 +466,22 @@ __device__ __forceinline__ void count_greater_ror(uint32_t key, int &rank) {
 // NORM: the logits still lack the RMSNorm's factor of the token row (they came with the output
 // projection's launch); the block's waves have left their sums of squares of the row's k columns in
 // `red` before the call, and the factor, which changes no order, goes into the weights alone.
+// `in`: this thread's logits and the shared gate's, asked for by the caller with the rest of what the kernel starts with (asked for
+// in here, behind the sums of squares, they were a second trip to memory: 1 us of the launch).
+struct RouteLoads {
+    float l0, l1, lsh;
+    __device__ __forceinline__ void ask(const float *lg, int n_expert) {
+        // no branch around a load: past the last expert the last one's, which nobody uses
+        l0 = lg[min(static_cast<int>(threadIdx.x), n_expert - 1)];
+        l1 = lg[min(static_cast<int>(threadIdx.x) + 256, n_expert - 1)];
+        lsh = lg[n_expert];
+    }
+};
+// Returns the expert of slot `slot`; sel_e and sel_w are filled for the block that asks for them (`all`): the others need
+// no weights, whose exponentials and sum stood between the selection and their weights' loads.
 template <bool NORM>
-__device__ __forceinline__ void route_block256(const float *lg, int n_expert, int n_used, bool shared_gate, int32_t *sel_e, float *sel_w, float *probs,
-                                               const float *red = nullptr, float mean_div = 1.f, float eps = 0.f) {
+__device__ __forceinline__ int route_block256(const RouteLoads &in, const float *lg, int n_expert, int n_used, bool shared_gate, int slot, bool all, int32_t *sel_e,
+                                              float *sel_w, float *probs, const float *red = nullptr, float mean_div = 1.f, float eps = 0.f) {
     __shared__ float s_max[4];
     __shared__ __align__(16) float s_gm[16];
     __shared__ int s_cnt[4];
@@ -478,8 +491,8 @@ __device__ __forceinline__ void route_block256(const float *lg, int n_expert, in
     const bool routing = tid < 256;
     const int e0 = tid, e1 = tid + 256;
     const bool has0 = routing && e0 < n_expert, has1 = routing && e1 < n_expert;
-    const float l0 = has0 ? lg[e0] : -INFINITY, l1 = has1 ? lg[e1] : -INFINITY;
-    const float lsh = (lane == 63 && shared_gate) ? lg[n_expert] : 0.f;  // every wave keeps the shared gate for itself
+    const float l0 = has0 ? in.l0 : -INFINITY, l1 = has1 ? in.l1 : -INFINITY;
+    const float lsh = (lane == 63 && shared_gate) ? in.lsh : 0.f;  // every wave keeps the shared gate for itself
     if (routing) {  // the block's maximum and the maxima of 16 groups of 16 threads
         float gm = fmaxf(l0, l1);
         gm = fmaxf(gm, dpp_f32<kDppXor1>(gm));
@@ -535,7 +548,7 @@ __device__ __forceinline__ void route_block256(const float *lg, int n_expert, in
             if (lane == 0) sel_w[n_used] = shared_gate ? sigmoid_exact(lg[n_expert] * scale) : 0.f;
         }
         __syncthreads();
-        return;
+        return sel_e[slot];
     }
     if (routing) {
         // the table's order does not matter to the ranks: each wave writes its candidates after
@@ -567,6 +580,10 @@ __device__ __forceinline__ void route_block256(const float *lg, int n_expert, in
         }
     }
     const int rank = (r4[0] + r4[1]) + (r4[2] + r4[3]);
+    const int e_mine = 0x7FFFFFFF - static_cast<int>(static_cast<uint32_t>(mine));
+    const unsigned long long at = __ballot(lane < total && rank == slot);
+    const int e_slot = __builtin_amdgcn_readlane(e_mine, __ffsll(static_cast<long long>(at)) - 1);
+    if (!all) return e_slot;
     // slot k's key goes to lane k through the wave's own table; the selected experts' exponentials,
     // then their sum over the slots in order, in float32: the reference's order of additions
     if (lane < total && rank < n_used) s_sel[wave][rank] = mine;
@@ -582,6 +599,7 @@ __device__ __forceinline__ void route_block256(const float *lg, int n_expert, in
     }
     if (lane == 63) sel_w[n_used] = shared_gate ? sigmoid_exact(lsh * scale) : 0.f;
     __builtin_amdgcn_wave_barrier();  // the wave reads what it has written itself (all waves write the same)
+    return e_slot;
 }
 
 // ------------------------------------------------------------------------------- up ----------
@@ -609,22 +627,28 @@ __global__ __launch_bounds__(kBlock) void moe_up_kernel(shv_moe_up_args a, int s
     const int gi = lane % LPR, rsub = lane / LPR, sb = gi >> 2, g = gi & 3;
     const int row0 = (blockIdx.x * 4 + wave) * P * RPP + rsub;  // row within the expert, first pass
 
-    // the activation row is requested before anything else and staged further down
+    // the router's logits and the activation row are requested before anything else
+    const bool routed = a.logits && slot < a.n_used;
+    const float *lg = a.logits + static_cast<size_t>(t) * (a.n_expert + 1);
+    RouteLoads logits{0.f, 0.f, 0.f};
+    if (routed) logits.ask(lg, a.n_expert);
     const float *x = a.xn + static_cast<size_t>(t) * K;
     constexpr int NVr = NV >= 1 ? NV : 1;
+    // a whole number of float4s a thread needs no test around its loads
+    constexpr bool WHOLE = K % (4 * kBlock) == 0;
     float4 xv[NVr];
     __shared__ float red[4];
 #pragma unroll
     for (int j = 0; j < NVr; j++) {
         const int c = 4 * (tid + kBlock * j);
-        xv[j] = c < K ? *reinterpret_cast<const float4 *>(x + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+        xv[j] = WHOLE || c < K ? *reinterpret_cast<const float4 *>(x + c) : make_float4(0.f, 0.f, 0.f, 0.f);
     }
     if constexpr (NORM) {
         float4 gm[NVr];
 #pragma unroll
         for (int j = 0; j < NVr; j++) {
             const int c = 4 * (tid + kBlock * j);
-            gm[j] = c < K ? *reinterpret_cast<const float4 *>(a.gamma + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+            gm[j] = WHOLE || c < K ? *reinterpret_cast<const float4 *>(a.gamma + c) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
         float ss = 0.f;
 #pragma unroll
@@ -645,7 +669,7 @@ __global__ __launch_bounds__(kBlock) void moe_up_kernel(shv_moe_up_args a, int s
 #pragma unroll
             for (int j = 0; j < NVr; j++) {
                 const int c = 4 * (tid + kBlock * j);
-                const float4 sg = c < K ? *reinterpret_cast<const float4 *>(a.shared_gate + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+                const float4 sg = WHOLE || c < K ? *reinterpret_cast<const float4 *>(a.shared_gate + c) : make_float4(0.f, 0.f, 0.f, 0.f);
                 dot = fmaf(sg.x, xv[j].x, fmaf(sg.y, xv[j].y, fmaf(sg.z, xv[j].z, fmaf(sg.w, xv[j].w, dot))));
             }
             dot = wave_sum_all(dot);
@@ -654,11 +678,13 @@ __global__ __launch_bounds__(kBlock) void moe_up_kernel(shv_moe_up_args a, int s
     }
 
     // the shared expert's blocks need no selection (the block that stores it is a routed slot's)
-    if (a.logits && slot < a.n_used) {
+    int e_routed = 0;
+    if (routed) {
         // route this block's token from the router's logits, all four waves together
-        const float *lg = a.logits + static_cast<size_t>(t) * (a.n_expert + 1);
-        route_block256<NORM>(lg, a.n_expert, a.n_used, a.no_shared_gate == 0 && !(NORM && a.shared_gate), s_topk, s_w, probs, red, 1.f / static_cast<float>(K), a.eps);
-        if (blockIdx.x == 0 && blockIdx.y == 0) {
+        const bool stores = blockIdx.x == 0 && blockIdx.y == 0;
+        e_routed = route_block256<NORM>(logits, lg, a.n_expert, a.n_used, a.no_shared_gate == 0 && !(NORM && a.shared_gate), slot, stores, s_topk, s_w, probs, red,
+                                        1.f / static_cast<float>(K), a.eps);
+        if (stores) {
             if (tid < a.n_used) a.topk[static_cast<size_t>(t) * a.n_used + tid] = s_topk[tid];
             if (tid < a.n_used + ((NORM && a.shared_gate) ? 0 : 1)) a.weights[static_cast<size_t>(t) * (a.n_used + 1) + tid] = s_w[tid];
         }
@@ -668,7 +694,7 @@ __global__ __launch_bounds__(kBlock) void moe_up_kernel(shv_moe_up_args a, int s
     const char *gbase, *ubase;
     if (slot < a.n_used) {
         int e;
-        if (a.logits) e = min(max(s_topk[slot], 0), a.n_expert - 1);  // whatever the selection gave, the address stays inside the bank
+        if (a.logits) e = min(max(e_routed, 0), a.n_expert - 1);  // whatever the selection gave, the address stays inside the bank
         else e = a.topk[static_cast<size_t>(t) * a.n_used + slot];
         gbase = static_cast<const char *>(a.gate_exps) + static_cast<size_t>(e) * a.ffn * ROWB;
         ubase = static_cast<const char *>(a.up_exps) + static_cast<size_t>(e) * a.ffn * ROWB;
@@ -686,7 +712,7 @@ __global__ __launch_bounds__(kBlock) void moe_up_kernel(shv_moe_up_args a, int s
 #pragma unroll
     for (int j = 0; j < NVr; j++) {
         const int c = 4 * (tid + kBlock * j);
-        if (c < K) {
+        if (WHOLE || c < K) {
             *reinterpret_cast<float4 *>(&xs[lds_slot(c)]) = xv[j];
             const float s8 = sum8_all((xv[j].x + xv[j].y) + (xv[j].z + xv[j].w));
             if ((lane & 7) == 0) xsum[c >> 5] = s8;
@@ -869,13 +895,15 @@ __global__ __launch_bounds__(768) void moe_down_slots_kernel(shv_moe_down_args a
     const int t = blockIdx.y, s = s_lo + wave, ns = a.n_used + 1;
     const int gi = lane % LPR, rsub = lane / LPR, sb = gi >> 2, g = gi & 3;
     const int row0 = blockIdx.x * P * RPP + rsub;
-    // this slot's activations, then its expert and weight (scalar loads), then the weights
+    // this slot's expert, which its weights' loads wait for, its activations, its weight, then the weights
+    int32_t e = 0;
+    if (s < a.n_used) e = load_in_turn(a.topk + static_cast<size_t>(t) * a.n_used + s);
     const float *act = a.act + (static_cast<size_t>(t) * ns + s) * K;
     float4 av[NV];
 #pragma unroll
     for (int j = 0; j < NV; j++) av[j] = *reinterpret_cast<const float4 *>(act + 4 * (lane + 64 * j));
     const char *base = static_cast<const char *>(a.down_sh);
-    if (s < a.n_used) base = static_cast<const char *>(a.down_exps) + static_cast<size_t>(a.topk[static_cast<size_t>(t) * a.n_used + s]) * a.n_embd * ROWB;
+    if (s < a.n_used) base = static_cast<const char *>(a.down_exps) + static_cast<size_t>(__builtin_amdgcn_readfirstlane(e)) * a.n_embd * ROWB;
     const float wt = a.weights[static_cast<size_t>(t) * ns + s];
     Q4kLane w[P];
 #pragma unroll

@@ -244,6 +244,15 @@ struct Q4kLane {
     }
 };
 
+// *p, the same for every lane, by a vector load: it takes its place in the order of the loads around it and is waited for where
+// it is used.  By a scalar load, which is what the compiler makes of it, the wave stands still from the next scalar it needs.
+template <typename T>
+__device__ __forceinline__ T load_in_turn(const T *p) {
+    int32_t zero = 0;
+    asm("" : "+v"(zero));  // (a volatile one would keep every later load from being a scalar one)
+    return p[zero];
+}
+
 // ---- handing results from many blocks to the last one to finish ---------------------------------
 // The L2 caches of the chip's eight dies are not coherent with one another, and a device-scope
 // release or acquire fence pays for that by writing back and invalidating a whole L2 — tens of
