@@ -8,14 +8,18 @@
 //   products   v_mfma_f32_16x16x32_f16, activations x weights: a lane holds one weight row (its scales, its d); the
 //              activations as two binary16 parts, the weights as the whole numbers n * sc, exact in binary16, one
 //              accumulator a super-block
-//   min term   per super-block one v_mfma_f32_16x16x16_f16 a part of the sub-blocks' sums with the rows' mins
+//   min term   per super-block one v_mfma_f32_16x16x32_bf16 of the sub-blocks' sums with the rows' mins: a float32 sum is exactly
+//              three bfloat16 parts, and it leaves binary16's range long before one of its 32 activations does.  (Two
+//              v_mfma_f32_16x16x4_f32 of the sums as they are: 12352 x 2048 of 150 rows 30.2 us, of 512 rows 78.9.)
 // Up to 64 rows the weights' way through memory and the two launches bound it; from there the fragments' way from L2: 128 KB
 // a tile and block of 64 weight rows go at 31 bytes a clock and compute unit (1.7 us a tile), whatever their number in
 // flight, where the products alone would take half of that.  More rows a block would need more registers than there are:
 // 64 rows of 2048 columns, formed, are 256 of a compute unit's 512 KB, and forming them again for each tile costs what it saves.
-// us, with the staging launch, against the launches of 16, of 64 rows and their joins before (n x k, rows):
-//   12352 x 2048   9: 20.3 -> 11.8   16: 24.6 -> 11.2   64: 29.9 -> 17.9   150: 69.1 -> 31   255: 49.0 -> 44   512: 90 -> 76
-//    2048 x 4096   9: 16.0 -> 10.9   16: 16.5 -> 10.7   64: 22.3 -> 13.3   150: 51.5 -> 22.7   255: 59.7 -> 26   512: 65 -> 40
+// us, with the staging launch, two dozen matrices in turn (n x k, rows), and what the launches of 16, of 64 rows and their joins
+// took that this kernel has replaced:
+//   12352 x 2048   9: 20.3, now 9.7   16: 24.6, 9.9   150: 69.1, 28.2   255: 49.0, 40.5   512: 90, 72.5
+//    2048 x 4096   9: 16.0, now 8.4   16: 16.5, 8.4   150: 51.5, 18.6   255: 59.7, 23.5   512: 65, 37.1
+// Error against float64 of 4096 x 2048 over normal activations: 0.4e-6; of the kernels of 16 and of 64 rows 2.1e-6.
 #include <atomic>
 #include "gemm_rows.hpp"
 #include "moe_staged.hpp"
@@ -28,9 +32,9 @@ using namespace shv_moe;
 
 // The staged activations of a pass: fragments [tile of 16 rows][super-block][v][part] of 1 KB, v = nibble half * 4 + block of
 // 8 columns: lane (row n, group kb) holds columns 64 kb + 32 half + 8 block .. + 7 of the super-block, in the order a
-// payload dword's nibbles come; then the sub-blocks' sums [tile][super-block][part] of 256 bytes: lane (n, kb) those of
-// sub-blocks 2 kb, 2 kb + 1; then where each row's outputs go (a ring's row takes divisions and two loads to find).
-constexpr int kMidFrag = 1024, kMidSb = 16 * kMidFrag, kMidSums = 2 * 256;
+// payload dword's nibbles come; then the sub-blocks' sums [tile][super-block] of 1 KB: lane (n, kb) those of sub-blocks
+// 2 kb and 2 kb + 1, first parts, second, third, two zeros; then where each row's outputs go (a ring's row takes divisions and two loads to find).
+constexpr int kMidFrag = 1024, kMidSb = 16 * kMidFrag, kMidSums = 64 * 16;
 __host__ __device__ constexpr size_t mid_sums_offset(int tiles, int k) { return static_cast<size_t>(tiles) * (k / 256) * kMidSb; }
 __host__ __device__ constexpr size_t mid_rows_offset(int tiles, int k) { return mid_sums_offset(tiles, k) + static_cast<size_t>(tiles) * (k / 256) * kMidSums; }
 __host__ __device__ constexpr size_t mid_bytes(int tiles, int k) { return mid_rows_offset(tiles, k) + static_cast<size_t>(tiles) * 16 * sizeof(size_t); }
@@ -62,10 +66,9 @@ __global__ __launch_bounds__(256) void gemm_mid_stage_kernel(shv_gemv_q4k_args a
         const int sub = c >> 5, kb = sub >> 1, v = (sub & 1) * 4 + ((c & 31) >> 3);
         const size_t at = static_cast<size_t>(blockIdx.z) * (K / 256) + sb;
         if ((c & 31) == 0) {
-            const _Float16 hi = static_cast<_Float16>(sum);
-            _Float16 *sp = reinterpret_cast<_Float16 *>(staged + mid_sums_offset(tiles, K) + at * kMidSums + (kb * 16 + n) * 4) + (sub & 1);
-            sp[0] = hi;
-            sp[128] = static_cast<_Float16>(sum - static_cast<float>(hi));
+            uint16_t *sp = reinterpret_cast<uint16_t *>(staged + mid_sums_offset(tiles, K) + at * kMidSums + (kb * 16 + n) * 16) + (sub & 1);
+            bf16_parts(sum, sp[0], sp[2], sp[4]);
+            sp[6] = 0;
         }
         const float o[4] = {x[0], x[2], x[1], x[3]};
         half4_t h, l;
@@ -115,23 +118,21 @@ __global__ __launch_bounds__(64 * W) void gemm_mid_kernel(shv_gemv_q4k_args a, c
         }
     }
     const char *frag = staged + (static_cast<size_t>(tile0) * SBS + wave * S) * kMidSb + lane * 16;
-    const char *sums = staged + mid_sums_offset(tiles, a.k) + (static_cast<size_t>(tile0) * SBS + wave * S) * kMidSums + lane * 4;
+    const char *sums = staged + mid_sums_offset(tiles, a.k) + (static_cast<size_t>(tile0) * SBS + wave * S) * kMidSums + lane * 16;
     constexpr int D = 4;  // fetches held; eight are no faster
     auto ask = [&](const char *fp, int i, half8_t (&f)[2]) {
 #pragma unroll
         for (int p = 0; p < 2; p++) f[p] = *reinterpret_cast<const half8_t *>(fp + (i * 2 + p) * kMidFrag);
     };
     half8_t f[D][2];
-    uint32_t sx[S][2];
+    bf16x8_t sx[S];
 #pragma unroll
     for (int i = 0; i < D - 1; i++) ask(frag, i, f[i]);
 #pragma unroll
-    for (int s = 0; s < S; s++)
-#pragma unroll
-        for (int p = 0; p < 2; p++) sx[s][p] = *reinterpret_cast<const uint32_t *>(sums + s * kMidSums + p * 256);
+    for (int s = 0; s < S; s++) sx[s] = *reinterpret_cast<const bf16x8_t *>(sums + s * kMidSums);
     // n * sc of the wave's columns, held for every tile of the chunk
     half8_t wt[S][R][8];
-    half4_t am[S][R];
+    uint32_t am[S][R];
     float d[S][R], dmin[S][R];
 #pragma unroll
     for (int s = 0; s < S; s++)
@@ -145,8 +146,7 @@ __global__ __launch_bounds__(64 * W) void gemm_mid_kernel(shv_gemv_q4k_args a, c
                 const uint32_t d0 = (v & 1) ? x.z : x.x, d1 = (v & 1) ? x.w : x.y;
                 wt[s][r][v] = v < 4 ? weights8<false>(d0, d1, sc & 0xFFu, nc) : weights8<true>(d0, d1, sc >> 8, nc);
             }
-            am[s][r] = half4_t{static_cast<_Float16>(static_cast<float>(mn & 0xFFu)), static_cast<_Float16>(static_cast<float>(mn >> 8)),
-                               static_cast<_Float16>(0.f), static_cast<_Float16>(0.f)};
+            am[s][r] = bf16_pair(mn & 0xFFu, mn >> 8);
             d[s][r] = f16_bits_to_f32(hdr[s][r].x);
             dmin[s][r] = f16_bits_to_f32(hdr[s][r].x >> 16);
         }
@@ -171,7 +171,7 @@ __global__ __launch_bounds__(64 * W) void gemm_mid_kernel(shv_gemv_q4k_args a, c
         const char *fnext = more ? frag + SBS * kMidSb : frag, *snext = more ? sums + SBS * kMidSums : sums;
         find(tile);  // asked for here, needed at the tile's end
         float4_t y[R];
-        uint32_t sn[S][2];
+        bf16x8_t sn[S];
 #pragma unroll
         for (int s = 0; s < S; s++) {
             float4_t acc[R];
@@ -184,9 +184,7 @@ __global__ __launch_bounds__(64 * W) void gemm_mid_kernel(shv_gemv_q4k_args a, c
                 else ask(fnext, to - S * 8, f[to % D]);
                 if (to == S * 8) {
 #pragma unroll
-                    for (int s2 = 0; s2 < S; s2++)
-#pragma unroll
-                        for (int p = 0; p < 2; p++) sn[s2][p] = *reinterpret_cast<const uint32_t *>(snext + s2 * kMidSums + p * 256);
+                    for (int s2 = 0; s2 < S; s2++) sn[s2] = *reinterpret_cast<const bf16x8_t *>(snext + s2 * kMidSums);
                 }
                 __builtin_amdgcn_sched_barrier(0);  // the fragments stay ahead of their use
 #pragma unroll
@@ -197,13 +195,8 @@ __global__ __launch_bounds__(64 * W) void gemm_mid_kernel(shv_gemv_q4k_args a, c
             // the super-block ends: its sums take the row's d, its mins the row's dmin
 #pragma unroll
             for (int r = 0; r < R; r++) {
-                float4_t cm = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int p = 0; p < 2; p++) {
-                    const half2_t s2 = __builtin_bit_cast(half2_t, sx[s][p]);
-                    const half4_t bs = {s2[0], s2[1], static_cast<_Float16>(0.f), static_cast<_Float16>(0.f)};
-                    cm = __builtin_amdgcn_mfma_f32_16x16x16f16(bs, am[s][r], cm, 0, 0, 0);
-                }
+                const u32x4_t m3 = {am[s][r], am[s][r], am[s][r], 0u};  // the same two mins against each part
+                const float4_t cm = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sx[s], __builtin_bit_cast(bf16x8_t, m3), float4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
                     const float m = -dmin[s][r] * cm[j];
@@ -213,9 +206,7 @@ __global__ __launch_bounds__(64 * W) void gemm_mid_kernel(shv_gemv_q4k_args a, c
         }
         frag = fnext; sums = snext;
 #pragma unroll
-        for (int s = 0; s < S; s++)
-#pragma unroll
-            for (int p = 0; p < 2; p++) sx[s][p] = sn[s][p];
+        for (int s = 0; s < S; s++) sx[s] = sn[s];
         // ---- the waves' columns meet: every lane adds up its share of the tile in wave order ----
         float *cp = cpart + buf * (W * R * 256);
 #pragma unroll
@@ -348,9 +339,9 @@ int launch_stage(shv_ctx *ctx, const shv_gemv_q4k_args &a, int tiles, float *x_o
 }  // namespace
 
 // From nine rows, where the kernels that form every weight once for up to eight of them end, to 512, but for 17 to 64, which
-// keep the kernel of one 64-row group: a prompt of that height is one pass whose routing (a token's tenth expert or its
-// eleventh) every token decoded after it carries on, and the fewer roundings of these sums would decide some of it otherwise
-// for 12 us a layer, once a prompt.  Past 512 the blocks
+// keep the kernel of one 64-row group.  That kernel is the slower there (12352 x 2048 of 64 rows 27.7 us, 17.9 here) and the less
+// exact (2.1e-6 against 0.4e-6): the line is one of results that stay what they were, since a prompt of that height is one pass
+// whose routing, where a token's tenth expert and its eleventh are level, every token decoded after it carries on.  Past 512 the blocks
 // that share their activations through LDS have rows enough for every compute unit and read less from L2 (9216 x 2048 of
 // 1024 rows: 114 us there, 133 here; of 512: 75 there, 73 here).
 bool shv_gemm_mid_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a) {

@@ -40,7 +40,6 @@ constexpr int kRing = 2 * kChunk;  // a wave's LDS: a chunk being multiplied, th
 
 typedef const __attribute__((address_space(1))) void *global_ptr_t;
 typedef __attribute__((address_space(3))) void *lds_ptr_t;
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef const __attribute__((address_space(3))) char *lds_bytes_t;
 typedef const __attribute__((address_space(3))) u32x4_t *lds_quad_t;
 

@@ -13,6 +13,8 @@ typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kStSubBytes = 128;  // a row's sub-block: 2 parts x 4 column blocks x 16 bytes
 
@@ -47,6 +49,21 @@ __device__ __forceinline__ void stage_list_quad(const float4 v, int t, int c, in
         sp[0] = hi;
         sp[8] = static_cast<_Float16>(sum - static_cast<float>(hi));
     }
+}
+
+// v as the exact sum of three bfloat16 values (bit patterns): eight bits of it each, cut off, so that what is left is exact.
+__device__ __forceinline__ void bf16_parts(float v, uint16_t &p0, uint16_t &p1, uint16_t &p2) {
+    const uint32_t b0 = __float_as_uint(v);
+    const float r1 = v - __uint_as_float(b0 & 0xFFFF0000u);
+    const uint32_t b1 = __float_as_uint(r1);
+    const float r2 = r1 - __uint_as_float(b1 & 0xFFFF0000u);
+    p0 = static_cast<uint16_t>(b0 >> 16);
+    p1 = static_cast<uint16_t>(b1 >> 16);
+    p2 = static_cast<uint16_t>(__float_as_uint(r2) >> 16);
+}
+// Two whole numbers below 256 (a sub-block's min is below 64) as a pair of bfloat16 values, exact.
+__device__ __forceinline__ uint32_t bf16_pair(uint32_t a, uint32_t b) {
+    return (__float_as_uint(static_cast<float>(a)) >> 16) | (__float_as_uint(static_cast<float>(b)) & 0xFFFF0000u);
 }
 
 // The masks and exponents of the two nibble positions a weight is read from.

@@ -64,3 +64,27 @@ def test_router_logits_of_a_long_pass(rows, H, E):
         assert np.abs(got - want).max() <= 1e-6 * np.abs(want).max() * 4
     finally:
         ctx.destroy()
+
+
+@pytest.mark.parametrize("n,k,rows", [(96, 2048, 9), (2048, 4096, 16), (70, 2048, 65), (2048, 4096, 192), (300, 2048, 512)])
+def test_sums_past_binary16(n, k, rows):
+    """Every activation is a binary16 number, the sum of a sub-block's 32 is not (65504 is the largest): the min term's sums are
+    float32.  The bound is on what the two terms of a row add up, which cancel here: 16 ulp of float32, a fourth of what 64 roundings
+    in a row could make."""
+    rng = np.random.default_rng(n + rows)
+    ctx = A.Context(0)
+    try:
+        w = (rng.standard_normal((n, k)) * 0.02).astype(np.float32)
+        wq = O.quantize_q4k(w)
+        w64 = O.dequant_q4k(wq, k).astype(np.float64)
+        x = (rng.standard_normal((rows, k)) * 500.0 + 3000.0 * np.where(np.arange(rows) % 2, 1.0, -1.0)[:, None]).astype(np.float32)
+        x[rows // 2] *= 1e-4  # and a row of ordinary size among them
+        assert np.abs(x.reshape(rows, -1, 32).sum(axis=2)).max() > 65504 and np.abs(x).max() < 65504
+        dy = ctx.alloc(rows * n * 4)
+        ctx.gemv_q4k(ctx.upload(wq), ctx.upload(x), dy, n, k, n_tok=rows)
+        got, x64 = dy.read(np.float32, rows * n).reshape(rows, n), x.astype(np.float64)
+        size = np.abs(x64) @ (np.abs(w64) + 2 * np.abs(w64).max(axis=1, keepdims=True)).T
+        assert np.isfinite(got).all()
+        assert (np.abs(got - x64 @ w64.T) <= 2.0 ** -20 * size).all()
+    finally:
+        ctx.destroy()
