@@ -1006,8 +1006,9 @@ bool shapes_covered(const shv_ctx *ctx, int n_tok, int n_embd, int ffn, int n_us
 // repeat, the shapes the kernels are built for, and a selection that is already made (topk from
 // the router).  The launchers in moe.hip have checked that every bank is Q4_K.
 bool shv_moe_up_grouped_covers(const shv_ctx *ctx, const shv_moe_up_args &a) {
+    const bool lists = shv_moe_list_tokens(a.n_tok, a.n_used, a.n_expert) > 0;
     return a.group && !a.logits && shv_aligned16(a.xn) && shapes_covered(ctx, a.n_tok, a.n_embd, a.ffn, a.n_used, a.n_expert) && ctx->gemm_stage &&
-           staged_bytes(a.n_tok, a.n_embd) <= static_cast<size_t>(shv_ctx::kGemmStageBytes);
+           (lists ? list_bytes(a.n_tok, a.n_embd) : staged_bytes(a.n_tok, a.n_embd)) <= static_cast<size_t>(shv_ctx::kGemmStageBytes);
 }
 
 bool shv_moe_down_grouped_covers(const shv_ctx *ctx, const shv_moe_down_args &a) {
@@ -1017,9 +1018,11 @@ bool shv_moe_down_grouped_covers(const shv_ctx *ctx, const shv_moe_down_args &a)
 // Lists, the rows as operands, then the grouped gate/up products.
 int shv_launch_moe_up_grouped(shv_ctx *ctx, const shv_moe_up_args &a) {
     // refused before anything is enqueued: an error return leaves no half pass on the stream
-    SHV_REQUIRE(!a.act_packed || (ctx->gemm_part && packed_sums_bytes(static_cast<long long>(a.n_tok) * (a.n_used + 1), a.ffn) <= static_cast<size_t>(shv_ctx::kGemmPartBytes)),
+    const bool short_lists = shv_moe_list_tokens(a.n_tok, a.n_used, a.n_expert) > 0;
+    const long long n_pairs = static_cast<long long>(a.n_tok) * (a.n_used + 1);
+    SHV_REQUIRE(!a.act_packed || (ctx->gemm_part && (short_lists ? list_act_bytes(n_pairs, a.ffn) : packed_sums_bytes(n_pairs, a.ffn)) <= static_cast<size_t>(shv_ctx::kGemmPartBytes)),
                 "moe_up: %d rows are too many for act_packed", a.n_tok);
-    if (shv_moe_list_tokens(a.n_tok, a.n_used, a.n_expert) > 0) {
+    if (short_lists) {
         // short lists: streamed, wave by wave
         if (const int rc = launch_group(ctx, a.topk, a.n_tok, a.n_used, a.n_expert, a.group, a.xn, a.n_embd); rc != SHV_OK) return rc;
         ctx->moe_stamp = {a.topk, a.group, a.act, a.n_tok, a.n_used, true, a.act_packed != 0};

@@ -9,8 +9,8 @@
 //                 token rows; the weights are the whole numbers n * sc, exact in binary16, one accumulator a super-block
 //   up to eight tokens: the high and the low parts of a token are two rows of ONE operand (a product for both parts,
 //                 the halves of a result in neighbouring registers of a lane); nine to sixteen: an operand for each part
-//   min term    = per super-block one v_mfma_f32_16x16x16_f16 of the sub-blocks' sums of x (as two halves) with the rows'
-//                 mins (whole numbers), times the row's dmin
+//   min term    = per super-block one v_mfma_f32_16x16x16_bf16 a part of the sub-blocks' sums of x (float32 values, each
+//                 exactly three bfloat16 ones) with the rows' mins (whole numbers), times the row's dmin
 // Gate/up of a 150-row pass 217 -> 131 us (4.4 TB/s), down 115 -> 64.  The chunks' loads alone take 100 us of the 131, the
 // arithmetic alone 87; two waves a SIMD hide most of one under the other.  The same waves as a persistent walk over a work
 // list, the next unit's loads behind the last one's products, measured the same (the waits are not at a unit's ends).
@@ -38,6 +38,7 @@ constexpr int kDownUnits = 4;  // 64-row units of the down projection a wave tak
 constexpr int kChunk = 9 * 1024;
 constexpr int kRing = 2 * kChunk;  // a wave's LDS: a chunk being multiplied, the next on its way
 
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 typedef const __attribute__((address_space(1))) void *global_ptr_t;
 typedef __attribute__((address_space(3))) void *lds_ptr_t;
 typedef const __attribute__((address_space(3))) char *lds_bytes_t;
@@ -96,7 +97,7 @@ __device__ __forceinline__ void stream_tiles(const char *w0, const char *w1, int
     const int lane = threadIdx.x & 63, n = lane & 15, kb = lane >> 4;
     const NibbleMasks nc = nibble_masks();
     half8_t b[S][8][PARTS];
-    uint32_t sx[S][PARTS];
+    short4_t sx[S][PARTS];
     auto ask_tok = [&](int sb, int s) {
 #pragma unroll
         for (int v = 0; v < 8; v++)
@@ -104,7 +105,7 @@ __device__ __forceinline__ void stream_tiles(const char *w0, const char *w1, int
             for (int p = 0; p < PARTS; p++)
                 b[s][v][p] = *reinterpret_cast<const half8_t *>(staged + sb * (8 * kStSubBytes) + (tok + v * 128 + p * 64));
 #pragma unroll
-        for (int p = 0; p < PARTS; p++) sx[s][p] = *reinterpret_cast<const uint32_t *>(sums + sb * 32 + (sum + p * 16));
+        for (int p = 0; p < PARTS; p++) sx[s][p] = *reinterpret_cast<const short4_t *>(sums + sb * kListSumBytes + (sum + p * 32));
     };
     // where chunk c of a step begins: tiles TC c .. of the unit
     auto chunk_at = [&](int st, int c) {
@@ -161,15 +162,10 @@ __device__ __forceinline__ void stream_tiles(const char *w0, const char *w1, int
                             for (int p = 0; p < PARTS; p++) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[s][v][p], w8, acc, 0, 0, 0);
                         }
                         // the super-block ends: its sums take the row's d, its mins the row's dmin
-                        const half4_t am = {static_cast<_Float16>(static_cast<float>(mn & 0xFFu)), static_cast<_Float16>(static_cast<float>(mn >> 8)),
-                                            static_cast<_Float16>(0.f), static_cast<_Float16>(0.f)};
+                        const u32x2_t am = static_cast<u32x2_t>(bf16_pair(mn & 0xFFu, mn >> 8));
                         float4_t cm = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                        for (int p = 0; p < PARTS; p++) {
-                            const half2_t s2 = __builtin_bit_cast(half2_t, sx[s][p]);
-                            const half4_t bs = {s2[0], s2[1], static_cast<_Float16>(0.f), static_cast<_Float16>(0.f)};
-                            cm = __builtin_amdgcn_mfma_f32_16x16x16f16(bs, am, cm, 0, 0, 0);
-                        }
+                        for (int p = 0; p < PARTS; p++) cm = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(sx[s][p], __builtin_bit_cast(short4_t, am), cm, 0, 0, 0);
                         const float d = f16_bits_to_f32(hdr.x), dmin = f16_bits_to_f32(hdr.x >> 16);
 #pragma unroll
                         for (int j = 0; j < 4; j++) y[r][j] = fmaf(-dmin, cm[j], fmaf(d, acc[j], y[r][j]));
@@ -228,7 +224,7 @@ __device__ __forceinline__ void up_list_pass(const shv_moe_up_args &a, const cha
     const int t = pair / (a.n_used + 1);
     const int part = PARTS == 1 ? n & 1 : 0;
     const uint32_t tok = t * ((K / 32) * kStSubBytes) + kb * 16 + part * 64;
-    const uint32_t sum = t * (K / 256 * 32) + part * 16 + kb * 4;
+    const uint32_t sum = t * (K / 256 * kListSumBytes) + part * 32 + kb * 8;
     const int row = row0 + n, sub = row0 >> 5;
     // column n (and n + 16) of the sub-block: its slot of [0, 2, 1, 3, 4, 6, 5, 7]
     const int p8 = n & 7, slot = (p8 & 4) | ((p8 & 1) << 1) | ((p8 & 2) >> 1);
@@ -261,12 +257,7 @@ __device__ __forceinline__ void up_list_pass(const shv_moe_up_args &a, const cha
                     *reinterpret_cast<_Float16 *>(e + r * 256) = hi;
                     *reinterpret_cast<_Float16 *>(e + r * 256 + 64) = static_cast<_Float16>(v[r] - static_cast<float>(hi));
                 }
-                if (n == 0) {
-                    const _Float16 hi = static_cast<_Float16>(sum32);
-                    _Float16 *sp = reinterpret_cast<_Float16 *>(act_sums + (to * (a.ffn / 256) + (sub >> 3)) * 32) + (sub & 7);
-                    sp[0] = hi;
-                    sp[8] = static_cast<_Float16>(sum32 - static_cast<float>(hi));
-                }
+                if (n == 0) list_sum_put(act_sums + (to * (a.ffn / 256) + (sub >> 3)) * kListSumBytes, sub, sum32);
             }
         }
     });
@@ -299,7 +290,7 @@ __device__ __forceinline__ void down_list_pass(const shv_moe_down_args &a, const
     const int pair = pair_at(u, t0, PARTS == 1 ? n >> 1 : n, m, a.n_used, a.n_expert, a.group);
     const int part = PARTS == 1 ? n & 1 : 0;
     const uint32_t tok = pair * ((K / 32) * kStSubBytes) + kb * 16 + part * 64;
-    const uint32_t sum = pair * (K / 256 * 32) + part * 16 + kb * 4;
+    const uint32_t sum = pair * (K / 256 * kListSumBytes) + part * 32 + kb * 8;
     stream_tiles<K, PARTS, 2>(base, base + 32 * ROWB, kDownUnits, 16 * kR * ROWB, ring, reinterpret_cast<const char *>(a.act), tok, act_sums, sum,
                               [&](int unit, const float4_t (&y)[kR]) {
         constexpr int NT = PARTS == 1 ? 2 : 4;

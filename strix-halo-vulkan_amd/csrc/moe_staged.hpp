@@ -3,7 +3,7 @@
 // A row of k columns is [sub-block of 32][part hi, lo][block of 8 columns] x 16 bytes, 128 bytes a sub-block, the eight
 // columns of a block in slot order [0, 2, 1, 3, 4, 6, 5, 7] (the order a payload dword's nibbles come out of the masks).
 // After all rows come their sums over the sub-blocks, as operands too: [row][super-block] x 32 bytes, the eight sums'
-// binary16 values and then what those leave.
+// binary16 values and then what those leave.  (The list kernels' sums are float32, in bfloat16 parts: list_sum_put.)
 #pragma once
 #include "shv_device.hpp"
 
@@ -11,6 +11,7 @@ namespace shv_moe {
 
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -24,9 +25,35 @@ __host__ __device__ constexpr size_t staged_bytes(int rows, int k) { return stag
 // own 4 * ffn bytes of act in the staged layout, and its sub-blocks' sums in the library's scratch.
 __host__ __device__ constexpr size_t packed_sums_bytes(long long pairs, int ffn) { return static_cast<size_t>(pairs) * (ffn / 256) * 32; }
 
+// v as the exact sum of three bfloat16 values (bit patterns): eight bits of it each, cut off, so that what is left is exact.
+__device__ __forceinline__ void bf16_parts(float v, uint16_t &p0, uint16_t &p1, uint16_t &p2) {
+    const uint32_t b0 = __float_as_uint(v);
+    const float r1 = v - __uint_as_float(b0 & 0xFFFF0000u);
+    const uint32_t b1 = __float_as_uint(r1);
+    const float r2 = r1 - __uint_as_float(b1 & 0xFFFF0000u);
+    p0 = static_cast<uint16_t>(b0 >> 16);
+    p1 = static_cast<uint16_t>(b1 >> 16);
+    p2 = static_cast<uint16_t>(__float_as_uint(r2) >> 16);
+}
+// Two whole numbers below 256 (a sub-block's min is below 64) as a pair of bfloat16 values, exact.
+__device__ __forceinline__ uint32_t bf16_pair(uint32_t a, uint32_t b) {
+    return (__float_as_uint(static_cast<float>(a)) >> 16) | (__float_as_uint(static_cast<float>(b)) & 0xFFFF0000u);
+}
+
 // Where the high part of columns 32 sub + 8 c .. + 7 lies in a row staged for the list kernels; its low part is 64 bytes on.
 // [super-block][low / high nibbles' sub-blocks][c][part][group]: what the lanes of one operand take of a token is a line.
 __host__ __device__ constexpr int list_block(int sub, int c) { return (sub >> 3) * 1024 + (sub & 1) * 512 + c * 128 + ((sub >> 1) & 3) * 16; }
+
+// The sums of a row staged for the list kernels: [super-block] x 64 bytes, [part 0, 1][group] x 8 bytes, the group's two
+// sub-blocks' first and second bfloat16 parts in part 0, their third in part 1 (and two zeros, which its owner writes).
+constexpr int kListSumBytes = 64;
+__host__ __device__ constexpr size_t list_bytes(int rows, int k) { return staged_sums_offset(rows, k) + static_cast<size_t>(rows) * (k / 256) * kListSumBytes; }
+__host__ __device__ constexpr size_t list_act_bytes(long long pairs, int ffn) { return static_cast<size_t>(pairs) * (ffn / 256) * kListSumBytes; }
+__device__ __forceinline__ void list_sum_put(char *sb_sums, int sub, float sum) {
+    uint16_t *p = reinterpret_cast<uint16_t *>(sb_sums + ((sub >> 1) & 3) * 8) + (sub & 1);
+    bf16_parts(sum, p[0], p[2], p[16]);
+    p[18] = 0;
+}
 
 // Four columns c .. c + 3 of row t for the list kernels, and (the lane of a sub-block's first columns) the sub-block's sum;
 // the eight lanes of a sub-block are neighbours and all here.
@@ -43,27 +70,7 @@ __device__ __forceinline__ void stage_list_quad(const float4 v, int t, int c, in
     *reinterpret_cast<half4_t *>(e) = h;
     *reinterpret_cast<half4_t *>(e + 64) = l;
     const float sum = shv::sum8_all((v.x + v.y) + (v.z + v.w));
-    if ((c & 31) == 0) {
-        const _Float16 hi = static_cast<_Float16>(sum);
-        _Float16 *sp = reinterpret_cast<_Float16 *>(staged + staged_sums_offset(rows, k) + (static_cast<size_t>(t) * (k / 256) + (c >> 8)) * 32) + ((c >> 5) & 7);
-        sp[0] = hi;
-        sp[8] = static_cast<_Float16>(sum - static_cast<float>(hi));
-    }
-}
-
-// v as the exact sum of three bfloat16 values (bit patterns): eight bits of it each, cut off, so that what is left is exact.
-__device__ __forceinline__ void bf16_parts(float v, uint16_t &p0, uint16_t &p1, uint16_t &p2) {
-    const uint32_t b0 = __float_as_uint(v);
-    const float r1 = v - __uint_as_float(b0 & 0xFFFF0000u);
-    const uint32_t b1 = __float_as_uint(r1);
-    const float r2 = r1 - __uint_as_float(b1 & 0xFFFF0000u);
-    p0 = static_cast<uint16_t>(b0 >> 16);
-    p1 = static_cast<uint16_t>(b1 >> 16);
-    p2 = static_cast<uint16_t>(__float_as_uint(r2) >> 16);
-}
-// Two whole numbers below 256 (a sub-block's min is below 64) as a pair of bfloat16 values, exact.
-__device__ __forceinline__ uint32_t bf16_pair(uint32_t a, uint32_t b) {
-    return (__float_as_uint(static_cast<float>(a)) >> 16) | (__float_as_uint(static_cast<float>(b)) & 0xFFFF0000u);
+    if ((c & 31) == 0) list_sum_put(staged + staged_sums_offset(rows, k) + (static_cast<size_t>(t) * (k / 256) + (c >> 8)) * kListSumBytes, c >> 5, sum);
 }
 
 // The masks and exponents of the two nibble positions a weight is read from.

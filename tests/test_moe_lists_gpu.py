@@ -1,8 +1,9 @@
 """The expert kernels that stream short per-expert lists (csrc/moe_lists.hip) against the per-(token, slot) kernels, on lists
-whose lengths are the edges of what a wave takes at a time."""
+whose lengths are the edges of what a wave takes at a time, and against float64 where activations or their sums leave binary16."""
 import numpy as np
 import pytest
 
+import oracle_lib as O
 import shv
 
 pytestmark = pytest.mark.gpu
@@ -80,3 +81,45 @@ def test_lists_are_the_slots(rig, lengths, used, packed):
     rel = np.linalg.norm(got - want) / np.linalg.norm(want)
     assert rel <= 1e-5, (topk.shape, rel)
     assert np.max(np.abs(got - want)) <= 1e-4 * np.sqrt(np.mean(want ** 2))
+
+
+LENGTHS = [0, 1, 2, 7, 8, 9, 6, 0] + [2] * 16  # 65 tokens of one expert each, eight listed tokens a time
+SIXTEENS = [0, 1, 8, 9, 15, 16, 17, 7] + [8] * 15 + [9]  # 202 tokens, sixteen a time
+
+
+def expert_rows(rig, bank, e, rows, k):
+    raw = rig[3][bank].read(np.uint8, rows * k // 256 * 144, e * rows * k // 256 * 144)
+    return O.dequant_q4k(raw, k).reshape(rows, k).astype(np.float64)
+
+
+def up64(x, gate, up):
+    """SwiGLU of a token's gate and up products, and what rounding them once in 2^20 of their terms' sizes makes of it."""
+    g, u = x @ gate.T, x @ up.T
+    size = lambda w: np.abs(x) @ (np.abs(w) + 2 * np.abs(w).max(axis=1, keepdims=True)).T
+    sig = 1 / (1 + np.exp(-np.clip(g, -700, 700)))
+    return g * sig * u, 2.0 ** -20 * (size(gate) * np.abs(u) * 1.1 + size(up) * np.abs(g) * sig)  # |d silu| <= 1.1
+
+
+@pytest.mark.parametrize("lengths", [LENGTHS, SIXTEENS])
+def test_sums_past_binary16(rig, lengths):
+    """Activations are binary16 numbers, a sub-block's sum of 32 is not: the min term's sums are float32."""
+    c, E, _, banks = rig
+    rng = np.random.default_rng(3)
+    topk = selection(lengths, 1, rng)
+    T = len(topk)
+    xn = (rng.standard_normal((T, H)) * 500 + 3000 * np.where(np.arange(T) % 2, 1, -1)[:, None]).astype(np.float32)
+    xn[T // 3] *= 1e-4
+    bufs = [c.upload(a) for a in (xn, topk)]
+    act, group = c.alloc(T * 2 * F * 4), c.alloc((2 * E + 1 + T) * 4)
+    ua = A.MoeUpArgs(bufs[0].ptr, bufs[1].ptr, banks[0].ptr, banks[1].ptr, banks[3].ptr, banks[4].ptr, act.ptr, T, H, 1, F, None, None, E, 0, 0, 0, 0, group.ptr, 0, 0)
+    c.dispatch_multi([A.make_op(A.OP_MOE_UP, ua)])
+    got = act.read(np.float32, T * 2 * F).reshape(T, 2, F)
+    for b in bufs + [act, group]:
+        b.free()
+    assert np.isfinite(got).all()
+    for e in range(1, 7):
+        at = np.flatnonzero(topk[:, 0] == e)
+        want, tol = up64(xn[at].astype(np.float64), expert_rows(rig, 0, e, F, H), expert_rows(rig, 1, e, F, H))
+        assert (np.abs(got[at, 0] - want) <= tol).all(), e
+    want, tol = up64(xn.astype(np.float64), expert_rows(rig, 3, 0, F, H), expert_rows(rig, 4, 0, F, H))
+    assert (np.abs(got[:, 1] - want) <= tol).all()
