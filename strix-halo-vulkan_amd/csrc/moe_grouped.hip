@@ -140,14 +140,25 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int32_t *topk, in
 // counts (an expert's total, and what the blocks before it hold of it), forms the starts, and places its own pairs
 // behind those of the blocks before it; block 0 also writes the starts and the experts' launch order.
 constexpr int kGroupBlocks = 16;
-// Blocks past the counting ones, when the launch has them, stage the rows x [rows][k] for the list kernels meanwhile.
+// Blocks past the counting ones, when the launch has them, stage the rows x [rows][k] for the list kernels meanwhile: whole
+// rows, k / 256 of a block's sixteen waves each.
 __global__ __launch_bounds__(1024) void moe_group_count_kernel(const int32_t *topk, int n_pairs, int chunk, int n_expert, int32_t *counts, const float *x, int rows, int k,
                                                                char *staged) {
     __shared__ int32_t s_cnt[kMaxExperts];
     const int tid = threadIdx.x;
     if (blockIdx.x >= kGroupBlocks) {
-        const int quad = (blockIdx.x - kGroupBlocks) * 1024 + tid, t = quad / (k / 4), c = (quad % (k / 4)) * 4;
-        if (t < rows) stage_list_quad(*reinterpret_cast<const float4 *>(x + static_cast<size_t>(t) * k + c), t, c, k, rows, staged);
+        __shared__ float s_max[16];
+        const int quad = (blockIdx.x - kGroupBlocks) * 1024 + tid, t = quad / (k / 4), c = (quad % (k / 4)) * 4, per = k / 256;
+        const float4 v = t < rows ? *reinterpret_cast<const float4 *>(x + static_cast<size_t>(t) * k + c) : float4{0.f, 0.f, 0.f, 0.f};
+        float largest = wave_max_all(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+        if ((tid & 63) == 0) s_max[tid >> 6] = largest;
+        __syncthreads();
+        for (int w = 0, w0 = (tid >> 6) / per * per; w < per; w++) largest = fmaxf(largest, s_max[w0 + w]);
+        const int e = biased_exponent(largest);
+        if (t < rows) {
+            stage_list_quad(v, e, t, c, k, rows, staged);
+            if (c == 0) reinterpret_cast<int32_t *>(staged + list_exps_offset(rows, k))[t] = e;
+        }
         return;
     }
     for (int e = tid; e < n_expert; e += 1024) s_cnt[e] = 0;
@@ -1012,6 +1023,8 @@ bool shv_moe_up_grouped_covers(const shv_ctx *ctx, const shv_moe_up_args &a) {
 }
 
 bool shv_moe_down_grouped_covers(const shv_ctx *ctx, const shv_moe_down_args &a) {
+    // (act as floats, rows that used to go slot by slot: they still do, in float32)
+    if (!a.act_packed && a.n_tok < 128 && !ctx->moe_group_forced) return false;
     return a.group && a.pairs && shv_aligned16(a.act) && shv_aligned16(a.pairs) && shapes_covered(ctx, a.n_tok, a.n_embd, a.ffn, a.n_used, a.n_expert);
 }
 

@@ -7,6 +7,11 @@
 //                 into its own LDS a chunk ahead of the products, the tokens' operands come to registers; no barrier
 //   products    = v_mfma_f32_16x16x32_f16, tokens x weights: a lane holds one weight row (its scales, its d) and four
 //                 token rows; the weights are the whole numbers n * sc, exact in binary16, one accumulator a super-block
+//   operands    = a token's values scaled by a power of two, as two binary16 parts (binary16_parts); what a token's products
+//                 come to is scaled back where they leave.  A token's own row has one exponent, known when it is staged; a
+//                 SwiGLU row is written by sixteen waves that know their sub-block's alone, and the waves that read it bring
+//                 its sub-blocks to the row's largest, 2^-k being exact.  Error of a layer's outputs against float64, whatever
+//                 the activations' size: 0.5e-6 to 0.7e-6 (slot by slot 4.2e-6; without the exponents 240e-6 at xn of 0.02)
 //   up to eight tokens: the high and the low parts of a token are two rows of ONE operand (a product for both parts,
 //                 the halves of a result in neighbouring registers of a lane); nine to sixteen: an operand for each part
 //   min term    = per super-block one v_mfma_f32_16x16x16_bf16 a part of the sub-blocks' sums of x (float32 values, each
@@ -14,6 +19,8 @@
 // Gate/up of a 150-row pass 217 -> 131 us (4.4 TB/s), down 115 -> 64.  The chunks' loads alone take 100 us of the 131, the
 // arithmetic alone 87; two waves a SIMD hide most of one under the other.  The same waves as a persistent walk over a work
 // list, the next unit's loads behind the last one's products, measured the same (the waits are not at a unit's ends).
+#include <type_traits>
+
 #include "moe_staged.hpp"
 #include "shv_internal.hpp"
 
@@ -81,16 +88,19 @@ struct TileSb {
     }
 };
 
+struct AsStaged {};
+
 // A wave's share of one expert: row tiles of K columns against the tokens whose operands the lane reads at tok (and sums
 // at sum).  A unit is four tiles, w0 and w1 the first rows of its two pairs (the same in every lane); `units` of them
 // follow one another unit_bytes apart.  done(unit, y) takes a unit's sums: y[r][j] of lane (n, kb) is weight row n of
 // tile r against operand row 4 kb + j.
+// settle(b, sx) brings operands that are not all of one exponent to one, when they have come (AsStaged: they are).
 // PARTS 1: operand row 2 t + p is part p of token t (up to eight); PARTS 2: operand row t, parts one after the other.
 // A lane (n, kb) of a tile takes group kb of row n's super-blocks, so one decode of the header serves a super-block.  The
 // tokens' operands of S super-blocks stay in registers over the chunks that meet them.
-template <int K, int PARTS, int S, typename Done>
+template <int K, int PARTS, int S, typename Settle, typename Done>
 __device__ __forceinline__ void stream_tiles(const char *w0, const char *w1, int units, int unit_bytes, char *ring, const char *staged, uint32_t tok, const char *sums, uint32_t sum,
-                                             Done &&done) {
+                                             Settle &&settle, Done &&done) {
     constexpr int SBS = K / SHV_Q4K_BLOCK, ROWB = SBS * SHV_Q4K_BYTES, STEPS = SBS / S;
     constexpr int TC = 4 / S, CHUNKS = kR / TC;  // tiles a chunk, chunks a step
     static_assert((S == 2 || S == 4) && CHUNKS % 2 == 0, "chunk shape");
@@ -112,9 +122,22 @@ __device__ __forceinline__ void stream_tiles(const char *w0, const char *w1, int
         const char *w = c * TC >= 2 ? w1 : w0;
         return w + ((c * TC) & 1) * (16 * ROWB) + st * (S * SHV_Q4K_BYTES);
     };
-    ask_chunk<ROWB, S>(chunk_at(0, 0), ring, lane);
+    if constexpr (!std::is_same_v<Settle, AsStaged>) {
+        // the operands first, settled while the first chunk is on its way (with the second chunk asked for here as well the
+        // loop has a case more, and 51 registers of the sixteen-token kernel go to memory where 27 do)
+        static_assert(STEPS == 1, "operands that stay");
 #pragma unroll
-    for (int s = 0; s < S; s++) ask_tok(s, s);
+        for (int s = 0; s < S; s++) ask_tok(s, s);
+        __builtin_amdgcn_sched_barrier(0);
+        ask_chunk<ROWB, S>(chunk_at(0, 0), ring, lane);
+        __builtin_amdgcn_s_waitcnt(0x0F79);  // vmcnt(9)
+        __builtin_amdgcn_sched_barrier(0);
+        settle(b, sx);
+    } else {
+        ask_chunk<ROWB, S>(chunk_at(0, 0), ring, lane);
+#pragma unroll
+        for (int s = 0; s < S; s++) ask_tok(s, s);
+    }
     float4_t y[kR];
 #pragma unroll 1
     for (int u = 0; u < units; u++) {
@@ -225,19 +248,23 @@ __device__ __forceinline__ void up_list_pass(const shv_moe_up_args &a, const cha
     const int part = PARTS == 1 ? n & 1 : 0;
     const uint32_t tok = t * ((K / 32) * kStSubBytes) + kb * 16 + part * 64;
     const uint32_t sum = t * (K / 256 * kListSumBytes) + part * 32 + kb * 8;
+    const int exponent = reinterpret_cast<const int32_t *>(staged + list_exps_offset(a.n_tok, K))[t];
     const int row = row0 + n, sub = row0 >> 5;
+    uint8_t *act_exps = reinterpret_cast<uint8_t *>(act_sums + list_act_exps_offset(static_cast<long long>(a.n_tok) * (a.n_used + 1), a.ffn));
     // column n (and n + 16) of the sub-block: its slot of [0, 2, 1, 3, 4, 6, 5, 7]
     const int p8 = n & 7, slot = (p8 & 4) | ((p8 & 1) << 1) | ((p8 & 2) >> 1);
-    stream_tiles<K, PARTS, PARTS == 1 ? 4 : 2>(gate, up, 1, 0, ring, staged, tok, staged + staged_sums_offset(a.n_tok, K), sum, [&](int, const float4_t (&y)[kR]) {
+    stream_tiles<K, PARTS, PARTS == 1 ? 4 : 2>(gate, up, 1, 0, ring, staged, tok, staged + staged_sums_offset(a.n_tok, K), sum,
+                                                  AsStaged(), [&](int, const float4_t (&y)[kR]) {
         constexpr int NT = PARTS == 1 ? 2 : 4;  // tokens whose sums this lane holds
 #pragma unroll
         for (int j = 0; j < NT; j++) {
             const int i = NT * kb + j;
+            const int back = __shfl(exponent, PARTS == 1 ? 2 * i : i, 64) - kListOne;
             float v[2];
 #pragma unroll
             for (int r = 0; r < 2; r++) {
-                const float gv = PARTS == 1 ? y[r][2 * (j & 1)] + y[r][2 * (j & 1) + 1] : y[r][j];
-                const float uv = PARTS == 1 ? y[2 + r][2 * (j & 1)] + y[2 + r][2 * (j & 1) + 1] : y[2 + r][j];
+                const float gv = ldexpf(PARTS == 1 ? y[r][2 * (j & 1)] + y[r][2 * (j & 1) + 1] : y[r][j], back);
+                const float uv = ldexpf(PARTS == 1 ? y[2 + r][2 * (j & 1)] + y[2 + r][2 * (j & 1) + 1] : y[2 + r][j], back);
                 v[r] = gv * sigmoid_exact(gv) * uv;
             }
             const size_t to = static_cast<size_t>(__shfl(pair, PARTS == 1 ? 2 * i : i, 64));
@@ -249,14 +276,17 @@ __device__ __forceinline__ void up_list_pass(const shv_moe_up_args &a, const cha
                 continue;
             }
             const float sum32 = group_sum<16>(v[0] + v[1]);
+            const int e = biased_exponent(max16_all(fmaxf(fabsf(v[0]), fabsf(v[1]))));
             if (i < m) {
-                char *e = reinterpret_cast<char *>(a.act) + to * (a.ffn / 32) * kStSubBytes + list_block(sub, n >> 3) + slot * 2;
+                char *at = reinterpret_cast<char *>(a.act) + to * (a.ffn / 32) * kStSubBytes + list_block(sub, n >> 3) + slot * 2;
 #pragma unroll
                 for (int r = 0; r < 2; r++) {
-                    const _Float16 hi = static_cast<_Float16>(v[r]);
-                    *reinterpret_cast<_Float16 *>(e + r * 256) = hi;
-                    *reinterpret_cast<_Float16 *>(e + r * 256 + 64) = static_cast<_Float16>(v[r] - static_cast<float>(hi));
+                    _Float16 hi, lo;
+                    binary16_parts(ldexpf(v[r], kListOne - e), hi, lo);
+                    *reinterpret_cast<_Float16 *>(at + r * 256) = hi;
+                    *reinterpret_cast<_Float16 *>(at + r * 256 + 64) = lo;
                 }
+                if (n == 0) act_exps[to * (a.ffn / 32) + sub] = static_cast<uint8_t>(e);
                 if (n == 0) list_sum_put(act_sums + (to * (a.ffn / 256) + (sub >> 3)) * kListSumBytes, sub, sum32);
             }
         }
@@ -291,17 +321,50 @@ __device__ __forceinline__ void down_list_pass(const shv_moe_down_args &a, const
     const int part = PARTS == 1 ? n & 1 : 0;
     const uint32_t tok = pair * ((K / 32) * kStSubBytes) + kb * 16 + part * 64;
     const uint32_t sum = pair * (K / 256 * kListSumBytes) + part * 32 + kb * 8;
-    stream_tiles<K, PARTS, 2>(base, base + 32 * ROWB, kDownUnits, 16 * kR * ROWB, ring, reinterpret_cast<const char *>(a.act), tok, act_sums, sum,
+    static_assert(K == 512, "sixteen sub-blocks, an exponent of a byte each");
+    const u32x4_t exps = *reinterpret_cast<const u32x4_t *>(act_sums + list_act_exps_offset(static_cast<long long>(a.n_tok) * (a.n_used + 1), K) + static_cast<size_t>(pair) * 16);
+    int exponent = 0;  // the row's: its largest sub-block's
+    auto settle = [&](half8_t(&b)[2][8][PARTS], short4_t(&sx)[2][PARTS]) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) exponent = max(exponent, static_cast<int>(exps[i >> 2] >> (8 * (i & 3)) & 255));
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            const uint32_t two = ((kb & 2) ? exps[2 * s + 1] : exps[2 * s]) >> (16 * (kb & 1));  // of this lane's sub-blocks 8 s + 2 kb and the next
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int down = static_cast<int>(two >> (8 * h) & 255) - exponent;
+                const _Float16 f = static_cast<_Float16>(ldexpf(1.f, max(down, -24)));
+#pragma unroll
+                for (int v = 4 * h; v < 4 * h + 4; v++)
+#pragma unroll
+                    for (int p = 0; p < PARTS; p++) b[s][v][p] *= static_cast<half8_t>(f);
+                if (__any(down < -24)) {  // binary16 knows no smaller power
+                    const _Float16 f2 = static_cast<_Float16>(ldexpf(1.f, min(down + 24, 0)));
+#pragma unroll
+                    for (int v = 4 * h; v < 4 * h + 4; v++)
+#pragma unroll
+                        for (int p = 0; p < PARTS; p++) b[s][v][p] *= static_cast<half8_t>(f2);
+                }
+            }
+#pragma unroll
+            for (int p = 0; p < PARTS; p++)
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    sx[s][p][i] = static_cast<short>(__float_as_uint(ldexpf(__uint_as_float(static_cast<uint32_t>(static_cast<uint16_t>(sx[s][p][i])) << 16), kListOne - exponent)) >> 16);
+        }
+    };
+    stream_tiles<K, PARTS, 2>(base, base + 32 * ROWB, kDownUnits, 16 * kR * ROWB, ring, reinterpret_cast<const char *>(a.act), tok, act_sums, sum, settle,
                               [&](int unit, const float4_t (&y)[kR]) {
         constexpr int NT = PARTS == 1 ? 2 : 4;
 #pragma unroll
         for (int j = 0; j < NT; j++) {
             const int i = NT * kb + j;
             const size_t to = static_cast<size_t>(__shfl(pair, PARTS == 1 ? 2 * i : i, 64));
+            const int back = __shfl(exponent, PARTS == 1 ? 2 * i : i, 64) - kListOne;
             float *dst = a.pairs + to * a.n_embd + row0 + unit * 16 * kR + n;
             if (i < m) {
 #pragma unroll
-                for (int r = 0; r < kR; r++) dst[16 * r] = PARTS == 1 ? y[r][2 * (j & 1)] + y[r][2 * (j & 1) + 1] : y[r][j];
+                for (int r = 0; r < kR; r++) dst[16 * r] = ldexpf(PARTS == 1 ? y[r][2 * (j & 1)] + y[r][2 * (j & 1) + 1] : y[r][j], back);
             }
         }
     });
@@ -335,10 +398,12 @@ __global__ __launch_bounds__(kListThreads, 2) void moe_down_list_kernel(shv_moe_
 //   64 (1.25)                      185 / 158 / 168      400 (7.8)       400 / 321 / 312
 //   150 (2.9)                      352 / 215 / 229      600 (11.7)      453 / 413 / 379
 //   200 (3.9)                      366 / 240 / 247      800 (15.6)      480 / 510 / 460      1000 (19.5)  494 / 608 / 542
-// Below the first line most experts a pass touches are touched once, and reading them row by row costs no list.  Up to 64
-// rows the passes keep the other kernels' sums all the same: the choice between a token's tenth and eleventh expert can hang
-// on the last bits, a short prompt's choices are carried through every token decoded after it, and the 15 % at 64 rows are one
-// part in two hundred of a reply of a hundred tokens.
+// (Taken with operands as they were and no exponents; with them 66 rows 182, 150 rows 224, 300 rows 270, 400 rows 315, 750 rows
+// 431, a part in a hundred to a part in thirty more: the line at 15 pairs an expert is as good as level.)
+// Below the first line most experts a pass touches are touched once, and reading them row by row costs no list.  Passes of 40
+// to 64 rows would be a seventh faster here and no less exact (5e-7 against 4e-6 of a layer's outputs, against float64): they
+// keep the other kernels so that a short prompt's results stay the ones they were, since where a token's tenth expert and
+// its eleventh are level its choice is carried through every token decoded after it.
 int shv_moe_list_tokens(int n_tok, int n_used, int n_expert) {
     const long long pairs = static_cast<long long>(n_tok) * n_used;
     if (n_tok <= 64 || 4 * pairs < 3ll * n_expert || pairs > 15ll * n_expert) return 0;

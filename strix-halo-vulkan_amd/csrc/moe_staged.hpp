@@ -3,7 +3,8 @@
 // A row of k columns is [sub-block of 32][part hi, lo][block of 8 columns] x 16 bytes, 128 bytes a sub-block, the eight
 // columns of a block in slot order [0, 2, 1, 3, 4, 6, 5, 7] (the order a payload dword's nibbles come out of the masks).
 // After all rows come their sums over the sub-blocks, as operands too: [row][super-block] x 32 bytes, the eight sums'
-// binary16 values and then what those leave.  (The list kernels' sums are float32, in bfloat16 parts: list_sum_put.)
+// binary16 values and then what those leave.  (The list kernels' sums are float32, in bfloat16 parts: list_sum_put; their
+// values are scaled: binary16_parts.)
 #pragma once
 #include "shv_device.hpp"
 
@@ -46,30 +47,44 @@ __host__ __device__ constexpr int list_block(int sub, int c) { return (sub >> 3)
 
 // The sums of a row staged for the list kernels: [super-block] x 64 bytes, [part 0, 1][group] x 8 bytes, the group's two
 // sub-blocks' first and second bfloat16 parts in part 0, their third in part 1 (and two zeros, which its owner writes).
+// Then the rows' exponents, an int each; of SwiGLU rows, whose sub-blocks have one each, a byte each.
 constexpr int kListSumBytes = 64;
-__host__ __device__ constexpr size_t list_bytes(int rows, int k) { return staged_sums_offset(rows, k) + static_cast<size_t>(rows) * (k / 256) * kListSumBytes; }
-__host__ __device__ constexpr size_t list_act_bytes(long long pairs, int ffn) { return static_cast<size_t>(pairs) * (ffn / 256) * kListSumBytes; }
+__host__ __device__ constexpr size_t list_exps_offset(int rows, int k) { return staged_sums_offset(rows, k) + static_cast<size_t>(rows) * (k / 256) * kListSumBytes; }
+__host__ __device__ constexpr size_t list_bytes(int rows, int k) { return list_exps_offset(rows, k) + static_cast<size_t>(rows) * sizeof(int32_t); }
+__host__ __device__ constexpr size_t list_act_exps_offset(long long pairs, int ffn) { return static_cast<size_t>(pairs) * (ffn / 256) * kListSumBytes; }
+__host__ __device__ constexpr size_t list_act_bytes(long long pairs, int ffn) { return list_act_exps_offset(pairs, ffn) + static_cast<size_t>(pairs) * (ffn / 32); }
 __device__ __forceinline__ void list_sum_put(char *sb_sums, int sub, float sum) {
     uint16_t *p = reinterpret_cast<uint16_t *>(sb_sums + ((sub >> 1) & 3) * 8) + (sub & 1);
     bf16_parts(sum, p[0], p[2], p[16]);
     p[18] = 0;
 }
 
-// Four columns c .. c + 3 of row t for the list kernels, and (the lane of a sub-block's first columns) the sub-block's sum;
-// the eight lanes of a sub-block are neighbours and all here.
-__device__ __forceinline__ void stage_list_quad(const float4 v, int t, int c, int k, int rows, char *staged) {
-    const float o[4] = {v.x, v.z, v.y, v.w};
+// The list kernels' values: times the power of two 2^(kListOne - e) that brings the largest of their row (of their sub-block)
+// to 2^14 .. 2^15, e being its biased exponent, as two binary16 parts: 22 bits or more of anything down to 2^-17 of the largest,
+// whatever their size (unscaled, values of 1e-4 keep 11 to 12 bits and values past 65504 none).
+constexpr int kListOne = 127 + 14;
+__device__ __forceinline__ int biased_exponent(float largest) { return __float_as_uint(largest) >> 23 & 255; }
+__device__ __forceinline__ void binary16_parts(float u, _Float16 &hi, _Float16 &lo) {
+    hi = static_cast<_Float16>(u);
+    lo = fabsf(u) < INFINITY ? static_cast<_Float16>(u - static_cast<float>(hi)) : static_cast<_Float16>(0.f);  // an infinity is all in hi
+}
+
+// Four columns c .. c + 3 of row t for the list kernels, e the row's exponent, and (the lane of a sub-block's first columns)
+// the sub-block's sum; the eight lanes of a sub-block are neighbours and all here.
+__device__ __forceinline__ void stage_list_quad(const float4 v, int e, int t, int c, int k, int rows, char *staged) {
+    const float o[4] = {ldexpf(v.x, kListOne - e), ldexpf(v.z, kListOne - e), ldexpf(v.y, kListOne - e), ldexpf(v.w, kListOne - e)};
     half4_t h, l;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-        const _Float16 hi = static_cast<_Float16>(o[j]);
+        _Float16 hi, lo;
+        binary16_parts(o[j], hi, lo);
         h[j] = hi;
-        l[j] = static_cast<_Float16>(o[j] - static_cast<float>(hi));
+        l[j] = lo;
     }
-    char *e = staged + static_cast<size_t>(t) * (k / 32) * kStSubBytes + list_block(c >> 5, (c & 31) >> 3) + ((c & 7) >> 2) * 8;
-    *reinterpret_cast<half4_t *>(e) = h;
-    *reinterpret_cast<half4_t *>(e + 64) = l;
-    const float sum = shv::sum8_all((v.x + v.y) + (v.z + v.w));
+    char *at = staged + static_cast<size_t>(t) * (k / 32) * kStSubBytes + list_block(c >> 5, (c & 31) >> 3) + ((c & 7) >> 2) * 8;
+    *reinterpret_cast<half4_t *>(at) = h;
+    *reinterpret_cast<half4_t *>(at + 64) = l;
+    const float sum = shv::sum8_all((o[0] + o[2]) + (o[1] + o[3]));
     if ((c & 31) == 0) list_sum_put(staged + staged_sums_offset(rows, k) + (static_cast<size_t>(t) * (k / 256) + (c >> 8)) * kListSumBytes, c >> 5, sum);
 }
 

@@ -231,6 +231,14 @@ __device__ __forceinline__ float sum8_all(float v) {
     return v;
 }
 
+// The largest of aligned groups of 16 lanes, in every lane of the group.
+__device__ __forceinline__ float max16_all(float v) {
+    v = fmaxf(v, dpp_f32<kDppXor1>(v));
+    v = fmaxf(v, dpp_f32<kDppXor2>(v));
+    v = fmaxf(v, dpp_f32<kDppHalfMirror>(v));
+    return fmaxf(v, dpp_f32<kDppMirror>(v));
+}
+
 // One lane's loads for one row: the super-block header and the 32 payload bytes of its group.
 struct Q4kLane {
     uint4 hdr, q0, q1;

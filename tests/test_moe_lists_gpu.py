@@ -123,3 +123,36 @@ def test_sums_past_binary16(rig, lengths):
         assert (np.abs(got[at, 0] - want) <= tol).all(), e
     want, tol = up64(xn.astype(np.float64), expert_rows(rig, 3, 0, F, H), expert_rows(rig, 4, 0, F, H))
     assert (np.abs(got[:, 1] - want) <= tol).all()
+
+
+# act as floats from 128 rows on goes to the grouped down projection, whose operands keep binary16's range
+@pytest.mark.parametrize("lengths,packed", [(LENGTHS, 1), (LENGTHS, 0), (SIXTEENS, 1)])
+def test_values_of_any_size(rig, lengths, packed):
+    """Rows whose activations, whose SwiGLU values or whose SwiGLU sub-blocks among one another are past binary16's range or far
+    below its normal numbers, against float64: each row as exact as any other."""
+    c, E, _, banks = rig
+    rng = np.random.default_rng(4)
+    topk = selection(lengths, 1, rng)
+    T = len(topk)
+    # SwiGLU goes with the square of a row's size: 1e-8 .. 1e12; from gates of some size on, half of its values are next to nothing
+    xn = (rng.standard_normal((T, H)) * 10.0 ** rng.uniform(-4, 6, size=(T, 1))).astype(np.float32)
+    wts = np.ones((T, 2), np.float32)
+    wts[:, 1] = rng.choice([0, 1], T)  # half of the rows without the shared expert, which would hide the routed one's small values
+    bufs = [c.upload(a) for a in (xn, topk, wts)]
+    act, out = c.alloc(T * 2 * F * 4), c.alloc(T * H * 4)
+    group, pairs = c.alloc((2 * E + 1 + T) * 4), c.alloc(T * 2 * H * 4)
+    g, u, d, gs, us, ds = (b.ptr for b in banks)
+    ua = A.MoeUpArgs(bufs[0].ptr, bufs[1].ptr, g, u, gs, us, act.ptr, T, H, 1, F, None, None, E, 0, 0, 0, 0, group.ptr, 0, packed)
+    da = A.MoeDownArgs(act.ptr, bufs[1].ptr, bufs[2].ptr, d, ds, None, out.ptr, T, H, 1, F, H, H, 0, 0, E, group.ptr, pairs.ptr, 1, packed)
+    c.dispatch_multi([A.make_op(A.OP_MOE_UP, ua), A.make_op(A.OP_MOE_DOWN, da)])
+    got = out.read(np.float32, T * H).reshape(T, H)
+    for b in bufs + [act, out, group, pairs]:
+        b.free()
+    x64 = xn.astype(np.float64)
+    shared = up64(x64, expert_rows(rig, 3, 0, F, H), expert_rows(rig, 4, 0, F, H))[0] @ expert_rows(rig, 5, 0, H, F).T
+    for e in range(1, 7):
+        at = np.flatnonzero(topk[:, 0] == e)
+        want = up64(x64[at], expert_rows(rig, 0, e, F, H), expert_rows(rig, 1, e, F, H))[0] @ expert_rows(rig, 2, e, H, F).T + wts[at, 1:] * shared[at]
+        err = np.linalg.norm(got[at] - want, axis=1) / np.linalg.norm(want, axis=1)
+        # three projections in a row of float32 sums, as the tests beside this one state it
+        assert err.max() <= 1e-5, (e, at[err.argmax()], float(err.max()))
