@@ -1861,7 +1861,9 @@ void Graph::Checkpoint(struct Checkpoint &c) {
     const size_t carried = dn_->CarriedLen() * 4;
     c.past = q.past;
     c.ids.resize(q.past);
-    if (!c.on_device || c.on_device->device != dev_.index() || c.on_device->bytes != carried) {
+    // Memory of a checkpoint taken before serves again when nothing else can be reading it: no copy of the checkpoint holds it,
+    // and it is this context's, whose stream orders this write behind its own readings (another context waits for those).
+    if (!c.on_device || c.on_device.use_count() > 1 || c.on_device->owner() != dev_.ctx() || c.on_device->bytes != carried) {
         c.on_device = nullptr;
         if (carried > 0) c.on_device = dev_.block(carried);
     }
@@ -1888,6 +1890,7 @@ void Graph::Restore(const struct Checkpoint &c) {
     if (!same) throw Error("llm: this slot no longer holds the checkpoint's tokens");
     if (c.on_device && c.on_device->device == dev_.index()) {
         dn_->RestoreCarriedOnDevice(static_cast<const float *>(c.on_device->ptr), slot_, q.plane, c.past);
+        if (c.on_device->owner() != dev_.ctx()) dev_.sync();  // the owner's next write is not ordered behind this stream
     } else if (c.on_device) {  // taken on another GPU
         const auto carried = c.on_device->Read();
         dn_->RestoreCarried(carried.data(), slot_, q.plane, c.past);

@@ -35,6 +35,7 @@ public:
     DeviceBlock(const DeviceBlock &) = delete;
     DeviceBlock &operator=(const DeviceBlock &) = delete;
     std::vector<float> Read() const;
+    const shv_ctx *owner() const { return ctx_.get(); }  // whose stream writes it
     const int device;
     void *const ptr;
     const size_t bytes;
@@ -432,7 +433,8 @@ struct Pass {
 // llm.Checkpoint (llm/graph.go:902-1003): a sequence's position, tokens and DeltaNet carry; the KV
 // cells need no copy, the ones past the checkpoint are simply written again.  The carry (77 MB at 48
 // layers) stays in device memory, where saving and restoring it is one launch; in host memory, as the
-// reference keeps it, only when the device has no room.
+// reference keeps it, only when the device has no room.  A copy shares the carry, which is not written again
+// while anyone else holds it: what a checkpoint holds stays what it held when it was taken.
 struct Checkpoint {
     int past = 0;
     std::vector<int32_t> ids;
