@@ -170,6 +170,49 @@ int shv_free(shv_ctx *ctx, void *dptr) {
     return SHV_OK;
 }
 
+namespace {
+// the calling thread's device for a call that names its own, and back
+struct OnDevice {
+    int before = 0;
+    hipError_t error;
+    explicit OnDevice(int device) {
+        error = hipGetDevice(&before);
+        if (error == hipSuccess && device != before) error = hipSetDevice(device);
+    }
+    ~OnDevice() { (void)hipSetDevice(before); }
+};
+}  // namespace
+
+int shv_block_alloc(int device, size_t bytes, void **dptr) {
+    SHV_REQUIRE(dptr && bytes > 0, "shv_block_alloc: NULL argument or zero bytes");
+    *dptr = nullptr;
+    const OnDevice on(device);
+    SHV_HIP_CHECK(on.error);
+    const hipError_t e = hipMalloc(dptr, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        return shv_set_error(SHV_E_NOMEM, "shv_block_alloc: %zu bytes do not fit in device memory", bytes);
+    }
+    SHV_HIP_CHECK(e);
+    return SHV_OK;
+}
+
+int shv_block_free(int device, void *dptr) {
+    if (!dptr) return SHV_OK;
+    const OnDevice on(device);
+    SHV_HIP_CHECK(on.error);
+    SHV_HIP_CHECK(hipFree(dptr));  // waits for the device's streams by itself
+    return SHV_OK;
+}
+
+int shv_block_read(int device, void *dst, const void *src, size_t bytes) {
+    SHV_REQUIRE(dst && src, "shv_block_read: NULL argument");
+    const OnDevice on(device);
+    SHV_HIP_CHECK(on.error);
+    SHV_HIP_CHECK(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost));
+    return SHV_OK;
+}
+
 int shv_upload(shv_ctx *ctx, void *dst, const void *src, size_t bytes) {
     SHV_REQUIRE(ctx && dst && src, "shv_upload: NULL argument");
     SHV_REQUIRE(!ctx->capturing, "shv_upload: not valid while recording");

@@ -174,7 +174,7 @@ def make_op(kind, args, flags=0):
 # every symbol include/shv_hip.h declares; the CPU test suite checks the library exports them all
 SYMBOLS = [
     "shv_last_error", "shv_device_count", "shv_init", "shv_destroy", "shv_device_props", "shv_sync",
-    "shv_submits", "shv_alloc", "shv_free", "shv_upload", "shv_upload_async", "shv_download", "shv_copy", "shv_zero", "shv_copy_spans", "shv_upload_words",
+    "shv_submits", "shv_alloc", "shv_free", "shv_upload", "shv_block_alloc", "shv_block_free", "shv_block_read", "shv_upload_async", "shv_download", "shv_copy", "shv_zero", "shv_copy_spans", "shv_upload_words",
     "shv_host_alloc", "shv_host_free", "shv_enqueue", "shv_dispatch_multi", "shv_prerecord",
     "shv_prerecorded_submit", "shv_prerecorded_launch", "shv_stamp", "shv_stamp_elapsed", "shv_prerecorded_count",
     "shv_prerecorded_destroy", "shv_gemv_q4k", "shv_dequant_q4k", "shv_dequant", "shv_gemv", "shv_quantize_q4k",
@@ -208,6 +208,9 @@ def load():
     L.shv_upload.argtypes = [vp, vp, vp, C.c_size_t]
     L.shv_upload_async.argtypes = [vp, vp, vp, C.c_size_t]
     L.shv_download.argtypes = [vp, vp, vp, C.c_size_t]
+    L.shv_block_alloc.argtypes = [C.c_int, C.c_size_t, vpp]
+    L.shv_block_free.argtypes = [C.c_int, vp]
+    L.shv_block_read.argtypes = [C.c_int, vp, vp, C.c_size_t]
     L.shv_copy.argtypes = [vp, vp, vp, C.c_size_t]
     L.shv_zero.argtypes = [vp, vp, C.c_size_t]
     L.shv_copy_spans.argtypes = [vp, C.POINTER(Span), C.c_int]

@@ -18,28 +18,25 @@ static uint64_t q4k_bytes(int64_t rows, int64_t cols) { return rows * (cols / SH
 
 // ------------------------------------------------------------------------------- Device -------
 
-Device::Device(int index) : index_(index) {
-    shv_ctx *c = nullptr;
-    check(shv_init(index, &c), "NewDevice");
-    ctx_ = std::shared_ptr<shv_ctx>(c, shv_destroy);
-}
+Device::Device(int index) : index_(index) { check(shv_init(index, &ctx_), "NewDevice"); }
 
 Device::~Device() {
     if (!ctx_) return;
     shv_sync(ctx());
     for (void *p : owned_) shv_free(ctx(), p);
     for (void *p : host_owned_) shv_host_free(ctx(), p);
+    shv_destroy(ctx_);
 }
 
 std::vector<float> DeviceBlock::Read() const {
     std::vector<float> v(bytes / 4);
-    check(shv_download(ctx_.get(), v.data(), ptr, bytes), "DeviceBlock.Read");
+    check(shv_block_read(device, v.data(), ptr, bytes), "DeviceBlock.Read");
     return v;
 }
 
 std::shared_ptr<DeviceBlock> Device::block(size_t bytes) {
     void *p = nullptr;
-    if (shv_alloc(ctx(), bytes, &p) != SHV_OK) return nullptr;
+    if (shv_block_alloc(index_, bytes, &p) != SHV_OK) return nullptr;
     return std::make_shared<DeviceBlock>(ctx_, index_, p, bytes);
 }
 

@@ -27,21 +27,21 @@ struct Error : std::runtime_error {
     using std::runtime_error::runtime_error;
 };
 
-// A device allocation that may outlive the Device it came from: it holds the context itself.
+// A device allocation that may outlive the Device it came from, and keeps nothing of it; any thread may drop it.
 class DeviceBlock {
 public:
-    DeviceBlock(std::shared_ptr<shv_ctx> ctx, int device, void *p, size_t bytes) : device(device), ptr(p), bytes(bytes), ctx_(std::move(ctx)) {}
-    ~DeviceBlock() { shv_free(ctx_.get(), ptr); }
+    DeviceBlock(const shv_ctx *owner, int device, void *p, size_t bytes) : device(device), ptr(p), bytes(bytes), owner_(owner) {}
+    ~DeviceBlock() { shv_block_free(device, ptr); }
     DeviceBlock(const DeviceBlock &) = delete;
     DeviceBlock &operator=(const DeviceBlock &) = delete;
     std::vector<float> Read() const;
-    const shv_ctx *owner() const { return ctx_.get(); }  // whose stream writes it
+    const shv_ctx *owner() const { return owner_; }  // whose stream writes it: a name, the context may be gone
     const int device;
     void *const ptr;
     const size_t bytes;
 
 private:
-    std::shared_ptr<shv_ctx> ctx_;
+    const shv_ctx *owner_;
 };
 
 // vk.Device (vk/engine.go:266-311): owns the context; every block borrows it.
@@ -51,7 +51,7 @@ public:
     ~Device();
     Device(const Device &) = delete;
     Device &operator=(const Device &) = delete;
-    shv_ctx *ctx() const { return ctx_.get(); }
+    shv_ctx *ctx() const { return ctx_; }
     int index() const { return index_; }
     std::shared_ptr<DeviceBlock> block(size_t bytes);  // nullptr where the device has no room
     void *alloc(size_t bytes);  // tracked; released with the device
@@ -69,7 +69,7 @@ public:
     size_t allocated() const { return allocated_; }
 
 private:
-    std::shared_ptr<shv_ctx> ctx_;
+    shv_ctx *ctx_ = nullptr;
     int index_ = 0;
     std::vector<void *> owned_, host_owned_;
     size_t allocated_ = 0;

@@ -41,6 +41,9 @@ void shv_destroy(shv_ctx *c) {
 int shv_sync(shv_ctx *c) { return c->unwaited = 0; }
 int shv_alloc(shv_ctx *, size_t bytes, void **p) { return take(bytes, p); }
 int shv_free(shv_ctx *, void *p) { return give(p); }
+int shv_block_alloc(int, size_t bytes, void **p) { return take(bytes, p); }
+int shv_block_free(int, void *p) { return give(p); }
+int shv_block_read(int, void *dst, const void *src, size_t n) { return std::memcpy(dst, src, n), 0; }
 int shv_host_alloc(shv_ctx *, size_t bytes, void **p) { return take(bytes, p); }
 int shv_host_free(shv_ctx *, void *p) { return give(p); }
 int shv_upload_async(shv_ctx *, void *dst, const void *src, size_t n) { return std::memcpy(dst, src, n), 0; }
@@ -135,5 +138,16 @@ int double_restored_elsewhere() {
     const int before = g_given;
     other.graph->Checkpoint(a);
     return g_given == before + 1;  // given back, which waits for the device, and other memory taken
+}
+
+// A checkpoint that outlives its model: the contexts still there, and a thousand times the allocations beside the checkpoint's own.
+int double_checkpoint_outlives_its_model() {
+    const size_t before = g_memory.size();
+    llm::Checkpoint a;
+    {
+        Rig r;
+        r.graph->Checkpoint(a);
+    }
+    return g_contexts + 1000 * static_cast<int>(g_memory.size() - before - 1);
 }
 }

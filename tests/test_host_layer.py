@@ -40,3 +40,7 @@ def test_a_checkpoint_taken_again_uses_its_memory_again(host):
 
 def test_a_checkpoint_another_graph_restores_is_read_to_the_end_and_not_written(host):
     assert host.double_restored_elsewhere() == 1
+
+
+def test_a_checkpoint_that_outlives_its_model_keeps_its_carry_alone(host):
+    assert host.double_checkpoint_outlives_its_model() == 0
