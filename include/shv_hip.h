@@ -69,8 +69,9 @@ int shv_free(shv_ctx *ctx, void *dptr);
 int shv_upload(shv_ctx *ctx, void *dst_dev, const void *src_host, size_t bytes);
 int shv_download(shv_ctx *ctx, void *dst_host, const void *src_dev, size_t bytes);
 /* Device memory that no context owns, for what outlives the model it came from (a saved sequence): any thread may give it
- * back, which waits for the device, and read it, which waits for nothing but the reading. */
-int shv_block_alloc(int device, size_t bytes, void **dptr);
+ * back, which waits for the device, and read it, which waits for nothing but the reading.  Refused with SHV_E_NOMEM
+ * where less than keep_free bytes of the device would be left to others. */
+int shv_block_alloc(int device, size_t bytes, size_t keep_free, void **dptr);
 int shv_block_free(int device, void *dptr);
 int shv_block_read(int device, void *dst_host, const void *src_dev, size_t bytes);
 /* shv_upload for a pass's control words and token ids (Buffer.WriteU32s on a host-visible buffer,

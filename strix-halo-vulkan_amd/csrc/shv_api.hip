@@ -183,11 +183,17 @@ struct OnDevice {
 };
 }  // namespace
 
-int shv_block_alloc(int device, size_t bytes, void **dptr) {
+int shv_block_alloc(int device, size_t bytes, size_t keep_free, void **dptr) {
     SHV_REQUIRE(dptr && bytes > 0, "shv_block_alloc: NULL argument or zero bytes");
     *dptr = nullptr;
     const OnDevice on(device);
     SHV_HIP_CHECK(on.error);
+    if (keep_free > 0) {
+        size_t left = 0, all = 0;
+        SHV_HIP_CHECK(hipMemGetInfo(&left, &all));
+        if (left < bytes || left - bytes < keep_free)
+            return shv_set_error(SHV_E_NOMEM, "shv_block_alloc: %zu bytes of %zu free would leave less than %zu", bytes, left, keep_free);
+    }
     const hipError_t e = hipMalloc(dptr, bytes);
     if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();

@@ -208,7 +208,7 @@ def load():
     L.shv_upload.argtypes = [vp, vp, vp, C.c_size_t]
     L.shv_upload_async.argtypes = [vp, vp, vp, C.c_size_t]
     L.shv_download.argtypes = [vp, vp, vp, C.c_size_t]
-    L.shv_block_alloc.argtypes = [C.c_int, C.c_size_t, vpp]
+    L.shv_block_alloc.argtypes = [C.c_int, C.c_size_t, C.c_size_t, vpp]
     L.shv_block_free.argtypes = [C.c_int, vp]
     L.shv_block_read.argtypes = [C.c_int, vp, vp, C.c_size_t]
     L.shv_copy.argtypes = [vp, vp, vp, C.c_size_t]

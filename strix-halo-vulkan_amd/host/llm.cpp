@@ -36,7 +36,9 @@ std::vector<float> DeviceBlock::Read() const {
 
 std::shared_ptr<DeviceBlock> Device::block(size_t bytes) {
     void *p = nullptr;
-    if (shv_block_alloc(index_, bytes, &p) != SHV_OK) return nullptr;
+    shv_props props;
+    check(shv_device_props(ctx(), &props), "block");
+    if (shv_block_alloc(index_, bytes, props.hbm_bytes / 16, &p) != SHV_OK) return nullptr;
     return std::make_shared<DeviceBlock>(ctx_, index_, p, bytes);
 }
 

@@ -53,7 +53,8 @@ public:
     Device &operator=(const Device &) = delete;
     shv_ctx *ctx() const { return ctx_; }
     int index() const { return index_; }
-    std::shared_ptr<DeviceBlock> block(size_t bytes);  // nullptr where the device has no room
+    // nullptr where the device has no room: a sixteenth of its memory stays free, for models and graphs staged later
+    std::shared_ptr<DeviceBlock> block(size_t bytes);
     void *alloc(size_t bytes);  // tracked; released with the device
     void *alloc_zero(size_t bytes);
     void release(void *p, size_t bytes);  // an alloc() handed back early; bytes as asked for
@@ -433,7 +434,7 @@ struct Pass {
 // llm.Checkpoint (llm/graph.go:902-1003): a sequence's position, tokens and DeltaNet carry; the KV
 // cells need no copy, the ones past the checkpoint are simply written again.  The carry (77 MB at 48
 // layers) stays in device memory, where saving and restoring it is one launch; in host memory, as the
-// reference keeps it, only when the device has no room.  A copy shares the carry, which is not written again
+// reference keeps it, only when the device has no room to spare (Device::block).  A copy shares the carry, which is not written again
 // while anyone else holds it: what a checkpoint holds stays what it held when it was taken.
 struct Checkpoint {
     int past = 0;

@@ -17,6 +17,7 @@ struct shv_prerecorded {
 
 namespace {
 int g_contexts = 0, g_recorded = 0, g_enqueued = 0, g_given = 0;
+size_t g_free = size_t(16) << 30;  // what the device claims to have left
 std::set<void *> g_memory;
 int take(size_t bytes, void **p) {
     *p = std::calloc(1, bytes);
@@ -41,7 +42,8 @@ void shv_destroy(shv_ctx *c) {
 int shv_sync(shv_ctx *c) { return c->unwaited = 0; }
 int shv_alloc(shv_ctx *, size_t bytes, void **p) { return take(bytes, p); }
 int shv_free(shv_ctx *, void *p) { return give(p); }
-int shv_block_alloc(int, size_t bytes, void **p) { return take(bytes, p); }
+int shv_device_props(shv_ctx *, shv_props *p) { return std::memset(p, 0, sizeof *p), p->hbm_bytes = 16ull << 30, 0; }
+int shv_block_alloc(int, size_t bytes, size_t keep, void **p) { return bytes + keep > g_free ? SHV_E_NOMEM : take(bytes, p); }
 int shv_block_free(int, void *p) { return give(p); }
 int shv_block_read(int, void *dst, const void *src, size_t n) { return std::memcpy(dst, src, n), 0; }
 int shv_host_alloc(shv_ctx *, size_t bytes, void **p) { return take(bytes, p); }
@@ -149,5 +151,16 @@ int double_checkpoint_outlives_its_model() {
         r.graph->Checkpoint(a);
     }
     return g_contexts + 1000 * static_cast<int>(g_memory.size() - before - 1);
+}
+
+// A checkpoint on a device with `free_mb` of its 16 GB left: 1 in device memory, 0 whole in host memory, and restored from there.
+int double_checkpoint_where_free(int free_mb) {
+    Rig r;
+    llm::Checkpoint a;
+    g_free = static_cast<size_t>(free_mb) << 20;
+    r.graph->Checkpoint(a);
+    g_free = static_cast<size_t>(16) << 30;
+    r.graph->Restore(a);
+    return a.on_device ? 1 : a.dn.empty() ? -1 : 0;
 }
 }

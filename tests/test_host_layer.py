@@ -44,3 +44,8 @@ def test_a_checkpoint_another_graph_restores_is_read_to_the_end_and_not_written(
 
 def test_a_checkpoint_that_outlives_its_model_keeps_its_carry_alone(host):
     assert host.double_checkpoint_outlives_its_model() == 0
+
+
+@pytest.mark.parametrize("free_mb,on_device", [(8000, 1), (1100, 1), (1023, 0), (0, 0)])
+def test_a_checkpoint_leaves_a_sixteenth_of_the_device_free(host, free_mb, on_device):
+    assert host.double_checkpoint_where_free(free_mb) == on_device

@@ -64,3 +64,16 @@ def test_spans_and_words_refuse_what_they_cannot_do(ctx):
     for w in (A.Words(None, v.ctypes.data, 4), A.Words(b.ptr, None, 4), A.Words(b.at(2), v.ctypes.data, 1)):
         with pytest.raises(A.ShvError):
             A.check(ctx.L.shv_upload_words(ctx.h, C.byref(w), 1))
+
+
+def test_blocks_no_context_owns(ctx):
+    p = C.c_void_p()
+    hbm = ctx.props().hbm_bytes
+    assert ctx.L.shv_block_alloc(0, 1 << 20, hbm, C.byref(p)) == -3 and p.value is None  # would leave less than all of it
+    A.check(ctx.L.shv_block_alloc(0, 1 << 20, hbm // 16, C.byref(p)))
+    want = np.random.default_rng(1).integers(0, 256, 1 << 20).astype(np.uint8)
+    A.check(ctx.L.shv_upload(ctx.h, p, want.ctypes.data, want.nbytes))
+    got = np.zeros_like(want)
+    A.check(ctx.L.shv_block_read(0, got.ctypes.data, p, got.nbytes))
+    assert np.array_equal(got, want)
+    A.check(ctx.L.shv_block_free(0, p))
