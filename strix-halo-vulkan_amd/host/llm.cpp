@@ -2009,21 +2009,28 @@ PassRows MTPHead::rows_of(int n) const {
     return r;
 }
 
-Pass &MTPHead::cell_pass(int n) {
-    const std::vector<int> key{slot_, n, 2, 0};
-    auto it = passes_.find(key);
-    if (it == passes_.end()) {
-        Pass p;
-        p.ops = input_ops(n, nullptr, &p.labels);
-        auto a = attn_->Dispatches(layer_, x_, x_, rows_of(n), &p.labels);
-        shv_attn_decode_args cells{};
-        std::memcpy(&cells, a[1].args, sizeof cells);
-        cells.out = nullptr;  // the rows' cells, nothing attended
-        p.ops.push_back(a[0]);
-        p.ops.push_back(make_op(SHV_OP_ATTN_DECODE, cells));
-        it = passes_.emplace(key, std::move(p)).first;
+std::vector<shv_op> MTPHead::cell_ops(int n) const {
+    std::vector<shv_op> ops = input_ops(n, nullptr, nullptr);
+    auto a = attn_->Dispatches(layer_, x_, x_, rows_of(n), nullptr);
+    shv_attn_decode_args cells{};
+    std::memcpy(&cells, a[1].args, sizeof cells);
+    cells.out = nullptr;  // the rows' cells, nothing attended
+    ops.push_back(a[0]);
+    ops.push_back(make_op(SHV_OP_ATTN_DECODE, cells));
+    return ops;
+}
+
+// The row counts that come again and again, a round's owed rows and a prompt's full chunks, are recorded; what a prompt's length
+// leaves of its last chunk is handed over op by op: any length costs its first prompt what it costs the next.
+void MTPHead::launch_cells(int n) {
+    if (n > max_tok_ && n < cell_rows_) {
+        for (const shv_op &op : cell_ops(n)) check(shv_enqueue(dev_.ctx(), op.kind, op.args, sizeof op.args), "draft cells");
+        return;
     }
-    return it->second;
+    Pass &p = passes_[{slot_, n, 2, 0}];
+    if (p.ops.empty()) p.ops = cell_ops(n);
+    if (!p.rec) check(shv_prerecord(dev_.ctx(), p.ops.data(), static_cast<int>(p.ops.size()), &p.rec), "draft cells");
+    check(shv_prerecorded_launch(dev_.ctx(), p.rec), "draft cells");
 }
 
 void MTPHead::check_rows(const std::vector<int32_t> &ids, int pos) const {
@@ -2040,12 +2047,10 @@ void MTPHead::WriteCells(const float *hs, const std::vector<int32_t> &ids, int p
     check_rows(ids, pos);
     for (int a = 0; a < n; a += cell_rows_) {
         const int k = std::min(cell_rows_, n - a);
-        Pass &pass = cell_pass(k);
         const int32_t p32 = pos + a;
         check(shv_copy(dev_.ctx(), h_, hs + static_cast<size_t>(a) * c_.NEmbd, static_cast<size_t>(k) * c_.NEmbd * 4), "draft input");
         dev_.words({{ids_, ids.data() + a, k}, {pos_ + slot_, &p32, 1}});
-        if (!pass.rec) check(shv_prerecord(dev_.ctx(), pass.ops.data(), static_cast<int>(pass.ops.size()), &pass.rec), "draft cells");
-        check(shv_prerecorded_launch(dev_.ctx(), pass.rec), "draft cells");
+        launch_cells(k);
         Steps++;
     }
     pasts_[slot_] = pos + n;

@@ -621,7 +621,8 @@ private:
     void check_rows(const std::vector<int32_t> &ids, int pos) const;
     std::vector<shv_op> input_ops(int n, int32_t *ring, std::vector<std::string> *labels) const;
     PassRows rows_of(int n) const;
-    Pass &cell_pass(int n);
+    std::vector<shv_op> cell_ops(int n) const;
+    void launch_cells(int n);
     Pass &draft_pass(int n, bool head, int k, int32_t *ring);
 };
 

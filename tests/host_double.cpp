@@ -163,4 +163,18 @@ int double_checkpoint_where_free(int free_mb) {
     r.graph->Restore(a);
     return a.on_device ? 1 : a.dn.empty() ? -1 : 0;
 }
+
+// The draft's cells over prompts of every length from 1 to 130: how many sequences of ops were recorded for them.
+int double_recordings_for_cells() {
+    Rig r(1);
+    llm::MTPHead head(*r.dev, *r.model, r.graph->Head(), 4, 1024, 1);
+    std::vector<float> rows(130 * 256);
+    const int before = g_recorded;
+    for (int n = 1; n <= 130; n++) {
+        head.Reset();
+        head.WriteCells(rows.data(), std::vector<int32_t>(n, 7), 0);
+        if (head.Past() != n) return -1;
+    }
+    return g_recorded - before;
+}
 }

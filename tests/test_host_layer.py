@@ -49,3 +49,8 @@ def test_a_checkpoint_that_outlives_its_model_keeps_its_carry_alone(host):
 @pytest.mark.parametrize("free_mb,on_device", [(8000, 1), (1100, 1), (1023, 0), (0, 0)])
 def test_a_checkpoint_leaves_a_sixteenth_of_the_device_free(host, free_mb, on_device):
     assert host.double_checkpoint_where_free(free_mb) == on_device
+
+
+def test_cells_of_a_prompt_are_recorded_for_the_counts_that_come_again(host):
+    # one to four rows (what the head was staged for) and a full chunk of 64, whatever the prompts' lengths
+    assert host.double_recordings_for_cells() == 5
