@@ -129,6 +129,7 @@ enum {
     SHV_OP_ROUTER_FOLD = 16,
     SHV_OP_QSA_INDEX = 17,
     SHV_OP_ARGMAX_STATIC = 18, /* shv_argmax_static as an op, so that a recorded sequence can hold it */
+    SHV_OP_ATTN_CELLS = 19,    /* shv_attn_decode_args: the rows' cells alone */
     SHV_OP__COUNT
 };
 
@@ -443,7 +444,7 @@ typedef struct {
     void *kcache;
     void *vcache;
     float *partial;
-    float *out;  /* NULL: the rows' cells are written and nothing is attended */
+    float *out;
     const int32_t *pos;
     const int32_t *slot;
     int32_t n_seq, seq_len;
@@ -456,6 +457,9 @@ typedef struct {
     const uint32_t *mask;
     int32_t mask_stride;
 } shv_attn_decode_args;
+
+/* SHV_OP_ATTN_CELLS takes the same arguments: the rows' cells are written, as shv_attn_decode writes them, and nothing is
+ * attended; out and partial are not used and may be NULL.  (A draft's cells over a prompt are all it needs of it.) */
 
 /* The block-sparse indexer beside a full-attention layer (AttnTrace.indexerAt, llm/attn.go:231-421;
  * topK / topKThreshold / f2ui :588-682; shaders llm_attn_idx / score / select / selblk.comp), for

@@ -967,9 +967,9 @@ int launch_rows(shv_ctx *ctx, const shv_attn_decode_args &a, int row0, int n_gro
 
 }  // namespace
 
-int shv_launch_attn_decode(shv_ctx *ctx, const shv_attn_decode_args *pa) {
-    const shv_attn_decode_args &a = *pa;
-    SHV_REQUIRE(a.qkv && a.q_norm && a.k_norm && a.rope && a.kcache && a.vcache && a.partial, "attn_decode: NULL argument");
+// What a call has to be whether its rows are attended to or only written.
+static int check_attn_args(const shv_attn_decode_args &a) {
+    SHV_REQUIRE(a.qkv && a.q_norm && a.k_norm && a.rope && a.kcache && a.vcache, "attn_decode: NULL argument");
     SHV_REQUIRE(a.head_dim == kD, "attn_decode: head_dim %d; built for %d", a.head_dim, kD);
     SHV_REQUIRE(a.n_head_kv >= 1 && a.n_head == a.n_head_kv * kRep, "attn_decode: %d query heads over %d KV heads; built for %d per KV head",
                 a.n_head, a.n_head_kv, kRep);
@@ -985,11 +985,21 @@ int shv_launch_attn_decode(shv_ctx *ctx, const shv_attn_decode_args *pa) {
     SHV_REQUIRE(shv_aligned16(a.qkv) && shv_aligned16(a.kcache) && shv_aligned16(a.vcache) && shv_aligned16(a.q_norm) &&
                     shv_aligned16(a.k_norm) && shv_aligned16(a.out) && shv_aligned16(a.partial) && a.qkv_stride % 4 == 0,
                 "attn_decode: qkv, caches, norms, partial and out must be 16-byte aligned");
-    if (!a.out) {
-        SHV_REQUIRE(a.seq_len <= 65535, "attn_decode: %d rows", a.seq_len);
-        SHV_LAUNCH(ctx, attn_append_kernel, dim3(a.n_head_kv, a.seq_len, a.n_seq), dim3(kBlock), 0, a);
-        return SHV_OK;
-    }
+    return SHV_OK;
+}
+
+int shv_launch_attn_cells(shv_ctx *ctx, const shv_attn_decode_args *pa) {
+    const shv_attn_decode_args &a = *pa;
+    if (const int rc = check_attn_args(a); rc != SHV_OK) return rc;
+    SHV_REQUIRE(a.seq_len <= 65535, "attn_cells: %d rows", a.seq_len);
+    SHV_LAUNCH(ctx, attn_append_kernel, dim3(a.n_head_kv, a.seq_len, a.n_seq), dim3(kBlock), 0, a);
+    return SHV_OK;
+}
+
+int shv_launch_attn_decode(shv_ctx *ctx, const shv_attn_decode_args *pa) {
+    const shv_attn_decode_args &a = *pa;
+    SHV_REQUIRE(a.partial && a.out, "attn_decode: NULL argument");
+    if (const int rc = check_attn_args(a); rc != SHV_OK) return rc;
     // The rows of a sequence go two at a time: both see one pass over the cache.  One or two rows
     // write their own cells on the way; more rows have all their cells written first and then go
     // through as pairs of one launch (a last pair of one row repeats it and drops the copy).

@@ -296,6 +296,7 @@ static int dispatch_one(shv_ctx *ctx, uint32_t kind, const void *args, size_t by
         case SHV_OP_MOE_DOWN: return run_as<shv_moe_down_args>(ctx, args, bytes, shv_launch_moe_down, "moe_down");
         case SHV_OP_DN_STEP: return run_as<shv_dn_step_args>(ctx, args, bytes, shv_launch_dn_step, "dn_step");
         case SHV_OP_ATTN_DECODE: return run_as<shv_attn_decode_args>(ctx, args, bytes, shv_launch_attn_decode, "attn_decode");
+        case SHV_OP_ATTN_CELLS: return run_as<shv_attn_decode_args>(ctx, args, bytes, shv_launch_attn_cells, "attn_cells");
         case SHV_OP_EMBED: return run_as<shv_embed_args>(ctx, args, bytes, shv_launch_embed, "embed");
         case SHV_OP_ARGMAX: return run_as<shv_argmax_args>(ctx, args, bytes, shv_launch_argmax, "argmax");
         case SHV_OP_ADVANCE: return run_as<shv_advance_args>(ctx, args, bytes, shv_launch_advance, "advance");

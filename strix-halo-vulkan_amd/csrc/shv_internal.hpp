@@ -181,6 +181,7 @@ int shv_launch_moe_up_lists(shv_ctx *ctx, const shv_moe_up_args &a);
 int shv_launch_moe_down_lists(shv_ctx *ctx, const shv_moe_down_args &a);
 int shv_launch_dn_step(shv_ctx *ctx, const shv_dn_step_args *a);
 int shv_launch_attn_decode(shv_ctx *ctx, const shv_attn_decode_args *a);
+int shv_launch_attn_cells(shv_ctx *ctx, const shv_attn_decode_args *a);
 // expert banks in other types than Q4_K: slots [slot0, slot0 + slots) of the up projection; slots
 // [s_lo, s_hi) of the down projection, added to out when `add` (another launch wrote the rest)
 int shv_launch_moe_up_any(shv_ctx *ctx, const shv_moe_up_args *a, int slot0, int slots);

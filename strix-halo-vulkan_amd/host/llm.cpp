@@ -2012,11 +2012,8 @@ PassRows MTPHead::rows_of(int n) const {
 std::vector<shv_op> MTPHead::cell_ops(int n) const {
     std::vector<shv_op> ops = input_ops(n, nullptr, nullptr);
     auto a = attn_->Dispatches(layer_, x_, x_, rows_of(n), nullptr);
-    shv_attn_decode_args cells{};
-    std::memcpy(&cells, a[1].args, sizeof cells);
-    cells.out = nullptr;  // the rows' cells, nothing attended
-    ops.push_back(a[0]);
-    ops.push_back(make_op(SHV_OP_ATTN_DECODE, cells));
+    a[1].kind = SHV_OP_ATTN_CELLS;  // the rows' cells, nothing attended
+    ops.insert(ops.end(), a.begin(), a.begin() + 2);
     return ops;
 }
 

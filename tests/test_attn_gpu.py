@@ -247,3 +247,33 @@ def test_attn_refuses_unsupported_shapes(ctx):
     for bad in (dict(head_dim=128), dict(n_head=24), dict(n_splits=1000), dict(qkv_stride=100)):
         with pytest.raises(shv.pkg.ShvError):
             ctx.enqueue(A.OP_ATTN_DECODE, mk(**bad))
+
+
+@pytest.mark.parametrize("n_seq,seq_len,first", [(1, 1, 0), (3, 2, 31), (2, 5, 29), (1, 70, 60)])
+def test_cells_alone_are_the_pass_cells(ctx, n_seq, seq_len, first):
+    """The cells written without attending are those the attention's own launch writes, bit for bit, and no others; attending without
+    an output is refused."""
+    case = AttnCase(ctx, seed=5)
+    max_cells, n_splits, c, rows = 160, 2, ctx, n_seq * seq_len
+    case.upload(max_cells)
+    qkv = case.rng.standard_normal((rows, case.width)).astype(np.float32)
+    slot, pos = case.rng.permutation(4)[:n_seq].astype(np.int32), (first + np.arange(n_seq)).astype(np.int32)
+    d_qkv, d_slot, d_pos = c.upload(qkv), c.upload(slot), c.upload(pos)
+    d_part, d_ctx = c.alloc(_part_floats(n_seq, n_splits, seq_len) * 4), c.alloc(rows * NH * D * 4)
+    size = 4 * max_cells * NKV * D
+    got = []
+    for kind, part, out in ((A.OP_ATTN_DECODE, d_part.ptr, d_ctx.ptr), (A.OP_ATTN_CELLS, None, None)):
+        d_kc, d_vc = c.alloc(size * 2).zero(), c.alloc(size * 2).zero()
+        args = A.AttnDecodeArgs(d_qkv.ptr, case.d_qn.ptr, case.d_kn.ptr, case.d_rope.ptr, d_kc.ptr, d_vc.ptr, part, out, d_pos.ptr, d_slot.ptr,
+                                n_seq, seq_len, NH, NKV, D, ROPE, max_cells, case.width, n_splits, EPS)
+        c.dispatch_multi([A.make_op(kind, args)])
+        got.append((d_kc.read(np.uint16, size), d_vc.read(np.uint16, size)))
+        for gone in ("out", "partial"):
+            if kind == A.OP_ATTN_DECODE:
+                keep = getattr(args, gone)
+                setattr(args, gone, None)
+                with pytest.raises(A.ShvError, match="NULL argument"):
+                    c.enqueue(kind, args)
+                setattr(args, gone, keep)
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+    assert np.count_nonzero(got[1][0].reshape(4, max_cells, -1).any(axis=2)) == rows
