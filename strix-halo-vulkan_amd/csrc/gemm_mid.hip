@@ -20,7 +20,9 @@
 //   12352 x 2048   9: 20.3, now 9.7   16: 24.6, 9.9   150: 69.1, 28.2   255: 49.0, 40.5   512: 90, 72.5
 //    2048 x 4096   9: 16.0, now 8.4   16: 16.5, 8.4   150: 51.5, 18.6   255: 59.7, 23.5   512: 65, 37.1
 // Error against float64 of 4096 x 2048 over normal activations: 0.4e-6; of the kernels of 16 and of 64 rows 2.1e-6.
+#include <algorithm>
 #include <atomic>
+
 #include "gemm_rows.hpp"
 #include "moe_staged.hpp"
 
@@ -305,6 +307,13 @@ __global__ __launch_bounds__(512) void router_rows_kernel(const float *W, const 
     }
 }
 
+// How many of a pass's tiles a block walks, `blocks` of them side by side over the weight rows: as few as blocks on every compute
+// unit, one each, leave it (more blocks would form the weights again).
+int tiles_a_block(const shv_ctx *ctx, int tiles, int blocks) {
+    const int chunks = std::min(std::max(ctx->prop.multiProcessorCount / blocks, 1), tiles);
+    return (tiles + chunks - 1) / chunks;
+}
+
 template <int R, int S, int W>
 int launch(shv_ctx *ctx, const shv_gemv_q4k_args &a, int tiles) {
     constexpr size_t lds = static_cast<size_t>(W) * R * 2048;
@@ -316,11 +325,7 @@ int launch(shv_ctx *ctx, const shv_gemv_q4k_args &a, int tiles) {
         }
     }
     const int blocks = (a.n + 16 * R - 1) / (16 * R);
-    // the pass's tiles go to as many blocks as a chip of 256 compute units holds one each of: more would form the weights again
-    int chunks = 256 / blocks;
-    if (chunks < 1) chunks = 1;
-    if (chunks > tiles) chunks = tiles;
-    const int per = (tiles + chunks - 1) / chunks;
+    const int per = tiles_a_block(ctx, tiles, blocks);
     SHV_LAUNCH(ctx, (gemm_mid_kernel<R, S, W>), dim3(blocks, (tiles + per - 1) / per), dim3(64 * W), lds, a, static_cast<const char *>(ctx->gemm_stage), tiles, per);
     return SHV_OK;
 }
@@ -383,10 +388,7 @@ int shv_launch_router_rows(shv_ctx *ctx, const shv_moe_router_args &a) {
     const int rc = launch_stage(ctx, g, tiles, a.xn);
     if (rc != SHV_OK) return rc;
     constexpr int R = 2;
-    const int blocks = (n_rows + 16 * R - 1) / (16 * R);
-    int chunks = 256 / blocks;
-    if (chunks < 1) chunks = 1;
-    const int per = (tiles + chunks - 1) / chunks;
+    const int blocks = (n_rows + 16 * R - 1) / (16 * R), per = tiles_a_block(ctx, tiles, blocks);
     SHV_LAUNCH(ctx, (router_rows_kernel<R>), dim3(blocks, (tiles + per - 1) / per), dim3(512), 0, a.router, a.shared_gate, n_rows, a.n_embd, a.n_tok,
                static_cast<const char *>(ctx->gemm_stage), a.logits, a.n_expert + 1, tiles, per);
     return SHV_OK;
