@@ -17,8 +17,8 @@
 // 64 rows of 2048 columns, formed, are 256 of a compute unit's 512 KB, and forming them again for each tile costs what it saves.
 // us, with the staging launch, two dozen matrices in turn (n x k, rows), and what the launches of 16, of 64 rows and their joins
 // took that this kernel has replaced:
-//   12352 x 2048   9: 20.3, now 9.7   16: 24.6, 9.9   150: 69.1, 28.2   255: 49.0, 40.5   512: 90, 72.5
-//    2048 x 4096   9: 16.0, now 8.4   16: 16.5, 8.4   150: 51.5, 18.6   255: 59.7, 23.5   512: 65, 37.1
+//   12352 x 2048   9: 20.3, now 9.6   16: 24.6, 9.5   150: 69.1, 27.3   255: 49.0, 40   512: 90, 72.4
+//    2048 x 4096   9: 16.0, now 8.5   16: 16.5, 8.8   150: 51.5, 18.6   255: 59.7, 23.5   512: 65, 36.0
 // Error against float64 of 4096 x 2048 over normal activations: 0.4e-6; of the kernels of 16 and of 64 rows 2.1e-6.
 #include <algorithm>
 #include <atomic>
@@ -67,11 +67,8 @@ __global__ __launch_bounds__(256) void gemm_mid_stage_kernel(shv_gemv_q4k_args a
         const float sum = sum8_all((x[0] + x[1]) + (x[2] + x[3]));
         const int sub = c >> 5, kb = sub >> 1, v = (sub & 1) * 4 + ((c & 31) >> 3);
         const size_t at = static_cast<size_t>(blockIdx.z) * (K / 256) + sb;
-        if ((c & 31) == 0) {
-            uint16_t *sp = reinterpret_cast<uint16_t *>(staged + mid_sums_offset(tiles, K) + at * kMidSums + (kb * 16 + n) * 16) + (sub & 1);
-            bf16_parts(sum, sp[0], sp[2], sp[4]);
-            sp[6] = 0;
-        }
+        const float next = dpp_f32<kDppMirror>(sum);  // the sub-block's after it, which the next eight lanes hold
+        if ((c & 63) == 0) *reinterpret_cast<u32x4_t *>(staged + mid_sums_offset(tiles, K) + at * kMidSums + (kb * 16 + n) * 16) = bf16_parts_pair(sum, next);
         const float o[4] = {x[0], x[2], x[1], x[3]};
         half4_t h, l;
 #pragma unroll

@@ -45,7 +45,6 @@ constexpr int kDownUnits = 4;  // 64-row units of the down projection a wave tak
 constexpr int kChunk = 9 * 1024;
 constexpr int kRing = 2 * kChunk;  // a wave's LDS: a chunk being multiplied, the next on its way
 
-typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 typedef const __attribute__((address_space(1))) void *global_ptr_t;
 typedef __attribute__((address_space(3))) void *lds_ptr_t;
 typedef const __attribute__((address_space(3))) char *lds_bytes_t;

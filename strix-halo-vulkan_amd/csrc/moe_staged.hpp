@@ -16,6 +16,7 @@ typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kStSubBytes = 128;  // a row's sub-block: 2 parts x 4 column blocks x 16 bytes
@@ -35,6 +36,13 @@ __device__ __forceinline__ void bf16_parts(float v, uint16_t &p0, uint16_t &p1, 
     p0 = static_cast<uint16_t>(b0 >> 16);
     p1 = static_cast<uint16_t>(b1 >> 16);
     p2 = static_cast<uint16_t>(__float_as_uint(r2) >> 16);
+}
+// The parts of two values side by side: first parts, second, third, two zeros.
+__device__ __forceinline__ u32x4_t bf16_parts_pair(float a, float b) {
+    uint16_t a0, a1, a2, b0, b1, b2;
+    bf16_parts(a, a0, a1, a2);
+    bf16_parts(b, b0, b1, b2);
+    return u32x4_t{a0 | static_cast<uint32_t>(b0) << 16, a1 | static_cast<uint32_t>(b1) << 16, a2 | static_cast<uint32_t>(b2) << 16, 0u};
 }
 // Two whole numbers below 256 (a sub-block's min is below 64) as a pair of bfloat16 values, exact.
 __device__ __forceinline__ uint32_t bf16_pair(uint32_t a, uint32_t b) {
@@ -69,8 +77,8 @@ __device__ __forceinline__ void binary16_parts(float u, _Float16 &hi, _Float16 &
     lo = fabsf(u) < INFINITY ? static_cast<_Float16>(u - static_cast<float>(hi)) : static_cast<_Float16>(0.f);  // an infinity is all in hi
 }
 
-// Four columns c .. c + 3 of row t for the list kernels, e the row's exponent, and (the lane of a sub-block's first columns)
-// the sub-block's sum; the eight lanes of a sub-block are neighbours and all here.
+// Four columns c .. c + 3 of row t for the list kernels, e the row's exponent, and (the lane of the first of 64)
+// the sums of two sub-blocks; the sixteen lanes of the two are neighbours and all here.
 __device__ __forceinline__ void stage_list_quad(const float4 v, int e, int t, int c, int k, int rows, char *staged) {
     const float o[4] = {ldexpf(v.x, kListOne - e), ldexpf(v.z, kListOne - e), ldexpf(v.y, kListOne - e), ldexpf(v.w, kListOne - e)};
     half4_t h, l;
@@ -85,7 +93,12 @@ __device__ __forceinline__ void stage_list_quad(const float4 v, int e, int t, in
     *reinterpret_cast<half4_t *>(at) = h;
     *reinterpret_cast<half4_t *>(at + 64) = l;
     const float sum = shv::sum8_all((o[0] + o[2]) + (o[1] + o[3]));
-    if ((c & 31) == 0) list_sum_put(staged + staged_sums_offset(rows, k) + (static_cast<size_t>(t) * (k / 256) + (c >> 8)) * kListSumBytes, c >> 5, sum);
+    const u32x4_t p = bf16_parts_pair(sum, shv::dpp_f32<shv::kDppMirror>(sum));  // and of the sub-block after it, which the next eight lanes hold
+    if ((c & 63) == 0) {
+        char *sums = staged + staged_sums_offset(rows, k) + (static_cast<size_t>(t) * (k / 256) + (c >> 8)) * kListSumBytes + ((c >> 6) & 3) * 8;
+        *reinterpret_cast<u32x2_t *>(sums) = u32x2_t{p.x, p.y};
+        *reinterpret_cast<u32x2_t *>(sums + 32) = u32x2_t{p.z, p.w};
+    }
 }
 
 // The masks and exponents of the two nibble positions a weight is read from.
