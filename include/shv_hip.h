@@ -155,7 +155,10 @@ enum {
  * y + (slot[s]*ring_slots + (pos[s]+i) % ring_slots) * ring_stride, slot[s] = s when slot is NULL,
  * instead of y + t*y_stride.  z_ring != 0 reads the prologue's z row from the same ring
  * geometry instead (z + (slot*ring_slots + (pos+i) % ring_slots) * ring_stride) and leaves y
- * plain: the DeltaNet output projection takes its gate z from the projection ring. */
+ * plain: the DeltaNet output projection takes its gate z from the projection ring.
+ * Range: up to four rows any float32; from five on the rows enter the matrix cores, after the
+ * prologue, as binary16 pairs: values up to 65504, and in passes past 512 rows the sums of 32
+ * neighbours too.  (shv_gemv_mrows' kernel, two to eight rows, scales them.) */
 typedef struct {
     const void *w;
     const float *x;
@@ -305,10 +308,12 @@ typedef struct {
  * When logits is given ([T][n_expert+1] from a router run with defer_route) every block first
  * routes its token from them exactly as the router would, and the selection is also stored to
  * topk [T][n_used] and weights [T][n_used+1] for the down projection; otherwise topk is read.
- * A pass of many rows (128 and more; SHV_MOE_GROUP_MIN) whose topk is given, with n_expert stated
+ * A pass of many rows (128 and more, or 65 and more where experts have 0.75 to 15 tokens each;
+ * SHV_MOE_GROUP_MIN) whose topk is given, with n_expert stated
  * and a `group` workspace of 2 * n_expert + 1 + T * n_used ints, is grouped by expert on the matrix
- * cores: an expert's weights are read once per 48 tokens that chose it (the prompt arm of
- * llm_moe_gemv.comp). */
+ * cores: an expert's weights are read once per 8 to 48 tokens that chose it (the prompt arm of
+ * llm_moe_gemv.comp).  Range: with up to 15 tokens an expert any float32 xn and act; with more, or with act as
+ * floats from 128 rows on, values and sums of 32 neighbours up to 65504, and values below 1e-3 lose bits. */
 typedef struct {
     const float *xn;
     int32_t *topk;
@@ -329,8 +334,8 @@ typedef struct {
                                 left logits[n_expert] unwritten), and weights[t][n_used] is stored as 0,
                                 as the router's own selection stores it */
     int32_t act_packed;      /* grouped path only: act is left as the matrix-core operands the grouped
-                                shv_moe_down reads (two binary16 parts of every value, same bytes a row)
-                                instead of floats; the shv_moe_down of this pass must be the library's
+                                shv_moe_down reads (two binary16 parts of every value, same bytes a row,
+                                sums and exponents in the library's scratch) instead of floats; the shv_moe_down of this pass must be the library's
                                 next call on the stream, with act_packed and group_ready set too */
     const float *gamma;      /* with logits, up to four rows: xn is the row BEFORE its RMSNorm and logits are the
                                 router's products without the norm's factor (shv_gemv_q4k's fold_out);

@@ -1316,10 +1316,15 @@ int shv_launch_gemm_q4k(shv_ctx *ctx, const shv_gemv_q4k_args &a) {
         SHV_REQUIRE(groups * wide_region(a.k) <= static_cast<size_t>(shv_ctx::kGemmStageBytes), "gemm_q4k: %d rows of %d columns do not fit the staging buffer", a.n_tok, a.k);
         SHV_LAUNCH(ctx, gemm_wide_stage_kernel, dim3(stage_parts(a, groups), kWideTok / 4, groups), dim3(256), 0, a, ctx->gemm_stage);
         if (groups >= 4) {
-            // Blocks of 256 rows and two groups form each weight once for 128 activation rows: an eighth less work in all (9216 x
-            // 2048 of 4096 rows 403 -> 380 us, 2048 x 4096 203 -> 180), when their rounds of the chip, one a compute unit, leave
-            // no more of it idle than the rounds of the blocks of 128 rows and one group, two a unit, do (12352 x 2048 of 2048
-            // rows 278 so and 290 with two groups).
+            // Blocks of 256 rows and two groups form each weight once for 128 activation rows: up to an eighth less work in all,
+            // where their rounds of the chip, one a compute unit, leave no more of it idle than the rounds of the blocks of 128
+            // rows and one group, two a unit, do.  us with one group / with two, over eight matrices in turn, the taken one first:
+            //              576 rows     768         1024        1531        2048        3000        4096
+            //   12352x2048 80 <- 92     112 <- 144  142 <- 150  211 <- 215  272 <- 280  364 <- 436  514 <- 524  (two, one, two, one, one, two, two)
+            //    9216x2048 72 <- 74      76 <- 90   111 <- 142  144 <- 153  196 <- 213  337 <- 285  369 <- 389  (two, two, one, two, one, one, two)
+            //    2048x4096 59 <- 130     58 <- 130   61 <- 130   87 <- 134  100 <- 137  143 <- 160  165 <- 190  (one up to 2048, two from there)
+            // The factor lies between the quotients of 9216 x 2048 of 4096 rows, 1.11, and of 12352 x 2048 of 2048, 1.13; of these
+            // shapes one, 9216 x 2048 of 3000 rows at 1.14, comes out wrong.
             const int cus = ctx->prop.multiProcessorCount;
             const auto filled = [](long long blocks, int slots) { return static_cast<double>(blocks) / static_cast<double>((blocks + slots - 1) / slots * slots); };
             const int pairs = (groups + 1) / 2;

@@ -1,7 +1,8 @@
 // y = W x for a weight matrix in any tensor type the reference's loader accepts: the CPU path's
 // matvec over Tensor.DequantizeRow (llm/hc.go:255-264, gguf/dequant.go:119-124) for the tensors
 // of a checkpoint that are not Q4_K (a UD-Q4_K_XL file keeps dense projections in Q8_0 and some
-// banks in Q5_K / Q6_K).  HBM-bound like the Q4_K kernel, not yet tuned like it (Q6_K and Q8_0 of 2048 columns go to gemv_q68.hip): a lane takes one
+// banks in Q5_K / Q6_K).  HBM-bound like the Q4_K kernel, not yet tuned like it (Q6_K and Q8_0 of
+// 2048 columns go to gemv_q68.hip): a lane takes one
 // 32-element group of a row, dequantises it exactly as the format's CPU arm does and multiplies
 // it with its 32 activations from LDS; a wave owns a row at a time and adds the lanes up.
 #include "group_dot.hpp"

@@ -388,8 +388,9 @@ int launch(shv_ctx *ctx, const shv_gemv_args &a) {
 
 }  // namespace
 
-// Columns whose activations, 96 registers of every wave, leave room for the rest (twice as many would not), and rows of x that
-// 16-byte loads can read.
+// The one row length that is built: a wave's 256 columns of it are 96 registers of activations, which leave room for the rest.
+// (4096 columns would take sixteen waves, or twice the registers; fewer columns fewer waves: neither has been built or measured,
+// such matrices go lane by lane, gemv_any.hip.)  And rows of x that 16-byte loads can read.
 bool shv_gemv_q68_covers(const shv_gemv_args &a) {
     if ((a.type != SHV_GGML_Q6_K && a.type != SHV_GGML_Q8_0) || a.k != 2048) return false;
     return shv_aligned16(a.x) && (!a.gamma || shv_aligned16(a.gamma)) && (a.n_tok <= 1 || a.x_stride % 4 == 0);

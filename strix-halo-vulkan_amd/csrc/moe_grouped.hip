@@ -2,19 +2,25 @@
 // MoETrace.Experts, llm/moe.go:289-409; the reference batches a chunk's tokens per expert in
 // llm_moe_gemv.comp's multi-row arm).  The per-(token, expert) GEMV reads and unpacks an expert's
 // weights once per token that chose it, this path once per 48 such tokens: it pays when tokens
-// outnumber experts (2048 rows choosing 10 of 512: 40 tokens an expert), not at 64 rows (1.9).
+// outnumber experts (2048 rows choosing 10 of 512: 40 tokens an expert).  Passes whose experts have
+// up to fifteen tokens each go on from the same lists in moe_lists.hip.
 //
 //   moe_group_kernel          per-expert lists of (token, slot) pairs from topk (one block; long passes:
 //                             moe_group_count_kernel + moe_group_place_kernel, sixteen blocks)
+//   moe_stage_kernel          xn made into matrix-core operands once: two halves hi + lo of every
+//                             value as it is, and of every sub-block's sum (both within 65504)
 //   moe_up_grouped_kernel     a block = (expert, half of its ffn rows) and up to 48 of its tokens
-//                             at a time: their xn rows go through LDS as matrix-core operands
-//                             (two halves hi + lo, as the projections do) in slabs of 512 columns,
-//                             each wave streams two gate tiles of 16 rows and the matching up
-//                             tiles, forms a sub-block's weights once (as the whole numbers n * sc,
-//                             exact in binary16) for all three token tiles, keeps one matrix
-//                             accumulator per super-block, SwiGLU in registers, act[pair] out
-//   moe_down_grouped_kernel   a block = (expert, quarter of n_embd rows): act rows staged the
-//                             same way (one slab), each wave two tiles, raw products to pairs[pair]
+//                             at a time: their staged rows come to LDS in slabs of 256 columns (by
+//                             the loads themselves, the next slab under this one's products), each
+//                             wave streams two gate tiles of 16 rows and the matching up tiles,
+//                             forms a sub-block's weights once (as the whole numbers n * sc, exact
+//                             in binary16) for all three token tiles, keeps one matrix accumulator
+//                             per super-block, SwiGLU in registers, act[pair] out: as operands
+//                             (act_packed) or floats
+//   moe_down_staged_kernel    a block = (expert, quarter of n_embd rows) over act rows that are
+//                             operands, four row tiles a wave, raw products to pairs[pair]
+//   moe_down_grouped_kernel   the same over act rows that are floats, made into operands by the
+//                             block, 512 columns (a whole row) at a time
 //   moe_combine_kernel        out[t] = residual[t] + sum over slots of weights[t][s]*pairs[t][s],
 //                             slots in order
 // The shared expert is an expert every token lists: its blocks take 48 tokens each.
