@@ -465,6 +465,36 @@ def test_checkpoint_restore_is_the_shorter_sequence(rig):
     m.checkpoint_free(c)
 
 
+def test_checkpoint_of_another_model_is_restored_after_that_one_is_closed(rig):
+    """A checkpoint holds nothing of the model it came from: one of the same weights takes it up, again after the first is gone, and
+    its carry is not what the owner writes when it takes its next one."""
+    m, cfg, _ = rig
+    rng = np.random.default_rng(78)
+    head, tail, other = (rng.integers(0, cfg.vocab, size=n).astype(np.int32) for n in (6, 4, 5))
+    fresh(m)
+    m.extend(head, want_logits=False)
+    want = [m.extend(np.array([t], np.int32))[0] for t in tail]
+    twin = LA.LLM(cfg)
+    twin.init_synthetic(4321)
+    twin.stage()
+    twin.extend(head, want_logits=False)
+    c = twin.checkpoint()
+    twin.extend(other, want_logits=False)
+    later = twin.checkpoint()
+    for closed in (False, True):
+        fresh(m)
+        m.extend(head, want_logits=False)  # the cells are the caller's own
+        m.extend(other, want_logits=False)
+        m.restore(c)
+        got = [m.extend(np.array([t], np.int32))[0] for t in tail]
+        for g, w in zip(got, want):
+            assert np.array_equal(g, w), closed
+        if not closed:
+            twin.checkpoint_free(later)
+            twin.close()
+    m.checkpoint_free(c)
+
+
 def test_chunk_size_does_not_matter_over_4096_tokens():
     """BASELINE's prefill shape: 4096 tokens through a period of three DeltaNet layers and one
     attention layer at the full widths, as one pass of 4096, in chunks of 2048 (either way every
