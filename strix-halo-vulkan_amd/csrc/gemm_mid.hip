@@ -340,15 +340,15 @@ int launch_stage(shv_ctx *ctx, const shv_gemv_q4k_args &a, int tiles, float *x_o
 
 }  // namespace
 
-// From nine rows, where the kernels that form every weight once for up to eight of them end, to 512, but for 17 to 64, which
-// keep the kernel of one 64-row group.  That kernel is the slower there (12352 x 2048 of 64 rows 27.7 us, 17.9 here) and the less
-// exact (2.1e-6 against 0.4e-6): the line is one of results that stay what they were, since a prompt of that height is one pass
-// whose routing, where a token's tenth expert and its eleventh are level, every token decoded after it carries on.  Past 512 the blocks
-// that share their activations through LDS have rows enough for every compute unit and read less from L2 (9216 x 2048 of
-// 1024 rows: 114 us there, 133 here; of 512: 75 there, 73 here).
+// From nine rows, where the kernels that form every weight once for up to eight of them end, to 512, but for 49 to 64, which
+// keep the kernel of one 64-row group.  That kernel is the slower there (12352 x 2048 of 64 rows 27.7 us, 15.9 here; of 40 rows 24.1
+// and 13.8, of 17 20.6 and 12.4; 2048 x 4096 of 40 rows 17.9 and 11.0) and the less exact (2.1e-6 against 0.4e-6): the line is one of
+// results that stay what they were, since a prompt's whole chunk of 64 rows is one pass whose routing, where a token's tenth expert and
+// its eleventh are level, every token decoded after it carries on (48 layers: the logits after 96 tokens parted by 1e-4 to 2e-3).
+// Past 512 gemm_long.hip's blocks read less from L2.
 bool shv_gemm_mid_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a) {
     if (!ctx->gemm_stage || (a.k != 2048 && a.k != 4096) || a.n_tok < 9 || a.n_tok > 512) return false;
-    if (a.n_tok > 16 && a.n_tok <= 64) return false;
+    if (a.n_tok > 48 && a.n_tok <= 64) return false;
     if (a.prologue == SHV_PRO_GATED_NORM && 256 % a.head_dim != 0) return false;
     return mid_bytes((a.n_tok + 15) / 16, a.k) <= static_cast<size_t>(shv_ctx::kGemmStageBytes);
 }

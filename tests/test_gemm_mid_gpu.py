@@ -44,6 +44,12 @@ def test_rows_of_a_pass(n, k, rows):
         ctx.destroy()
 
 
+@pytest.mark.parametrize("n,k,rows", [(300, 2048, 17), (2055, 4096, 33), (12352, 2048, 48), (2048, 4096, 49)])
+def test_rows_of_a_short_prompt(n, k, rows):
+    """17 to 48 rows take these kernels too; 49 the kernel of one 64-row group."""
+    test_rows_of_a_pass(n, k, rows)
+
+
 @pytest.mark.parametrize("rows,H,E", [(128, 256, 7), (129, 1024, 31), (145, 2304, 64), (2001, 512, 32)])
 def test_router_logits_of_a_long_pass(rows, H, E):
     """Columns of one super-block, of fewer than the block's waves and of more; router rows (the experts and the shared
