@@ -637,7 +637,7 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(shv_gemv_q4k_ar
     }
 }
 
-// ---------------------------------------------------------------- passes of 17 to 64 rows -------
+// ---------------------------------------------------------------- passes of 49 to 64 rows, and of other widths than gemm_mid.hip's from 17 to 192 -------
 // A prompt chunk has more rows than one block can keep in LDS for the whole width of the matrix,
 // so its operands stream: the activations of 64 rows are made once into `staged` as slabs of 128
 // columns (four sub-blocks), each slab in the order the products read it, and every block of the
@@ -651,12 +651,7 @@ constexpr int kWideFrag = 64 * 16;                           // one operand: a l
 constexpr int kWideSlabA = 4 * 4 * 2 * kWideFrag;            // [sub-block 4][token tile 4][hi, lo]
 constexpr int kWideSlab = kWideSlabA + 4 * kWideTok * 4;     // + the sub-blocks' sums of x
 
-// After a group's slabs, the same sums as operands of the min term: for every 1024 columns (four
-// super-blocks) a fragment per (token tile, part): lane = token in the tile + 16 * (super-block of
-// the four), the super-block's eight sums' binary16 values (part 0) and what those leave (part 1).
-constexpr int kWideSumFrags = 4 * 2 * kWideFrag;
-__host__ __device__ constexpr size_t wide_sums_offset(int k) { return static_cast<size_t>(k / 128) * kWideSlab; }
-__host__ __device__ constexpr size_t wide_region(int k) { return wide_sums_offset(k) + static_cast<size_t>((k + 1023) / 1024) * kWideSumFrags; }
+__host__ __device__ constexpr size_t wide_region(int k) { return static_cast<size_t>(k / 128) * kWideSlab; }
 
 // The same for a pass of up to 64 rows a group, in the slab order gemm_wide_kernel streams.
 // grid: (parts of the k/256 column blocks, 16 quartets of rows, groups of 64 rows), 256 threads: a wave takes one row's 64
@@ -692,14 +687,7 @@ __global__ __launch_bounds__(256) void gemm_wide_stage_kernel(shv_gemv_q4k_args 
         sum += __shfl_xor(sum, 1, 64);
         sum += __shfl_xor(sum, 2, 64);
         sum += __shfl_xor(sum, 4, 64);
-        if ((c & 31) == 0) {
-            reinterpret_cast<float *>(slab + kWideSlabA)[sub * kWideTok + tl] = sum;
-            const _Float16 hi = static_cast<_Float16>(sum);
-            _Float16 *sp = reinterpret_cast<_Float16 *>(region + wide_sums_offset(K) + static_cast<size_t>(((c >> 10) * 4 + (tl >> 4)) * 2) * kWideFrag +
-                                                        (((c >> 8) & 3) * 16 + (tl & 15)) * 16) + ((c >> 5) & 7);
-            sp[0] = hi;
-            sp[kWideFrag / 2] = static_cast<_Float16>(sum - static_cast<float>(hi));
-        }
+        if ((c & 31) == 0) reinterpret_cast<float *>(slab + kWideSlabA)[sub * kWideTok + tl] = sum;
         // slot order of a lane's eight columns: [0, 2, 1, 3, 4, 6, 5, 7]
         const float o[4] = {x[0], x[2], x[1], x[3]};
         half4_t h, l;
@@ -891,234 +879,6 @@ __global__ __launch_bounds__(NW * 64) void gemm_wide_kernel(shv_gemv_q4k_args a,
     }
 }
 
-// The same product for a pass of many groups, every group in one launch, with the second operand
-// formed as the experts' grouped kernels form theirs: a sub-block's eight weights a lane become the
-// whole numbers n * sc (exact in binary16), one matrix accumulator runs over a super-block and takes
-// its d at the end, and the min term is the only per-sub-block vector work: half the vector
-// instructions per matrix instruction of the kernel above, and no branch inside a step.
-// grid: (row blocks of NW*R*16 rows) x bundles of TG groups; all token tiles are multiplied whatever the
-// groups hold (rows they do not have were staged as zeros).
-template <int NW, int R, int TG>
-__global__ __launch_bounds__(NW * 64) void gemm_pass_kernel(shv_gemv_q4k_args a, const char *staged_all, int groups) {
-    extern __shared__ __align__(16) char smem[];
-    char *sumf = smem + 2 * TG * kWideSlab;   // the sums of the quarter of the columns in hand, as operands
-    size_t *yoffs = reinterpret_cast<size_t *>(sumf + TG * kWideSumFrags);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int n = lane & 15, kb = lane >> 4;
-    const int sbs = a.k / SHV_Q4K_BLOCK;
-    const size_t row_bytes = static_cast<size_t>(sbs) * SHV_Q4K_BYTES;
-    const int bundles = (groups + TG - 1) / TG, grp = blockIdx.x % bundles * TG, xb = blockIdx.x / bundles;
-    const int t0 = grp * kWideTok;
-    const int nt = a.n_tok - t0 < TG * kWideTok ? a.n_tok - t0 : TG * kWideTok;
-    const char *staged[TG];
-#pragma unroll
-    for (int u = 0; u < TG; u++) staged[u] = staged_all + static_cast<size_t>(grp + u < groups ? grp + u : grp) * wide_region(a.k);  // past the last: one again, not stored
-    const int row0 = (xb * NW + wave) * (R * kTileRows);
-    const int steps = a.k / 128;
-
-    const char *rp[R];
-    uint4 hdr[R], hdrn[R];
-    uint2 q[R][2], qn[R][2];
-    // step s: the 128 columns s*128.. of the row = groups 2(s&1), 2(s&1)+1 of super-block s>>1
-    auto load_q = [&](int s, uint2 (&dst)[R][2]) {
-#pragma unroll
-        for (int r = 0; r < R; r++)
-#pragma unroll
-            for (int g = 0; g < 2; g++)
-                dst[r][g] = *reinterpret_cast<const uint2 *>(rp[r] + static_cast<size_t>(s >> 1) * SHV_Q4K_BYTES + 16 + ((s & 1) * 2 + g) * 32 + kb * 8);
-    };
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        const int row = row0 + r * kTileRows + n;
-        rp[r] = static_cast<const char *>(a.w) + static_cast<size_t>(row < a.n ? row : a.n - 1) * row_bytes;
-        hdr[r] = *reinterpret_cast<const uint4 *>(rp[r]);
-    }
-    load_q(0, q);
-    if (tid < nt) yoffs[tid] = out_offset(a, t0 + tid);
-    // A slab is 33 pieces of 1 KB that lie in `staged` as they will in LDS: the loads place them
-    // there themselves (lane l's 16 bytes at 16 l of the piece), through no register.
-    constexpr int kPieces = kWideSlab / 1024;
-    static_assert(kPieces * 1024 == kWideSlab, "whole pieces");
-    auto ask_slab = [&](int s, char *buf) {
-#pragma unroll
-        for (int u = 0; u < TG; u++) {
-            const char *src = staged[u] + static_cast<size_t>(s) * kWideSlab + lane * 16;
-            for (int c = wave; c < kPieces; c += NW)
-                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(src + c * 1024),
-                                                 (__attribute__((address_space(3))) void *)(buf + u * kWideSlab + c * 1024), 16, 0, 0);
-        }
-    };
-    // the min term of columns [1024 qt, 1024 qt + 1024): the tokens' sums (wave w asks for fragment w of eight) and this lane's
-    // rows' headers of super-block 4 qt + kb, both a step ahead of their use
-    static_assert(NW >= 8, "a fragment of sums a wave");
-    uint4 hq[R];
-    auto ask_quarter = [&](int qt) {
-        if (wave < 8) {
-#pragma unroll
-            for (int u = 0; u < TG; u++)
-                __builtin_amdgcn_global_load_lds(
-                    (const __attribute__((address_space(1))) void *)(staged[u] + wide_sums_offset(a.k) + static_cast<size_t>(qt * 8 + wave) * kWideFrag + lane * 16),
-                    (__attribute__((address_space(3))) void *)(sumf + u * kWideSumFrags + wave * kWideFrag), 16, 0, 0);
-        }
-        const int sb = 4 * qt + kb < sbs ? 4 * qt + kb : 0;
-#pragma unroll
-        for (int r = 0; r < R; r++) hq[r] = *reinterpret_cast<const uint4 *>(rp[r] + static_cast<size_t>(sb) * SHV_Q4K_BYTES);
-    };
-    ask_slab(0, smem);
-    ask_quarter(0);
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    __syncthreads();
-
-    const NibbleConsts nc = nibble_consts();
-    uint32_t m0 = 0x000F000Fu, o0 = 0x64006400u;   // bits 0..3 of both halves under the exponent of 1024
-    asm volatile("" : "+s"(m0));
-    asm volatile("" : "+v"(o0));
-    float4_t y[R][4 * TG], acc[R][4 * TG];
-#pragma unroll
-    for (int r = 0; r < R; r++)
-#pragma unroll
-        for (int tt = 0; tt < 4 * TG; tt++) y[r][tt] = acc[r][tt] = float4_t{0.f, 0.f, 0.f, 0.f};
-
-    for (int s = 0; s < steps; s++) {
-        const int cur = s & 1;
-        const bool more = s + 1 < steps;
-        {
-            const int sn = more ? s + 1 : s;
-            if (more) ask_slab(sn, smem + (cur ^ 1) * (TG * kWideSlab));   // the other buffer was read to its end before the barrier that ended the last step
-            if (more && (sn & 7) == 0) {
-                // the sums in LDS were read at this quarter's first step, steps ago; every wave is past that
-                ask_quarter(sn >> 3);
-            }
-            load_q(sn, qn);
-            if (s & 1) {
-#pragma unroll
-                for (int r = 0; r < R; r++) hdrn[r] = *reinterpret_cast<const uint4 *>(rp[r] + static_cast<size_t>(sn >> 1) * SHV_Q4K_BYTES);
-            }
-        }
-        const char *A = smem + cur * (TG * kWideSlab);
-        if ((s & 7) == 0) {
-            // y -= sum over the quarter's sub-blocks of dmin * m * sum(x), as three matrix products a token tile:
-            // -dmin * m has 17 significant bits and goes as two halves, the sums come as two halves too
-            // (the small halves' product is below float32's last bit)
-            const bool on = 4 * (s >> 3) + kb < sbs;
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                const float nd = on ? -f16_bits_to_f32(hq[r].x >> 16) : 0.f;
-                const uint32_t m03 = hq[r].z & 0x3F3F3F3Fu, m47 = ((hq[r].w >> 4) & 0x0F0F0F0Fu) | ((hq[r].z >> 2) & 0x30303030u);
-                half8_t bh, bl;
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const float p = nd * static_cast<float>(((j < 4 ? m03 : m47) >> (8 * (j & 3))) & 0xFFu);
-                    const _Float16 hi = static_cast<_Float16>(p);
-                    bh[j] = hi;
-                    bl[j] = static_cast<_Float16>(p - static_cast<float>(hi));
-                }
-#pragma unroll
-                for (int tt = 0; tt < 4 * TG; tt++) {
-                    half8_t sh = *reinterpret_cast<const half8_t *>(sumf + (tt * 2) * kWideFrag + lane * 16);
-                    half8_t sl = *reinterpret_cast<const half8_t *>(sumf + (tt * 2 + 1) * kWideFrag + lane * 16);
-                    if (!on) sh = sl = static_cast<half8_t>(static_cast<_Float16>(0.f));   // a super-block past the row: nothing was staged there
-                    y[r][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(sh, bh, y[r][tt], 0, 0, 0);
-                    y[r][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(sl, bh, y[r][tt], 0, 0, 0);
-                    y[r][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(sh, bl, y[r][tt], 0, 0, 0);
-                }
-            }
-        }
-#pragma unroll
-        for (int g = 0; g < 2; g++) {
-            uint32_t sc[R];
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                uint32_t mn;
-                q4k_group_scale_min(hdr[r], (s & 1) * 2 + g, sc[r], mn);
-            }
-#pragma unroll
-            for (int hi = 0; hi < 2; hi++) {
-                const int sub = g * 2 + hi;
-                half8_t b[R];
-#pragma unroll
-                for (int r = 0; r < R; r++) {
-                    const uint32_t q0 = q[r][g].x, q1 = q[r][g].y;
-                    typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-                    // A nibble in the low bits of a half's mantissa reads, under the right exponent, as
-                    // C + n: bits 0..3 under 1024's, bits 4..7 under 64's (the odd bytes' nibbles take
-                    // one shift down there).  One fused multiply-add then makes (C + n) * sc - C * sc =
-                    // n * sc: a whole number up to 15 * 63, exact in binary16, as are C * sc.
-                    // slot order of the eight columns: bytes [0, 2, 1, 3, 4, 6, 5, 7]
-                    const _Float16 s1 = static_cast<_Float16>(static_cast<float>(hi ? sc[r] >> 8 : sc[r] & 0xFFu));
-                    const half2_t s2 = {s1, s1};
-                    half2_t w[4], c[4];
-                    if (hi == 0) {
-                        w[0] = __builtin_bit_cast(half2_t, (q0 & m0) | o0); w[1] = __builtin_bit_cast(half2_t, ((q0 >> 4) & nc.mask) | nc.one);
-                        w[2] = __builtin_bit_cast(half2_t, (q1 & m0) | o0); w[3] = __builtin_bit_cast(half2_t, ((q1 >> 4) & nc.mask) | nc.one);
-                        c[0] = c[2] = s2 * static_cast<half2_t>(static_cast<_Float16>(-1024.f));
-                        c[1] = c[3] = s2 * static_cast<half2_t>(static_cast<_Float16>(-64.f));
-                    } else {
-                        w[0] = __builtin_bit_cast(half2_t, (q0 & nc.mask) | nc.one); w[1] = __builtin_bit_cast(half2_t, ((q0 >> 8) & nc.mask) | nc.one);
-                        w[2] = __builtin_bit_cast(half2_t, (q1 & nc.mask) | nc.one); w[3] = __builtin_bit_cast(half2_t, ((q1 >> 8) & nc.mask) | nc.one);
-                        c[0] = c[1] = c[2] = c[3] = s2 * static_cast<half2_t>(static_cast<_Float16>(-64.f));
-                    }
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const half2_t p = __builtin_elementwise_fma(w[i], s2, c[i]);
-                        b[r][2 * i] = p[0];
-                        b[r][2 * i + 1] = p[1];
-                    }
-                }
-#pragma unroll
-                for (int tt = 0; tt < 4 * TG; tt++) {
-                    const char *f = A + (tt >> 2) * kWideSlab + static_cast<size_t>((sub * 4 + (tt & 3)) * 2) * kWideFrag + lane * 16;
-                    const half8_t xh = *reinterpret_cast<const half8_t *>(f);
-                    const half8_t xl = *reinterpret_cast<const half8_t *>(f + kWideFrag);
-#pragma unroll
-                    for (int r = 0; r < R; r++) {
-                        acc[r][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, b[r], acc[r][tt], 0, 0, 0);
-                        acc[r][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, b[r], acc[r][tt], 0, 0, 0);
-                    }
-                }
-            }
-        }
-        if (s & 1) {
-            // the super-block ends: its sums take its d, the next one's header moves in
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                const float dd = f16_bits_to_f32(hdr[r].x);
-#pragma unroll
-                for (int tt = 0; tt < 4 * TG; tt++) {
-#pragma unroll
-                    for (int j = 0; j < 4; j++) y[r][tt][j] = fmaf(dd, acc[r][tt][j], y[r][tt][j]);
-                    acc[r][tt] = float4_t{0.f, 0.f, 0.f, 0.f};
-                }
-                hdr[r] = hdrn[r];
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < R; r++)
-#pragma unroll
-            for (int g = 0; g < 2; g++) q[r][g] = qn[r][g];
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's pieces of the next slab have landed, then everybody's
-        __syncthreads();
-    }
-
-    // C[token 16 tt + 4 kb + j][row n] of each tile
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        const int row = row0 + r * kTileRows + n;
-        if (row >= a.n) continue;
-#pragma unroll
-        for (int tt = 0; tt < 4 * TG; tt++) {
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int tok = tt * kTileRows + 4 * kb + j;
-                if (tok >= nt) continue;
-                float v = y[r][tt][j];
-                if (a.residual) v += a.residual[static_cast<size_t>(t0 + tok) * a.y_stride + row];
-                a.y[yoffs[tok] + row] = v;
-            }
-        }
-    }
-}
-
 // The column parts of a split product added up in a fixed order.  grid: (ceil(n/256), nt), one
 // wave a block; a thread takes four neighbouring outputs, with 16-byte moves when the row count
 // and the addresses allow them.
@@ -1267,23 +1027,6 @@ bool rows_kernel_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a) {
     return true;
 }
 
-// Every group of 64 rows of a long pass in one launch (the operands of all of them are in
-// ctx->gemm_stage): no split along the columns, the groups themselves fill the chip.
-template <int NW, int R, int TG>
-int launch_wide_all(shv_ctx *ctx, const shv_gemv_q4k_args &a, int groups) {
-    constexpr int kRows = NW * R * kTileRows;
-    const int bx = (a.n + kRows - 1) / kRows;
-    const size_t lds = TG * (2 * kWideSlab + kWideSumFrags + kWideTok * sizeof(size_t));
-    static std::atomic<bool> raised{false};
-    if (!raised.load(std::memory_order_acquire)) {
-        SHV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_pass_kernel<NW, R, TG>), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-        raised.store(true, std::memory_order_release);
-    }
-    SHV_REQUIRE(static_cast<long long>(bx) * groups <= 0x7fffffffll, "gemm_q4k: %d row blocks of %d groups", bx, groups);
-    SHV_LAUNCH(ctx, (gemm_pass_kernel<NW, R, TG>), dim3(bx * ((groups + TG - 1) / TG)), dim3(NW * 64), lds, a, static_cast<const char *>(ctx->gemm_stage), groups);
-    return SHV_OK;
-}
-
 }  // namespace
 
 // Whether the matrix-core kernel takes this call: arguments are already validated by the GEMV's
@@ -1307,6 +1050,7 @@ bool shv_gemm_q4k_covers(const shv_gemv_q4k_args &a) {
 
 int shv_launch_gemm_q4k(shv_ctx *ctx, const shv_gemv_q4k_args &a) {
     if (rows_kernel_covers(ctx, a)) return a.k == 2048 ? launch_rows_k<2048, 3>(ctx, a) : launch_rows_k<4096, 1>(ctx, a);
+    if (shv_gemm_long_covers(ctx, a)) return shv_launch_gemm_long(ctx, a);
     if (shv_gemm_mid_covers(ctx, a)) return shv_launch_gemm_mid(ctx, a);
     // the fragments of 16 rows of 4096 columns do not fit LDS: such a pass goes 8 rows at a time
     const int cap = a.k > 2048 ? 8 : 16;
@@ -1315,22 +1059,6 @@ int shv_launch_gemm_q4k(shv_ctx *ctx, const shv_gemv_q4k_args &a) {
         const int groups = (a.n_tok + kWideTok - 1) / kWideTok;
         SHV_REQUIRE(groups * wide_region(a.k) <= static_cast<size_t>(shv_ctx::kGemmStageBytes), "gemm_q4k: %d rows of %d columns do not fit the staging buffer", a.n_tok, a.k);
         SHV_LAUNCH(ctx, gemm_wide_stage_kernel, dim3(stage_parts(a, groups), kWideTok / 4, groups), dim3(256), 0, a, ctx->gemm_stage);
-        if (groups >= 4) {
-            // Blocks of 256 rows and two groups form each weight once for 128 activation rows: up to an eighth less work in all,
-            // where their rounds of the chip, one a compute unit, leave no more of it idle than the rounds of the blocks of 128
-            // rows and one group, two a unit, do.  us with one group / with two, over eight matrices in turn, the taken one first:
-            //              576 rows     768         1024        1531        2048        3000        4096
-            //   12352x2048 80 <- 92     112 <- 144  142 <- 150  211 <- 215  272 <- 280  364 <- 436  514 <- 524  (two, one, two, one, one, two, two)
-            //    9216x2048 72 <- 74      76 <- 90   111 <- 142  144 <- 153  196 <- 213  337 <- 285  369 <- 389  (two, two, one, two, one, one, two)
-            //    2048x4096 59 <- 130     58 <- 130   61 <- 130   87 <- 134  100 <- 137  143 <- 160  165 <- 190  (one up to 2048, two from there)
-            // The factor lies between the quotients of 9216 x 2048 of 4096 rows, 1.11, and of 12352 x 2048 of 2048, 1.13; of these
-            // shapes one, 9216 x 2048 of 3000 rows at 1.14, comes out wrong.
-            const int cus = ctx->prop.multiProcessorCount;
-            const auto filled = [](long long blocks, int slots) { return static_cast<double>(blocks) / static_cast<double>((blocks + slots - 1) / slots * slots); };
-            const int pairs = (groups + 1) / 2;
-            const double two = filled(static_cast<long long>((a.n + 255) / 256) * pairs, cus) * groups / (2 * pairs), one = filled(static_cast<long long>((a.n + 127) / 128) * groups, 2 * cus);
-            return 1.12 * two >= one ? launch_wide_all<16, 1, 2>(ctx, a, groups) : launch_wide_all<8, 1, 1>(ctx, a, groups);
-        }
         for (int g = 0; g < groups; g++) {
             const int t0 = g * kWideTok;
             const int nt = a.n_tok - t0 < kWideTok ? a.n_tok - t0 : kWideTok;

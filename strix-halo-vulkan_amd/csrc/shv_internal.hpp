@@ -157,6 +157,8 @@ bool shv_gemv_mrows_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a);
 int shv_launch_gemv_mrows(shv_ctx *ctx, const shv_gemv_q4k_args &a);
 bool shv_gemm_mid_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a);
 int shv_launch_gemm_mid(shv_ctx *ctx, const shv_gemv_q4k_args &a);
+bool shv_gemm_long_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a);
+int shv_launch_gemm_long(shv_ctx *ctx, const shv_gemv_q4k_args &a);
 int shv_launch_gemm_q4k(shv_ctx *ctx, const shv_gemv_q4k_args &a);
 bool shv_router_rows_covers(const shv_ctx *ctx, const shv_moe_router_args &a);
 int shv_launch_router_rows(shv_ctx *ctx, const shv_moe_router_args &a);
@@ -179,6 +181,10 @@ int shv_launch_moe_down_grouped(shv_ctx *ctx, const shv_moe_down_args &a);
 int shv_moe_list_tokens(int n_tok, int n_used, int n_expert);
 int shv_launch_moe_up_lists(shv_ctx *ctx, const shv_moe_up_args &a);
 int shv_launch_moe_down_lists(shv_ctx *ctx, const shv_moe_down_args &a);
+// ... and passes whose lists are long (moe_long.hip)
+size_t shv_moe_long_stage_bytes(int n_tok, int n_embd);
+int shv_launch_moe_up_long(shv_ctx *ctx, const shv_moe_up_args &a);
+int shv_launch_moe_down_long(shv_ctx *ctx, const shv_moe_down_args &a);
 int shv_launch_dn_step(shv_ctx *ctx, const shv_dn_step_args *a);
 int shv_launch_attn_decode(shv_ctx *ctx, const shv_attn_decode_args *a);
 int shv_launch_attn_cells(shv_ctx *ctx, const shv_attn_decode_args *a);

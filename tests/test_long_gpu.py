@@ -1,0 +1,84 @@
+"""Passes of hundreds of rows (csrc/long_tiles.hpp): projections against float64 (gemm_long.hip), expert lists around the tiles of 32, 64
+and 96 rows against the per-(token, slot) kernels (moe_long.hip)."""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+import shv
+from test_moe_lists_gpu import block, rig, selection  # noqa: F401 (rig is a fixture)
+
+pytestmark = pytest.mark.gpu
+A = shv.api
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = A.Context(0)
+    yield c
+    c.destroy()
+
+
+# every width; the fewest rows of each, whole and ragged groups of 64; weight rows inside a tile, a block of 128, of 256; blocks of either
+# kind (256 weight rows from 2048 x 4096 of 1800 rows on), in strips of eight groups and in a last one that is narrower
+@pytest.mark.parametrize("n,k,rows", [(17, 256, 193), (300, 512, 256), (513, 1024, 449), (129, 2048, 513), (2055, 2048, 1090), (70, 4096, 577), (2048, 4096, 1801)])
+def test_rows_of_a_long_pass(ctx, n, k, rows):
+    """The norm folded in and the residual in place, then no prologue and a ring that wraps.  2^-17: 32 bits' sums of up to 4096 products
+    in a fixed order, each product as exact as one float32."""
+    rng = np.random.default_rng(n + k + rows)
+    w = (rng.standard_normal((n, k)) * 0.02).astype(np.float32)
+    w[n // 2] = 0.015  # constant rows: a super-block whose d is zero, whose mins are not
+    wq = O.quantize_q4k(w)
+    w64 = O.dequant_q4k(wq, k).astype(np.float64)
+    x = (rng.standard_normal((rows, k)) * 10.0 ** rng.uniform(-6, 9, size=(rows, 1))).astype(np.float32)  # the sums of 32, too, leave binary16
+    x[rows // 3] = 0.0
+    x[rows // 5] += 5 * np.abs(x[rows // 5]).max()
+    gamma = (1 + 0.1 * rng.standard_normal(k)).astype(np.float32)
+    x64, res = x.astype(np.float64), rng.standard_normal((rows, n)).astype(np.float32)
+    bufs = dw, dx, dg, dy = ctx.upload(wq), ctx.upload(x), ctx.upload(gamma), ctx.upload(res)
+    ctx.gemv_q4k(dw, dx, dy, n, k, n_tok=rows, prologue=A.PRO_RMSNORM, gamma=dg, residual=dy)
+    xn = x64 / np.sqrt((x64 * x64).mean(axis=1, keepdims=True) + 1e-6) * gamma
+    want, got = xn @ w64.T + res, dy.read(np.float32, rows * n).reshape(rows, n)
+    size = np.abs(xn) @ (np.abs(w64) + 2 * np.abs(w64).max(axis=1, keepdims=True)).T + np.abs(res)
+    assert (np.abs(got - want) <= 2.0 ** -17 * size).all()
+    err = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+    assert np.sqrt(np.mean(err ** 2)) <= 1e-5, float(err.max())
+    slots, pos = rows + 3, np.array([rows - 2], np.int32)
+    ring, dpos = ctx.upload(np.full((slots, n), -7.0, np.float32)), ctx.upload(pos)
+    ctx.gemv_q4k(dw, dx, ring, n, k, n_tok=rows, pos=dpos, seq_len=rows, ring_slots=slots, ring_stride=n)
+    got, at = ring.read(np.float32, slots * n).reshape(slots, n), (pos[0] + np.arange(rows)) % slots
+    want = x64 @ w64.T
+    size = np.abs(x64) @ (np.abs(w64) + 2 * np.abs(w64).max(axis=1, keepdims=True)).T
+    assert (np.abs(got[at] - want) <= 2.0 ** -17 * size).all() and (got[at][rows // 3] == 0).all()
+    assert (np.delete(got, at, axis=0) == -7.0).all()
+    for b in bufs + (ring, dpos):
+        b.free()
+
+
+def test_an_infinity_stays_in_its_row(ctx):
+    n, k, rows = 96, 2048, 600
+    rng = np.random.default_rng(2)
+    wq = O.quantize_q4k((rng.standard_normal((n, k)) * 0.02).astype(np.float32))
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    x[70, 5], x[71, 9] = np.inf, np.nan
+    dw, dx, dy = ctx.upload(wq), ctx.upload(x), ctx.alloc(rows * n * 4)
+    ctx.gemv_q4k(dw, dx, dy, n, k, n_tok=rows)
+    got = dy.read(np.float32, rows * n).reshape(rows, n)
+    assert not np.isfinite(got[70:72]).any()
+    keep = np.delete(np.arange(rows), [70, 71])
+    want = x[keep].astype(np.float64) @ O.dequant_q4k(wq, k).astype(np.float64).T
+    assert np.linalg.norm(got[keep] - want) <= 1e-5 * np.linalg.norm(want)
+
+
+# (lengths, used): lists on the edges of one, two and three tiles and of what a pass takes, and the shared expert's last pass of each height
+@pytest.mark.parametrize("lengths,used", [
+    ([0, 1, 31, 32, 33, 63, 64, 65, 95, 96, 97, 128, 129, 193] + [40] * 9 + [41], 4),  # 357 tokens
+    ([16] * 22 + [20, 24], 2),                                                           # 198
+    ([0] + [17] * 20 + [30] * 3, 1),                                                     # 430
+])
+@pytest.mark.parametrize("packed", [1, 0])
+def test_long_lists_are_the_slots(rig, lengths, used, packed):  # noqa: F811
+    topk = selection(lengths, used, np.random.default_rng(sum(lengths)))
+    want, got = block(rig, topk, False, 0), block(rig, topk, True, packed)
+    rel = np.linalg.norm(got - want) / np.linalg.norm(want)
+    assert rel <= 1e-5, (topk.shape, rel)
+    assert np.max(np.abs(got - want)) <= 1e-4 * np.sqrt(np.mean(want ** 2))
