@@ -157,8 +157,8 @@ enum {
  * geometry instead (z + (slot*ring_slots + (pos+i) % ring_slots) * ring_stride) and leaves y
  * plain: the DeltaNet output projection takes its gate z from the projection ring.
  * Range: up to four rows any float32; from five on the rows enter the matrix cores, after the
- * prologue, as binary16 pairs: values up to 65504, and in passes past 512 rows the sums of 32
- * neighbours too.  (shv_gemv_mrows' kernel, two to eight rows, scales them.) */
+ * prologue, as binary16 pairs: values up to 65504.  (shv_gemv_mrows' kernel, two to eight rows, and
+ * the kernels of passes past 512 rows scale them: any float32.) */
 typedef struct {
     const void *w;
     const float *x;
@@ -311,9 +311,9 @@ typedef struct {
  * A pass of many rows (128 and more, or 65 and more where experts have 0.75 to 15 tokens each;
  * SHV_MOE_GROUP_MIN) whose topk is given, with n_expert stated
  * and a `group` workspace of 2 * n_expert + 1 + T * n_used ints, is grouped by expert on the matrix
- * cores: an expert's weights are read once per 8 to 48 tokens that chose it (the prompt arm of
- * llm_moe_gemv.comp).  Range: with up to 15 tokens an expert any float32 xn and act; with more, or with act as
- * floats from 128 rows on, values and sums of 32 neighbours up to 65504, and values below 1e-3 lose bits. */
+ * cores: an expert's weights are read once per 8 to 96 tokens that chose it (the prompt arm of
+ * llm_moe_gemv.comp).  Range: any float32 xn; with up to 15 tokens an expert any act; with more, or with act as
+ * floats from 128 rows on, act values and their sums of 32 neighbours up to 65504, and act values below 1e-3 lose bits. */
 typedef struct {
     const float *xn;
     int32_t *topk;

@@ -1,29 +1,19 @@
 // The experts of a pass of many rows, grouped by expert on the matrix cores (the prompt side of
 // MoETrace.Experts, llm/moe.go:289-409; the reference batches a chunk's tokens per expert in
 // llm_moe_gemv.comp's multi-row arm).  The per-(token, expert) GEMV reads and unpacks an expert's
-// weights once per token that chose it, this path once per 48 such tokens: it pays when tokens
+// weights once per token that chose it, this path once per 96 such tokens: it pays when tokens
 // outnumber experts (2048 rows choosing 10 of 512: 40 tokens an expert).  Passes whose experts have
 // up to fifteen tokens each go on from the same lists in moe_lists.hip.
 //
 //   moe_group_kernel          per-expert lists of (token, slot) pairs from topk (one block; long passes:
 //                             moe_group_count_kernel + moe_group_place_kernel, sixteen blocks)
-//   moe_stage_kernel          xn made into matrix-core operands once: two halves hi + lo of every
-//                             value as it is, and of every sub-block's sum (both within 65504)
-//   moe_up_grouped_kernel     a block = (expert, half of its ffn rows) and up to 48 of its tokens
-//                             at a time: their staged rows come to LDS in slabs of 256 columns (by
-//                             the loads themselves, the next slab under this one's products), each
-//                             wave streams two gate tiles of 16 rows and the matching up tiles,
-//                             forms a sub-block's weights once (as the whole numbers n * sc, exact
-//                             in binary16) for all three token tiles, keeps one matrix accumulator
-//                             per super-block, SwiGLU in registers, act[pair] out: as operands
-//                             (act_packed) or floats
-//   moe_down_staged_kernel    a block = (expert, quarter of n_embd rows) over act rows that are
-//                             operands, four row tiles a wave, raw products to pairs[pair]
-//   moe_down_grouped_kernel   the same over act rows that are floats, made into operands by the
-//                             block, 512 columns (a whole row) at a time
+//   moe_long.hip              the rows made into operands, gate/up + SwiGLU, and the down projection
+//                             over act rows that are operands (act_packed)
+//   moe_down_grouped_kernel   the down projection over act rows that are floats, 48 at a time, made into
+//                             operands by the block, 512 columns (a whole row) at a time
 //   moe_combine_kernel        out[t] = residual[t] + sum over slots of weights[t][s]*pairs[t][s],
 //                             slots in order
-// The shared expert is an expert every token lists: its blocks take 48 tokens each.
+// The shared expert is an expert every token lists.
 #include "moe_staged.hpp"
 #include "shv_internal.hpp"
 
@@ -309,16 +299,6 @@ struct RowStream {
         for (int r = 0; r < R; r++)
             q_next[r] = *reinterpret_cast<const uint2 *>(rp[r] + static_cast<size_t>(Gc >> 2) * SHV_Q4K_BYTES + 16 + (Gc & 3) * 32 + kb * 8);
     }
-    // A lane's 16 bytes of a PAIR of groups (pair Pg = groups 2 Pg, 2 Pg + 1: 64 payload bytes a row, one line's
-    // worth in one load where two 8-byte loads of a group each took a half line apiece): lane (row, kb) holds bytes
-    // 16 kb .. 16 kb + 15 of the pair, i.e. columns 16 (kb & 1) .. + 15 of group 2 Pg + (kb >> 1), low and high nibbles.
-    uint4 pair_next[R];
-    __device__ __forceinline__ void ask_pair(const char *const (&rp)[R], int Pg, int P_last, int kb) {
-        const int Pc = Pg < P_last ? Pg : P_last;
-#pragma unroll
-        for (int r = 0; r < R; r++)
-            pair_next[r] = *reinterpret_cast<const uint4 *>(rp[r] + static_cast<size_t>(Pc >> 1) * SHV_Q4K_BYTES + 16 + (Pc & 1) * 64 + kb * 16);
-    }
     __device__ __forceinline__ void ask_header(const char *const (&rp)[R], int sb, int sb_last) {
         const int sc = sb < sb_last ? sb : sb_last;
 #pragma unroll
@@ -452,301 +432,6 @@ __device__ __forceinline__ void rows_times_tiles(const char *const (&rp)[kTiles]
     }
 }
 
-// The same product over rows that a launch before this one has made into operands, a row's
-// own bytes together (moe_stage_kernel): [row][sub-block][part hi, lo][block of 8 columns] x 16
-// bytes, 128 bytes a sub-block, the eight columns in slot order.  A slab of 256 columns is 48
-// fragments which the loads place in LDS themselves, a lane's 16 bytes each from the listed row it
-// stands for (the four lanes of a row read 64 bytes in a line, the other part the line's other
-// half), so staging costs no vector work and no registers, and the next slab is on its way while
-// this one is multiplied.  Wave w asks for sub-block w of the slab: its two parts for every token
-// tile.  The sub-blocks' sums of x come from the operands (slab_times_tiles with SXS 0).
-// tok_s: the listed rows' numbers in the staged array.
-typedef const __attribute__((address_space(1))) void *global_ptr_t;
-typedef __attribute__((address_space(3))) void *lds_ptr_t;
-constexpr int kStWaves = kWaves;                 // waves of a block of the staged kernels: two such blocks share a compute unit, one's waits under the other's work
-constexpr int kStThreads = kStWaves * 64;
-constexpr int kStSubs = kStWaves;             // sub-blocks of a staged slab: one a wave
-constexpr int kStQuarter = 1024 / (32 * kStSubs);  // slabs in the 1024 columns one min-term product covers
-constexpr int kStSlab = 32 * kStSubs;
-constexpr int kStFrags = kStSubs * 2 * kTT * kFrag;
-constexpr int kStSumFrags = kTT * 2 * kFrag;   // the sums of a quarter of the columns (four super-blocks): [token tile][part]
-constexpr int kStMinHdrs = kStWaves * kTiles * kFrag;   // every lane's row header of its super-block of the quarter, a wave's own
-constexpr size_t kStagedLds = 2 * static_cast<size_t>(kStFrags) + 2 * kStSumFrags + kStMinHdrs + 2 * kTok * 4;
-
-// Where the eight columns of block blk of sub-block `sub` stand in a row's operands, part 0 (part 1: 64 on): [super-block]
-// [product][part][lane kb of the products] x 16 bytes, so that the four lanes of a row ask for 64 bytes in a line.  Product
-// pr * 4 + hi * 2 + half: pair pr of the super-block's groups, low or high nibbles, first or second eight of a lane's sixteen.
-__device__ __forceinline__ size_t group_block(int sub, int blk) {
-    const int product = ((sub >> 2) & 1) * 4 + (sub & 1) * 2 + (blk & 1), kb = ((sub >> 1) & 1) * 2 + (blk >> 1);
-    return static_cast<size_t>(sub >> 3) * (8 * kStSubBytes) + product * 128 + kb * 16;
-}
-
-// grid: (k / 1024, rows), 256 threads, a quad of columns each.
-__global__ __launch_bounds__(256) void moe_stage_kernel(const float *x, int x_stride, int k, int rows, char *staged) {
-    const int t = blockIdx.y, c = (blockIdx.x * 256 + threadIdx.x) * 4;
-    if (c >= k) return;
-    const float4 v = *reinterpret_cast<const float4 *>(x + static_cast<size_t>(t) * x_stride + c);
-    const float o[4] = {v.x, v.z, v.y, v.w};
-    half4_t h, l;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const _Float16 hi = static_cast<_Float16>(o[j]);
-        h[j] = hi;
-        l[j] = static_cast<_Float16>(o[j] - static_cast<float>(hi));
-    }
-    char *e = staged + static_cast<size_t>(t) * (k / 32) * kStSubBytes + group_block(c >> 5, (c & 31) >> 3) + ((c & 7) >> 2) * 8;
-    *reinterpret_cast<half4_t *>(e) = h;
-    *reinterpret_cast<half4_t *>(e + 64) = l;
-    // the sub-block's sum: eight neighbouring lanes (k is a multiple of 32, so they are all here)
-    float sum = (v.x + v.y) + (v.z + v.w);
-    sum += __shfl_xor(sum, 1, 64);
-    sum += __shfl_xor(sum, 2, 64);
-    sum += __shfl_xor(sum, 4, 64);
-    if ((c & 31) == 0) {
-        const _Float16 hi = static_cast<_Float16>(sum);
-        _Float16 *sp = reinterpret_cast<_Float16 *>(staged + staged_sums_offset(rows, k) + (static_cast<size_t>(t) * (k / 256) + (c >> 8)) * 32) + ((c >> 5) & 7);
-        sp[0] = hi;
-        sp[8] = static_cast<_Float16>(sum - static_cast<float>(hi));
-    }
-}
-
-// Where lane (row n, piece kb) of the products finds its sixteen bytes of a fragment that ask_staged_slab has brought.
-__device__ __forceinline__ int frag_at(int lane) { return (lane & 15) * 64 + (((lane >> 4) ^ (lane >> 2)) & 3) * 16; }
-
-template <int K>
-__device__ __forceinline__ void ask_staged_slab(const char *staged, const int32_t *tok_s, int m, int n_tt, int sl, char *buf, int lane, int wave) {
-    // Wave w asks for product w of the slab's eight.  Four neighbouring lanes ask for a row's four pieces, which lie in a
-    // line of 64 bytes and are one request; which of them asks for which is turned with the row, so that the products' lanes
-    // (row n, piece kb), reading at frag_at, find eight rows' pieces in different banks.
-    const int n = lane >> 2, kb = (lane & 3) ^ ((n >> 2) & 3);
-#pragma unroll
-    for (int tt = 0; tt < kTT; tt++) {
-        if (tt >= n_tt) break;
-        const int i = 16 * tt + n;
-        const int t = tok_s[i < m ? i : 0];  // a column past the list repeats the first row; nobody reads its products
-        const char *g = staged + (static_cast<size_t>(t) * (K / 32) + sl * kStSubs) * kStSubBytes + wave * 128 + kb * 16;
-        char *f = buf + ((wave * 2) * kTT + tt) * kFrag;
-        __builtin_amdgcn_global_load_lds((global_ptr_t)(g), (lds_ptr_t)(f), 16, 0, 0);
-        __builtin_amdgcn_global_load_lds((global_ptr_t)(g + 64), (lds_ptr_t)(f + kTT * kFrag), 16, 0, 0);
-    }
-}
-
-// The sums of x of columns [1024 q, 1024 q + 1024), four super-blocks, as the operands of the
-// min term: fragment (token tile, part), lane = token in the tile + 16 * (super-block of the four).
-// The waves share the fragments out.
-template <int K>
-__device__ __forceinline__ void ask_staged_sums(const char *sums, const int32_t *tok_s, int m, int n_tt, int q, char *buf, int lane, int wave) {
-    const int n = lane & 15, kb = lane >> 4;
-    const int sb = 4 * q + kb < K / 256 ? 4 * q + kb : K / 256 - 1;  // past the row: a real sum against a zero weight
-    for (int f = wave; f < 2 * n_tt; f += kStWaves) {
-        const int tt = f >> 1, part = f & 1;
-        const int i = 16 * tt + n;
-        const int t = tok_s[i < m ? i : 0];
-        const char *g = sums + (static_cast<size_t>(t) * (K / 256) + sb) * 32 + part * 16;
-        __builtin_amdgcn_global_load_lds((global_ptr_t)(g), (lds_ptr_t)(buf + f * kFrag), 16, 0, 0);
-    }
-}
-
-// The headers min_terms reads, on their way a slab ahead: lane (row, kb) asks for its R rows'
-// headers of super-block 4 q + kb, into the wave's own kTiles fragments at hbuf.
-template <int K, int R>
-__device__ __forceinline__ void ask_min_headers(const char *const (&rp)[R], int q, char *hbuf, int lane) {
-    const int sb = 4 * q + (lane >> 4) < K / 256 ? 4 * q + (lane >> 4) : 0;
-#pragma unroll
-    for (int r = 0; r < R; r++)
-        __builtin_amdgcn_global_load_lds((global_ptr_t)(rp[r] + static_cast<size_t>(sb) * SHV_Q4K_BYTES), (lds_ptr_t)(hbuf + r * kFrag), 16, 0, 0);
-}
-
-// y -= sum over the quarter's sub-blocks of dmin * m * sum(x), on the matrix cores: lane (row,
-// kb) forms its row's eight -dmin * m of super-block 4 q + kb as two halves each (the product has
-// 17 significant bits), the tokens' sums come as two halves too, and three products (the small
-// halves' one is below float32's last bit) add to the accumulators what the vector units would
-// subtract sub-block by sub-block.
-template <int K, int R, int NTT>
-__device__ __forceinline__ void min_terms(int q, const char *sfr, const char *hbuf, int lane, float4_t (&y)[R][NTT]) {
-    const int kb = lane >> 4;
-    const bool on = 4 * q + kb < K / 256;
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        const uint4 h = *reinterpret_cast<const uint4 *>(hbuf + r * kFrag + lane * 16);
-        const float nd = on ? -f16_bits_to_f32(h.x >> 16) : 0.f;
-        const uint32_t m03 = h.z & 0x3F3F3F3Fu, m47 = ((h.w >> 4) & 0x0F0F0F0Fu) | ((h.z >> 2) & 0x30303030u);
-        half8_t bh, bl;
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const float p = nd * static_cast<float>(((j < 4 ? m03 : m47) >> (8 * (j & 3))) & 0xFFu);
-            const _Float16 hi = static_cast<_Float16>(p);
-            bh[j] = hi;
-            bl[j] = static_cast<_Float16>(p - static_cast<float>(hi));
-        }
-#pragma unroll
-        for (int tt = 0; tt < NTT; tt++) {
-            const half8_t sh = *reinterpret_cast<const half8_t *>(sfr + (tt * 2) * kFrag + lane * 16);
-            const half8_t sl = *reinterpret_cast<const half8_t *>(sfr + (tt * 2 + 1) * kFrag + lane * 16);
-            y[r][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(sh, bh, y[r][tt], 0, 0, 0);
-            y[r][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(sl, bh, y[r][tt], 0, 0, 0);
-            y[r][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(sh, bl, y[r][tt], 0, 0, 0);
-        }
-    }
-}
-
-// slab_times_tiles for staged rows and NTT token tiles, without the min term (min_terms has it):
-// the (sub-block, token tile) steps of a 64-weight group run as one pipeline in which the
-// fragments of the step after this one are read from LDS before this step's products are issued,
-// so no product waits for an LDS read.
-template <int NG, int R, int NTT, typename Ask>
-__device__ __forceinline__ void staged_slab_times_tiles(const char *const (&rp)[R], RowStream<R> &st, int G0, int G_last, const char *frags, const char *hbuf,
-                                                        int lane, float4_t (&acc)[R][NTT], float4_t (&y)[R][NTT], Ask &&ask_next) {
-    static_assert(NG == 4, "a slab is one super-block: its header is read once, where the slab begins");
-    const int kb = lane >> 4;
-    const NibbleMasks nc = nibble_masks();
-    // The rows' headers of this super-block are in LDS already: min_terms' loads brought the quarter's (lane (row, kb)
-    // holds super-block 4 q + kb's), a slab and more ahead.  Asked for from memory where a super-block ends they were
-    // waited for where the next begins; kept in registers they cost sixteen, so each pair of groups reads them again.
-    typedef uint32_t u32x4_lds __attribute__((ext_vector_type(4)));
-    const __attribute__((address_space(3))) char *hl = (const __attribute__((address_space(3))) char *)(hbuf) + ((lane & 15) + 16 * ((G0 >> 2) & 3)) * 16;
-    // LDS addresses are 32 bits wide: kept as such, a fragment's place costs no 64-bit arithmetic
-    typedef const __attribute__((address_space(3))) char *lds_bytes_t;
-    typedef const __attribute__((address_space(3))) half8_t *lds_half8_t;
-    const lds_bytes_t fl = (lds_bytes_t)(frags) + frag_at(lane);
-    half8_t nh = *(lds_half8_t)(fl), nl = *(lds_half8_t)(fl + kTT * kFrag);
-#pragma unroll 1
-    for (int pi = 0; pi < NG / 2; pi++) {
-        const int Pg = (G0 >> 1) + pi;                                          // the pair of groups: 2 Pg, 2 Pg + 1
-        const lds_bytes_t fp = fl + pi * (8 * kTT * kFrag);                     // this pair's four products
-        const lds_bytes_t fn = pi + 1 < NG / 2 ? fp + 8 * kTT * kFrag : fl;    // the pair after it (the slab's first again past its last, unused)
-        uint4 q[R];
-#pragma unroll
-        for (int r = 0; r < R; r++) q[r] = st.pair_next[r];
-        // the pair's bytes are here: only now the loads that nothing in this slab waits for (a
-        // wait for loaded registers also waits for every load issued before them)
-        asm volatile("" : "+v"(q[0].x), "+v"(q[1].x), "+v"(q[2].x), "+v"(q[3].x));
-        // this lane's group of the pair, within the super-block: its scales, and the rows' d
-        const int g = (2 * Pg + (kb >> 1)) & 3;
-        uint32_t sc[R], dd16[R];
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            const u32x4_lds h = *reinterpret_cast<const __attribute__((address_space(3))) u32x4_lds *>(hl + r * kFrag);
-            uint32_t mn;
-            q4k_group_scale_min(make_uint4(h.x, h.y, h.z, h.w), g, sc[r], mn);
-            dd16[r] = h.x;
-        }
-        // read to the end before the loads of the quarter after this one may be asked for (they land in the same place)
-        asm volatile("" : "+v"(sc[0]), "+v"(sc[1]), "+v"(sc[2]), "+v"(sc[3]), "+v"(dd16[0]), "+v"(dd16[1]), "+v"(dd16[2]), "+v"(dd16[3]));
-        // the next pair's bytes first: a wait for them then does not wait for the slab's loads behind them
-        st.ask_pair(rp, Pg + 1, G_last >> 1, kb);
-        ask_next(pi);
-        __builtin_amdgcn_sched_barrier(0);  // the loads stay up here, a pair ahead of their use
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int hi = u >> 1;  // products 0, 1: the low nibbles of bytes 0..7 and 8..15; 2, 3: the high nibbles
-            half8_t b[R];
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                const uint32_t q0 = (u & 1) ? q[r].z : q[r].x, q1 = (u & 1) ? q[r].w : q[r].y;
-                // A nibble in the low bits of a half's mantissa reads, under the right exponent, as
-                // C + n: bits 0..3 under 1024's, bits 4..7 under 64's (the odd bytes' nibbles take
-                // one shift down there).  One fused multiply-add then makes (C + n) * sc - C * sc =
-                // n * sc: a whole number up to 15 * 63, exact in binary16, as are C * sc.
-                const _Float16 s1 = static_cast<_Float16>(static_cast<float>(hi ? sc[r] >> 8 : sc[r] & 0xFFu));
-                const half2_t s2 = {s1, s1};
-                half2_t w[4], c[4];
-                if (hi == 0) {
-                    w[0] = __builtin_bit_cast(half2_t, (q0 & nc.m0) | nc.o0); w[1] = __builtin_bit_cast(half2_t, ((q0 >> 4) & nc.m4) | nc.o4);
-                    w[2] = __builtin_bit_cast(half2_t, (q1 & nc.m0) | nc.o0); w[3] = __builtin_bit_cast(half2_t, ((q1 >> 4) & nc.m4) | nc.o4);
-                    c[0] = c[2] = s2 * static_cast<half2_t>(static_cast<_Float16>(-1024.f));
-                    c[1] = c[3] = s2 * static_cast<half2_t>(static_cast<_Float16>(-64.f));
-                } else {
-                    w[0] = __builtin_bit_cast(half2_t, (q0 & nc.m4) | nc.o4); w[1] = __builtin_bit_cast(half2_t, ((q0 >> 8) & nc.m4) | nc.o4);
-                    w[2] = __builtin_bit_cast(half2_t, (q1 & nc.m4) | nc.o4); w[3] = __builtin_bit_cast(half2_t, ((q1 >> 8) & nc.m4) | nc.o4);
-                    c[0] = c[1] = c[2] = c[3] = s2 * static_cast<half2_t>(static_cast<_Float16>(-64.f));
-                }
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const half2_t p = __builtin_elementwise_fma(w[i], s2, c[i]);
-                    b[r][2 * i] = p[0];
-                    b[r][2 * i + 1] = p[1];
-                }
-            }
-            // the matrix instructions of a step win the SIMD's issue slot over the other wave's vector
-            // instructions, which then run under them instead of between them
-            __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-            for (int tt = 0; tt < NTT; tt++) {
-                const half8_t xh = nh, xl = nl;
-                // the step after this one: the next token tile, the next product's first, or (past
-                // the slab's last) the first again, unused
-                const int ntt = tt + 1 < NTT ? tt + 1 : 0;
-                const lds_bytes_t f = tt + 1 < NTT ? fp + ((u * 2) * kTT + ntt) * kFrag : (u < 3 ? fp + ((u + 1) * 2) * kTT * kFrag : fn);
-                nh = *(lds_half8_t)(f);
-                nl = *(lds_half8_t)(f + kTT * kFrag);
-#pragma unroll
-                for (int r = 0; r < R; r++) acc[r][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, b[r], acc[r][tt], 0, 0, 0);
-#pragma unroll
-                for (int r = 0; r < R; r++) acc[r][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, b[r], acc[r][tt], 0, 0, 0);
-            }
-            __builtin_amdgcn_s_setprio(0);
-        }
-        if (Pg & 1) {
-            // the super-block ends: its sums take its d
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                const float dd = f16_bits_to_f32(dd16[r]);
-#pragma unroll
-                for (int tt = 0; tt < NTT; tt++) {
-#pragma unroll
-                    for (int j = 0; j < 4; j++) y[r][tt][j] = fmaf(dd, acc[r][tt][j], y[r][tt][j]);
-                    acc[r][tt] = float4_t{0.f, 0.f, 0.f, 0.f};
-                }
-            }
-        }
-    }
-}
-
-template <int K, int NTT>
-__device__ __forceinline__ void staged_times_tiles(const char *const (&rp)[kTiles], const char *staged, const char *sums, const int32_t *tok_s, int m,
-                                                   char *bufs, int lane, int wave, float4_t (&y)[kTiles][NTT]) {
-    constexpr int GROUPS = K / 64, NG = kStSlab / 64, SLABS = K / kStSlab;
-    static_assert(K % kStSlab == 0, "whole slabs");
-#pragma unroll
-    for (int r = 0; r < kTiles; r++)
-#pragma unroll
-        for (int tt = 0; tt < NTT; tt++) y[r][tt] = float4_t{0.f, 0.f, 0.f, 0.f};
-    float4_t acc[kTiles][NTT];
-#pragma unroll
-    for (int r = 0; r < kTiles; r++)
-#pragma unroll
-        for (int tt = 0; tt < NTT; tt++) acc[r][tt] = float4_t{0.f, 0.f, 0.f, 0.f};
-    char *sum_bufs = bufs + 2 * kStFrags;
-    char *hbuf = sum_bufs + 2 * kStSumFrags + wave * (kTiles * kFrag);
-    ask_staged_slab<K>(staged, tok_s, m, NTT, 0, bufs, lane, wave);
-    ask_staged_sums<K>(sums, tok_s, m, NTT, 0, sum_bufs, lane, wave);
-    ask_min_headers<K, kTiles>(rp, 0, hbuf, lane);
-    RowStream<kTiles> st;
-    st.ask_pair(rp, 0, GROUPS / 2 - 1, lane >> 4);
-#pragma unroll 1
-    for (int sl = 0; sl < SLABS; sl++) {
-        char *buf = bufs + (sl & 1) * kStFrags;
-        // this wave's loads have landed, then everybody's: the slab is whole, and the buffer the
-        // next one goes to has been read to its end
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-        __syncthreads();
-        if (sl % kStQuarter == 0) min_terms<K, kTiles, NTT>(sl / kStQuarter, sum_bufs + ((sl / kStQuarter) & 1) * kStSumFrags, hbuf, lane, y);
-        staged_slab_times_tiles<NG, kTiles, NTT>(rp, st, sl * NG, GROUPS - 1, buf, hbuf, lane, acc, y, [&](int pi) {
-            // the next slab at the slab's first pair of groups; the next quarter's sums and headers at its second, behind
-            // the last reading of this quarter's headers
-            if (sl + 1 < SLABS) {
-                if (pi == 0) ask_staged_slab<K>(staged, tok_s, m, NTT, sl + 1, bufs + ((sl + 1) & 1) * kStFrags, lane, wave);
-                if (pi == 1 && (sl + 1) % kStQuarter == 0) {
-                    const int q = (sl + 1) / kStQuarter;
-                    ask_staged_sums<K>(sums, tok_s, m, NTT, q, sum_bufs + (q & 1) * kStSumFrags, lane, wave);
-                    ask_min_headers<K, kTiles>(rp, q, hbuf, lane);
-                }
-            }
-        });
-    }
-}
-
 // Which expert, which part of its rows and which of its tokens a block takes.  The first
 // parts * ceil(n_tok / 16) blocks are the shared expert, one per (part, tile of 16 tokens); the
 // rest are the routed experts (every token tile of the expert's list in turn).
@@ -787,99 +472,6 @@ struct Staging {
 };
 constexpr size_t kGroupedLds = static_cast<size_t>(kSlabSubs) * 2 * kTT * kFrag + static_cast<size_t>(kSlabSubs) * kTok * 4 + kTok * sizeof(float *) + kTok * 4;
 
-// One pass of a block of the gate/up kernel over up to 16 NTT of its tokens: the products, SwiGLU, act out
-// (as floats, or, packed, as the operands the grouped down projection stages from).
-template <int K, int NTT>
-__device__ __forceinline__ void up_pass(const shv_moe_up_args &a, const char *const (&rp)[kTiles], const char *staged, const int32_t *tok_s,
-                                        const int32_t *pair_s, int m, char *smem, int row, char *act_sums) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, kb = lane >> 4, n = lane & 15;
-    float4_t y[kTiles][NTT];
-    staged_times_tiles<K, NTT>(rp, staged, staged + staged_sums_offset(a.n_tok, K), tok_s, m, smem, lane, wave, y);
-    // this wave's 32 columns are one sub-block of the down projection's rows
-    const int sub = row >> 5;   // row = 32 * sub + n
-    // column 16 r + n of the sub-block: block of 8 columns 2 r + n / 8, slot of [0, 2, 1, 3, 4, 6, 5, 7]
-    const int p8 = n & 7, slot = (p8 & 4) | ((p8 & 1) << 1) | ((p8 & 2) >> 1);
-#pragma unroll
-    for (int tt = 0; tt < NTT; tt++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int i = 16 * tt + 4 * kb + j;
-            float v[2];
-#pragma unroll
-            for (int r = 0; r < 2; r++) {
-                const float gv = y[r][tt][j];
-                v[r] = gv * sigmoid_exact(gv) * y[2 + r][tt][j];
-            }
-            if (!a.act_packed) {
-                if (i < m) {
-#pragma unroll
-                    for (int r = 0; r < 2; r++) a.act[static_cast<size_t>(pair_s[i]) * a.ffn + row + 16 * r] = v[r];
-                }
-            } else {
-                // the sub-block's sum: both tiles, the 16 lanes of the token
-                float sum = v[0] + v[1];
-                sum += __shfl_xor(sum, 1, 64);
-                sum += __shfl_xor(sum, 2, 64);
-                sum += __shfl_xor(sum, 4, 64);
-                sum += __shfl_xor(sum, 8, 64);
-                if (i < m) {
-                    const size_t pair = static_cast<size_t>(pair_s[i]);
-                    char *e = reinterpret_cast<char *>(a.act) + pair * (a.ffn / 32) * kStSubBytes + slot * 2;
-#pragma unroll
-                    for (int r = 0; r < 2; r++) {
-                        const _Float16 hi = static_cast<_Float16>(v[r]);
-                        const size_t at = group_block(sub, 2 * r + (n >> 3));
-                        *reinterpret_cast<_Float16 *>(e + at) = hi;
-                        *reinterpret_cast<_Float16 *>(e + at + 64) = static_cast<_Float16>(v[r] - static_cast<float>(hi));
-                    }
-                    if (n == 0) {
-                        const _Float16 hi = static_cast<_Float16>(sum);
-                        _Float16 *sp = reinterpret_cast<_Float16 *>(act_sums + (pair * (a.ffn / 256) + (sub >> 3)) * 32) + (sub & 7);
-                        sp[0] = hi;
-                        sp[8] = static_cast<_Float16>(sum - static_cast<float>(hi));
-                    }
-                }
-            }
-        }
-}
-
-// grid: n_expert * parts + parts * ceil(n_tok / 48) blocks of 8 waves, parts = ffn / 256; K = n_embd.
-// A part is 256 gate rows and the same 256 up rows = 16 + 16 tiles; wave w takes gate tiles 2w and
-// 2w + 1 and the up tiles of the same rows, so SwiGLU stays in registers.
-template <int K>
-__global__ __launch_bounds__(kStThreads, 2) void moe_up_grouped_kernel(shv_moe_up_args a, const char *staged, char *act_sums) {
-    extern __shared__ __align__(16) char smem[];
-    // the two slab buffers, then the listed rows' pair and token numbers
-    int32_t *pair_s = reinterpret_cast<int32_t *>(smem + 2 * kStFrags + 2 * kStSumFrags + kStMinHdrs);
-    int32_t *tok_s = pair_s + kTok;
-    const int32_t *group = a.group;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int n = lane & 15;
-    const int parts = a.ffn / (32 * kStWaves);
-    const Unit u = unit_of(blockIdx.x, parts, a.n_expert, a.n_tok, a.n_used, group);
-    if (u.count <= 0) return;
-    const size_t row_bytes = static_cast<size_t>(K / SHV_Q4K_BLOCK) * SHV_Q4K_BYTES;
-    const int row = u.part * (32 * kStWaves) + wave * 32 + n;   // this lane's first row of the expert, gate and up alike; its second is 16 on
-    const size_t wrow = static_cast<size_t>(u.expert < 0 ? 0 : u.expert) * a.ffn + row;
-    const char *gp = static_cast<const char *>(u.expert < 0 ? a.gate_sh : a.gate_exps) + wrow * row_bytes;
-    const char *up = static_cast<const char *>(u.expert < 0 ? a.up_sh : a.up_exps) + wrow * row_bytes;
-    const char *rp[kTiles] = {gp, gp + 16 * row_bytes, up, up + 16 * row_bytes};
-    for (int t0 = 0; t0 < u.count; t0 += kTok) {
-        const int m = u.count - t0 < kTok ? u.count - t0 : kTok;
-        if (tid < m) {
-            const int pair = u.expert < 0 ? (u.first + t0 + tid) * (a.n_used + 1) + a.n_used : group[a.n_expert + 1 + u.first + t0 + tid];
-            pair_s[tid] = pair;
-            tok_s[tid] = pair / (a.n_used + 1);
-        }
-        __syncthreads();   // the list is written; the pass before this one has read its last slab
-        const int n_tt = (m + 15) >> 4;
-        if (n_tt == 3) up_pass<K, 3>(a, rp, staged, tok_s, pair_s, m, smem, row, act_sums);
-        else if (n_tt == 2) up_pass<K, 2>(a, rp, staged, tok_s, pair_s, m, smem, row, act_sums);
-        else up_pass<K, 1>(a, rp, staged, tok_s, pair_s, m, smem, row, act_sums);
-        __syncthreads();   // the list is read to the end before the next one replaces it
-    }
-}
-
 // grid: n_expert * parts + parts * ceil(n_tok / 48) blocks, parts = n_embd / 512: a part is 512
 // output rows = 32 tiles, wave w takes tiles 4w .. 4w + 3.  K = ffn.
 template <int K>
@@ -919,55 +511,6 @@ __global__ __launch_bounds__(kThreads) void moe_down_grouped_kernel(shv_moe_down
                 }
             }
         __syncthreads();
-    }
-}
-
-// One pass of a block of the staged down kernel: the products of up to 16 NTT listed pairs, raw, to pairs[pair].
-template <int K, int NTT>
-__device__ __forceinline__ void down_pass(const shv_moe_down_args &a, const char *const (&rp)[kTiles], const char *act_sums, const int32_t *pair_s,
-                                          int m, char *smem, int row0) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, kb = lane >> 4;
-    float4_t y[kTiles][NTT];
-    staged_times_tiles<K, NTT>(rp, reinterpret_cast<const char *>(a.act), act_sums, pair_s, m, smem, lane, wave, y);
-#pragma unroll
-    for (int tt = 0; tt < NTT; tt++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int i = 16 * tt + 4 * kb + j;
-            if (i < m) {
-                float *dst = a.pairs + static_cast<size_t>(pair_s[i]) * a.n_embd + row0;
-#pragma unroll
-                for (int r = 0; r < kTiles; r++) dst[16 * r] = y[r][tt][j];
-            }
-        }
-}
-
-// The down projection over act rows that the gate/up kernel left as operands (act_packed): the
-// same blocks and tiles as moe_down_grouped_kernel, the rows staged by the loads themselves.
-template <int K>
-__global__ __launch_bounds__(kStThreads, 2) void moe_down_staged_kernel(shv_moe_down_args a, const char *act_sums) {
-    extern __shared__ __align__(16) char smem[];
-    int32_t *pair_s = reinterpret_cast<int32_t *>(smem + 2 * kStFrags + 2 * kStSumFrags + kStMinHdrs);
-    const int32_t *group = a.group;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int n = lane & 15;
-    const int parts = a.n_embd / (64 * kStWaves);
-    const Unit u = unit_of(blockIdx.x, parts, a.n_expert, a.n_tok, a.n_used, group);
-    if (u.count <= 0) return;
-    const size_t row_bytes = static_cast<size_t>(K / SHV_Q4K_BLOCK) * SHV_Q4K_BYTES;
-    const int row0 = u.part * (64 * kStWaves) + wave * 64 + n;
-    const char *base = static_cast<const char *>(u.expert < 0 ? a.down_sh : a.down_exps) +
-                       (static_cast<size_t>(u.expert < 0 ? 0 : u.expert) * a.n_embd + row0) * row_bytes;
-    const char *rp[kTiles] = {base, base + 16 * row_bytes, base + 32 * row_bytes, base + 48 * row_bytes};
-    for (int t0 = 0; t0 < u.count; t0 += kTok) {
-        const int m = u.count - t0 < kTok ? u.count - t0 : kTok;
-        if (tid < m) pair_s[tid] = u.expert < 0 ? (u.first + t0 + tid) * (a.n_used + 1) + a.n_used : group[a.n_expert + 1 + u.first + t0 + tid];
-        __syncthreads();   // the list is written; the pass before this one has read its last slab
-        const int n_tt = (m + 15) >> 4;
-        if (n_tt == 3) down_pass<K, 3>(a, rp, act_sums, pair_s, m, smem, row0);
-        else if (n_tt == 2) down_pass<K, 2>(a, rp, act_sums, pair_s, m, smem, row0);
-        else down_pass<K, 1>(a, rp, act_sums, pair_s, m, smem, row0);
-        __syncthreads();   // the list is read to the end before the next one replaces it
     }
 }
 
@@ -1025,7 +568,7 @@ bool shapes_covered(const shv_ctx *ctx, int n_tok, int n_embd, int ffn, int n_us
 bool shv_moe_up_grouped_covers(const shv_ctx *ctx, const shv_moe_up_args &a) {
     const bool lists = shv_moe_list_tokens(a.n_tok, a.n_used, a.n_expert) > 0;
     return a.group && !a.logits && shv_aligned16(a.xn) && shapes_covered(ctx, a.n_tok, a.n_embd, a.ffn, a.n_used, a.n_expert) && ctx->gemm_stage &&
-           (lists ? list_bytes(a.n_tok, a.n_embd) : staged_bytes(a.n_tok, a.n_embd)) <= static_cast<size_t>(shv_ctx::kGemmStageBytes);
+           (lists ? list_bytes(a.n_tok, a.n_embd) : shv_moe_long_stage_bytes(a.n_tok, a.n_embd)) <= static_cast<size_t>(shv_ctx::kGemmStageBytes);
 }
 
 bool shv_moe_down_grouped_covers(const shv_ctx *ctx, const shv_moe_down_args &a) {
@@ -1048,13 +591,7 @@ int shv_launch_moe_up_grouped(shv_ctx *ctx, const shv_moe_up_args &a) {
         return shv_launch_moe_up_lists(ctx, a);
     }
     if (const int rc = launch_group(ctx, a.topk, a.n_tok, a.n_used, a.n_expert, a.group); rc != SHV_OK) return rc;
-    SHV_LAUNCH(ctx, moe_stage_kernel, dim3((a.n_embd + 1023) / 1024, a.n_tok), dim3(256), 0, a.xn, a.n_embd, a.n_embd, a.n_tok, ctx->gemm_stage);
-    constexpr size_t lds = kStagedLds;
-    static const int raised = raise_lds(&moe_up_grouped_kernel<2048>, lds);
-    if (raised != SHV_OK) return raised;
-    const int parts = a.ffn / (32 * kStWaves), tiles = (a.n_tok + kTok - 1) / kTok;
-    SHV_LAUNCH(ctx, moe_up_grouped_kernel<2048>, dim3(a.n_expert * parts + parts * tiles), dim3(kStThreads), lds, a, static_cast<const char *>(ctx->gemm_stage),
-               reinterpret_cast<char *>(ctx->gemm_part));
+    if (const int rc = shv_launch_moe_up_long(ctx, a); rc != SHV_OK) return rc;
     ctx->moe_stamp = {a.topk, a.group, a.act, a.n_tok, a.n_used, true, a.act_packed != 0};
     return SHV_OK;
 }
@@ -1078,11 +615,7 @@ int shv_launch_moe_down_grouped(shv_ctx *ctx, const shv_moe_down_args &a) {
     if (a.act_packed && shv_moe_list_tokens(a.n_tok, a.n_used, a.n_expert) > 0) {
         if (const int rc = shv_launch_moe_down_lists(ctx, a); rc != SHV_OK) return rc;
     } else if (a.act_packed) {
-        constexpr size_t lds = kStagedLds;
-        static const int raised = raise_lds(&moe_down_staged_kernel<512>, lds);
-        if (raised != SHV_OK) return raised;
-        static_assert(64 * kStWaves == 512, "a part is 512 rows");
-        SHV_LAUNCH(ctx, moe_down_staged_kernel<512>, dim3(a.n_expert * parts + parts * tiles), dim3(kStThreads), lds, a, reinterpret_cast<const char *>(ctx->gemm_part));
+        if (const int rc = shv_launch_moe_down_long(ctx, a); rc != SHV_OK) return rc;
     } else {
         constexpr size_t lds = kGroupedLds;
         static const int raised = raise_lds(&moe_down_grouped_kernel<512>, lds);

@@ -1,10 +1,8 @@
 // What the expert kernels of long passes share: rows of activations as matrix-core operands, a row's own bytes together.
 //
-// A row of k columns is [sub-block of 32][part hi, lo][block of 8 columns] x 16 bytes, 128 bytes a sub-block, the eight
-// columns of a block in slot order [0, 2, 1, 3, 4, 6, 5, 7] (the order a payload dword's nibbles come out of the masks).
-// After all rows come their sums over the sub-blocks, as operands too: [row][super-block] x 32 bytes, the eight sums'
-// binary16 values and then what those leave.  (The list kernels' sums are float32, in bfloat16 parts: list_sum_put; their
-// values are scaled: binary16_parts.)
+// For the list kernels a row of k columns is [sub-block of 32] x 128 bytes (list_block), the eight columns of a block in slot
+// order [0, 2, 1, 3, 4, 6, 5, 7] (the order a payload dword's nibbles come out of the masks), its sums over the sub-blocks
+// float32, in bfloat16 parts (list_sum_put), its values scaled (binary16_parts).  moe_long.hip's rows: long_tiles.hpp.
 #pragma once
 #include "shv_device.hpp"
 
@@ -22,9 +20,7 @@ typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 constexpr int kStSubBytes = 128;  // a row's sub-block: 2 parts x 4 column blocks x 16 bytes
 
 __host__ __device__ constexpr size_t staged_sums_offset(int rows, int k) { return static_cast<size_t>(rows) * (k / 32) * 128; }
-__host__ __device__ constexpr size_t staged_bytes(int rows, int k) { return staged_sums_offset(rows, k) + static_cast<size_t>(rows) * (k / 256) * 32; }
-// Where the grouped down projection finds a pair's act row when it comes as operands: the row's
-// own 4 * ffn bytes of act in the staged layout, and its sub-blocks' sums in the library's scratch.
+// Where a pair's act row comes as operands (moe_long.hip): its sub-blocks' sums, in the library's scratch.
 __host__ __device__ constexpr size_t packed_sums_bytes(long long pairs, int ffn) { return static_cast<size_t>(pairs) * (ffn / 256) * 32; }
 
 // v as the exact sum of three bfloat16 values (bit patterns): eight bits of it each, cut off, so that what is left is exact.
