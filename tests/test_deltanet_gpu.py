@@ -241,6 +241,39 @@ def test_chunked_rows_equal_the_row_by_row_rule(ctx, T, pos0, n_seq):
         assert O.rel_l2(got_state[0], s_state) <= TOL
 
 
+@pytest.mark.parametrize("T,n_seq,hk,hv", [(65, 1, 2, 2), (65, 2, 2, 2), (127, 1, 4, 16), (128, 2, 2, 4), (129, 1, 16, 32), (193, 3, 2, 8), (640, 1, 2, 4)])
+def test_the_walk_over_records_at_its_edges(ctx, T, n_seq, hk, hv):
+    """Two chunks and more with the records' room, the last of 1, 63 and 64 rows; one, two and four value heads a key
+    head; several sequences whose states are in slots of another order, with two planes.  Against this library's row-by-row kernel on the same inputs; both compute in float32, the
+    chunked form on 22-bit operands: 2e-5, as the other chunked passes are held to."""
+    c, d, conv = ctx, 128, 4
+    rng = np.random.default_rng(T + 10 * n_seq + hk + hv)
+    cw, vw = 2 * hk * d + hv * d, hv * d
+    width, slots, planes = cw + vw + 2 * hv, T + 3, 2
+    f32 = lambda *s: rng.standard_normal(s).astype(np.float32)
+    d_conv, d_a, d_dt = c.upload(f32(cw, conv) * 0.3), c.upload(-np.exp(f32(hv))), c.upload(f32(hv))
+    d_ring = c.upload(f32(n_seq + 1, slots, width))
+    s0 = f32((n_seq + 1) * planes * hv * d * d) * 0.1
+    d_pos, d_slot = c.upload(5 + np.arange(n_seq, dtype=np.int32)), c.upload(np.arange(n_seq, 0, -1).astype(np.int32))
+    d_plane = c.upload((np.arange(n_seq + 1) % planes).astype(np.int32))
+    floats = ((n_seq * T * (cw + 2 * hv) + 3) & ~3) + n_seq * ((T + 63) // 64) * hv * 10880
+    got = []
+    for work in (c.alloc(floats * 4), None):
+        d_state, d_out = c.upload(s0), c.alloc(n_seq * T * vw * 4)
+        c.dispatch_multi([A.make_op(A.OP_DN_STEP, A.DnStepArgs(
+            d_ring.ptr, d_conv.ptr, d_a.ptr, d_dt.ptr, d_state.ptr, d_out.ptr, d_pos.ptr, d_slot.ptr, n_seq, T, hk, hv, d, conv,
+            slots, width, EPS, 0, d_plane.ptr, planes, 0, A.ptr(work), floats if work is not None else 0))])
+        got.append((d_out.read(np.float32, n_seq * T * vw), d_state.read(np.float32, s0.size)))
+        d_state.free(), d_out.free()
+        if work is not None:
+            work.free()
+    (rows, state), (want_rows, want_state) = got
+    e_r, e_s = O.rel_l2(rows, want_rows), O.rel_l2(state, want_state)
+    print(f"deltanet walk over records T={T} x{n_seq} {hk}+{hv} heads: rows {e_r:.3e} state {e_s:.3e}")
+    assert e_r <= 2e-5 and e_s <= 2e-5
+    assert max(O.rel_l2(rows.reshape(n_seq * T, vw)[t], want_rows.reshape(n_seq * T, vw)[t]) for t in range(n_seq * T)) <= 1e-4
+
+
 def test_dn_step_refuses_unsupported_shapes(ctx):
     d = ctx.alloc(1 << 16)
     with pytest.raises(shv.pkg.ShvError):
