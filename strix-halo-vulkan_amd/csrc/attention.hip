@@ -605,12 +605,15 @@ __global__ __launch_bounds__(kBlock) void attn_append_kernel(shv_attn_decode_arg
 // takes (64 lanes x 16 bytes, in lane order: no bank is asked twice), and the loads put them
 // there themselves: a lane names the 16 bytes of the cache that belong at its place in the chunk
 // and the load writes LDS, so a tile passes through no register and costs no vector work.  Four
-// tiles are in the ring: three on their way while one is multiplied.  Every wave forms its
+// tiles are in the ring: two on their way while one is multiplied and the values of the one before.  Every wave forms its
 // products from there, as v_mfma_f32_16x16x32_f16 (eight dims or eight cells a lane), slices the
 // cache and writes its records exactly as a block of the kernel above would for that pair, so the
 // same merge follows.
+// What bounds it: the matrix cores (64 products a wave and tile) and the LDS reads (32 KB a wave and tile, as long as the
+// products), while the softmax between the two halves of a tile has neither at work.  16 + 2 heads, us a layer, 4096 rows behind
+// 4096 cells / from an empty cache: 944 / 460 with all waves in step, blocks in the order of their rows, reads waited for all
+// together; half the waves half a tile apart 892 / 423, the longest blocks first 810 / 344, reads four ahead 751 / 324.
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-typedef const __attribute__((address_space(1))) void *global_ptr_t;
 typedef __attribute__((address_space(3))) void *lds_ptr_t;
 constexpr int kPfWaves = 8;
 constexpr int kPfThreads = kPfWaves * 64;
@@ -627,12 +630,12 @@ struct PrefillSmem {
     } u;
 };
 
-// The barrier between two tiles.  A wave's loads complete in order, so "at most eight of mine still
-// out" says that all but its two youngest tiles' loads have written LDS; the LDS reads of the tile
+// The barrier between two tiles.  A wave's loads complete in order, so "at most four of mine still
+// out" says that all but its youngest tile's loads have written LDS; the LDS reads of the tile
 // just multiplied have returned (their values were used); then the workgroup meets.  Written out
 // because __syncthreads() would first wait for every load in flight, the tiles ahead included.
 __device__ __forceinline__ void tile_barrier() {
-    asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 // The same for the kernel that also loads mask words between the tiles' loads, which the count above
 // does not know of: it waits for everything (the tiles ahead included; that build gives up their
@@ -660,6 +663,8 @@ __global__ __launch_bounds__(kPfThreads) void attn_prefill_kernel(shv_attn_decod
             bx = (id >> 3) * per + die / a.n_head_kv;
         }
     }
+    // later rows see more cells: the longest blocks go first, so that those behind them even out what a compute unit has to do
+    bx = gridDim.x - 1 - bx;
     const int split = blockIdx.z;
     const int bps = (n_groups + kPfWaves - 1) / kPfWaves;
     const int seq = bx / bps, g0 = (bx % bps) * kPfWaves;
@@ -714,25 +719,20 @@ __global__ __launch_bounds__(kPfThreads) void attn_prefill_kernel(shv_attn_decod
     // ---- the tile copy: four chunks a wave, waves 0..3 the keys, 4..7 the values ----
     // K chunk (T, i): lane (n, q) stands for score-tile slot n = cell 8 (n / 4) + 4 T + n % 4 of the tile, dims 32 i + 8 q ..;
     // V chunk db: lane (n, q) stands for dim 16 db + n, cells 8 q .. of the tile.  A tile past the last repeats it.
+    // (As buffer loads: the loads to LDS that take a flat address count as LDS reads too, and every wait for a read then waits for all.)
     const int last_tile = (hi - 1) / kTile;
+    const bool keys = __builtin_amdgcn_readfirstlane(wave) < 4;
+    const int k_cell = 8 * (n >> 2) + 4 * (wave >> 1) + (n & 3);
+    const uint32_t v_at = static_cast<uint32_t>((64 * (wave - 4) + n) * kTile + 8 * q) * 2;
     auto ask_tile = [&](int t0, int stage) {
-        char *ring = sm.u.ring[stage];
         const int tile = t0 / kTile < last_tile ? t0 / kTile : last_tile;
+        const int left = hi - 1 - tile * kTile;   // cells past the pass's last: that one again
+        const uint16_t *from = keys ? kc + static_cast<size_t>(tile) * kTile * kvw : vtg + static_cast<size_t>(tile) * vtile;
+        const __amdgpu_buffer_rsrc_t tile_bytes = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(from), 0, static_cast<uint32_t>(kTile * kvw) * 2, 0x00027000);
+        const uint32_t at = keys ? static_cast<uint32_t>((k_cell < left ? k_cell : left) * kvw + 128 * (wave & 1) + 8 * q) * 2 : v_at;
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int ch = 4 * wave + u;
-            const uint16_t *g;
-            if (wave < 4) {
-                const int T = ch >> 3, i = ch & 7;
-                int c = tile * kTile + 8 * (n >> 2) + 4 * T + (n & 3);
-                c = c < hi ? c : hi - 1;
-                g = kc + static_cast<size_t>(c) * kvw + 32 * i + 8 * q;
-            } else {
-                const int db = ch - 16;
-                g = vtg + static_cast<size_t>(tile) * vtile + (16 * db + n) * kTile + 8 * q;
-            }
-            __builtin_amdgcn_global_load_lds((global_ptr_t)(g), (lds_ptr_t)(ring + ch * kChunk), 16, 0, 0);
-        }
+        for (int u = 0; u < 4; u++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(tile_bytes, (lds_ptr_t)(sm.u.ring[stage] + (4 * wave + u) * kChunk), 16, at, u * (keys ? 64 : 1024), 0, 0);
     };
 
     // ---- the wave's 16 query rows: norm, rotation, scale, operand order ----
@@ -780,9 +780,8 @@ __global__ __launch_bounds__(kPfThreads) void attn_prefill_kernel(shv_attn_decod
     __syncthreads();   // every wave holds its queries: the bytes become the ring of tiles
     ask_tile(lo, 0);
     ask_tile(lo + kTile, 1);
-    ask_tile(lo + 2 * kTile, 2);
     if constexpr (QSA) tile_barrier_all();
-    else tile_barrier();   // the first tile has landed: all but the two youngest tiles' loads of every wave
+    else tile_barrier();   // the first tile has landed: all but the youngest tile's loads of every wave
     const uint32_t *mrow = nullptr;
     if constexpr (QSA) {
         const int jr = (n >> 3) < me.valid ? (n >> 3) : me.valid - 1;
@@ -795,51 +794,50 @@ __global__ __launch_bounds__(kPfThreads) void attn_prefill_kernel(shv_attn_decod
     float m_run = -INFINITY, l_run = 0.f;
     const int my_row_pos = me.p_first + (n >> 3);
 
-    int b = 0;
-    for (int t0 = lo; t0 < hi; t0 += kTile, b = (b + 1) & (kPfStages - 1)) {
-        // three tiles on: into the stage read a tile ago (every wave has passed the barrier that ended that tile)
-        ask_tile(t0 + 3 * kTile, (b + 3) & (kPfStages - 1));
-        uint32_t mw = 0xFFFFFFFFu;
-        if constexpr (QSA) mw = mrow[t0 >> 5];
-        // tiles wholly outside the wave's slice or beyond what its rows see are skipped
-        if (me.mine && t0 < me.c1 && t0 + kTile > me.c0 && t0 <= me.p_first + 1 && (!QSA || __ballot(mw != 0u) != 0ull)) {
-            const char *kt = sm.u.ring[b], *vt = sm.u.ring[b] + 16 * kChunk;
-            // operands come from LDS four reads ahead of the products that use them: a read's
-            // latency is about what eight products take, and asked for one at a time it is paid 32 times a tile
-            float4_t st[2];
-            half8_t vb[2][4];
-            {
-                float4_t acc[2][2];
+    // scores of the tile in stage b: cell 8 q + 4 T + i of it against query row n
+    float4_t st[2];
+    auto scores = [&](int b) {
+        const char *kt = sm.u.ring[b];
+        // operands come from LDS four reads ahead of the products that use them: a read's
+        // latency is about what eight products take, and asked for one at a time it is paid 32 times a tile
+        float4_t acc[2][2];
 #pragma unroll
-                for (int T = 0; T < 2; T++)
+        for (int T = 0; T < 2; T++)
 #pragma unroll
-                    for (int e = 0; e < 2; e++) acc[T][e] = float4_t{0.f, 0.f, 0.f, 0.f};
-                half8_t kb[2][4];
-                auto read_k = [&](half8_t (&dst)[4], int g4) {   // batch g4: dim steps 2 g4, 2 g4 + 1 of both score tiles
+            for (int e = 0; e < 2; e++) acc[T][e] = float4_t{0.f, 0.f, 0.f, 0.f};
+        half8_t kb[2][4];
+        auto read_k = [&](half8_t (&dst)[4], int g4) {   // batch g4: dim steps 2 g4, 2 g4 + 1 of both score tiles
 #pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const int i = 2 * g4 + (e >> 1), T = e & 1;
-                        dst[e] = *reinterpret_cast<const half8_t *>(kt + (8 * T + i) * kChunk + lane * 16);
-                    }
-                };
-                read_k(kb[0], 0);
-#pragma unroll
-                for (int g4 = 0; g4 < 4; g4++) {
-                    if (g4 + 1 < 4) read_k(kb[(g4 + 1) & 1], g4 + 1);
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const int i = 2 * g4 + (e >> 1), T = e & 1;
-                        acc[T][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kb[g4 & 1][e], qh[i], acc[T][0], 0, 0, 0);
-                        acc[T][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kb[g4 & 1][e], ql[i], acc[T][1], 0, 0, 0);
-                    }
-                }
-                // the first values go out now, under the softmax arithmetic
-#pragma unroll
-                for (int e = 0; e < 4; e++) vb[0][e] = *reinterpret_cast<const half8_t *>(vt + e * kChunk + lane * 16);
-                st[0] = acc[0][0] + acc[0][1];
-                st[1] = acc[1][0] + acc[1][1];
+            for (int e = 0; e < 4; e++) {
+                const int i = 2 * g4 + (e >> 1), T = e & 1;
+                dst[e] = *reinterpret_cast<const half8_t *>(kt + (8 * T + i) * kChunk + lane * 16);
             }
-            float mx = -INFINITY;
+        };
+        read_k(kb[0], 0);
+#pragma unroll
+        for (int g4 = 0; g4 < 4; g4++) {
+            if (g4 + 1 < 4) read_k(kb[(g4 + 1) & 1], g4 + 1);
+            __builtin_amdgcn_sched_barrier(0);  // (left to itself the compiler puts the reads just before their use)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int i = 2 * g4 + (e >> 1), T = e & 1;
+                acc[T][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kb[g4 & 1][e], qh[i], acc[T][0], 0, 0, 0);
+                acc[T][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kb[g4 & 1][e], ql[i], acc[T][1], 0, 0, 0);
+            }
+        }
+        st[0] = acc[0][0] + acc[0][1];
+        st[1] = acc[1][0] + acc[1][1];
+    };
+    // the tile at t0, whose scores are in st, whose values in stage b and whose mask word is mw, into the sums
+    auto attend = [&](int t0, int b, uint32_t mw) {
+        const char *vt = sm.u.ring[b] + 16 * kChunk;
+        half8_t vb[2][4];
+        // the first values go out now, under the softmax arithmetic
+#pragma unroll
+        for (int e = 0; e < 4; e++) vb[0][e] = *reinterpret_cast<const half8_t *>(vt + e * kChunk + lane * 16);
+        __builtin_amdgcn_sched_barrier(0);
+        // a tile that every row sees whole (all but a row's last, and a slice's first and last) needs no comparisons
+        if (QSA || t0 < me.c0 || t0 + kTile > me.c1 || t0 + kTile - 1 > me.p_first) {
 #pragma unroll
             for (int T = 0; T < 2; T++)
 #pragma unroll
@@ -848,58 +846,85 @@ __global__ __launch_bounds__(kPfThreads) void attn_prefill_kernel(shv_attn_decod
                     bool ok = c >= me.c0 && c < me.c1 && c <= my_row_pos;
                     if constexpr (QSA) ok = ok && ((mw >> (8 * q + 4 * T + i)) & 1u) != 0u;
                     st[T][i] = ok ? st[T][i] : -INFINITY;
-                    mx = fmaxf(mx, st[T][i]);
                 }
-            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            const float m_new = fmaxf(m_run, mx);
-            const float m_use = m_new == -INFINITY ? 0.f : m_new;
-            float sum = 0.f;
-            half8_t ph, pl;
+        }
+        float mx = -INFINITY;
 #pragma unroll
-            for (int T = 0; T < 2; T++)
+        for (int T = 0; T < 2; T++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const float pv = __expf(st[T][i] - m_use);
-                    sum += pv;
-                    const _Float16 hi16 = static_cast<_Float16>(pv);
-                    ph[4 * T + i] = hi16;
-                    pl[4 * T + i] = static_cast<_Float16>(pv - static_cast<float>(hi16));
-                }
-            sum += __shfl_xor(sum, 16, 64);
-            sum += __shfl_xor(sum, 32, 64);
-            const float alpha = __expf(m_run - m_use);
-            l_run = l_run * alpha + sum;
-            m_run = m_new;
-            if (__ballot(alpha != 1.f) != 0ull) {
-                // a lane's four accumulator rows are query rows 4 q + i: their factors sit in lanes 4 q + i
-                float av[4];
+            for (int i = 0; i < 4; i++) mx = fmaxf(mx, st[T][i]);
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const float m_new = fmaxf(m_run, mx);
+        const float m_use = m_new == -INFINITY ? 0.f : m_new;
+        float sum = 0.f;
+        half8_t ph, pl;
 #pragma unroll
-                for (int i = 0; i < 4; i++) av[i] = __shfl(alpha, 4 * q + i, 64);
+        for (int T = 0; T < 2; T++)
 #pragma unroll
-                for (int db = 0; db < 16; db++)
-#pragma unroll
-                    for (int i = 0; i < 4; i++) o[db][i] *= av[i];
+            for (int i = 0; i < 4; i++) {
+                const float pv = __expf(st[T][i] - m_use);
+                sum += pv;
+                const _Float16 hi16 = static_cast<_Float16>(pv);
+                ph[4 * T + i] = hi16;
+                pl[4 * T + i] = static_cast<_Float16>(pv - static_cast<float>(hi16));
             }
+        sum += __shfl_xor(sum, 16, 64);
+        sum += __shfl_xor(sum, 32, 64);
+        const float alpha = __expf(m_run - m_use);
+        l_run = l_run * alpha + sum;
+        m_run = m_new;
+        if (__ballot(alpha != 1.f) != 0ull) {
+            // a lane's four accumulator rows are query rows 4 q + i: their factors sit in lanes 4 q + i
+            float av[4];
 #pragma unroll
-            for (int g4 = 0; g4 < 4; g4++) {
-                if (g4 + 1 < 4) {
+            for (int i = 0; i < 4; i++) av[i] = __shfl(alpha, 4 * q + i, 64);
 #pragma unroll
-                    for (int e = 0; e < 4; e++) vb[(g4 + 1) & 1][e] = *reinterpret_cast<const half8_t *>(vt + (4 * (g4 + 1) + e) * kChunk + lane * 16);
-                }
+            for (int db = 0; db < 16; db++)
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const int db = 4 * g4 + e;
-                    float4_t acc = o[db];
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, vb[g4 & 1][e], acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl, vb[g4 & 1][e], acc, 0, 0, 0);
-                    o[db] = acc;
-                }
+                for (int i = 0; i < 4; i++) o[db][i] *= av[i];
+        }
+#pragma unroll
+        for (int g4 = 0; g4 < 4; g4++) {
+            if (g4 + 1 < 4) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) vb[(g4 + 1) & 1][e] = *reinterpret_cast<const half8_t *>(vt + (4 * (g4 + 1) + e) * kChunk + lane * 16);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int db = 4 * g4 + e;
+                float4_t acc = o[db];
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, vb[g4 & 1][e], acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl, vb[g4 & 1][e], acc, 0, 0, 0);
+                o[db] = acc;
             }
         }
+    };
+
+    // Between two barriers the first four waves take a tile's scores, its softmax and its values; the other four, which share
+    // their matrix cores, the softmax and the values of the tile before and then this one's scores: in step all eight would
+    // leave the matrix cores idle through the softmax and then wait for them together.
+    const bool late = wave >= kPfWaves / 2;
+    bool pending = false;   // late: st holds the tile before's scores
+    uint32_t mw_before = 0xFFFFFFFFu;
+    int b = 0;
+    for (int t0 = lo; t0 < hi; t0 += kTile, b = (b + 1) & (kPfStages - 1)) {
+        // two tiles on: into the stage whose values were read up to the barrier before
+        ask_tile(t0 + 2 * kTile, (b + 2) & (kPfStages - 1));
+        uint32_t mw = 0xFFFFFFFFu;
+        if constexpr (QSA) mw = mrow[t0 >> 5];
+        // tiles wholly outside the wave's slice or beyond what its rows see are skipped
+        const bool live = me.mine && t0 < me.c1 && t0 + kTile > me.c0 && t0 <= me.p_first + 1 && (!QSA || __ballot(mw != 0u) != 0ull);
+        if (live && !late) scores(b);
+        if (late ? pending : live) attend(late ? t0 - kTile : t0, late ? (b + kPfStages - 1) & (kPfStages - 1) : b, late ? mw_before : mw);
+        if (live && late) scores(b);
+        pending = live;
+        mw_before = mw;
         if constexpr (QSA) tile_barrier_all();
-        else tile_barrier();   // the next tile has landed, this one has been read
+        else tile_barrier();   // the next tile has landed, this one's keys have been read, and the values of the one before
     }
+    if (late && pending) attend(lo + ((hi - 1 - lo) / kTile) * kTile, (b + kPfStages - 1) & (kPfStages - 1), mw_before);
     // the loads asked for past the last tile still write LDS: none may be out when the wave ends and its LDS goes to another workgroup
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (!me.mine) return;

@@ -249,6 +249,38 @@ def test_attn_refuses_unsupported_shapes(ctx):
             ctx.enqueue(A.OP_ATTN_DECODE, mk(**bad))
 
 
+@pytest.mark.parametrize("n_seq,rows,past,n_splits", [(1, 15, 0, 1), (1, 16, 17, 1), (2, 17, 47, 1), (1, 34, 1, 64), (3, 31, 480, 64),
+                                                       (1, 257, 0, 8), (1, 130, 900, 64), (1, 600, 1000, 64)])
+def test_a_prompt_pass_against_its_rows_alone(ctx, n_seq, rows, past, n_splits):
+    """A pass of fifteen rows and more, whose blocks share the cache's tiles (one tile, a first and a last that a row sees in part, tiles
+    seen whole; one slice a row pair and several; a last block and a last pair not full), against the same rows one at a time over the
+    cells the pass has written.  Both hold the queries and the weights of the cells to 22 bits and add in float32: 2e-5."""
+    case = AttnCase(ctx, seed=17 + rows)
+    c, rng, max_cells = ctx, case.rng, (past + n_seq + rows + 31) // 32 * 32
+    case.upload(max_cells)
+    qkv = rng.standard_normal((n_seq, rows, case.width)).astype(np.float32)
+    cells = rng.standard_normal((2, n_seq, max_cells, NKV * D)).astype(np.float16)
+    pos = (past + np.arange(n_seq)).astype(np.int32)
+    for s in range(n_seq):
+        cells[:, s, pos[s]:] = 0
+    d_kc, d_vc = c.upload(cells[0]), c.upload(v_dev(cells[1].reshape(n_seq, max_cells, NKV, D)))
+    d_pos, d_out, d_part = c.upload(pos), c.alloc(n_seq * rows * NH * D * 4), c.alloc(_part_floats(n_seq, n_splits, rows) * 4)
+
+    def attend(d_qkv, d_at, n):
+        c.dispatch_multi([A.make_op(A.OP_ATTN_DECODE, A.AttnDecodeArgs(
+            d_qkv.ptr, case.d_qn.ptr, case.d_kn.ptr, case.d_rope.ptr, d_kc.ptr, d_vc.ptr, d_part.ptr, d_out.ptr, d_at.ptr, None, n_seq, n, NH, NKV,
+            D, ROPE, max_cells, case.width, n_splits, EPS))])
+        return d_out.read(np.float32, n_seq * n * NH * D).reshape(n_seq, n, NH * D)
+
+    got = attend(c.upload(qkv), d_pos, rows)
+    worst = 0.0
+    for t in sorted({0, 1, rows // 2, rows - 2, rows - 1, *range(0, rows, 37)}):
+        one = attend(c.upload(qkv[:, t]), c.upload(pos + t), 1)
+        worst = max(worst, *(O.rel_l2(got[s, t], one[s, 0]) for s in range(n_seq)))
+    print(f"attention of {n_seq} x {rows} rows behind {past} cells, {n_splits} slices: {worst:.2e}")
+    assert worst <= 2e-5
+
+
 @pytest.mark.parametrize("n_seq,seq_len,first", [(1, 1, 0), (3, 2, 31), (2, 5, 29), (1, 70, 60)])
 def test_cells_alone_are_the_pass_cells(ctx, n_seq, seq_len, first):
     """The cells written without attending are those the attention's own launch writes, bit for bit, and no others; attending without
