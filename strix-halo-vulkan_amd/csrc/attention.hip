@@ -33,6 +33,7 @@ constexpr int kD = 256;        // head dimension the kernel is built for
 constexpr int kRep = 8;        // query heads per KV head
 constexpr int kTile = 32;         // cells a wave takes at a time
 constexpr int kSliceCells = 128;  // cells a slice gets while there are slices to spare: one tile a wave
+constexpr int kPfSliceCells = 192;  // and a slice of a prompt pass's blocks, each of which forms its 128 query rows anew
 constexpr int kMaxSplits = 512;
 constexpr int kRec = kRep * (kD + 2);  // floats of one (slice, row) record: per head d values, max, sum
 
@@ -574,6 +575,42 @@ __global__ __launch_bounds__(64 * NW) void attn_merge_kernel(shv_attn_decode_arg
     a.out[static_cast<size_t>(seq * a.seq_len + row0 + j) * a.n_head * kD + static_cast<size_t>(head) * kD + d] = nt / dt;
 }
 
+// The same for the rows of a prompt pass, whose pairs have few slices: a block a row and head, a thread a dim.  A pair with one
+// slice has its rows already (attn_prefill_kernel).  grid: (n_head, 2, row pairs).
+template <int MB>
+__global__ __launch_bounds__(kD) void attn_merge_rows_kernel(shv_attn_decode_args a, int n_groups, int slice_cells) {
+    const int head = blockIdx.x, d = threadIdx.x, j = blockIdx.y;
+    const int seq = blockIdx.z / n_groups, row0 = 2 * (blockIdx.z % n_groups);
+    const int kvh = head / kRep, hh = head % kRep;
+    const int valid = a.seq_len - row0 < 2 ? a.seq_len - row0 : 2;
+    const int n_cells = (a.pos ? a.pos[seq] : 0) + row0 + valid;
+    int n_active = (n_cells + slice_cells - 1) / slice_cells;
+    if (n_active > a.n_splits) n_active = a.n_splits;
+    if (j >= valid || n_active == 1) return;
+    const float *pin = a.partial + (static_cast<size_t>(blockIdx.z) * a.n_head_kv + kvh) * a.n_splits * 2 * kRec + j * kRec + hh * (kD + 2);
+    float num = 0.f, den = 0.f, M = -INFINITY;
+    for (int s0 = 0; s0 < n_active; s0 += MB) {
+        float v[MB];
+        float2 ml[MB];
+#pragma unroll
+        for (int u = 0; u < MB; u++) {
+            const float *rec = pin + static_cast<size_t>(s0 + u < n_active ? s0 + u : s0) * 2 * kRec;
+            v[u] = rec[d];
+            ml[u] = *reinterpret_cast<const float2 *>(rec + kD);
+        }
+#pragma unroll
+        for (int u = 0; u < MB; u++) {
+            if (s0 + u >= n_active || ml[u].x == -INFINITY) continue;
+            const float Mn = fmaxf(M, ml[u].x);
+            const float shrink = __expf(M - Mn), w = __expf(ml[u].x - Mn);  // shrink is 0 while M is -inf
+            den = fmaf(den, shrink, w * ml[u].y);
+            num = fmaf(num, shrink, w * v[u]);
+            M = Mn;
+        }
+    }
+    a.out[static_cast<size_t>(seq * a.seq_len + row0 + j) * a.n_head * kD + static_cast<size_t>(head) * kD + d] = num / den;
+}
+
 // grid: (n_head_kv, seq_len, n_seq): the cells of every row of a pass, written before any of
 // them is read: K normed and rotated by the first wave, V transposed into its tile by all threads.
 __global__ __launch_bounds__(kBlock) void attn_append_kernel(shv_attn_decode_args a) {
@@ -646,7 +683,7 @@ __device__ __forceinline__ void tile_barrier_all() {
 
 // grid: (n_seq * ceil(n_groups / 8), n_head_kv, n_splits); the cells of the pass are in the cache already.
 template <bool QSA>
-__global__ __launch_bounds__(kPfThreads) void attn_prefill_kernel(shv_attn_decode_args a, int n_groups, int slice_cells, int direct) {
+__global__ __launch_bounds__(kPfThreads) void attn_prefill_kernel(shv_attn_decode_args a, int n_groups, int slice_cells) {
     extern __shared__ __align__(16) char praw[];
     PrefillSmem &sm = *reinterpret_cast<PrefillSmem *>(praw);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -671,7 +708,7 @@ __global__ __launch_bounds__(kPfThreads) void attn_prefill_kernel(shv_attn_decod
     const int slot = a.slot ? a.slot[seq] : seq;
     const int pos_first = a.pos ? a.pos[seq] : 0;
     // pair gg of the sequence: its rows, what it sees, its slice of that
-    struct Slice { int c0, c1, p_first, valid; bool mine, empty; };
+    struct Slice { int c0, c1, p_first, valid; bool mine, empty, alone; };
     auto slice_of = [&](int gg) {
         Slice s;
         const bool live = gg < n_groups;
@@ -687,6 +724,7 @@ __global__ __launch_bounds__(kPfThreads) void attn_prefill_kernel(shv_attn_decod
         s.c0 = split * cps;
         s.c1 = s.c0 + cps < n_cells ? s.c0 + cps : n_cells;
         s.mine = live && split < n_active && s.c1 > s.c0;
+        s.alone = n_active == 1;
         // slices start on a tile of V: rounded up, the last of a pair's slices can start past its cells
         s.empty = live && split < n_active && s.c1 <= s.c0;
         return s;
@@ -928,8 +966,8 @@ __global__ __launch_bounds__(kPfThreads) void attn_prefill_kernel(shv_attn_decod
     // the loads asked for past the last tile still write LDS: none may be out when the wave ends and its LDS goes to another workgroup
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (!me.mine) return;
-    if (direct) {
-        // one slice a pair: what the merge would make of its single record, sums / sum, goes straight out
+    if (me.alone) {
+        // one slice: what the merge would make of its single record, sums / sum, goes straight out
         float lr[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) lr[i] = __shfl(l_run, 4 * q + i, 64);   // query row 4 q + i keeps its sum in lane 4 q + i
@@ -961,28 +999,36 @@ int launch_rows(shv_ctx *ctx, const shv_attn_decode_args &a, int row0, int n_gro
     // of many sequences) brings its own parallelism, and every block pays the query prologue
     // (norms and rotation of its 16 rows) whatever its slice holds: such a pass takes as many
     // slices as make two blocks a compute unit, no more (64 rows at 32 768 cells: 359 to 214 us).
+    // A block of attn_prefill_kernel has eight pairs, and a compute unit holds one (the ring of tiles): there
+    // as many slices as still find a compute unit each, of kPfSliceCells and more.  Counted by pairs instead, us:
+    // 121 rows behind 32 768 cells 358 (now 177), 512 behind 32 000 1600 (518), 300 behind 4000 148 (88), 37 behind
+    // 3000 39 (41).  Two slices where a compute unit is there for more than half of the blocks: 1531 rows from an
+    // empty cache 143 for 112, most of it writing and merging the slices' sums.
     shv_attn_decode_args b = a;
     const int lanes = a.n_seq * n_groups * a.n_head_kv;
     const int want = (2 * ctx->prop.multiProcessorCount + lanes - 1) / lanes;
-    if (b.n_splits > want) b.n_splits = want < 1 ? 1 : want;
+    const bool shared = R == 2 && !append && row0 == 0 && n_groups >= 8;  // a prompt pass: eight pairs a block share the cache's tiles
+    int most = shared ? ctx->prop.multiProcessorCount / (a.n_seq * ((n_groups + kPfWaves - 1) / kPfWaves) * a.n_head_kv) : want;
+    if (most < 1) most = 1;
+    if (b.n_splits > most) b.n_splits = most;
     // one row pair: slices of one tile while there are slices to spare, so that as many compute
     // units as possible pull the cache (a unit issues a wave's 16-byte loads at about 25 B a clock;
     // 36 units over 2 300 cells took 2.2 us to ask for them, 144 take a quarter of that)
-    const int slice_cells = a.n_seq * n_groups == 1 ? kTile : kSliceCells;
-    if (R == 2 && !append && row0 == 0 && n_groups >= 8) {
-        // a prompt pass: eight pairs a block share the cache's tiles
+    const int slice_cells = a.n_seq * n_groups == 1 ? kTile : shared ? kPfSliceCells : kSliceCells;
+    if (shared) {
         static std::atomic<bool> raised{false};
         if (!raised.load(std::memory_order_acquire)) {
             SHV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_prefill_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(sizeof(PrefillSmem))));
             SHV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_prefill_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(sizeof(PrefillSmem))));
             raised.store(true, std::memory_order_release);
         }
-        // with one slice a pair there is nothing to merge: the kernel writes the rows themselves
-        const int direct = b.n_splits == 1 ? 1 : 0;
         const dim3 grid(a.n_seq * ((n_groups + kPfWaves - 1) / kPfWaves), a.n_head_kv, b.n_splits);
-        if (a.mask) SHV_LAUNCH(ctx, attn_prefill_kernel<true>, grid, dim3(kPfThreads), sizeof(PrefillSmem), b, n_groups, slice_cells, direct);
-        else SHV_LAUNCH(ctx, attn_prefill_kernel<false>, grid, dim3(kPfThreads), sizeof(PrefillSmem), b, n_groups, slice_cells, direct);
-        if (direct) return SHV_OK;
+        if (a.mask) SHV_LAUNCH(ctx, attn_prefill_kernel<true>, grid, dim3(kPfThreads), sizeof(PrefillSmem), b, n_groups, slice_cells);
+        else SHV_LAUNCH(ctx, attn_prefill_kernel<false>, grid, dim3(kPfThreads), sizeof(PrefillSmem), b, n_groups, slice_cells);
+        // the slices' sums are read sixteen at a time where there may be that many (or four: what is not there is read as the first again)
+        if (b.n_splits > 4) SHV_LAUNCH(ctx, attn_merge_rows_kernel<16>, dim3(a.n_head, 2, a.n_seq * n_groups), dim3(kD), 0, b, n_groups, slice_cells);
+        else if (b.n_splits > 1) SHV_LAUNCH(ctx, attn_merge_rows_kernel<4>, dim3(a.n_head, 2, a.n_seq * n_groups), dim3(kD), 0, b, n_groups, slice_cells);
+        return SHV_OK;
     } else {
         dim3 grid(a.n_seq * n_groups, a.n_head_kv, b.n_splits);
         if (a.mask) SHV_LAUNCH(ctx, (attn_decode_kernel<R, true>), grid, dim3(kBlock), 0, b, row0, n_groups, append, slice_cells);

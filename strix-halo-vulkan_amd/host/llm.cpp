@@ -1017,8 +1017,9 @@ AttnGPU::AttnGPU(Device &dev, const Model &m, int maxTokens, int nKV, int slots,
     // one set of slice records per sequence of a batched pass (an ordinary pass is one sequence)
     // Slice records: a pass of P row pairs over all its sequences takes min(splits, ceil(2 CUs / (P kv)))
     // slices a pair, two rows of 8 heads a record.  One pair can take every slice; many pairs
-    // take at most 2 CUs + P kv records in all, and P is at most the pass's rows.
-    partial_records_ = static_cast<size_t>(c_.NHeadKV) * kMaxSplits + 2 * 512 + (T + 1) * c_.NHeadKV;
+    // take at most 2 CUs + P kv records in all, and P is at most the pass's rows.  A sequence's eight pairs
+    // and more go in blocks of eight, with as many slices as leave a block a CU: 8 CUs records at most.
+    partial_records_ = std::max(static_cast<size_t>(c_.NHeadKV) * kMaxSplits + 2 * 512 + (T + 1) * c_.NHeadKV, size_t{8 * 512});
     partial_ = static_cast<float *>(dev.alloc(partial_records_ * 2 * 8 * (c_.HeadDim + 2) * 4));
     const std::vector<float> rt = rope_table(nKV, c_.RopeDims, c_.RopeBase);
     rope_ = static_cast<float *>(dev.alloc(rt.size() * 4));
@@ -1086,7 +1087,9 @@ std::vector<shv_op> AttnGPU::Dispatches(int l, const float *in, float *out, cons
     {
         // the slice records this pass writes (the launcher's own arithmetic) against what was staged
         const size_t pairs = static_cast<size_t>(r.n_seq) * ((r.seq_len + 1) / 2);
-        const size_t per_pair = std::min<size_t>(splits_, (2 * 512 + pairs * c_.NHeadKV - 1) / (pairs * c_.NHeadKV));
+        const size_t groups = (r.seq_len + 1) / 2, blocks = r.n_seq * ((groups + 7) / 8) * c_.NHeadKV;
+        const size_t most = groups >= 8 ? std::max<size_t>(1, 512 / blocks) : (2 * 512 + pairs * c_.NHeadKV - 1) / (pairs * c_.NHeadKV);
+        const size_t per_pair = std::min<size_t>(splits_, most);
         if (pairs * c_.NHeadKV * per_pair > partial_records_)
             throw Error("llm: AttnGPU: " + std::to_string(r.n_seq) + " sequences of " + std::to_string(r.seq_len) + " rows need more slice records than were staged");
     }
