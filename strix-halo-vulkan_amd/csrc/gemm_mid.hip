@@ -233,6 +233,8 @@ __global__ __launch_bounds__(64 * W) void gemm_mid_kernel(shv_gemv_q4k_args a, c
 // Bound by the fragments' way from L2, as above, and below some 500 rows by the launches.  Slabs of 64 rows staged through LDS
 // took 46 us whatever the pass's height, 27 blocks of them at 150 rows: with its staging and the selection after it the router
 // went from 58 to 24 us a layer at 150 rows of 513 x 2048, from 60 to 31 at 512, from 76 to 62 at 2048.
+// A fragment of the next tile asked for when this tile's is multiplied: 98.5 to 90.2 us at 4096 rows, 50.4 to 46.7 at 1531; a
+// die's blocks on neighbouring tiles: to 80.7 and 43.3 (150 rows 25.1 to 24.6).
 template <int R>
 __global__ __launch_bounds__(512) void router_rows_kernel(const float *W, const float *extra_row, int n_rows, int K, int n_tok, const char *staged, float *logits,
                                                           int logits_stride, int tiles, int per_chunk) {
@@ -240,7 +242,11 @@ __global__ __launch_bounds__(512) void router_rows_kernel(const float *W, const 
     __shared__ __align__(16) float cpart[2][NW][R * 256];
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, kb = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int sbs = K / 256, row0 = blockIdx.x * (16 * R), tile0 = blockIdx.y * per_chunk;
+    // Workgroup i goes to die i % 8, each with an L2 of its own: a die takes neighbouring (chunk, rows), so that it reads two or
+    // three chunks of the staged rows and not all of them.
+    const int count = gridDim.x * gridDim.y, id = blockIdx.x + gridDim.x * blockIdx.y, die = id & 7;
+    const int item = die * (count >> 3) + min(die, count & 7) + (id >> 3);
+    const int sbs = K / 256, row0 = item % gridDim.x * (16 * R), tile0 = item / gridDim.x * per_chunk;
     const int tile_end = tile0 + per_chunk < tiles ? tile0 + per_chunk : tiles;
     half8_t wh[R][8], wl[R][8];
     auto form = [&](int sb) {  // this lane's 64 columns of every row
@@ -263,7 +269,18 @@ __global__ __launch_bounds__(512) void router_rows_kernel(const float *W, const 
             }
         }
     };
-    if (wave < sbs) form(wave);
+    // a fragment of the next tile is asked for as soon as this tile's is multiplied (and the first tile's before the weights are formed)
+    half8_t f[8][2];
+    auto ask = [&](int tile, int sb, int v) {
+        const char *frag = staged + (static_cast<size_t>(tile) * sbs + sb) * kMidSb + lane * 16;
+#pragma unroll
+        for (int p = 0; p < 2; p++) f[v][p] = *reinterpret_cast<const half8_t *>(frag + (v * 2 + p) * kMidFrag);
+    };
+    if (wave < sbs) {
+#pragma unroll
+        for (int v = 0; v < 8; v++) ask(tile0, wave, v);
+        form(wave);
+    }
     const int o = tid % (R * 256), out_row = row0 + 16 * (o >> 8) + ((o >> 2) & 15), t_in = 4 * (o >> 6 & 3) + (o & 3);
     const bool mine = tid < R * 256 && out_row < n_rows;
     int buf = 0;
@@ -273,20 +290,18 @@ __global__ __launch_bounds__(512) void router_rows_kernel(const float *W, const 
         for (int r = 0; r < R; r++) ym[r] = yl[r] = float4_t{0.f, 0.f, 0.f, 0.f};
         for (int sb = wave; sb < sbs; sb += NW) {
             if (sbs > NW) form(sb);
-            const char *frag = staged + (static_cast<size_t>(tile) * sbs + sb) * kMidSb + lane * 16;
-            half8_t f[8][2];
+            const int sb_next = sb + NW < sbs ? sb + NW : wave, tile_next = sb + NW < sbs ? tile : tile + 1 < tile_end ? tile + 1 : tile;
 #pragma unroll
-            for (int v = 0; v < 8; v++)
-#pragma unroll
-                for (int p = 0; p < 2; p++) f[v][p] = *reinterpret_cast<const half8_t *>(frag + (v * 2 + p) * kMidFrag);
-#pragma unroll
-            for (int v = 0; v < 8; v++)
+            for (int v = 0; v < 8; v++) {
 #pragma unroll
                 for (int r = 0; r < R; r++) {
                     ym[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f[v][0], wh[r][v], ym[r], 0, 0, 0);
                     ym[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f[v][1], wh[r][v], ym[r], 0, 0, 0);
                     yl[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f[v][0], wl[r][v], yl[r], 0, 0, 0);
                 }
+                ask(tile_next, sb_next, v);
+                __builtin_amdgcn_sched_barrier(0);  // (here, and not all of them behind the last product)
+            }
         }
 #pragma unroll
         for (int r = 0; r < R; r++)
