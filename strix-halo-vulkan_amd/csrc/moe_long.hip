@@ -123,11 +123,16 @@ __device__ __forceinline__ void up_pass(const shv_moe_up_args &a, const char *ga
         const int col = col0 + c;
         const float *from = act_s + i * kActPitch + (R == 2 ? c : (c >> 4) * 32 + (c & 15));
         float v[8], sum = 0.f;
+        {
+            // the sum is of the values as they are stored (no product and sum in one rounding where R is 1), so that a pair's result
+            // is the same bit for bit whichever pass of its list it falls to: the order of a list changes from call to call
+#pragma clang fp contract(off)
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            v[j] = from[j];
-            if constexpr (R == 1) v[j] = v[j] * sigmoid_exact(v[j]) * from[16 + j];
-            sum += v[j];
+            for (int j = 0; j < 8; j++) {
+                v[j] = from[j];
+                if constexpr (R == 1) v[j] = v[j] * sigmoid_exact(v[j]) * from[16 + j];
+                sum += v[j];
+            }
         }
         const float o[8] = {v[0], v[2], v[1], v[3], v[4], v[6], v[5], v[7]};
         sum += __shfl_xor(sum, 1, 64);

@@ -82,3 +82,13 @@ def test_long_lists_are_the_slots(rig, lengths, used, packed):  # noqa: F811
     rel = np.linalg.norm(got - want) / np.linalg.norm(want)
     assert rel <= 1e-5, (topk.shape, rel)
     assert np.max(np.abs(got - want)) <= 1e-4 * np.sqrt(np.mean(want ** 2))
+
+
+@pytest.mark.parametrize("packed", [1, 0])
+def test_a_token_is_the_same_in_any_place_of_a_list(rig, packed):  # noqa: F811
+    """A list's order is the order in which its tokens were counted, another one from call to call: a token's result must not depend on
+    which pass over the list it falls to, nor on its row there.  Bit for bit, the tokens in another order and turned round."""
+    topk = selection([97, 98, 101, 128, 129, 160, 193] + [40] * 16 + [42], 4, np.random.default_rng(3))
+    want = block(rig, topk, True, packed)
+    for order in (np.arange(len(topk))[::-1], np.random.default_rng(4).permutation(len(topk))):
+        assert np.array_equal(block(rig, topk, True, packed, order), want[order])

@@ -42,13 +42,13 @@ def selection(lengths, used, rng):
     return np.ascontiguousarray(flat[rng.permutation(tokens)], dtype=np.int32)
 
 
-def block(rig, topk, grouped, packed):
+def block(rig, topk, grouped, packed, order=slice(None)):
     c, E, _, banks = rig
     T, U = topk.shape
     rng = np.random.default_rng(T)
     xn, res = rng.standard_normal((T, H)).astype(np.float32), rng.standard_normal((T, H)).astype(np.float32)
     wts = rng.random((T, U + 1)).astype(np.float32)
-    bufs = [c.upload(a) for a in (xn, topk, wts, res)]
+    bufs = [c.upload(a[order]) for a in (xn, topk, wts, res)]
     act, out = c.alloc(T * (U + 1) * F * 4), c.alloc(T * H * 4)
     group, pairs = c.alloc((2 * E + 1 + T * U) * 4), c.alloc(T * (U + 1) * H * 4)
     g, u, d, gs, us, ds = (b.ptr for b in banks)
