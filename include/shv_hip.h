@@ -400,7 +400,7 @@ typedef struct {
  * multiple of 4 floats) for 10 880 more floats per (sequence, chunk of 64 rows, value head), what a
  * chunk needs that does not depend on the state is formed for every chunk of the pass at once, by a
  * launch of its own, instead of inside the walk over the chunks by each of a head's eight blocks;
- * the walk is then a kernel of its own, a third as long.  The reference scans row by row at every pass length
+ * the walk is then a kernel of its own, half as long.  The reference scans row by row at every pass length
  * (shaders/llm_dn_scan.comp; llm/gpu_deltanet.go:48-52 names the chunked form as not built there). */
 typedef struct {
     const float *ring;

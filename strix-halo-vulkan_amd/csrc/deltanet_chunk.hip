@@ -558,7 +558,7 @@ __global__ __launch_bounds__(kThreads, 1) void dn_chunk_kernel(shv_dn_step_args 
 // by columns, goes past the registers into LDS (its sixteen-byte pieces exchanged so that either way of reading it meets all
 // banks) and its columns are read by the transposing load.  LDS holds the state's halves, B, U and U e^(G_C - G_s) besides.
 // 16 + 32 heads, 4096 rows, the walk alone: 158 us (2.4 us a chunk; 310 with four waves, every operand by registers to LDS and
-// no wave beside the chain), 1531 rows about 55 (116).  Tried beside it: W2 behind the first barrier, the four waves beside the chain
+// no wave beside the chain), 1531 rows 63 (116).  Tried beside it: W2 behind the first barrier, the four waves beside the chain
 // loading all of k^, a third buffer of it: 4 to 35 us longer at 4096 rows.
 constexpr int kWalkThreads = 512;
 constexpr int kRowBytes = kD * 4;  // of k^ in LDS: [octet of columns] hi, lo x 16 bytes
