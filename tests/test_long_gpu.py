@@ -84,6 +84,18 @@ def test_long_lists_are_the_slots(rig, lengths, used, packed):  # noqa: F811
     assert np.max(np.abs(got - want)) <= 1e-4 * np.sqrt(np.mean(want ** 2))
 
 
+# walks of up to 32, 64 and 96 tokens, on either side of both lines (24 and 60 tokens an expert), lists on the edges of each
+@pytest.mark.parametrize("lengths,used", [
+    ([24] * 16 + [1, 31, 32, 33, 64, 6, 1, 24], 3),
+    ([24] * 16 + [1, 31, 32, 33, 64, 65, 0, 2], 4),
+    ([60] * 16 + [63, 64, 65, 66, 97, 95, 29, 1], 4),
+    ([60] * 15 + [63, 64, 65, 96, 97, 129, 31, 32, 103], 4),
+])
+@pytest.mark.parametrize("packed", [1, 0])
+def test_walks_of_every_height(rig, lengths, used, packed):  # noqa: F811
+    test_long_lists_are_the_slots(rig, lengths, used, packed)
+
+
 @pytest.mark.parametrize("packed", [1, 0])
 def test_a_token_is_the_same_in_any_place_of_a_list(rig, packed):  # noqa: F811
     """A list's order is the order in which its tokens were counted, another one from call to call: a token's result must not depend on
