@@ -37,8 +37,8 @@ constexpr int kMaxExperts = 1024;
 // then n_tok * n_used pair ids (token * (n_used + 1) + slot), then the experts in the order their
 // blocks are launched: longest list first, so that the blocks which walk their weights two or
 // three times start early and the launch does not end on them.  A list's order is whatever the
-// arrivals made it; every pair's products are formed in a matrix-core column of their own, so no
-// value depends on it.
+// arrivals made it, but for the list kernels (moe_group_place_kernel): in the others no value depends
+// on it, every pair's products being formed and added alike in whatever column they are.
 __global__ __launch_bounds__(1024) void moe_group_kernel(const int32_t *topk, int n_tok, int n_used, int n_expert, int32_t *group) {
     __shared__ int32_t s_cnt[kMaxExperts + 1];
     __shared__ __align__(16) int32_t s_len[kMaxExperts];
@@ -135,6 +135,10 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int32_t *topk, in
 // First launch: every block's count of its pairs per expert, to counts[b][e].  Second: every block adds up the
 // counts (an expert's total, and what the blocks before it hold of it), forms the starts, and places its own pairs
 // behind those of the blocks before it; block 0 also writes the starts and the experts' launch order.
+// In order: a list's pairs lie by token (chunks of at most a pair a thread).  The list kernels add a token's two parts earlier
+// or later as a pass over its list has more than eight tokens or not, so a place that changes from call to call would change
+// its last bit.  The waves then place their pairs one after the other, a lane behind the lanes before it with the same expert
+// (150 rows of ten experts: 224.2 us a layer with the pairs as they arrive, 224.9 so; 750 rows 430.5 and 430.9).
 constexpr int kGroupBlocks = 16;
 // Blocks past the counting ones, when the launch has them, stage the rows x [rows][k] for the list kernels meanwhile: whole
 // rows, k / 256 of a block's sixteen waves each.
@@ -169,7 +173,7 @@ __global__ __launch_bounds__(1024) void moe_group_count_kernel(const int32_t *to
 }
 
 __global__ __launch_bounds__(1024) void moe_group_place_kernel(const int32_t *topk, int n_pairs, int chunk, int n_used, int n_expert, const int32_t *counts,
-                                                               int32_t *group) {
+                                                               int32_t *group, int in_order) {
     __shared__ int32_t s_cnt[kMaxExperts + 1];
     __shared__ __align__(16) int32_t s_len[kMaxExperts];
     __shared__ int32_t s_wsum[16];
@@ -230,6 +234,25 @@ __global__ __launch_bounds__(1024) void moe_group_place_kernel(const int32_t *to
     __syncthreads();
     int32_t *list = group + n_expert + 1;
     const int lo = b * chunk, hi = lo + chunk < n_pairs ? lo + chunk : n_pairs;
+    if (in_order) {
+        const int i = lo + tid, e = i < hi ? topk[i] : -1;
+        const bool on = e >= 0 && e < n_expert;
+        uint64_t same = __ballot(on);  // the lanes with this lane's expert
+        for (int bit = 1; bit < kMaxExperts; bit <<= 1) {
+            const uint64_t set = __ballot(e & bit);
+            same &= e & bit ? set : ~set;
+        }
+        const int ahead = __popcll(same & ((1ull << lane) - 1));
+        for (int w = 0; w * 64 < hi - lo; w++) {
+            if (wave == w && on) {
+                const int at = s_cnt[e];
+                if (ahead == 0) s_cnt[e] = at + __popcll(same);
+                list[at + ahead] = (i / n_used) * (n_used + 1) + i % n_used;
+            }
+            __syncthreads();
+        }
+        return;
+    }
     for (int i = lo + tid; i < hi; i += 1024) {
         const int e = topk[i];
         if (e >= 0 && e < n_expert) list[atomicAdd(&s_cnt[e], 1)] = (i / n_used) * (n_used + 1) + i % n_used;
@@ -533,7 +556,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(shv_moe_down_args a) {
 // The per-expert lists of a pass: one block for short passes of few experts, kGroupBlocks in two launches from 2048
 // pairs or 128 experts on (ranking the experts by length is E^2 comparisons, a block's share of them a sixteenth)
 // (their counts meet in the library's scratch, which nothing else on the stream is using between the two).
-// x: rows of k floats to stage for the list kernels in the first launch.
+// x: rows of k floats to stage for the list kernels in the first launch; their lists are in order.
 int launch_group(shv_ctx *ctx, const int32_t *topk, int n_tok, int n_used, int n_expert, int32_t *group, const float *x = nullptr, int k = 0) {
     const int n_pairs = n_tok * n_used;
     if (!x && ((n_pairs < 2048 && n_expert < 128) || !ctx->gemm_part || ctx->moe_group_one_block)) {
@@ -545,7 +568,7 @@ int launch_group(shv_ctx *ctx, const int32_t *topk, int n_tok, int n_used, int n
     const int chunk = (n_pairs + kGroupBlocks - 1) / kGroupBlocks;
     const int stage_blocks = x ? static_cast<int>((static_cast<long long>(n_tok) * (k / 4) + 1023) / 1024) : 0;
     SHV_LAUNCH(ctx, moe_group_count_kernel, dim3(kGroupBlocks + stage_blocks), dim3(1024), 0, topk, n_pairs, chunk, n_expert, counts, x, n_tok, k, ctx->gemm_stage);
-    SHV_LAUNCH(ctx, moe_group_place_kernel, dim3(kGroupBlocks), dim3(1024), 0, topk, n_pairs, chunk, n_used, n_expert, counts, group);
+    SHV_LAUNCH(ctx, moe_group_place_kernel, dim3(kGroupBlocks), dim3(1024), 0, topk, n_pairs, chunk, n_used, n_expert, counts, group, x && chunk <= 1024 ? 1 : 0);
     return SHV_OK;
 }
 

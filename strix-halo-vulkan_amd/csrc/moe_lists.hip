@@ -14,6 +14,8 @@
 //                 the activations' size: 0.5e-6 to 0.7e-6 (slot by slot 4.2e-6; without the exponents 240e-6 at xn of 0.02)
 //   up to eight tokens: the high and the low parts of a token are two rows of ONE operand (a product for both parts,
 //                 the halves of a result in neighbouring registers of a lane); nine to sixteen: an operand for each part
+//                 (the parts of a sum are added at its end in the one, along it in the other: the lists come in order of
+//                 their tokens, so that a pair meets the same one from call to call)
 //   min term    = per super-block one v_mfma_f32_16x16x16_bf16 a part of the sub-blocks' sums of x (float32 values, each
 //                 exactly three bfloat16 ones) with the rows' mins (whole numbers), times the row's dmin
 // Gate/up of a 150-row pass 217 -> 131 us (4.4 TB/s), down 115 -> 64.  The chunks' loads alone take 100 us of the 131, the

@@ -156,3 +156,41 @@ def test_values_of_any_size(rig, lengths, packed):
         err = np.linalg.norm(got[at] - want, axis=1) / np.linalg.norm(want, axis=1)
         # three projections in a row of float32 sums, as the tests beside this one state it
         assert err.max() <= 1e-5, (e, at[err.argmax()], float(err.max()))
+
+
+@pytest.mark.parametrize("T", [106, 380])  # eight listed tokens a time and sixteen; 67 and 238 pairs a block that places them: waves of one that race
+def test_the_same_pass_again_is_the_same(T):
+    """Lists of every length, most of them in several passes or past eight: bit for bit, from call to call."""
+    c, E, U = A.Context(), 256, 10
+    import ctypes as C
+
+    def bank(rows, k, seed):
+        src, dst = c.alloc(rows * k * 4), c.alloc(rows * k // 256 * 144)
+        A.check(c.L.shv_fill_normal(c.h, C.byref(A.FillNormalArgs(src.ptr, rows * k, seed, 0.0, 0.02, 0))))
+        A.check(c.L.shv_quantize_q4k(c.h, C.byref(A.QuantizeQ4KArgs(src.ptr, dst.ptr, rows, k))))
+        c.sync()
+        src.free()
+        return dst
+
+    rows, down = bank(E * F, H, 1), bank(E * H, F, 2)  # gate and up the same bank, the shared expert the first of it
+    rng = np.random.default_rng(T)
+    topk = np.argsort(rng.random((T, E)) * (1 + np.arange(E)), axis=1)[:, :U].astype(np.int32)
+    xn, res, wts = (rng.standard_normal((T, H)).astype(np.float32) for _ in range(3))
+    bufs = dx, dt, dr, dw = [c.upload(a) for a in (xn, topk, res, wts[:, :U + 1].copy())]
+    act, out = c.alloc(T * (U + 1) * F * 4), c.alloc(T * H * 4)
+    group, pairs = c.alloc((2 * E + 1 + T * U) * 4), c.alloc(T * (U + 1) * H * 4)
+    ua = A.MoeUpArgs(dx.ptr, dt.ptr, rows.ptr, rows.ptr, rows.ptr, rows.ptr, act.ptr, T, H, U, F, None, None, E, 0, 0, 0, 0, group.ptr, 0, 1)
+    da = A.MoeDownArgs(act.ptr, dt.ptr, dw.ptr, down.ptr, down.ptr, dr.ptr, out.ptr, T, H, U, F, H, H, 0, 0, E, group.ptr, pairs.ptr, 1, 1)
+    first = None
+    for _ in range(8):
+        c.dispatch_multi([A.make_op(A.OP_MOE_UP, ua), A.make_op(A.OP_MOE_DOWN, da)])
+        got, lists = out.read(np.float32, T * H), group.read(np.int32, 2 * E + 1 + T * U)
+        if first is None:
+            first = got, lists
+            for e in range(E):
+                want = np.flatnonzero((topk == e).any(axis=1))
+                assert np.array_equal(lists[E + 1 + lists[e]:E + 1 + lists[e + 1]] // (U + 1), want)
+        assert np.array_equal(got, first[0]) and np.array_equal(lists, first[1])
+    for b in bufs + [act, out, group, pairs, rows, down]:
+        b.free()
+    c.destroy()
