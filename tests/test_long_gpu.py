@@ -104,3 +104,32 @@ def test_a_token_is_the_same_in_any_place_of_a_list(rig, packed):  # noqa: F811
     want = block(rig, topk, True, packed)
     for order in (np.arange(len(topk))[::-1], np.random.default_rng(4).permutation(len(topk))):
         assert np.array_equal(block(rig, topk, True, packed, order), want[order])
+
+
+@pytest.mark.parametrize("lengths,used", [([24] * 24, 3), ([15] * 24, 3)])  # long lists, and the list kernels'
+@pytest.mark.parametrize("packed", [1, 0])
+def test_act_on_a_floats_grid(rig, lengths, used, packed):  # noqa: F811
+    """shv_moe_up writes act wherever a float may lie, the same bytes; operands off the sixteen-byte grid are refused by the down
+    projection that would read them, and the pass after that is nobody's but its own."""
+    c, E, _, banks = rig
+    topk = selection(lengths, used, np.random.default_rng(5))
+    T = len(topk)
+    dx, dt = c.upload(np.random.default_rng(6).standard_normal((T, 2048)).astype(np.float32)), c.upload(topk)
+    words = T * (used + 1) * 512
+    act, group = c.upload(np.zeros(words + 4, np.float32)), c.alloc((2 * E + 1 + T * used) * 4)
+    pairs, out, wts = c.alloc(T * (used + 1) * 2048 * 4), c.alloc(T * 2048 * 4), c.upload(np.ones((T, used + 1), np.float32))
+    g, u, d, gs, us, ds = (b.ptr for b in banks)
+
+    def up(at):
+        c.dispatch_multi([A.make_op(A.OP_MOE_UP, A.MoeUpArgs(dx.ptr, dt.ptr, g, u, gs, us, act.ptr + at, T, 2048, used, 512, None, None, E, 0, 0, 0, 0, group.ptr, 0, packed))])
+        return act.read(np.uint32, words, at)
+
+    want = up(0)
+    for at in (4, 8, 12):
+        assert np.array_equal(up(at), want)
+    if packed:
+        with pytest.raises(A.ShvError, match="left act as matrix-core operands"):
+            c.dispatch_multi([A.make_op(A.OP_MOE_DOWN, A.MoeDownArgs(act.ptr + 12, dt.ptr, wts.ptr, d, ds, None, out.ptr, T, 2048, used, 512, 2048, 2048, 0, 0, E, group.ptr, pairs.ptr, 1, 1))])
+    assert np.array_equal(up(0), want)
+    for b in (dx, dt, act, group, pairs, out, wts):
+        b.free()
