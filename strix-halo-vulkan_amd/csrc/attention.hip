@@ -21,6 +21,9 @@
 // A second, small kernel merges the slices: one wave a (row, head, 64 dims), every slice's value
 // requested at once.  (Merging in the last block to arrive instead costs more than the launch: that
 // block walks all the records alone, a few dependent round trips to memory.)
+#include <atomic>
+#include <type_traits>
+
 #include "shv_device.hpp"
 #include "shv_internal.hpp"
 
@@ -34,7 +37,26 @@ constexpr int kRep = 8;        // query heads per KV head
 constexpr int kTile = 32;         // cells a wave takes at a time
 constexpr int kSliceCells = 128;  // cells a slice gets while there are slices to spare: one tile a wave
 constexpr int kPfSliceCells = 192;  // and a slice of a prompt pass's blocks, each of which forms its 128 query rows anew
+constexpr int kPfOneSlice = 96;  // a pass that short takes one such slice (15 rows behind 110 cells 25.6 us with one, 22.6 with two)
+constexpr int kPfFewSlices = 24;  // where there are compute units for this many slices, a prompt pass takes them at kSliceCells cells (launch_rows)
 constexpr int kMaxSplits = 512;
+// Slices of the row pairs of a prompt pass whose last row sees pass_cells; a pair with one has its rows put straight out.
+// Slices of kSliceCells: one for every pair of a short pass, two and more for every pair of another, since one pair with two costs the
+// pass the merge, one pair with one its length.
+struct PrefillSlices {
+    int cells, least, most;
+    __device__ __forceinline__ PrefillSlices(int pass_cells, int slice_cells, int n_splits) : cells(slice_cells), least(1), most(n_splits) {
+        if (slice_cells == kSliceCells) {
+            if (pass_cells <= kPfOneSlice) most = 1;
+            else least = 2;
+        }
+    }
+    __device__ __forceinline__ int of(int n_cells) const {
+        const int n = (n_cells + cells - 1) / cells;
+        return min(max(n, least), most);
+    }
+};
+
 constexpr int kRec = kRep * (kD + 2);  // floats of one (slice, row) record: per head d values, max, sum
 
 // RMS norm over the 256 dims of one head by one wave (4 dims per lane: lane l holds dims 4l..4l+3),
@@ -577,19 +599,18 @@ __global__ __launch_bounds__(64 * NW) void attn_merge_kernel(shv_attn_decode_arg
 
 // The same for the rows of a prompt pass, whose pairs have few slices: a block a row and head, a thread a dim.  A pair with one
 // slice has its rows already (attn_prefill_kernel).  grid: (n_head, 2, row pairs).
-template <int MB>
 __global__ __launch_bounds__(kD) void attn_merge_rows_kernel(shv_attn_decode_args a, int n_groups, int slice_cells) {
     const int head = blockIdx.x, d = threadIdx.x, j = blockIdx.y;
     const int seq = blockIdx.z / n_groups, row0 = 2 * (blockIdx.z % n_groups);
     const int kvh = head / kRep, hh = head % kRep;
     const int valid = a.seq_len - row0 < 2 ? a.seq_len - row0 : 2;
-    const int n_cells = (a.pos ? a.pos[seq] : 0) + row0 + valid;
-    int n_active = (n_cells + slice_cells - 1) / slice_cells;
-    if (n_active > a.n_splits) n_active = a.n_splits;
+    const int pos = a.pos ? a.pos[seq] : 0;
+    const int n_active = PrefillSlices(pos + a.seq_len, slice_cells, a.n_splits).of(pos + row0 + valid);
     if (j >= valid || n_active == 1) return;
     const float *pin = a.partial + (static_cast<size_t>(blockIdx.z) * a.n_head_kv + kvh) * a.n_splits * 2 * kRec + j * kRec + hh * (kD + 2);
     float num = 0.f, den = 0.f, M = -INFINITY;
-    for (int s0 = 0; s0 < n_active; s0 += MB) {
+    auto fold = [&](int s0, auto batch) {
+        constexpr int MB = decltype(batch)::value;
         float v[MB];
         float2 ml[MB];
 #pragma unroll
@@ -598,6 +619,10 @@ __global__ __launch_bounds__(kD) void attn_merge_rows_kernel(shv_attn_decode_arg
             v[u] = rec[d];
             ml[u] = *reinterpret_cast<const float2 *>(rec + kD);
         }
+        // Asked for together: what only some records need the compiler would ask for behind each one's test, a trip to memory a record
+        // (300 rows behind 300 cells 47.6 us a layer, 40.4 so)
+#pragma unroll
+        for (int u = 0; u < MB; u++) asm volatile("" : "+v"(v[u]));
 #pragma unroll
         for (int u = 0; u < MB; u++) {
             if (s0 + u >= n_active || ml[u].x == -INFINITY) continue;
@@ -607,7 +632,11 @@ __global__ __launch_bounds__(kD) void attn_merge_rows_kernel(shv_attn_decode_arg
             num = fmaf(num, shrink, w * v[u]);
             M = Mn;
         }
-    }
+    };
+    // sixteen records at a time, or four where there are no more (what is not there is read as the batch's first again)
+    if (n_active <= 4) fold(0, std::integral_constant<int, 4>());
+    else
+        for (int s0 = 0; s0 < n_active; s0 += 16) fold(s0, std::integral_constant<int, 16>());
     a.out[static_cast<size_t>(seq * a.seq_len + row0 + j) * a.n_head * kD + static_cast<size_t>(head) * kD + d] = num / den;
 }
 
@@ -709,6 +738,7 @@ __global__ __launch_bounds__(kPfThreads) void attn_prefill_kernel(shv_attn_decod
     const int pos_first = a.pos ? a.pos[seq] : 0;
     // pair gg of the sequence: its rows, what it sees, its slice of that
     struct Slice { int c0, c1, p_first, valid; bool mine, empty, alone; };
+    const PrefillSlices slices(pos_first + a.seq_len, slice_cells, a.n_splits);
     auto slice_of = [&](int gg) {
         Slice s;
         const bool live = gg < n_groups;
@@ -717,8 +747,7 @@ __global__ __launch_bounds__(kPfThreads) void attn_prefill_kernel(shv_attn_decod
         s.valid = a.seq_len - row0 < 2 ? a.seq_len - row0 : 2;
         s.p_first = pos_first + row0;
         const int n_cells = s.p_first + s.valid;
-        int n_active = (n_cells + slice_cells - 1) / slice_cells;
-        if (n_active > a.n_splits) n_active = a.n_splits;
+        const int n_active = slices.of(n_cells);
         int cps = (n_cells + n_active - 1) / n_active;
         cps = (cps + kTile - 1) & ~(kTile - 1);
         s.c0 = split * cps;
@@ -1000,10 +1029,15 @@ int launch_rows(shv_ctx *ctx, const shv_attn_decode_args &a, int row0, int n_gro
     // (norms and rotation of its 16 rows) whatever its slice holds: such a pass takes as many
     // slices as make two blocks a compute unit, no more (64 rows at 32 768 cells: 359 to 214 us).
     // A block of attn_prefill_kernel has eight pairs, and a compute unit holds one (the ring of tiles): there
-    // as many slices as still find a compute unit each, of kPfSliceCells and more.  Counted by pairs instead, us:
-    // 121 rows behind 32 768 cells 358 (now 177), 512 behind 32 000 1600 (518), 300 behind 4000 148 (88), 37 behind
-    // 3000 39 (41).  Two slices where a compute unit is there for more than half of the blocks: 1531 rows from an
-    // empty cache 143 for 112, most of it writing and merging the slices' sums.
+    // as many slices as still find a compute unit each.  Counted by pairs instead, us: 121 rows behind 32 768 cells 358 (now 177),
+    // 512 behind 32 000 1600 (518), 300 behind 4000 148 (88).  Two slices where a compute unit is there for more than half of the
+    // blocks: 1531 rows from an empty cache 143 for 112, most of it writing and merging the slices' sums.
+    // Where that is 24 slices and more (up to 80 rows of one sequence) they have kSliceCells cells instead of kPfSliceCells: there are compute
+    // units for them.  us counted by pairs / of kPfSliceCells with a merge that read its records one after the other / now:
+    //   cells behind       150                300                1500               3000               12 000
+    //   15 rows    28.7 / 28.8 / 24.3  31.0 / 29.0 / 26.0  34.3 / 34.6 / 28.7  37.1 / 37.2 / 32.3  54.2 / 60.4 / 43.1
+    //   37         27.8 / 29.3 / 24.5  30.2 / 31.1 / 26.5  35.4 / 37.2 / 32.6  42.0 / 40.9 / 37.4  82.7 / 62.7 / 51.2
+    //   80         32.2 / 33.2 / 27.2  33.7 / 33.2 / 28.2  50.3 / 41.0 / 37.1  56.5 / 44.9 / 43.5   136 / 72.9 / 69.1
     shv_attn_decode_args b = a;
     const int lanes = a.n_seq * n_groups * a.n_head_kv;
     const int want = (2 * ctx->prop.multiProcessorCount + lanes - 1) / lanes;
@@ -1014,7 +1048,7 @@ int launch_rows(shv_ctx *ctx, const shv_attn_decode_args &a, int row0, int n_gro
     // one row pair: slices of one tile while there are slices to spare, so that as many compute
     // units as possible pull the cache (a unit issues a wave's 16-byte loads at about 25 B a clock;
     // 36 units over 2 300 cells took 2.2 us to ask for them, 144 take a quarter of that)
-    const int slice_cells = a.n_seq * n_groups == 1 ? kTile : shared ? kPfSliceCells : kSliceCells;
+    const int slice_cells = a.n_seq * n_groups == 1 ? kTile : shared && b.n_splits < kPfFewSlices ? kPfSliceCells : kSliceCells;
     if (shared) {
         static std::atomic<bool> raised{false};
         if (!raised.load(std::memory_order_acquire)) {
@@ -1025,9 +1059,7 @@ int launch_rows(shv_ctx *ctx, const shv_attn_decode_args &a, int row0, int n_gro
         const dim3 grid(a.n_seq * ((n_groups + kPfWaves - 1) / kPfWaves), a.n_head_kv, b.n_splits);
         if (a.mask) SHV_LAUNCH(ctx, attn_prefill_kernel<true>, grid, dim3(kPfThreads), sizeof(PrefillSmem), b, n_groups, slice_cells);
         else SHV_LAUNCH(ctx, attn_prefill_kernel<false>, grid, dim3(kPfThreads), sizeof(PrefillSmem), b, n_groups, slice_cells);
-        // the slices' sums are read sixteen at a time where there may be that many (or four: what is not there is read as the first again)
-        if (b.n_splits > 4) SHV_LAUNCH(ctx, attn_merge_rows_kernel<16>, dim3(a.n_head, 2, a.n_seq * n_groups), dim3(kD), 0, b, n_groups, slice_cells);
-        else if (b.n_splits > 1) SHV_LAUNCH(ctx, attn_merge_rows_kernel<4>, dim3(a.n_head, 2, a.n_seq * n_groups), dim3(kD), 0, b, n_groups, slice_cells);
+        if (b.n_splits > 1) SHV_LAUNCH(ctx, attn_merge_rows_kernel, dim3(a.n_head, 2, a.n_seq * n_groups), dim3(kD), 0, b, n_groups, slice_cells);
         return SHV_OK;
     } else {
         dim3 grid(a.n_seq * n_groups, a.n_head_kv, b.n_splits);

@@ -250,7 +250,10 @@ def test_attn_refuses_unsupported_shapes(ctx):
 
 
 @pytest.mark.parametrize("n_seq,rows,past,n_splits", [(1, 15, 0, 1), (1, 16, 17, 1), (2, 17, 47, 1), (1, 34, 1, 64), (3, 31, 480, 64),
-                                                       (1, 257, 0, 8), (1, 130, 900, 64), (1, 600, 1000, 64)])
+                                                       (1, 257, 0, 8), (1, 130, 900, 64), (1, 600, 1000, 64),
+                                                       # few blocks, 128 cells a slice: the last pass with one slice a pair and the first with two, whose
+                                                       # first pair has a cell alone in the second; 16 records a merge and more; the line at 24 slices
+                                                       (1, 16, 80, 64), (1, 16, 81, 64), (1, 72, 33, 24), (3, 15, 250, 24), (1, 16, 1936, 64), (1, 16, 2300, 64), (1, 80, 1100, 24), (1, 80, 1100, 23)])
 def test_a_prompt_pass_against_its_rows_alone(ctx, n_seq, rows, past, n_splits):
     """A pass of fifteen rows and more, whose blocks share the cache's tiles (one tile, a first and a last that a row sees in part, tiles
     seen whole; one slice a row pair and several; a last block and a last pair not full), against the same rows one at a time over the
