@@ -126,8 +126,21 @@ int padded_rows(int n_tok) { return (n_tok + kTok - 1) / kTok * kTok; }
 template <int K>
 int launch_k(shv_ctx *ctx, const shv_gemv_q4k_args &a) {
     static_assert(kLds <= 48 * 1024, "no more than a launch may have without asking");
-    const int padded = padded_rows(a.n_tok);
+    const int padded = padded_rows(a.n_tok), cus = ctx->prop.multiProcessorCount;
+    const long long groups = padded / kTok;
     SHV_LAUNCH(ctx, gemm_long_stage_kernel<K>, dim3(padded / 4), dim3(256), 0, a, ctx->gemm_stage, padded);
+    // Short rows: blocks of 128.  Of 256 columns up to two of them a compute unit, and past that as longer rows: what such a block does is write
+    // its sums, and three and four at a time on a unit do it faster on some cards and slower on others (2048 x 256 of 3000 rows, blocks of 128
+    // 16.8 to 27.4 us, of 256 18.6 to 21.4).  us, before (slabs, 16 x 16 tiles) / chosen as longer rows are / so:
+    //                     512 rows             1024                 1531                 2048                 4096
+    //    2048 x 256   10.4 / 10.0 / 10.0   11.1 / 11.0 / 11.0   13.7 / 15.2 / 13.1   15.4 / 16.5 / 14.6   23.4 / 23.8 / 23.8
+    //    2048 x 512   12.8 / 13.1 / 13.1   13.9 / 15.0 / 14.8   19.0 / 21.6 / 19.8   21.7 / 23.0 / 21.1   33.0 / 34.5 / 33.2
+    //    2048 x 1024  18.5 / 19.1 / 19.1   21.2 / 22.5 / 22.2   29.6 / 32.1 / 30.1   32.7 / 35.8 / 34.0   51.7 / 53.9 / 52.6
+    //    4096 x 512   13.6 / 14.1 / 14.1   20.1 / 22.2 / 20.1   28.8 / 27.0 / 27.0   31.1 / 32.2 / 30.9   54.7 / 55.2 / 51.1
+    //   12352 x 512   26.6 / 27.9 / 26.7   48.2 / 48.4 / 41.8   63.6 / 61.0 / 57.7   82.0 / 79.7 / 71.2    174 / 148  / 134
+    //   12352 x 1024  41.5 / 42.3 / 42.1   84.8 / 77.4 / 69.9    111 / 97   / 97      145 / 135  / 124     289 / 241  / 233
+    // (2048 x 1024 of 1024 and 2048 rows, 4096 x 1024 of 2048 and 300 x 512 are left 4 to 7 % behind the slabs.)
+    if (K == 512 || K == 1024 || (K == 256 && (a.n + 127) / 128 * groups <= 2ll * cus)) return launch<K, 1>(ctx, a, padded);
     // Blocks of 256 weight rows, two a compute unit, or of 128, four a unit, which read the activations twice as often but leave less of the
     // chip idle where there are few.  Their rounds of the chip, in rounds of full units: a unit with one block of 256 takes 0.58 of what two
     // take; 1, 2, 3 blocks of 128 take 0.37, 0.6, 0.82 of what four take, and four a tenth more than two of 256.  us, of 256 / of 128:
@@ -135,13 +148,11 @@ int launch_k(shv_ctx *ctx, const shv_gemv_q4k_args &a) {
     //   12352x2048  75 / 80   135 / 130  172 / 184  236 / 236  434 / 453
     //    9216x2048  70 / 65   109 / 99   139 / 137  176 / 175  316 / 338
     //    2048x4096  72 / 52    74 / 56    78 / 82    89 / 92   159 / 168
-    const int cus = ctx->prop.multiProcessorCount;
     const auto rounds = [cus](long long blocks, int a_unit, const double *part) {
         const long long full = blocks / (static_cast<long long>(cus) * a_unit), rest = blocks - full * cus * a_unit;
         return static_cast<double>(full) + part[(rest + cus - 1) / cus];
     };
     static const double two[] = {0., 0.58, 1.}, four[] = {0., 0.37, 0.6, 0.82, 1.};
-    const long long groups = padded / kTok;
     const double wide = rounds((a.n + 255) / 256 * groups, 2, two), narrow = 1.1 * rounds((a.n + 127) / 128 * groups, 4, four);
     return narrow < wide ? launch<K, 1>(ctx, a, padded) : launch<K, 2>(ctx, a, padded);
 }

@@ -181,8 +181,9 @@ __device__ __forceinline__ void landed_barrier() {
 // against activation row 8 (i / 4) + 4 h + i % 4 of tile tt.  (A chunk that nobody reads may be on its way to LDS still.)
 // rows[i] (chunk_piece in it) is where this lane's line of its wave's i-th eight rows begins in `staged`, sum where its sixteen bytes of the
 // sums of tile `wave` (waves 0 .. NTT - 1) begin in `sums`, in units of sum_unit.  A chunk's weights are asked for four chunks ahead, as soon
-// as their registers are free; where a row is short (SBS 1, 2), a super-block's all together, so that a line is fetched once (2048 x 512
-// expert rows 5 % faster; rows of eight super-blocks, whose waves wait for more at a time then, as much slower).
+// as their registers are free; where a row is short (SBS 1, 2; 4 of one tile), a super-block's all together, so that a line is fetched once
+// (2048 x 512 expert rows 5 % faster, 12352 x 1024 of 4096 rows, one tile, 247 to 235 us; rows of eight super-blocks, whose waves wait for
+// more at a time then, 5 % slower).
 // Every wave of a block of four calls it; smem: stream_lds(NTT).
 //
 // What bounds it: the card's power, then vector issue.  12352 x 2048 of 4096 rows: the clock falls to 1.9 GHz, the matrix cores are busy 53 %
@@ -193,7 +194,7 @@ template <int SBS, int R, int NTT, typename Done>
 __device__ __forceinline__ void stream_products(const char *const (&first)[R], int units, int unit_bytes, char *smem, int wave, buffer_t staged, const uint32_t (&rows)[NTT],
                                                 buffer_t sums, uint32_t sum, float sum_unit, Done &&done) {
     static_assert(NTT <= 4, "a tile's sums a wave");
-    constexpr bool whole = SBS <= 2;
+    constexpr bool whole = SBS <= 2 || (R == 1 && SBS <= 4);
     const int lane = threadIdx.x & 63, h = lane >> 5;
     const ChunkReader at(lane);
     char *sums_s = smem + 2 * chunk_lds(NTT);

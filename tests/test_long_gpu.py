@@ -19,8 +19,8 @@ def ctx():
 
 
 # every width; the fewest rows of each, whole and ragged groups of 64; weight rows inside a tile, a block of 128, of 256; blocks of either
-# kind (256 weight rows from 2048 x 4096 of 1800 rows on), in strips of eight groups and in a last one that is narrower
-@pytest.mark.parametrize("n,k,rows", [(17, 256, 193), (300, 512, 256), (513, 1024, 449), (129, 2048, 513), (2055, 2048, 1090), (70, 4096, 577), (2048, 4096, 1801)])
+# kind (256 weight rows from 2048 x 4096 of 1800 rows on, of 256 columns where 128 make more than two blocks a compute unit), in strips of eight groups and in a last one that is narrower
+@pytest.mark.parametrize("n,k,rows", [(17, 256, 193), (2055, 256, 1920), (2055, 256, 2950), (300, 512, 256), (513, 1024, 449), (129, 2048, 513), (2055, 2048, 1090), (70, 4096, 577), (2048, 4096, 1801)])
 def test_rows_of_a_long_pass(ctx, n, k, rows):
     """The norm folded in and the residual in place, then no prologue and a ring that wraps.  2^-17: 32 bits' sums of up to 4096 products
     in a fixed order, each product as exact as one float32."""
