@@ -584,6 +584,14 @@ __device__ __forceinline__ half4_t transposed4(const char *at) {
 // LDS written is there for the block; loads from memory stay in flight
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// A wave's loads complete in order, so that k^ of the next chunk, asked for first, is in LDS when as many loads are out as follow it.  What
+// follows in every turn of the loop, the last one too, each a vector load at an address of the lane's own, of a wave of the chain: G, beta,
+// v, the tiles (G_C, at one address for all lanes, may be a scalar load and does not count); of one beside it: q^, G, the tiles.
+// The loop is one copy of its turn (unroll 1), whose loads stay between the clobbers of memory they are written between.
+constexpr int kGateLoads = 1, kTileLoads = 4;
+constexpr int kChainLoads = 2 * kGateLoads + 4 + kTileLoads, kBesideLoads = 8 + kGateLoads + kTileLoads;
+constexpr int kLoadsBehindK = kChainLoads < kBesideLoads ? kChainLoads : kBesideLoads;
+
 // The walk of a wave of the chain, or of one beside it; both meet the same barriers.
 template <bool CHAIN>
 __device__ __forceinline__ void dn_walk(const shv_dn_step_args &a, const float *prep, int pw, const char *recs, int wave, WalkLds &L) {
@@ -645,7 +653,7 @@ __device__ __forceinline__ void dn_walk(const shv_dn_step_args &a, const float *
     };
     auto load_tiles = [&](const u32x4_t (*from)[64]) {
 #pragma unroll
-        for (int cb = 0; cb < 4; cb++) tiles[cb] = from[tri_tile(w, cb < w ? cb : w)][lane];  // four loads in every wave, so that what follows them can be counted
+        for (int cb = 0; cb < kTileLoads; cb++) tiles[cb] = from[tri_tile(w, cb < w ? cb : w)][lane];  // four loads in every wave, so that what follows them can be counted
     };
     auto load_v = [&](int c) {
 #pragma unroll
@@ -703,6 +711,7 @@ __device__ __forceinline__ void dn_walk(const shv_dn_step_args &a, const float *
         k_col[p] = t * kRowBytes + ((2 * (2 * wave + ((n & 3) >> 1)) + p) ^ walk_swizzle(t)) * 16 + (n & 1) * 8;
     }
 
+#pragma unroll 1
     for (int c = 0; c < n_chunks; c++) {
         const char *k = L.k[c & 1];
         const int next = c + 1 < n_chunks ? c + 1 : c;  // loaded after the last chunk too, so that the loads in flight can be counted
@@ -794,9 +803,10 @@ __device__ __forceinline__ void dn_walk(const shv_dn_step_args &a, const float *
             for (int r = 0; r < 4; r++) S[r] = fmaf(gC, S[r], fmaf(low[r], kLoInv, main[r]));
         }
         publish_state();
-        // k^ of the next chunk has landed: at least ten loads follow it in every wave that asked for it
-        asm volatile("s_waitcnt vmcnt(10) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        // k^ of the next chunk has landed
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kLoadsBehindK) : "memory");
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load to LDS is out when the wave ends
     if constexpr (!CHAIN) put_rows(n_chunks - 1, w2);
     *reinterpret_cast<float4_t *>(state + static_cast<size_t>(n) * kD + i0) = S;
 }
