@@ -91,8 +91,7 @@ class QsaDevice:
         self.stride = max_cells // 32
         self.d_mask = c.alloc(max_rows * self.stride * 4)
         self.d_qkv, self.d_ctx, self.d_out = c.alloc(max_rows * case.width * 4), c.alloc(max_rows * NH * D * 4), c.alloc(max_rows * H * 4)
-        # slice records: short passes take up to n_splits slices a row pair, long ones two or four (the launcher's own rule)
-        self.d_part = c.alloc((_part_floats(1, n_splits, min(max_rows, 64)) + _part_floats(1, 4, max_rows)) * 4)
+        self.d_part = c.alloc(_part_floats(1, n_splits, max_rows) * 4)  # as the declaration of the call states
         self.d_pos = c.alloc(4)
 
     def run(self, x, past, masked=True):
