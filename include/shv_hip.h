@@ -397,7 +397,7 @@ typedef struct {
  * row are prepared into work first, then each chunk is a few 64-row products and one triangular
  * solve against the state, which is read and written once per pass); results agree with the
  * row-by-row rule to float32 rounding.  With room behind those rows (their count rounded up to a
- * multiple of 4 floats) for 10 880 more floats per (sequence, chunk of 64 rows, value head), what a
+ * multiple of 4 floats) for 5248 more floats per (sequence, chunk of 64 rows, value head), what a
  * chunk needs that does not depend on the state is formed for every chunk of the pass at once, by a
  * launch of its own, instead of inside the walk over the chunks by each of a head's eight blocks;
  * the walk is then a kernel of its own, half as long.  The reference scans row by row at every pass length

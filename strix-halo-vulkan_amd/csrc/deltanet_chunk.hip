@@ -154,9 +154,7 @@ struct WalkRec {
     u32x4_t inv[kTriTiles][64], m[kTriTiles][64];
     float G[kC], beta[kC];
 };
-// from one record to the next, as the declaration of the workspace says
-constexpr size_t kRecStride = 43520;
-static_assert(sizeof(WalkRec) <= kRecStride && kRecStride % 16 == 0, "moved 16 bytes at a time");
+static_assert(sizeof(WalkRec) == 5248 * 4 && sizeof(WalkRec) % 16 == 0, "the floats that the declaration of the workspace states; moved 16 bytes at a time");
 
 struct ChunkLds {
     _Float16 kh[kC][kKS], kl[kC][kKS], qh[kC][kKS], ql[kC][kKS];  // k^ and q^ of the chunk, hi and scaled lo
@@ -402,7 +400,7 @@ __global__ __launch_bounds__(kThreads, 1) void dn_chunk_kernel(shv_dn_step_args 
                 }
             }
             __syncthreads();
-            WalkRec &rec = *reinterpret_cast<WalkRec *>(recs + (static_cast<size_t>(seq * n_chunks + c) * a.n_head_v + h) * kRecStride);
+            WalkRec &rec = reinterpret_cast<WalkRec *>(recs)[static_cast<size_t>(seq * n_chunks + c) * a.n_head_v + h];
 #pragma unroll
             for (int i = 0; i < 2 * kTriTiles / 4; i++) {
                 const int tile = 4 * i + w, tri = tile < kTriTiles ? tile : tile - kTriTiles;
@@ -637,7 +635,7 @@ __device__ __forceinline__ void dn_walk(const shv_dn_step_args &a, const float *
                                  to + (8 * wave + 2 * u) * kRowBytes);
         }
     };
-    auto rec_of = [&](int c) { return reinterpret_cast<const WalkRec *>(recs + (static_cast<size_t>(seq * n_chunks + c) * a.n_head_v + h) * kRecStride); };
+    auto rec_of = [&](int c) { return reinterpret_cast<const WalkRec *>(recs) + static_cast<size_t>(seq * n_chunks + c) * a.n_head_v + h; };
     auto row_of = [&](int t) { return rows + static_cast<size_t>(t < a.seq_len ? t : a.seq_len - 1) * pw; };
 
     // In registers from one chunk to the next: the gates of the wave's rows, G_C, and
@@ -846,7 +844,7 @@ int shv_launch_dn_chunk(shv_ctx *ctx, const shv_dn_step_args &a) {
     // part is then formed for all of them at once, and the walk over the chunks only reads it.
     const long long prep_floats = (static_cast<long long>(a.n_seq) * a.seq_len * pw + 3) & ~3ll;
     const int n_chunks = (a.seq_len + kC - 1) / kC;
-    const long long rec_floats = static_cast<long long>(a.n_seq) * n_chunks * a.n_head_v * static_cast<long long>(kRecStride / 4);
+    const long long rec_floats = static_cast<long long>(a.n_seq) * n_chunks * a.n_head_v * static_cast<long long>(sizeof(WalkRec) / 4);
     const dim3 grid(a.n_head_v * (kD / kJ), a.n_seq);
     if (n_chunks >= 2 && n_chunks <= 65535 && a.n_seq <= 65535 && prep_floats + rec_floats <= a.work_floats && !ctx->dn_chunk_no_recs) {
         char *recs = reinterpret_cast<char *>(a.work + prep_floats);

@@ -204,7 +204,7 @@ def test_chunked_rows_equal_the_row_by_row_rule(ctx, T, pos0, n_seq):
     d_x, d_pos = c.upload(xn.reshape(n_seq * T, case.H)), c.upload(pos)
     results = []
     prep_floats = (n_seq * T * (case.cw + 2 * case.hv) + 3) & ~3
-    rec_floats = n_seq * ((T + 63) // 64) * case.hv * 10880
+    rec_floats = n_seq * ((T + 63) // 64) * case.hv * 5248
     for chunked in ("records", "in the walk", None):
         d_ring, d_state = c.upload(ring), c.upload(s0)
         d_attn, d_res = c.alloc(n_seq * T * case.vw * 4), c.alloc(n_seq * T * case.H * 4)
@@ -256,7 +256,7 @@ def test_the_walk_over_records_at_its_edges(ctx, T, n_seq, hk, hv):
     s0 = f32((n_seq + 1) * planes * hv * d * d) * 0.1
     d_pos, d_slot = c.upload(5 + np.arange(n_seq, dtype=np.int32)), c.upload(np.arange(n_seq, 0, -1).astype(np.int32))
     d_plane = c.upload((np.arange(n_seq + 1) % planes).astype(np.int32))
-    floats = ((n_seq * T * (cw + 2 * hv) + 3) & ~3) + n_seq * ((T + 63) // 64) * hv * 10880
+    floats = ((n_seq * T * (cw + 2 * hv) + 3) & ~3) + n_seq * ((T + 63) // 64) * hv * 5248
     got = []
     for work in (c.alloc(floats * 4), None):
         d_state, d_out = c.upload(s0), c.alloc(n_seq * T * vw * 4)
