@@ -158,7 +158,8 @@ enum {
  * plain: the DeltaNet output projection takes its gate z from the projection ring.
  * Range: up to four rows any float32; from five on the rows enter the matrix cores, after the
  * prologue, as binary16 pairs: values up to 65504.  (shv_gemv_mrows' kernel, two to eight rows, and
- * the kernels of passes past 512 rows scale them: any float32.) */
+ * the kernels of long passes, past 512 rows of 2048 or 4096 columns and past 192 of 256, 512 or 1024,
+ * scale them: any float32.) */
 typedef struct {
     const void *w;
     const float *x;

@@ -5,10 +5,11 @@ import pytest
 
 import oracle_lib as O
 import shv
-from test_moe_lists_gpu import block, rig, selection  # noqa: F401 (rig is a fixture)
+from test_moe_lists_gpu import block, expert_rows, rig, selection, up64  # noqa: F401 (rig is a fixture)
 
 pytestmark = pytest.mark.gpu
 A = shv.api
+H, F = 2048, 512
 
 
 @pytest.fixture(scope="module")
@@ -51,6 +52,51 @@ def test_rows_of_a_long_pass(ctx, n, k, rows):
     assert (np.abs(got[at] - want) <= 2.0 ** -17 * size).all() and (got[at][rows // 3] == 0).all()
     assert (np.delete(got, at, axis=0) == -7.0).all()
     for b in bufs + (ring, dpos):
+        b.free()
+
+
+@pytest.mark.parametrize("gate", ["ring", "rows", "heads"])
+@pytest.mark.parametrize("rows", [577, 1801])
+def test_gated_rows_of_a_long_pass(ctx, rows, gate):
+    """The output projections' prologues: the norm of each head of 128 and the gate of a ring that wraps, or the gate of rows of its own;
+    the gate beside each head of 256's queries.  2^-16: a prologue of float32 (a head's sum of squares, a square root, the gate's
+    exponential: 2^-18 and less of a value each) before 2^-17 as above."""
+    rng = np.random.default_rng(rows)
+    n, k = 2048, 4096
+    wq = O.quantize_q4k((rng.standard_normal((n, k)) * 0.02).astype(np.float32))
+    w64 = O.dequant_q4k(wq, k).astype(np.float64)
+    x, res = rng.standard_normal((rows, k)).astype(np.float32), rng.standard_normal((rows, n)).astype(np.float32)
+    x[rows // 2] *= 1e6
+    x[rows // 3] *= 1e-4
+    z = rng.standard_normal((rows, k)).astype(np.float32) * 3
+    gamma = (1 + 0.1 * rng.standard_normal(128)).astype(np.float32)
+    bufs = [ctx.upload(wq), ctx.upload(x), ctx.upload(res), ctx.upload(gamma)]
+    dw, dx, dy, dg = bufs
+    x64 = x.astype(np.float64)
+    if gate == "heads":
+        held = np.concatenate([rng.standard_normal((rows, k // 256, 256)).astype(np.float32), z.reshape(rows, k // 256, 256)], axis=2)
+        bufs.append(ctx.upload(held))
+        ctx.gemv_q4k(dw, dx, dy, n, k, n_tok=rows, prologue=A.PRO_MUL_SIGMOID, z=bufs[-1], head_dim=256, z_stride=2 * k, residual=dy)
+    else:
+        heads = x64.reshape(rows, -1, 128)
+        x64 = (heads / np.sqrt((heads * heads).mean(axis=2, keepdims=True) + 1e-6) * gamma).reshape(rows, k)
+        if gate == "ring":
+            slots, pos = rows + 5, 2 * rows
+            ring = np.full((2, slots, k + 32), np.nan, np.float32)
+            ring[1, (pos + np.arange(rows)) % slots, 16:16 + k] = z
+            bufs += [ctx.upload(ring), ctx.upload(np.array([pos], np.int32)), ctx.upload(np.array([1], np.int32))]
+            ctx.gemv_q4k(dw, dx, dy, n, k, n_tok=rows, prologue=A.PRO_GATED_NORM, gamma=dg, z=bufs[4].at(64), head_dim=128, residual=dy,
+                         pos=bufs[5], slot=bufs[6], seq_len=rows, ring_slots=slots, ring_stride=k + 32, z_ring=1)
+        else:
+            bufs.append(ctx.upload(z))
+            ctx.gemv_q4k(dw, dx, dy, n, k, n_tok=rows, prologue=A.PRO_GATED_NORM, gamma=dg, z=bufs[4], head_dim=128, residual=dy)
+    x64 /= 1 + np.exp(-z.astype(np.float64))
+    want, got = x64 @ w64.T + res, dy.read(np.float32, rows * n).reshape(rows, n)
+    size = np.abs(x64) @ (np.abs(w64) + 2 * np.abs(w64).max(axis=1, keepdims=True)).T + np.abs(res)
+    assert (np.abs(got - want) <= 2.0 ** -16 * size).all()
+    err = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+    assert np.sqrt(np.mean(err ** 2)) <= 1e-5, float(err.max())
+    for b in bufs:
         b.free()
 
 
@@ -133,3 +179,33 @@ def test_act_on_a_floats_grid(rig, lengths, used, packed):  # noqa: F811
     assert np.array_equal(up(0), want)
     for b in (dx, dt, act, group, pairs, out, wts):
         b.free()
+
+
+# the kernels of walks of up to one, two and three tiles, lists of all their passes
+@pytest.mark.parametrize("lengths", [[17, 31, 32, 33, 1, 65] + [20] * 18, [33, 63, 64, 65, 1, 95] + [40] * 18, [97, 64, 65, 128, 193, 31] + [70] * 18])
+def test_gate_and_up_of_rows_of_any_size(rig, lengths):  # noqa: F811
+    """Rows whose values or whose sums of 32 are past binary16 or far below its normal numbers, against float64, each as exact as any other;
+    an infinity stays in its row.  2^-18: the two projections' sums of 2048 products and their scales, each product as exact as one float32."""
+    c, E, _, banks = rig
+    rng = np.random.default_rng(sum(lengths))
+    topk = selection(lengths, 1, rng)
+    T = len(topk)
+    xn = (rng.standard_normal((T, H)) * 500 + 3000 * np.where(np.arange(T) % 2, 1, -1)[:, None]) * 10.0 ** rng.uniform(-7, 5, size=(T, 1))
+    xn = xn.astype(np.float32)
+    lost = [int(np.flatnonzero(topk[:, 0] == 1)[4]), int(np.flatnonzero(topk[:, 0] == 3)[-1])]
+    xn[lost[0], 700], xn[lost[1], 31] = np.inf, np.nan
+    bufs = [c.upload(a) for a in (xn, topk)]
+    act, group = c.alloc(T * 2 * F * 4), c.alloc((2 * E + 1 + T) * 4)
+    ua = A.MoeUpArgs(bufs[0].ptr, bufs[1].ptr, banks[0].ptr, banks[1].ptr, banks[3].ptr, banks[4].ptr, act.ptr, T, H, 1, F, None, None, E, 0, 0, 0, 0, group.ptr, 0, 0)
+    c.dispatch_multi([A.make_op(A.OP_MOE_UP, ua)])
+    got = act.read(np.float32, T * 2 * F).reshape(T, 2, F)
+    for b in bufs + [act, group]:
+        b.free()
+    assert not np.isfinite(got[lost]).any()
+    kept = np.delete(np.arange(T), lost)
+    assert np.isfinite(got[kept]).all()
+    for e in range(E + 1):  # the last: the shared expert, whose rows are every token's
+        at = np.intersect1d(kept, np.flatnonzero(topk[:, 0] == e)) if e < E else kept
+        gate, up = (expert_rows(rig, 0, e, F, H), expert_rows(rig, 1, e, F, H)) if e < E else (expert_rows(rig, 3, 0, F, H), expert_rows(rig, 4, 0, F, H))
+        want, tol = up64(xn[at].astype(np.float64), gate, up)
+        assert (np.abs(got[at, int(e == E)] - want) <= 4 * tol).all(), (e, float(np.max(np.abs(got[at, int(e == E)] - want) / np.maximum(tol, 1e-300))))
