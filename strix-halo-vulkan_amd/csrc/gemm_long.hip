@@ -8,9 +8,6 @@
 //    9216 x 2048        73 / 65         111 / 99          147 / 138         192 / 175         363 / 316
 //    2048 x 4096        58 / 52          59 / 56           86 / 78           97 / 89          163 / 159
 // Error against float64 of 4096 x 2048: 0.40e-6 (before 0.45e-6; activations of 0.02 2.1e-6, of mean 3 6.5e-6 against 4.0e-6 now).
-#include <algorithm>
-#include <atomic>
-
 #include "gemm_rows.hpp"
 #include "long_tiles.hpp"
 

@@ -335,7 +335,7 @@ struct RowStream {
 // A sub-block's eight weights per lane are formed once, as the whole numbers n * sc, and multiplied
 // with every token tile; the matrix accumulators run over a super-block and take its d at its end,
 // the min term is subtracted per sub-block: y = sum_sb d * (sum x * n * sc) - sum_sub dmin * m * sum(x).
-template <int NG, int R, int SXS = kTok>
+template <int NG, int R>
 __device__ __forceinline__ void slab_times_tiles(const char *const (&rp)[R], RowStream<R> &st, int G0, int G_last, const char *frags,
                                                  const float *sxs, int lane, int n_tt, float4_t (&acc)[R][kTT], float4_t (&y)[R][kTT]) {
     const int kb = lane >> 4;
@@ -383,18 +383,8 @@ __device__ __forceinline__ void slab_times_tiles(const char *const (&rp)[R], Row
                 const char *f = frags + static_cast<size_t>((sub * 2) * kTT + tt) * kFrag + lane * 16;
                 const half8_t xh = *reinterpret_cast<const half8_t *>(f);
                 const half8_t xl = *reinterpret_cast<const half8_t *>(f + kTT * kFrag);
-                float sxv[4];
-                if constexpr (SXS > 0) {
-                    const float4 sx = *reinterpret_cast<const float4 *>(sxs + sub * SXS + 16 * tt + 4 * kb);
-                    sxv[0] = sx.x, sxv[1] = sx.y, sxv[2] = sx.z, sxv[3] = sx.w;
-                } else {
-                    // the sub-block's sum of x per token, from the operands themselves: a product
-                    // with ones leaves token 4 kb + j's sum in register j of every lane
-                    const half8_t ones = static_cast<half8_t>(static_cast<_Float16>(1.f));
-                    float4_t s4 = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, ones, float4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                    s4 = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, ones, s4, 0, 0, 0);
-                    sxv[0] = s4[0], sxv[1] = s4[1], sxv[2] = s4[2], sxv[3] = s4[3];
-                }
+                const float4 sx = *reinterpret_cast<const float4 *>(sxs + sub * kTok + 16 * tt + 4 * kb);
+                const float sxv[4] = {sx.x, sx.y, sx.z, sx.w};
 #pragma unroll
                 for (int r = 0; r < R; r++) {
                     acc[r][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, b[r], acc[r][tt], 0, 0, 0);
