@@ -585,7 +585,8 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // A wave's loads complete in order, so that k^ of the next chunk, asked for first, is in LDS when as many loads are out as follow it.  What
 // follows in every turn of the loop, the last one too, each a vector load at an address of the lane's own, of a wave of the chain: G, beta,
 // v, the tiles (G_C, at one address for all lanes, may be a scalar load and does not count); of one beside it: q^, G, the tiles.
-// The loop is one copy of its turn (unroll 1), whose loads stay between the clobbers of memory they are written between.
+// The loads stay between the clobbers of memory they are written between, and are all used behind the loop, so that no copy of its last
+// turn can go without them.  (The loop held to one copy instead: 162 us at 4096 rows, 158 so.)
 constexpr int kGateLoads = 1, kTileLoads = 4;
 constexpr int kChainLoads = 2 * kGateLoads + 4 + kTileLoads, kBesideLoads = 8 + kGateLoads + kTileLoads;
 constexpr int kLoadsBehindK = kChainLoads < kBesideLoads ? kChainLoads : kBesideLoads;
@@ -709,7 +710,6 @@ __device__ __forceinline__ void dn_walk(const shv_dn_step_args &a, const float *
         k_col[p] = t * kRowBytes + ((2 * (2 * wave + ((n & 3) >> 1)) + p) ^ walk_swizzle(t)) * 16 + (n & 1) * 8;
     }
 
-#pragma unroll 1
     for (int c = 0; c < n_chunks; c++) {
         const char *k = L.k[c & 1];
         const int next = c + 1 < n_chunks ? c + 1 : c;  // loaded after the last chunk too, so that the loads in flight can be counted
@@ -805,6 +805,13 @@ __device__ __forceinline__ void dn_walk(const shv_dn_step_args &a, const float *
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kLoadsBehindK) : "memory");
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load to LDS is out when the wave ends
+    if constexpr (CHAIN) {
+        asm volatile("" ::"v"(Gt), "v"(bt), "v"(v), "v"(tiles[0]), "v"(tiles[1]), "v"(tiles[2]), "v"(tiles[3]));
+    } else {
+        asm volatile("" ::"v"(Gt));
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) asm volatile("" ::"v"(q[ks][0]), "v"(q[ks][1]));
+    }
     if constexpr (!CHAIN) put_rows(n_chunks - 1, w2);
     *reinterpret_cast<float4_t *>(state + static_cast<size_t>(n) * kD + i0) = S;
 }
