@@ -359,7 +359,10 @@ int launch_stage(shv_ctx *ctx, const shv_gemv_q4k_args &a, int tiles, float *x_o
 // keep the kernel of one 64-row group.  That kernel is the slower there (12352 x 2048 of 64 rows 27.7 us, 15.9 here; of 40 rows 24.1
 // and 13.8, of 17 20.6 and 12.4; 2048 x 4096 of 40 rows 17.9 and 11.0) and the less exact (2.1e-6 against 0.4e-6): the line is one of
 // results that stay what they were, since a prompt's whole chunk of 64 rows is one pass whose routing, where a token's tenth expert and
-// its eleventh are level, every token decoded after it carries on (48 layers: the logits after 96 tokens parted by 1e-4 to 2e-3).
+// its eleventh are level, every token decoded after it carries on (48 layers: the logits after 96 tokens parted by 1e-4 to 2e-3).  It is a
+// line of the results' continuity, of neither speed nor precision: eight layers' logits against the CPU's, median of ten prompts, 56 rows
+// 1.5e-5 there and 1.1e-5 here, 64 rows 1.4e-5 and 1.0e-5 (one of the ten 3.6e-3 there: another expert), where 17 to 48 rows went over
+// from 2.1e-5 to 1.6e-5 at 20 rows, 1.6e-5 to 1.1e-5 at 48.
 // Past 512 gemm_long.hip's blocks read less from L2.
 bool shv_gemm_mid_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a) {
     if (!ctx->gemm_stage || (a.k != 2048 && a.k != 4096) || a.n_tok < 9 || a.n_tok > 512) return false;

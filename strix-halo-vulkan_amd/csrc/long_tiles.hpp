@@ -186,8 +186,8 @@ __device__ __forceinline__ void landed_barrier() {
 // more at a time then, 5 % slower).
 // Every wave of a block of four calls it; smem: stream_lds(NTT).
 //
-// What bounds it: the card's power, then vector issue.  12352 x 2048 of 4096 rows: the clock falls to 1.9 GHz, the matrix cores are busy 53 %
-// of it, vector instructions (4.6 a matrix instruction) 34 %; without forming weights the same time, without LDS reads 10 % less, with the
+// What bounds it: the card's power, then vector issue.  12352 x 2048 of 4096 rows: the clock falls to 1.8 GHz, the matrix cores are busy 55 %
+// of it, vector instructions (five beside each matrix instruction) issue 41 %; without forming weights the same time, without LDS reads 10 % less, with the
 // matrix instructions alone 27 % less.  More chunks on their way (two to four buffers), fragments read a step ahead, a wave's priority and
 // the order of its instructions changed nothing beyond 2 %.
 template <int SBS, int R, int NTT, typename Done>

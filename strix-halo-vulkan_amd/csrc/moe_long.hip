@@ -4,7 +4,7 @@
 // tokens, whose accumulators fill the registers, and a weight is formed once for all of them: with 64 at most an expert of 80 tokens would
 // form its weights twice (4096 rows over 512 experts: 1016 us a layer, 908 so).  Three blocks a compute unit instead of two, with fewer
 // registers: 960.
-// Bounded by vector issue and the matrix cores at 2 GHz (4096 rows: 39 % and 39 % of the time), below 20 tokens an expert by forming weights
+// Bounded by the matrix cores and vector issue at 2.0 to 2.2 GHz (4096 rows: up 41 % and 34 % of the time, down 34 % and 26 %), below 20 tokens an expert by forming weights
 // for tiles half empty.  us, gate/up + down of one layer of 512 experts, top 10, lists and staging included, before (16 x 16 tiles, up to 48
 // tokens a walk) / now:   800 rows 462 / 387   1024 505 / 403   1531 558 / 468   2048 625 / 559   4096 1102 / 908
 // Error of a layer's outputs against float64 0.71e-6 (before 0.78e-6).
@@ -290,6 +290,10 @@ int launch_down(shv_ctx *ctx, const shv_moe_down_args &a) {
 // spilled, of one; 256 and 13 spilled of two, 39 of three).  us a layer with one, two and three, lists drawn evenly:
 //   15.6 tokens an expert 387 / 403 / 416   22.5: 412 / 425 / 434   25.4: 448 / 438 / 454   30: 510 / 468 / 491   40: 698 / 559 / 578
 //   58.6: 840 / 686 / 695   64.5: 921 / 777 / 757   80: 1111 / 961 / 920
+// Of lists drawn unevenly the longest, which one expert's blocks walk pass after pass, takes longer than all the others, whichever kernel it is:
+// us by the logarithms' deviation over the experts, 0 / 1 / 2 / one expert that every token chose (before: 16 x 16 tiles, up to 48 tokens a walk)
+//    800 rows 382 / 418 / 568 / 1009 (before 459 / 444 / 636 / 1255)   1531: 477 / 565 / 1199 / 1357 (563 / 780 / 1984 / 2349)
+//   4096: 910 / 1300 / 3022 / 4343 (1095 / 1647 / 4303 / 6187)
 int walk_tiles(int n_tok, int n_used, int n_expert) {
     const long long pairs = static_cast<long long>(n_tok) * n_used;
     return pairs <= 24ll * n_expert ? 1 : pairs <= 60ll * n_expert ? 2 : 3;
