@@ -50,6 +50,52 @@ def test_rows_of_a_short_prompt(n, k, rows):
     test_rows_of_a_pass(n, k, rows)
 
 
+@pytest.mark.parametrize("rows,k,head_dim,n_seq", [(9, 2048, 4, 1), (12, 4096, 128, 3), (16, 2048, 8, 2), (40, 4096, 16, 1), (48, 2048, 32, 4), (65, 4096, 64, 5),
+                                                   (66, 2048, 256, 1), (150, 4096, 128, 1), (12, 2048, 0, 2), (81, 4096, 0, 1)])
+def test_gates_of_a_pass(rows, k, head_dim, n_seq):
+    """The staging launch's gated prologues: every width of a head that a super-block holds, gates in rows of their own and in a ring
+    that wraps, by a slot table in another order; sigmoid gates behind each head's query half and as plain rows (head_dim 0)."""
+    n, rng = 40, np.random.default_rng(rows + k + head_dim)
+    ctx = A.Context(0)
+    try:
+        wq = O.quantize_q4k((rng.standard_normal((n, k)) * 0.02).astype(np.float32))
+        w64 = O.dequant_q4k(wq, k).astype(np.float64)
+        x, z = rng.standard_normal((rows, k)).astype(np.float32), (2 * rng.standard_normal((rows, k))).astype(np.float32)
+        sig = 1 / (1 + np.exp(-z.astype(np.float64)))
+        dw, dx, dy = ctx.upload(wq), ctx.upload(x), ctx.alloc(rows * n * 4)
+
+        def check(want):
+            want, got = want @ w64.T, dy.read(np.float32, rows * n).reshape(rows, n)
+            err = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+            assert err.max() <= 1e-5, (int(err.argmax()), float(err.max()))
+            dy.zero()
+
+        if head_dim == 0:
+            ctx.gemv_q4k(dw, dx, dy, n, k, n_tok=rows, prologue=A.PRO_MUL_SIGMOID, z=ctx.upload(z))
+            return check(x.astype(np.float64) * sig)
+        pair = np.concatenate([rng.standard_normal((rows, k // head_dim, head_dim)).astype(np.float32), z.reshape(rows, -1, head_dim)], axis=2)
+        ctx.gemv_q4k(dw, dx, dy, n, k, n_tok=rows, prologue=A.PRO_MUL_SIGMOID, z=ctx.upload(pair), head_dim=head_dim, z_stride=2 * k)
+        check(x.astype(np.float64) * sig)
+        if head_dim < 32:
+            return
+        gamma = (1 + 0.1 * rng.standard_normal(head_dim)).astype(np.float32)
+        h = x.astype(np.float64).reshape(rows, -1, head_dim)
+        want = (h / np.sqrt((h * h).mean(axis=2, keepdims=True) + 1e-6) * gamma).reshape(rows, k) * sig
+        ctx.gemv_q4k(dw, dx, dy, n, k, n_tok=rows, prologue=A.PRO_GATED_NORM, gamma=ctx.upload(gamma), z=ctx.upload(z), head_dim=head_dim)
+        check(want)
+        seq_len, stride = rows // n_seq, k + 8
+        slots, pos, slot = seq_len + 1, np.arange(n_seq, dtype=np.int32) + 1, np.arange(n_seq, 0, -1).astype(np.int32)
+        ring = np.zeros((n_seq + 1, slots, stride), np.float32)
+        for s in range(n_seq):
+            for i in range(seq_len):
+                ring[slot[s], (pos[s] + i) % slots, :k] = z[s * seq_len + i]
+        ctx.gemv_q4k(dw, dx, dy, n, k, n_tok=rows, prologue=A.PRO_GATED_NORM, gamma=ctx.upload(gamma), z=ctx.upload(ring), head_dim=head_dim,
+                     pos=ctx.upload(pos), slot=ctx.upload(slot), seq_len=seq_len, ring_slots=slots, ring_stride=stride, z_ring=1)
+        check(want)
+    finally:
+        ctx.destroy()
+
+
 @pytest.mark.parametrize("rows,H,E", [(128, 256, 7), (129, 1024, 31), (145, 2304, 64), (2001, 512, 32)])
 def test_router_logits_of_a_long_pass(rows, H, E):
     """Columns of one super-block, of fewer than the block's waves and of more; router rows (the experts and the shared
