@@ -657,7 +657,7 @@ def main():
             st4 = dict(m.profile_chunk(rng.integers(0, cfg.vocab, size=big).astype(np.int32)))
             us4 = sum(v for k, v in st4.items() if k != "total") / 1e3
             n_dn = cfg.n_layer - cfg.n_layer // cfg.attn_every
-            dn_us = sum(st4.get(k, 0) for k in ("dn.hist", "dn.qkv", "dn.step", "dn.out")) / 1e3
+            dn_us = sum(st4.get(k, 0) for k in ("dn.qkv", "dn.step", "dn.out")) / 1e3
             at_us = sum(st4.get(k, 0) for k in ("attn.qkv", "attn.attn", "attn.out")) / 1e3
             rec["prefill_chunk_4096"] = {
                 "rows": big, "context_before": m.past() - big, "us": round(us4, 1), "tok_s": round(big / us4 * 1e6, 1),

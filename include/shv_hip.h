@@ -130,6 +130,7 @@ enum {
     SHV_OP_QSA_INDEX = 17,
     SHV_OP_ARGMAX_STATIC = 18, /* shv_argmax_static as an op, so that a recorded sequence can hold it */
     SHV_OP_ATTN_CELLS = 19,    /* shv_attn_decode_args: the rows' cells alone */
+    SHV_OP_DN_PASS = 20,
     SHV_OP__COUNT
 };
 
@@ -540,10 +541,10 @@ typedef struct {
 /* Rows of one ring of projection rows copied into another: positions pos[0]+first ..
  * pos[0]+first+count-1 (those below zero are skipped), row p from src[(p % src_slots) * stride] to
  * dst[(p % dst_slots) * stride], n floats each.  A prompt pass of many rows keeps its DeltaNet
- * projection rows in a ring of its own, sized for the pass: the conv's three rows of history are
- * brought into it before the step, and the pass's last three rows are left in the sequence's small
- * ring after it.  (No counterpart in the reference, whose conv window lives in the layer's own
- * activation buffer, llm/gpu_deltanet.go:1046-1052.) */
+ * projection rows in a ring of its own, sized for the pass; shv_dn_pass moves the conv's history
+ * between the two rings, by this where no kernel of the pass does it.  (No counterpart in the
+ * reference, whose conv window lives in the layer's own activation buffer,
+ * llm/gpu_deltanet.go:1046-1052.) */
 typedef struct {
     const float *src;
     float *dst;
@@ -551,6 +552,18 @@ typedef struct {
     int32_t src_slots, dst_slots, stride, n;
     int32_t first, count;
 } shv_ring_rows_args;
+
+/* shv_dn_step over one sequence whose pass has a ring of its own: step.ring holds the pass's rows
+ * alone (written by the projection before), the conv's history lies in hist, a ring of hist_slots
+ * rows ring_stride floats apart.  Rows pos-3 .. pos-1 are taken from hist, and the conv channels
+ * (2*hk*d + hv*d floats) of the pass's last three rows are left there for the next pass.
+ * n_seq 1, slot NULL, hist_slots >= 3, hist 16-byte aligned; step.ring must have room for three rows
+ * more than the pass, which a pass that shv_dn_step takes row by row uses. */
+typedef struct {
+    shv_dn_step_args step;
+    float *hist;
+    int32_t hist_slots, reserved;
+} shv_dn_pass_args;
 
 typedef struct {
     uint32_t kind;
@@ -595,6 +608,7 @@ int shv_moe_router(shv_ctx *ctx, const shv_moe_router_args *a);
 int shv_moe_up(shv_ctx *ctx, const shv_moe_up_args *a);
 int shv_moe_down(shv_ctx *ctx, const shv_moe_down_args *a);
 int shv_dn_step(shv_ctx *ctx, const shv_dn_step_args *a);
+int shv_dn_pass(shv_ctx *ctx, const shv_dn_pass_args *a);
 int shv_attn_decode(shv_ctx *ctx, const shv_attn_decode_args *a);
 int shv_embed(shv_ctx *ctx, const shv_embed_args *a);
 int shv_argmax(shv_ctx *ctx, const shv_argmax_args *a);

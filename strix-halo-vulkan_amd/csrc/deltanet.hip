@@ -402,8 +402,7 @@ __global__ __launch_bounds__(kBlock + 64 * kPrepWaves) void dn_step_pipe_kernel(
 
 }  // namespace
 
-int shv_launch_dn_step(shv_ctx *ctx, const shv_dn_step_args *pa) {
-    const shv_dn_step_args &a = *pa;
+static int check_step(const shv_dn_step_args &a) {
     SHV_REQUIRE(a.ring && a.conv1d && a.a && a.dt_bias && a.state && a.out, "dn_step: NULL argument");
     SHV_REQUIRE(a.head_dim == kD, "dn_step: head_dim %d; built for %d", a.head_dim, kD);
     SHV_REQUIRE(a.conv == 4, "dn_step: conv kernel %d; built for 4", a.conv);
@@ -418,7 +417,13 @@ int shv_launch_dn_step(shv_ctx *ctx, const shv_dn_step_args *pa) {
     SHV_REQUIRE(!a.spec || (a.n_planes > 1 && a.seq_len < a.n_planes), "dn_step: a rewindable pass of %d rows needs more than %d state planes",
                 a.seq_len, a.n_planes);
     SHV_REQUIRE(!a.work || a.work_floats >= 0, "dn_step: work_floats %lld", static_cast<long long>(a.work_floats));
-    if (shv_dn_chunk_covers(a)) return shv_launch_dn_chunk(ctx, a);
+    return SHV_OK;
+}
+
+int shv_launch_dn_step(shv_ctx *ctx, const shv_dn_step_args *pa) {
+    const shv_dn_step_args &a = *pa;
+    if (int rc = check_step(a)) return rc;
+    if (shv_dn_chunk_covers(a)) return shv_launch_dn_chunk(ctx, a, nullptr, 0);
     dim3 grid(kD / kRowsPerBlock, a.n_head_v, a.n_seq);
     // more than one group of rows: preparation and rule overlap
     if (a.seq_len > kPrep) SHV_LAUNCH(ctx, dn_step_pipe_kernel, grid, dim3(kBlock + 64 * kPrepWaves), 0, a);
@@ -427,4 +432,21 @@ int shv_launch_dn_step(shv_ctx *ctx, const shv_dn_step_args *pa) {
     else if (a.n_seq >= 4) SHV_LAUNCH(ctx, dn_step_kernel<4>, dim3(kD / 16, a.n_head_v, a.n_seq), dim3(kBlock), 0, a);
     else SHV_LAUNCH(ctx, dn_step_kernel<2>, grid, dim3(kBlock), 0, a);
     return SHV_OK;
+}
+
+// The history goes through the chunked form's preparation, which reads the rows it needs anyway; the forms that walk row
+// by row find it in the pass's ring, where a copy of three rows puts it (and another takes the last three out again).
+int shv_launch_dn_pass(shv_ctx *ctx, const shv_dn_pass_args *pa) {
+    const shv_dn_step_args &a = pa->step;
+    if (int rc = check_step(a)) return rc;
+    SHV_REQUIRE(a.n_seq == 1 && !a.slot, "dn_pass: one sequence without a slot table, not %d", a.n_seq);
+    SHV_REQUIRE(pa->hist && pa->hist_slots >= a.conv - 1, "dn_pass: a history of %d rows", pa->hist_slots);
+    SHV_REQUIRE(shv_aligned16(a.ring) && shv_aligned16(pa->hist) && a.ring_stride % 4 == 0, "dn_pass: rings must be 16-byte aligned, rows a multiple of 4 floats apart");
+    if (shv_dn_chunk_covers(a)) return shv_launch_dn_chunk(ctx, a, pa->hist, pa->hist_slots);
+    const int n = 2 * a.n_head_k * kD + a.n_head_v * kD, keep = a.conv - 1;
+    const shv_ring_rows_args in{pa->hist, const_cast<float *>(a.ring), a.pos, pa->hist_slots, a.ring_slots, a.ring_stride, n, -keep, keep};
+    const shv_ring_rows_args out{a.ring, pa->hist, a.pos, a.ring_slots, pa->hist_slots, a.ring_stride, n, a.seq_len - keep, keep};
+    if (int rc = shv_launch_ring_rows(ctx, &in)) return rc;
+    if (int rc = shv_launch_dn_step(ctx, &a)) return rc;
+    return shv_launch_ring_rows(ctx, &out);
 }

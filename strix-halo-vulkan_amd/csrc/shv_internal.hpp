@@ -186,6 +186,7 @@ size_t shv_moe_long_stage_bytes(int n_tok, int n_embd);
 int shv_launch_moe_up_long(shv_ctx *ctx, const shv_moe_up_args &a);
 int shv_launch_moe_down_long(shv_ctx *ctx, const shv_moe_down_args &a);
 int shv_launch_dn_step(shv_ctx *ctx, const shv_dn_step_args *a);
+int shv_launch_dn_pass(shv_ctx *ctx, const shv_dn_pass_args *a);
 int shv_launch_attn_decode(shv_ctx *ctx, const shv_attn_decode_args *a);
 int shv_launch_attn_cells(shv_ctx *ctx, const shv_attn_decode_args *a);
 // expert banks in other types than Q4_K: slots [slot0, slot0 + slots) of the up projection; slots
@@ -201,7 +202,7 @@ int shv_launch_ring_rows(shv_ctx *ctx, const shv_ring_rows_args *a);
 int shv_launch_router_fold(shv_ctx *ctx, const shv_router_fold_args *a);
 int shv_launch_qsa_index(shv_ctx *ctx, const shv_qsa_index_args *a);
 bool shv_dn_chunk_covers(const shv_dn_step_args &a);
-int shv_launch_dn_chunk(shv_ctx *ctx, const shv_dn_step_args &a);
+int shv_launch_dn_chunk(shv_ctx *ctx, const shv_dn_step_args &a, float *hist, int hist_slots);
 int shv_launch_copy_spans(shv_ctx *ctx, const shv_span *spans, int n);
 int shv_launch_upload_words(shv_ctx *ctx, const shv_words *words, int n);
 int shv_static_scratch_bind(shv_ctx *ctx);  // at shv_init, with ctx->device current

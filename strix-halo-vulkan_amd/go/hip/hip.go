@@ -294,6 +294,18 @@ type DNStepArgs struct {
 
 // DNStep is the gated delta rule over the ring rows of a pass.
 func DNStep(d DNStepArgs) Op {
+	a := d.args()
+	return mk(C.SHV_OP_DN_STEP, unsafe.Pointer(&a), C.sizeof_shv_dn_step_args)
+}
+
+// DNPass is DNStep over a pass whose ring holds its rows alone: the conv's history is taken from hist, a ring of
+// histSlots rows, and the pass's last rows are left there.
+func DNPass(d DNStepArgs, hist *Buffer, histSlots int) Op {
+	a := C.shv_dn_pass_args{step: d.args(), hist: fp(hist), hist_slots: C.int32_t(histSlots)}
+	return mk(C.SHV_OP_DN_PASS, unsafe.Pointer(&a), C.sizeof_shv_dn_pass_args)
+}
+
+func (d DNStepArgs) args() C.shv_dn_step_args {
 	var a C.shv_dn_step_args
 	a.ring, a.conv1d, a.a, a.dt_bias = fp(d.Ring), fp(d.Conv1D), fp(d.A), fp(d.DtBias)
 	a.state, a.out = fp(d.State), fp(d.Out)
@@ -308,7 +320,7 @@ func DNStep(d DNStepArgs) Op {
 	if d.Work != nil {
 		a.work, a.work_floats = fp(d.Work), C.int64_t(d.Work.size/4)
 	}
-	return mk(C.SHV_OP_DN_STEP, unsafe.Pointer(&a), C.sizeof_shv_dn_step_args)
+	return a
 }
 
 // AttnArgs are the fields of shv_attn_decode_args a caller sets (llm_attn_pack.comp,

@@ -85,11 +85,8 @@ func (g *deltanetHIP) graph(layer int, in, out *hip.Buffer, r hip.PassRows, f fo
 	}
 	kinds := []string{"dn.qkv", "dn.step", "dn.out"}
 	if big {
-		// the conv's history into the pass's ring, and the pass's last rows back into the sequence's own
-		hist := c.SSMConv - 1
-		ops = []hip.Op{hip.RingRows(g.ring[layer], g.bigRing, r.Pos, g.ringSlots, g.bigSlots, width, c.ConvWidth(), -hist, hist), ops[0], ops[1],
-			hip.RingRows(g.bigRing, g.ring[layer], r.Pos, g.bigSlots, g.ringSlots, width, c.ConvWidth(), rows-hist, hist), ops[2]}
-		kinds = []string{"dn.hist", "dn.qkv", "dn.step", "dn.hist", "dn.out"}
+		// the pass's rows lie in the big ring, the conv's history before and after it in the sequence's own
+		ops[1] = hip.DNPass(step, g.ring[layer], g.ringSlots)
 	}
 	return ops, kinds, nil
 }

@@ -11,7 +11,7 @@ Q4K_BYTES = 144
 OP_GEMV_Q4K, OP_DEQUANT_Q4K, OP_QUANTIZE_Q4K, OP_FILL_NORMAL = 1, 2, 3, 4
 OP_MOE_ROUTER, OP_MOE_UP, OP_MOE_DOWN, OP_DN_STEP, OP_ATTN_DECODE = 5, 6, 7, 8, 9
 OP_EMBED, OP_ARGMAX, OP_ADVANCE, OP_DEQUANT, OP_GEMV, OP_RING_ROWS, OP_ROUTER_FOLD, OP_QSA_INDEX = 10, 11, 12, 13, 14, 15, 16, 17
-OP_ARGMAX_STATIC, OP_ATTN_CELLS = 18, 19
+OP_ARGMAX_STATIC, OP_ATTN_CELLS, OP_DN_PASS = 18, 19, 20
 PRO_NONE, PRO_RMSNORM, PRO_GATED_NORM, PRO_MUL_SIGMOID, PRO_RMSNORM_PAIR = 0, 1, 2, 3, 4
 
 
@@ -110,6 +110,10 @@ class DnStepArgs(C.Structure):
                 ("work", C.c_void_p), ("work_floats", C.c_int64)]
 
 
+class DnPassArgs(C.Structure):
+    _fields_ = [("step", DnStepArgs), ("hist", C.c_void_p), ("hist_slots", C.c_int32), ("reserved", C.c_int32)]
+
+
 class AttnDecodeArgs(C.Structure):
     _fields_ = [("qkv", C.c_void_p), ("q_norm", C.c_void_p), ("k_norm", C.c_void_p),
                 ("rope", C.c_void_p), ("kcache", C.c_void_p), ("vcache", C.c_void_p),
@@ -178,7 +182,7 @@ SYMBOLS = [
     "shv_host_alloc", "shv_host_free", "shv_enqueue", "shv_dispatch_multi", "shv_prerecord",
     "shv_prerecorded_submit", "shv_prerecorded_launch", "shv_stamp", "shv_stamp_elapsed", "shv_prerecorded_count",
     "shv_prerecorded_destroy", "shv_gemv_q4k", "shv_dequant_q4k", "shv_dequant", "shv_gemv", "shv_quantize_q4k",
-    "shv_fill_normal", "shv_moe_router", "shv_moe_up", "shv_moe_down", "shv_dn_step", "shv_attn_decode", "shv_embed", "shv_argmax", "shv_advance",
+    "shv_fill_normal", "shv_moe_router", "shv_moe_up", "shv_moe_down", "shv_dn_step", "shv_dn_pass", "shv_attn_decode", "shv_embed", "shv_argmax", "shv_advance",
     "shv_argmax_static", "shv_ring_rows", "shv_router_fold", "shv_qsa_index",
 ]
 
@@ -238,6 +242,7 @@ def load():
     L.shv_moe_up.argtypes = [vp, C.POINTER(MoeUpArgs)]
     L.shv_moe_down.argtypes = [vp, C.POINTER(MoeDownArgs)]
     L.shv_dn_step.argtypes = [vp, C.POINTER(DnStepArgs)]
+    L.shv_dn_pass.argtypes = [vp, C.POINTER(DnPassArgs)]
     L.shv_attn_decode.argtypes = [vp, C.POINTER(AttnDecodeArgs)]
     L.shv_embed.argtypes = [vp, C.POINTER(EmbedArgs)]
     L.shv_argmax.argtypes = [vp, C.POINTER(ArgmaxArgs)]

@@ -886,16 +886,12 @@ std::vector<shv_op> DeltaNetGPU::Dispatches(int l, const float *in, float *out, 
         o.ring_stride = width;
         o.z_ring = 1;
     }
-    if (big) {
-        // history in, the pass, history out: only the conv's channels (q, k, v) are read back later
-        const int hist = c_.SSMConv - 1;
-        shv_ring_rows_args hin{slot_ring, big_ring_, r.pos, ring_slots_, big_slots_, width, c_.ConvWidth(), -hist, hist};
-        shv_ring_rows_args hout{big_ring_, slot_ring, r.pos, big_slots_, ring_slots_, width, c_.ConvWidth(), nTok - hist, hist};
-        if (labels) labels->insert(labels->end(), {"dn.hist", "dn.qkv", "dn.step", "dn.hist", "dn.out"});
-        return {make_op(SHV_OP_RING_ROWS, hin), make_op(SHV_OP_GEMV_Q4K, p), make_op(SHV_OP_DN_STEP, s), make_op(SHV_OP_RING_ROWS, hout),
-                make_op(SHV_OP_GEMV_Q4K, o)};
-    }
     if (labels) labels->insert(labels->end(), {"dn.qkv", "dn.step", "dn.out"});
+    if (big) {
+        // the pass's rows lie in the big ring, the conv's history before and after it in the slot's own
+        const shv_dn_pass_args d{s, slot_ring, ring_slots_, 0};
+        return {make_op(SHV_OP_GEMV_Q4K, p), make_op(SHV_OP_DN_PASS, d), make_op(SHV_OP_GEMV_Q4K, o)};
+    }
     return {make_op(SHV_OP_GEMV_Q4K, p), make_op(SHV_OP_DN_STEP, s), make_op(SHV_OP_GEMV_Q4K, o)};
 }
 

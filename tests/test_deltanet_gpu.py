@@ -274,6 +274,46 @@ def test_the_walk_over_records_at_its_edges(ctx, T, n_seq, hk, hv):
     assert max(O.rel_l2(rows.reshape(n_seq * T, vw)[t], want_rows.reshape(n_seq * T, vw)[t]) for t in range(n_seq * T)) <= 1e-4
 
 
+@pytest.mark.parametrize("T,pos,hist_slots,chunked", [(1, 0, 3, False), (2, 4, 3, False), (17, 0, 3, True), (18, 1, 4, True), (20, 2, 19, True),
+                                                      (64, 37, 19, True), (65, 5, 19, True), (150, 1000, 3, True), (70, 9, 8, False)])
+def test_a_pass_moves_its_history_between_two_rings(ctx, T, pos, hist_slots, chunked):
+    """shv_dn_pass against the step over one ring that holds the history too: the same rows and state bit for bit, the pass's
+    last three rows' conv channels in the history ring, and nothing else of it changed."""
+    c, d, hk, hv = ctx, 128, 4, 8
+    rng = np.random.default_rng(T + pos)
+    cw, vw = 2 * hk * d + hv * d, hv * d
+    width, slots = cw + vw + 2 * hv, T + 3
+    f32 = lambda *s: rng.standard_normal(s).astype(np.float32)
+    w = [c.upload(f32(cw, 4) * 0.3), c.upload(-np.exp(f32(hv))), c.upload(f32(hv))]
+    rows, hist, s0 = f32(slots, width), f32(hist_slots, width), f32(hv * d * d) * 0.1
+    whole, after = rows.copy(), hist.copy()
+    for p in range(max(pos - 3, 0), pos):
+        whole[p % slots, :cw] = hist[p % hist_slots, :cw]
+    for p in range(max(pos + T - 3, 0), pos + T):
+        after[p % hist_slots, :cw] = whole[p % slots, :cw]
+    floats = ((T * (cw + 2 * hv) + 3) & ~3) + ((T + 63) // 64) * hv * 5248
+    work = c.alloc(floats * 4) if chunked else None
+    d_pos, d_hist = c.upload(np.array([pos], np.int32)), c.upload(hist)
+    got = []
+    for ring in (whole, rows):
+        d_ring, d_state, d_out = c.upload(ring), c.upload(s0), c.alloc(T * vw * 4)
+        step = A.DnStepArgs(d_ring.ptr, w[0].ptr, w[1].ptr, w[2].ptr, d_state.ptr, d_out.ptr, d_pos.ptr, None, 1, T, hk, hv, d, 4,
+                            slots, width, EPS, 0, None, 0, 0, A.ptr(work), floats if chunked else 0)
+        c.dispatch_multi([A.make_op(A.OP_DN_STEP, step) if ring is whole else A.make_op(A.OP_DN_PASS, A.DnPassArgs(step, d_hist.ptr, hist_slots))])
+        got.append((d_out.read(np.float32, T * vw), d_state.read(np.float32, s0.size)))
+    for a, b in zip(*got):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    assert np.array_equal(d_hist.read(np.float32, hist.size).reshape(hist.shape), after)
+
+
+def test_dn_pass_refuses_what_it_does_not_cover(ctx):
+    d = ctx.alloc(1 << 16)
+    step = lambda n_seq, slot: A.DnStepArgs(d.ptr, d.ptr, d.ptr, d.ptr, d.ptr, d.ptr, d.ptr, slot, n_seq, 1, 16, 32, 128, 4, 4, 12352, EPS, 0)
+    for n_seq, slot, hist, slots in ((2, None, d.ptr, 3), (1, d.ptr, d.ptr, 3), (1, None, None, 3), (1, None, d.ptr, 2), (1, None, d.ptr + 4, 3)):
+        with pytest.raises(shv.pkg.ShvError):
+            ctx.enqueue(A.OP_DN_PASS, A.DnPassArgs(step(n_seq, slot), hist, slots))
+
+
 def test_dn_step_refuses_unsupported_shapes(ctx):
     d = ctx.alloc(1 << 16)
     with pytest.raises(shv.pkg.ShvError):
