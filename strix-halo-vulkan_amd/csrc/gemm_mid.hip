@@ -297,11 +297,15 @@ __global__ __launch_bounds__(64 * W) void gemm_mid_kernel(shv_gemv_q4k_args a, c
 // went from 58 to 24 us a layer at 150 rows of 513 x 2048, from 60 to 31 at 512, from 76 to 62 at 2048.
 // A fragment of the next tile asked for when this tile's is multiplied: 98.5 to 90.2 us at 4096 rows, 50.4 to 46.7 at 1531; a
 // die's blocks on neighbouring tiles: to 80.7 and 43.3 (150 rows 25.1 to 24.6).
+// A router row's 64 columns asked for by the lane that multiplies them are sixteen bytes of 64 lines a load, all eight waves' more
+// than L1 holds; by four lanes 64 bytes at a time and exchanged through LDS (the whole router op of 513 x 2048, launches overlapping):
+// 128 rows 18.6 to 13.7 us, 150 19.1 to 14.5, 512 23.3 to 18.9, 1531 32.8 to 29.0, 4096 60.4 to 56.7.
 template <int R>
 __global__ __launch_bounds__(512) void router_rows_kernel(const float *W, const float *extra_row, int n_rows, int K, int n_tok, const char *staged, float *logits,
                                                           int logits_stride, int tiles, int per_chunk) {
     constexpr int NW = 8;
     __shared__ __align__(16) float cpart[2][NW][R * 256];
+    __shared__ float4_t turn[NW][256];
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, kb = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // Workgroup i goes to die i % 8, each with an L2 of its own: a die takes neighbouring (chunk, rows), so that it reads two or
@@ -311,15 +315,26 @@ __global__ __launch_bounds__(512) void router_rows_kernel(const float *W, const 
     const int sbs = K / 256, row0 = item % gridDim.x * (16 * R), tile0 = item / gridDim.x * per_chunk;
     const int tile_end = tile0 + per_chunk < tiles ? tile0 + per_chunk : tiles;
     half8_t wh[R][8], wl[R][8];
-    auto form = [&](int sb) {  // this lane's 64 columns of every row
+    auto form = [&](int sb) {  // this lane's 64 columns of every row, read 64 bytes of a row by four lanes and turned in the wave's corner of LDS
+        const int lr = lane >> 2, ls = lane & 3;
+        // a row's sixteen quads, places exchanged by row: neither the four rows of a store nor the sixteen of a load meet in a bank
+        float4_t *mine = turn[wave];
+        const int to_x = ((lr & 3) << 2) | (lr >> 2), from_x = ((n & 3) << 2) | (n >> 2);
 #pragma unroll
         for (int r = 0; r < R; r++) {
             // rows past the end read the last row (their results are dropped); row n_rows - 1 may live apart
-            const int rr = row0 + 16 * r + n < n_rows ? row0 + 16 * r + n : n_rows - 1;
-            const float *wp = ((extra_row && rr == n_rows - 1) ? extra_row : W + static_cast<size_t>(rr) * K) + sb * 256 + kb * 64;
+            const int rr = row0 + 16 * r + lr < n_rows ? row0 + 16 * r + lr : n_rows - 1;
+            const float *wp = ((extra_row && rr == n_rows - 1) ? extra_row : W + static_cast<size_t>(rr) * K) + sb * 256 + ls * 4;
+            float4_t w[16];  // 16 columns of each 64, of all four
+#pragma unroll
+            for (int i = 0; i < 16; i++) w[i] = *reinterpret_cast<const float4_t *>(wp + (i & 3) * 64 + (i >> 2) * 16);
 #pragma unroll
             for (int v = 0; v < 8; v++) {
-                const float4 p = *reinterpret_cast<const float4 *>(wp + v * 8), q = *reinterpret_cast<const float4 *>(wp + v * 8 + 4);
+                if (v % 2 == 0) {
+#pragma unroll
+                    for (int g = 0; g < 4; g++) mine[lr * 16 + ((g * 4 + ls) ^ to_x)] = w[2 * v + g];
+                }
+                const float4_t p = mine[n * 16 + ((kb * 4 + v % 2 * 2) ^ from_x)], q = mine[n * 16 + ((kb * 4 + v % 2 * 2 + 1) ^ from_x)];
                 // slot order of the eight columns, as the rows were staged: [0, 2, 1, 3, 4, 6, 5, 7]
                 const float o[8] = {p.x, p.z, p.y, p.w, q.x, q.z, q.y, q.w};
 #pragma unroll
