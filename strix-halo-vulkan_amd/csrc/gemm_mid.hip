@@ -396,6 +396,127 @@ __global__ __launch_bounds__(512) void router_rows_kernel(const float *W, const 
     }
 }
 
+// The same logits for lower passes of 2048 columns, where launches and trips to memory are the time and not the products: a block
+// takes 16 R experts and 16 tokens, each of its eight waves an eighth of the columns, on the float32 matrix instruction (nothing
+// is split into halves), and no staging launch comes before.  The norm's factor is the last thing applied:
+// logit = factor * sum((h * gamma) . w); xn = h * (factor * gamma) for whoever needs the row.  Rows come and are exchanged as above.
+// No chain is longer than 16 products: against float64 the logits' error is 0.9 of the row kernel's below 128 rows (rms 4.4e-7 and
+// 4.9e-7 of logits of 3.7) and 0.63 of the staged form's.  Of the time, 3 us a block are its 256 KB by way of L1; with sixteen bytes
+// of 16 rows a load it took 7.  The whole op, 513 x 2048, before (row kernel to 127 rows, staged from there) and now: 65 rows 15.0
+// and 7.8 us, 100 19.9 and 8.0, 121 22.4 and 8.1, 150 14.5 and 10.4, 256 16.7 and 10.6, 300 17.9 and 16.0, 384 19.2 and 16.7.
+template <int R, int PER_CU>
+__global__ __launch_bounds__(512, 2 * PER_CU) void router_norm_kernel(shv_moe_router_args a, int tiles) {
+    constexpr int K = 2048, NW = 8;
+    __shared__ __align__(16) float g[K];
+    __shared__ float squares[NW][16], gate[NW][16], part[NW][R * 256];
+    __shared__ float4_t turn[NW][256];
+    const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, kb = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // a die takes neighbouring items, the tiles of 16 experts one behind the other: it reads an eighth of the router and all tokens
+    const int count = gridDim.x, die = blockIdx.x & 7, item = die * (count >> 3) + min(die, count & 7) + (blockIdx.x >> 3);
+    const int group = item / tiles, row0 = group * 16 * R, t0 = item % tiles * 16, groups = count / tiles;
+    const int c0 = wave * 256, lr = lane >> 2, ls = lane & 3;
+    // rows past the end read the last one: what they give is dropped
+    const float *hp = a.h + static_cast<size_t>(min(t0 + lr, a.n_tok - 1)) * a.h_stride + c0 + 4 * ls, *wp[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) wp[r] = a.router + static_cast<size_t>(min(row0 + 16 * r + lr, a.n_expert - 1)) * K + c0 + 4 * ls;
+    // sixteen columns of each 64 at a time, the next asked for when these are in LDS (two steps ahead: 0.3 us more)
+    float4_t h[4], w[R][4], sum[R];
+    const auto ask = [&](int q) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) h[i] = *reinterpret_cast<const float4_t *>(hp + (q * 4 + i) * 16);
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) w[r][i] = *reinterpret_cast<const float4_t *>(wp[r] + (q * 4 + i) * 16);
+    };
+    const float4_t gm = *reinterpret_cast<const float4_t *>(a.gamma + c0 + 4 * lane);
+    ask(0);
+    *reinterpret_cast<float4_t *>(g + c0 + 4 * lane) = gm;  // read by this wave, and behind the barrier by all
+    float4_t *mine = turn[wave];
+    const int to_x = ((lr & 3) << 2) | (lr >> 2), from_x = ((n & 3) << 2) | (n >> 2);
+    float ss = 0.f;
+#pragma unroll
+    for (int r = 0; r < R; r++) sum[r] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        __builtin_amdgcn_sched_barrier(0);
+        float4_t x[4], wq[R][4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) mine[lr * 16 + ((i * 4 + ls) ^ to_x)] = h[i];
+#pragma unroll
+        for (int i = 0; i < 4; i++) x[i] = mine[n * 16 + ((kb * 4 + i) ^ from_x)];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float4_t gi = *reinterpret_cast<const float4_t *>(g + c0 + (q * 4 + kb) * 16 + 4 * i);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                ss = fmaf(x[i][j], x[i][j], ss);
+                x[i][j] *= gi[j];
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) mine[lr * 16 + ((i * 4 + ls) ^ to_x)] = w[r][i];
+#pragma unroll
+            for (int i = 0; i < 4; i++) wq[r][i] = mine[n * 16 + ((kb * 4 + i) ^ from_x)];
+        }
+        if (PER_CU > 1) __builtin_amdgcn_sched_barrier(0);  // (not before these are read: two blocks of a compute unit share its registers)
+        if (q < 3) ask(q + 1);
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            float4_t acc[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc[j] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i][j], wq[r][i][j], acc[j], 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < 4; j++) sum[r][j] += (acc[0][j] + acc[1][j]) + (acc[2][j] + acc[3][j]);
+        }
+    }
+    ss += __shfl_xor(ss, 16, 64);
+    ss += __shfl_xor(ss, 32, 64);
+    if (kb == 0) squares[wave][n] = ss;
+    // the shared expert's gate, one row more: a token of the tile to each of its blocks
+    for (int t = group; a.shared_gate && t < 16; t += groups) {
+        const float4_t x = *reinterpret_cast<const float4_t *>(a.h + static_cast<size_t>(min(t0 + t, a.n_tok - 1)) * a.h_stride + c0 + 4 * lane);
+        const float4_t v = *reinterpret_cast<const float4_t *>(a.shared_gate + c0 + 4 * lane);
+        const float gs = wave_sum_all((x[0] * gm[0] * v[0] + x[1] * gm[1] * v[1]) + (x[2] * gm[2] * v[2] + x[3] * gm[3] * v[3]));
+        if (lane == 0) gate[wave][t] = gs;
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) part[wave][(r * 64 + lane) * 4 + j] = sum[r][j];
+    __syncthreads();
+    const auto over_waves = [](const float *v, int stride) {
+        return ((v[0] + v[stride]) + (v[2 * stride] + v[3 * stride])) + ((v[4 * stride] + v[5 * stride]) + (v[6 * stride] + v[7 * stride]));
+    };
+    const auto factor = [&](int t) { return 1.f / sqrtf(over_waves(&squares[0][t], 16) / static_cast<float>(K) + a.eps); };
+    if (tid < R * 256) {
+        // value j of a product's lane l: token 4 (l / 16) + j, router row l % 16
+        const int r = tid >> 8, t = tid >> 4 & 15, row = row0 + 16 * r + (tid & 15), o = (r * 64 + (t >> 2) * 16 + (tid & 15)) * 4 + (t & 3);
+        if (t0 + t < a.n_tok && row < a.n_expert) a.logits[static_cast<size_t>(t0 + t) * (a.n_expert + 1) + row] = over_waves(&part[0][o], R * 256) * factor(t);
+    }
+    if (a.shared_gate && tid < 16 && tid % groups == group && t0 + tid < a.n_tok)
+        a.logits[static_cast<size_t>(t0 + tid) * (a.n_expert + 1) + a.n_expert] = over_waves(&gate[0][tid], 16) * factor(tid);
+    // the normed rows themselves, 128 columns at a time by the tile's blocks in turn
+    const int t = tid >> 5;
+    if (t0 + t < a.n_tok) {
+        const float f = factor(t);
+        for (int c = group * 128 + (tid & 31) * 4; c < K; c += groups * 128) {
+            const float4_t v = *reinterpret_cast<const float4_t *>(a.h + static_cast<size_t>(t0 + t) * a.h_stride + c), gc = *reinterpret_cast<const float4_t *>(g + c);
+            float4_t x;
+#pragma unroll
+            for (int j = 0; j < 4; j++) x[j] = v[j] * (f * gc[j]);
+            *reinterpret_cast<float4_t *>(a.xn + static_cast<size_t>(t0 + t) * K + c) = x;
+        }
+    }
+}
+
 // How many of a pass's tiles a block walks, `blocks` of them side by side over the weight rows: as few as blocks on every compute
 // unit, one each, leave it (more blocks would form the weights again).
 int tiles_a_block(const shv_ctx *ctx, int tiles, int blocks) {
@@ -439,8 +560,6 @@ int launch_stage(shv_ctx *ctx, const shv_gemv_q4k_args &a, int tiles, float *x_o
     return SHV_OK;
 }
 
-}  // namespace
-
 // From nine rows, where the kernels that form every weight once for up to eight of them end, to 512, but for 49 to 64, which
 // keep the kernel of one 64-row group.  That kernel is the slower there (12352 x 2048 of 64 rows 27.7 us, 15.9 here; of 40 rows 24.1
 // and 13.8, of 17 20.6 and 12.4; 2048 x 4096 of 40 rows 17.9 and 11.0) and the less exact (2.1e-6 against 0.4e-6): the line is one of
@@ -450,6 +569,8 @@ int launch_stage(shv_ctx *ctx, const shv_gemv_q4k_args &a, int tiles, float *x_o
 // 1.5e-5 there and 1.1e-5 here, 64 rows 1.4e-5 and 1.0e-5 (one of the ten 3.6e-3 there: another expert), where 17 to 48 rows went over
 // from 2.1e-5 to 1.6e-5 at 20 rows, 1.6e-5 to 1.1e-5 at 48.
 // Past 512 gemm_long.hip's blocks read less from L2.
+}  // namespace
+
 bool shv_gemm_mid_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a) {
     if (!ctx->gemm_stage || (a.k != 2048 && a.k != 4096) || a.n_tok < 9 || a.n_tok > 512) return false;
     if (a.n_tok > 48 && a.n_tok <= 64) return false;
@@ -467,16 +588,43 @@ int shv_launch_gemm_mid(shv_ctx *ctx, const shv_gemv_q4k_args &a) {
     return tiles == 1 ? launch<1, 2, 8>(ctx, a, tiles) : launch<2, 2, 8>(ctx, a, tiles);
 }
 
-// The router of a pass of many rows: xn = rmsnorm(h) * gamma staged (and written out as float32), then every token's
-// n_expert (+ 1, the shared expert's gate) logits on the matrix cores.
+// The router of a pass of many rows: xn = rmsnorm(h) * gamma written as float32 (and staged, by the form that multiplies staged
+// rows), then every token's n_expert (+ 1, the shared expert's gate) logits on the matrix cores.
+// Which form, of 2048 columns: the float32 blocks while one a compute unit is enough, of 16 experts or of 32 (150 rows of 512 experts,
+// 256 compute units: 11.5 and 10.4 us), and by turns while three are (384 rows 16.7 us, staged 19.2); at 512 rows they lose, 20.3 to 18.9.
+// Their line below is 65 rows: the selection of a pass of one 64-row group stays what the row kernel's sums make it.
+namespace {
+
+bool router_aligned(const shv_moe_router_args &a) {
+    return a.gamma && a.xn && a.h_stride % 4 == 0 && shv_aligned16(a.h) && shv_aligned16(a.gamma) && shv_aligned16(a.xn) && shv_aligned16(a.router) &&
+           (!a.shared_gate || shv_aligned16(a.shared_gate));
+}
+
+enum class RouterNorm { none, sixteen, thirty_two, sixteen_by_turns };
+RouterNorm router_norm_form(const shv_ctx *ctx, const shv_moe_router_args &a) {
+    const long long cus = ctx->prop.multiProcessorCount, tiles = (a.n_tok + 15) / 16, ones = (a.n_expert + 15) / 16 * tiles, twos = (a.n_expert + 31) / 32 * tiles;
+    if (a.n_embd != 2048 || a.n_tok < 65 || ones > 3 * cus) return RouterNorm::none;
+    return ones <= cus ? RouterNorm::sixteen : twos <= cus ? RouterNorm::thirty_two : RouterNorm::sixteen_by_turns;
+}
+
+}  // namespace
+
 bool shv_router_rows_covers(const shv_ctx *ctx, const shv_moe_router_args &a) {
-    if (!ctx->gemm_stage || a.n_tok < 128 || !a.gamma || !a.xn) return false;
-    if (a.n_embd % 256 != 0 || a.n_embd < 256 || a.h_stride % 4 != 0) return false;
-    if (!shv_aligned16(a.h) || !shv_aligned16(a.gamma) || !shv_aligned16(a.xn) || !shv_aligned16(a.router) || (a.shared_gate && !shv_aligned16(a.shared_gate))) return false;
+    if (!router_aligned(a)) return false;
+    if (router_norm_form(ctx, a) != RouterNorm::none) return true;
+    if (!ctx->gemm_stage || a.n_tok < 128 || a.n_embd % 256 != 0 || a.n_embd < 256) return false;
     return mid_bytes((a.n_tok + 15) / 16, a.n_embd) <= static_cast<size_t>(shv_ctx::kGemmStageBytes);
 }
 
 int shv_launch_router_rows(shv_ctx *ctx, const shv_moe_router_args &a) {
+    const int tiles = (a.n_tok + 15) / 16;
+    const dim3 ones((a.n_expert + 15) / 16 * tiles), twos((a.n_expert + 31) / 32 * tiles), block(512);
+    switch (router_norm_form(ctx, a)) {
+        case RouterNorm::sixteen: SHV_LAUNCH(ctx, (router_norm_kernel<1, 1>), ones, block, 0, a, tiles); return SHV_OK;
+        case RouterNorm::thirty_two: SHV_LAUNCH(ctx, (router_norm_kernel<2, 1>), twos, block, 0, a, tiles); return SHV_OK;
+        case RouterNorm::sixteen_by_turns: SHV_LAUNCH(ctx, (router_norm_kernel<1, 2>), ones, block, 0, a, tiles); return SHV_OK;
+        case RouterNorm::none: break;
+    }
     shv_gemv_q4k_args g{};
     g.x = a.h;
     g.gamma = a.gamma;
@@ -485,7 +633,7 @@ int shv_launch_router_rows(shv_ctx *ctx, const shv_moe_router_args &a) {
     g.prologue = SHV_PRO_RMSNORM;
     g.eps = a.eps;
     g.x_stride = a.h_stride;
-    const int tiles = (a.n_tok + 15) / 16, n_rows = a.n_expert + (a.shared_gate ? 1 : 0);
+    const int n_rows = a.n_expert + (a.shared_gate ? 1 : 0);
     const int rc = launch_stage(ctx, g, tiles, a.xn);
     if (rc != SHV_OK) return rc;
     constexpr int R = 2;

@@ -118,6 +118,40 @@ def test_router_logits_of_a_long_pass(rows, H, E):
         ctx.destroy()
 
 
+@pytest.mark.parametrize("rows,E,gate", [(65, 512, True), (80, 512, False), (121, 512, True), (128, 512, True), (129, 512, True), (256, 512, True), (257, 512, True),
+                                         (384, 512, True), (385, 512, True), (70, 7, True), (100, 17, True), (300, 31, False), (2000, 33, True)])
+def test_router_of_a_lower_pass(rows, E, gate):
+    """Blocks of 16 experts, of 32, of 16 again and the staged form behind them; experts that end inside a block, fewer of them
+    than a tile's tokens and columns need blocks; with and without the shared expert's gate; a row of another size beside every
+    other; an infinity that stays in its row.  Sums of 2048 float32 products in chains of 16 and some ten levels over them: at
+    most 26 roundings a logit of its largest partial sum, which the products' root sum of squares bounds five times over."""
+    H, rng = 2048, np.random.default_rng(rows + E)
+    ctx = A.Context(0)
+    try:
+        h = (rng.standard_normal((rows, H)) * rng.uniform(0.01, 30.0, size=(rows, 1))).astype(np.float32)
+        bad = rows - 2
+        h[bad, 77] = np.inf
+        gamma = (1 + 0.1 * rng.standard_normal(H)).astype(np.float32)
+        router, shared = (rng.standard_normal((E, H)) * 0.08).astype(np.float32), (rng.standard_normal(H) * 0.08).astype(np.float32)
+        xn, logits = ctx.alloc(rows * H * 4), ctx.upload(np.full((rows, E + 1), -7.0, np.float32))
+        args = A.MoeRouterArgs(ctx.upload(h).ptr, ctx.upload(gamma).ptr, ctx.upload(router).ptr, ctx.upload(shared).ptr if gate else None, xn.ptr, logits.ptr,
+                               ctx.alloc(rows * 4 * 4).ptr, ctx.alloc(rows * 5 * 4).ptr, rows, H, E, 4, 1e-6, H, 0)
+        ctx.dispatch_multi([A.make_op(A.OP_MOE_ROUTER, args)])
+        ok = np.arange(rows) != bad
+        h64 = h[ok].astype(np.float64)
+        want_x = h64 / np.sqrt((h64 * h64).mean(axis=1, keepdims=True) + 1e-6) * gamma
+        every = np.vstack([router, shared]).astype(np.float64)
+        got_x, got = xn.read(np.float32, rows * H).reshape(rows, H), logits.read(np.float32, rows * (E + 1)).reshape(rows, E + 1)
+        assert np.abs(got_x[ok] - want_x).max() <= 1e-6 * np.abs(want_x).max()
+        bound = 26 * 2.0 ** -24 * 5 * np.sqrt((want_x * want_x) @ (every * every).T)
+        n = E + 1 if gate else E
+        assert (np.abs(got[ok] - want_x @ every.T) <= bound)[:, :n].all()
+        assert gate or (got[:, E] == -7.0).all()
+        assert not np.isfinite(got[bad, :n]).any()
+    finally:
+        ctx.destroy()
+
+
 @pytest.mark.parametrize("n,k,rows", [(96, 2048, 9), (2048, 4096, 16), (70, 2048, 65), (2048, 4096, 192), (300, 2048, 512)])
 def test_sums_past_binary16(n, k, rows):
     """Every activation is a binary16 number, the sum of a sub-block's 32 is not (65504 is the largest): the min term's sums are
