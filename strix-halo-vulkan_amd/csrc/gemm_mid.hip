@@ -592,7 +592,8 @@ int shv_launch_gemm_mid(shv_ctx *ctx, const shv_gemv_q4k_args &a) {
 // rows), then every token's n_expert (+ 1, the shared expert's gate) logits on the matrix cores.
 // Which form, of 2048 columns: the float32 blocks while one a compute unit is enough, of 16 experts or of 32 (150 rows of 512 experts,
 // 256 compute units: 11.5 and 10.4 us), and by turns while three are (384 rows 16.7 us, staged 19.2); at 512 rows they lose, 20.3 to 18.9.
-// Their line below is 65 rows: the selection of a pass of one 64-row group stays what the row kernel's sums make it.
+// Below, the row kernel goes through its tokens a few at a time (17 rows 7.8 us to 7.6, 32 10.4 to 7.7, 48 12.5 to 7.8) and is quicker
+// of 16; 49 to 64 rows stay with it as they do with the projections of one 64-row group: a line of the results' continuity.
 namespace {
 
 bool router_aligned(const shv_moe_router_args &a) {
@@ -603,7 +604,7 @@ bool router_aligned(const shv_moe_router_args &a) {
 enum class RouterNorm { none, sixteen, thirty_two, sixteen_by_turns };
 RouterNorm router_norm_form(const shv_ctx *ctx, const shv_moe_router_args &a) {
     const long long cus = ctx->prop.multiProcessorCount, tiles = (a.n_tok + 15) / 16, ones = (a.n_expert + 15) / 16 * tiles, twos = (a.n_expert + 31) / 32 * tiles;
-    if (a.n_embd != 2048 || a.n_tok < 65 || ones > 3 * cus) return RouterNorm::none;
+    if (a.n_embd != 2048 || a.n_tok < 17 || (a.n_tok > 48 && a.n_tok <= 64) || ones > 3 * cus) return RouterNorm::none;
     return ones <= cus ? RouterNorm::sixteen : twos <= cus ? RouterNorm::thirty_two : RouterNorm::sixteen_by_turns;
 }
 

@@ -118,7 +118,7 @@ def test_router_logits_of_a_long_pass(rows, H, E):
         ctx.destroy()
 
 
-@pytest.mark.parametrize("rows,E,gate", [(65, 512, True), (80, 512, False), (121, 512, True), (128, 512, True), (129, 512, True), (256, 512, True), (257, 512, True),
+@pytest.mark.parametrize("rows,E,gate", [(17, 512, True), (48, 512, True), (49, 512, True), (65, 512, True), (80, 512, False), (121, 512, True), (128, 512, True), (129, 512, True), (256, 512, True), (257, 512, True),
                                          (384, 512, True), (385, 512, True), (70, 7, True), (100, 17, True), (300, 31, False), (2000, 33, True)])
 def test_router_of_a_lower_pass(rows, E, gate):
     """Blocks of 16 experts, of 32, of 16 again and the staged form behind them; experts that end inside a block, fewer of them
