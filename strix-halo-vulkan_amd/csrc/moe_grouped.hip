@@ -140,27 +140,9 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int32_t *topk, in
 // its last bit.  The waves then place their pairs one after the other, a lane behind the lanes before it with the same expert
 // (150 rows of ten experts: 224.2 us a layer with the pairs as they arrive, 224.9 so; 750 rows 430.5 and 430.9).
 constexpr int kGroupBlocks = 16;
-// Blocks past the counting ones, when the launch has them, stage the rows x [rows][k] for the list kernels meanwhile: whole
-// rows, k / 256 of a block's sixteen waves each.
-__global__ __launch_bounds__(1024) void moe_group_count_kernel(const int32_t *topk, int n_pairs, int chunk, int n_expert, int32_t *counts, const float *x, int rows, int k,
-                                                               char *staged) {
+__global__ __launch_bounds__(1024) void moe_group_count_kernel(const int32_t *topk, int n_pairs, int chunk, int n_expert, int32_t *counts) {
     __shared__ int32_t s_cnt[kMaxExperts];
     const int tid = threadIdx.x;
-    if (blockIdx.x >= kGroupBlocks) {
-        __shared__ float s_max[16];
-        const int quad = (blockIdx.x - kGroupBlocks) * 1024 + tid, t = quad / (k / 4), c = (quad % (k / 4)) * 4, per = k / 256;
-        const float4 v = t < rows ? *reinterpret_cast<const float4 *>(x + static_cast<size_t>(t) * k + c) : float4{0.f, 0.f, 0.f, 0.f};
-        float largest = wave_max_all(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-        if ((tid & 63) == 0) s_max[tid >> 6] = largest;
-        __syncthreads();
-        for (int w = 0, w0 = (tid >> 6) / per * per; w < per; w++) largest = fmaxf(largest, s_max[w0 + w]);
-        const int e = biased_exponent(largest);
-        if (t < rows) {
-            stage_list_quad(v, e, t, c, k, rows, staged);
-            if (c == 0) reinterpret_cast<int32_t *>(staged + list_exps_offset(rows, k))[t] = e;
-        }
-        return;
-    }
     for (int e = tid; e < n_expert; e += 1024) s_cnt[e] = 0;
     __syncthreads();
     const int lo = blockIdx.x * chunk, hi = lo + chunk < n_pairs ? lo + chunk : n_pairs;
@@ -172,15 +154,51 @@ __global__ __launch_bounds__(1024) void moe_group_count_kernel(const int32_t *to
     for (int e = tid; e < n_expert; e += 1024) counts[blockIdx.x * n_expert + e] = s_cnt[e];
 }
 
+// Rows x [rows][k] staged for the list kernels: whole rows, k / 256 of a block's sixteen waves each.
+__device__ __forceinline__ void stage_rows(const float *x, int rows, int k, char *staged, int block) {
+    __shared__ float s_max[16];
+    const int tid = threadIdx.x, quad = block * 1024 + tid, t = quad / (k / 4), c = (quad % (k / 4)) * 4, per = k / 256;
+    const float4 v = t < rows ? *reinterpret_cast<const float4 *>(x + static_cast<size_t>(t) * k + c) : float4{0.f, 0.f, 0.f, 0.f};
+    float largest = wave_max_all(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+    if ((tid & 63) == 0) s_max[tid >> 6] = largest;
+    __syncthreads();
+    for (int w = 0, w0 = (tid >> 6) / per * per; w < per; w++) largest = fmaxf(largest, s_max[w0 + w]);
+    const int e = biased_exponent(largest);
+    if (t < rows) {
+        stage_list_quad(v, e, t, c, k, rows, staged);
+        if (c == 0) reinterpret_cast<int32_t *>(staged + list_exps_offset(rows, k))[t] = e;
+    }
+}
+
+// counts NULL: no launch before; every block counts all pairs itself, those before its own chunk apart.  Blocks past the sixteen,
+// when the launch has them, stage the list kernels' rows x meanwhile.
 __global__ __launch_bounds__(1024) void moe_group_place_kernel(const int32_t *topk, int n_pairs, int chunk, int n_used, int n_expert, const int32_t *counts,
-                                                               int32_t *group, int in_order) {
+                                                               int32_t *group, int in_order, const float *x, int rows, int k, char *staged) {
+    if (blockIdx.x >= kGroupBlocks) return stage_rows(x, rows, k, staged, blockIdx.x - kGroupBlocks);
     __shared__ int32_t s_cnt[kMaxExperts + 1];
     __shared__ __align__(16) int32_t s_len[kMaxExperts];
     __shared__ int32_t s_wsum[16];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nb = gridDim.x, b = blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nb = kGroupBlocks, b = blockIdx.x;
     // thread e: expert e's total, and the pairs of it the blocks before this one hold
     int c = 0, before = 0;
-    if (tid < n_expert) {
+    if (!counts) {
+        s_cnt[tid] = s_len[tid] = 0;
+        __syncthreads();
+        constexpr int NB = 8;
+        for (int i0 = tid; i0 < n_pairs; i0 += NB * 1024) {
+            int e[NB];
+#pragma unroll
+            for (int u = 0; u < NB; u++) e[u] = i0 + u * 1024 < n_pairs ? topk[i0 + u * 1024] : -1;
+#pragma unroll
+            for (int u = 0; u < NB; u++)
+                if (e[u] >= 0 && e[u] < n_expert) {
+                    atomicAdd(&s_len[e[u]], 1);
+                    if (i0 + u * 1024 < b * chunk) atomicAdd(&s_cnt[e[u]], 1);
+                }
+        }
+        __syncthreads();
+        c = s_len[tid], before = s_cnt[tid];
+    } else if (tid < n_expert) {
         // all of them asked for together: one after the other they are sixteen trips to memory
         int v[kGroupBlocks];
 #pragma unroll
@@ -546,7 +564,9 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(shv_moe_down_args a) {
 // The per-expert lists of a pass: one block for short passes of few experts, kGroupBlocks in two launches from 2048
 // pairs or 128 experts on (ranking the experts by length is E^2 comparisons, a block's share of them a sixteenth)
 // (their counts meet in the library's scratch, which nothing else on the stream is using between the two).
-// x: rows of k floats to stage for the list kernels in the first launch; their lists are in order.
+// x: rows of k floats to stage for the list kernels, whose lists are in order and few enough pairs for every block to count them
+// all: one launch (a pass of 16 layers, with the count in a launch of its own and so: 65 rows 3749 and 3720 us, 150 rows 4989
+// and 4965, 300 rows 6600 and 6580, 700 rows 10844 and 10837; the long passes' lists gain nothing, 1531 rows 14298 and 14297).
 int launch_group(shv_ctx *ctx, const int32_t *topk, int n_tok, int n_used, int n_expert, int32_t *group, const float *x = nullptr, int k = 0) {
     const int n_pairs = n_tok * n_used;
     if (!x && ((n_pairs < 2048 && n_expert < 128) || !ctx->gemm_part || ctx->moe_group_one_block)) {
@@ -557,8 +577,9 @@ int launch_group(shv_ctx *ctx, const int32_t *topk, int n_tok, int n_used, int n
     int32_t *counts = reinterpret_cast<int32_t *>(ctx->gemm_part);
     const int chunk = (n_pairs + kGroupBlocks - 1) / kGroupBlocks;
     const int stage_blocks = x ? static_cast<int>((static_cast<long long>(n_tok) * (k / 4) + 1023) / 1024) : 0;
-    SHV_LAUNCH(ctx, moe_group_count_kernel, dim3(kGroupBlocks + stage_blocks), dim3(1024), 0, topk, n_pairs, chunk, n_expert, counts, x, n_tok, k, ctx->gemm_stage);
-    SHV_LAUNCH(ctx, moe_group_place_kernel, dim3(kGroupBlocks), dim3(1024), 0, topk, n_pairs, chunk, n_used, n_expert, counts, group, x && chunk <= 1024 ? 1 : 0);
+    if (!x) SHV_LAUNCH(ctx, moe_group_count_kernel, dim3(kGroupBlocks), dim3(1024), 0, topk, n_pairs, chunk, n_expert, counts);
+    SHV_LAUNCH(ctx, moe_group_place_kernel, dim3(kGroupBlocks + stage_blocks), dim3(1024), 0, topk, n_pairs, chunk, n_used, n_expert, x ? nullptr : counts, group,
+               x && chunk <= 1024 ? 1 : 0, x, n_tok, k, ctx->gemm_stage);
     return SHV_OK;
 }
 

@@ -194,3 +194,26 @@ def test_the_same_pass_again_is_the_same(T):
     for b in bufs + [act, out, group, pairs, rows, down]:
         b.free()
     c.destroy()
+
+
+@pytest.mark.parametrize("T,E,U", [(65, 24, 1), (820, 600, 10), (896, 600, 10)])  # 65 pairs; 8200 and 8960: past a block's first 8192
+def test_the_lists_themselves(T, E, U):
+    """Starts, lists by token and the experts by length, made by one launch whose blocks each count every pair; experts nobody chose,
+    one that every token did."""
+    c, rng = A.Context(), np.random.default_rng(T)
+    p = rng.random((T, E)) * (1 + np.arange(E) % 7)
+    p[:, 3], p[:, 5] = 9.0, -1.0
+    topk = np.argsort(-p, axis=1)[:, :U].astype(np.int32)
+    bank = c.alloc(E * F * (H // 256) * 144).zero()
+    act, group = c.alloc(T * (U + 1) * F * 4), c.alloc((2 * E + 1 + T * U) * 4)
+    x, tk = c.upload(rng.standard_normal((T, H)).astype(np.float32)), c.upload(topk)
+    c.dispatch_multi([A.make_op(A.OP_MOE_UP, A.MoeUpArgs(x.ptr, tk.ptr, bank.ptr, bank.ptr, bank.ptr, bank.ptr, act.ptr, T, H, U, F, None, None, E,
+                                                         0, 0, 0, 0, group.ptr, 0, 1))])
+    got = group.read(np.int32, 2 * E + 1 + T * U)
+    flat = topk.ravel()
+    count = np.bincount(flat, minlength=E)
+    assert np.array_equal(got[:E + 1], np.concatenate([[0], np.cumsum(count)]))
+    order = np.argsort(flat, kind="stable")
+    assert np.array_equal(got[E + 1:E + 1 + T * U], order // U * (U + 1) + order % U)
+    assert np.array_equal(got[E + 1 + T * U:], np.argsort(-count, kind="stable"))
+    c.destroy()
