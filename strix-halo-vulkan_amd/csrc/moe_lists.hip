@@ -52,16 +52,20 @@ typedef __attribute__((address_space(3))) void *lds_ptr_t;
 typedef const __attribute__((address_space(3))) char *lds_bytes_t;
 typedef const __attribute__((address_space(3))) u32x4_t *lds_quad_t;
 
-// w: the first row of the chunk's (first) tile, at the first of its super-blocks (the same in every lane)
+// w: the first row of the chunk's (first) tile, at the first of its super-blocks (the same in every lane).  on false: as many
+// loads, all of the chunk's first lines.  A wave's last chunk is waited for by their count; with the whole first chunk asked for
+// again behind it a ninth of what the kernels read was read for nothing: a layer of 66 rows 176 to 168 us, of 150 rows 232 to
+// 223, of 700 rows 410 to 399 (prompts of 65, 150 and 700 rows of 16 layers 3725 to 3679 us, 5000 to 4938, 10793 to 10723).
+// A branch around the loads costs the gate/up kernel 156 spills.
 template <int ROWB, int S>
-__device__ __forceinline__ void ask_chunk(const char *w, char *lds, int lane) {
+__device__ __forceinline__ void ask_chunk(const char *w, char *lds, int lane, bool on = true) {
     const int n = lane & 15, kb = lane >> 4;
-    const uint32_t at = n * ROWB + kb * 16;
+    const uint32_t at = on ? n * ROWB + kb * 16 : 0;
     if constexpr (S == 4) {
 #pragma unroll
         for (int i = 0; i < 9; i++) __builtin_amdgcn_global_load_lds((global_ptr_t)(w + i * 64 + at), (lds_ptr_t)(lds + i * 1024), 16, 0, 0);
     } else {
-        const uint32_t tail = ((kb >> 1) * 16 + n) * ROWB + 256 + (kb & 1) * 16;
+        const uint32_t tail = on ? ((kb >> 1) * 16 + n) * ROWB + 256 + (kb & 1) * 16 : 0;
 #pragma unroll
         for (int t = 0; t < 2; t++)
 #pragma unroll
@@ -148,7 +152,8 @@ __device__ __forceinline__ void stream_tiles(const char *w0, const char *w1, int
         for (int st = 0; st < STEPS; st++) {
 #pragma unroll
             for (int c = 0; c < CHUNKS; c++) {
-                // the chunk after this one; behind the last of the last unit its first again (loads nobody reads)
+                // the chunk after this one; behind the last of the last unit loads that nobody reads
+                const bool more = c + 1 < CHUNKS || st + 1 < STEPS || u + 1 < units;
                 const char *next;
                 if (c + 1 < CHUNKS) next = chunk_at(st, c + 1);
                 else if (st + 1 < STEPS) next = chunk_at(st + 1, 0);
@@ -158,7 +163,7 @@ __device__ __forceinline__ void stream_tiles(const char *w0, const char *w1, int
                 }
                 const int sn = st + 1 < STEPS ? S * (st + 1) : 0;  // and the super-blocks whose operands it meets
                 __builtin_amdgcn_sched_barrier(0);  // everything read from the slot the next chunk goes to has been used
-                ask_chunk<ROWB, S>(next, ring + ((c + 1) & 1) * kChunk, lane);
+                ask_chunk<ROWB, S>(next, ring + ((c + 1) & 1) * kChunk, lane, more);
                 __builtin_amdgcn_s_waitcnt(0x0F79);  // vmcnt(9), all but those nine: this chunk has landed, and the tokens' operands
                 __builtin_amdgcn_sched_barrier(0);
                 const lds_bytes_t head = (lds_bytes_t)(ring + (c & 1) * kChunk) + n * 16, body = head + kb * 512;
