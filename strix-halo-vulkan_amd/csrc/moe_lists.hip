@@ -54,8 +54,8 @@ typedef const __attribute__((address_space(3))) u32x4_t *lds_quad_t;
 
 // w: the first row of the chunk's (first) tile, at the first of its super-blocks (the same in every lane).  on false: as many
 // loads, all of the chunk's first lines.  A wave's last chunk is waited for by their count; with the whole first chunk asked for
-// again behind it a ninth of what the kernels read was read for nothing: a layer of 66 rows 176 to 168 us, of 150 rows 232 to
-// 223, of 700 rows 410 to 399 (prompts of 65, 150 and 700 rows of 16 layers 3725 to 3679 us, 5000 to 4938, 10793 to 10723).
+// again behind it a ninth of what the kernels read was read for nothing: a layer of 66 rows 171 to 168 us, of 150 rows 226 to
+// 223, of 700 rows 404 to 399 (prompts of 65, 150 and 700 rows of 16 layers 3725 to 3679 us, 5000 to 4938, 10793 to 10723).
 // A branch around the loads costs the gate/up kernel 156 spills.
 template <int ROWB, int S>
 __device__ __forceinline__ void ask_chunk(const char *w, char *lds, int lane, bool on = true) {
