@@ -1,6 +1,7 @@
 // MoE FFN decode step: router logits, softmax/top-k selection, expert-gathered
 // gate/up GEMV with SwiGLU, down GEMV with weighting and combine.  Only the rows of the selected
 // experts (and the shared one) are read from HBM.
+#include <algorithm>
 #include "shv_device.hpp"
 #include "shv_internal.hpp"
 
@@ -939,6 +940,70 @@ __global__ __launch_bounds__(768) void moe_down_slots_kernel(shv_moe_down_args a
     }
 }
 
+// The same for more tokens than one round of those blocks takes (a compute unit holds one, of eleven waves): a block keeps
+// its token's activations and walks a run of passes, the next D on their way, and there are as many blocks as compute units.
+// Bound by HBM as far as its eleven waves hide their products.  us of 5 / 8 / 9 / 12 rows (10 of 512 experts, 2048 x 512; the same
+// bits): rounds of blocks of four passes 12.4 / 14.0 / 17.6 / 19.4, here 10.6 / 12.9 / 14.4 / 17.4 with one pass ahead (two: 11.2 / 13.0 /
+// 14.6 / 18.2); 13 / 16 / 40 / 48 rows: moe_down_kernel, whose waves walk three slots each, 23.5 / 26.9 / 51.4 / 57.8, here with two
+// ahead 18.8 / 21.1 / 44.7 / 51.5 (one: 18.5 / 22.6 / 45.1), its error against float64 0.95 of that kernel's.  49 to 64 rows, 73 us there and
+// 62 here at 64, stay with it as they do with the projections of one 64-row group.
+// grid: (runs of a token, n_tok), (s_hi - s_lo) * 64 threads; a run is at most kWalkRows rows.
+constexpr int kWalkRows = 512;
+template <int K, int D>
+__global__ __launch_bounds__(768) void moe_down_walk_kernel(shv_moe_down_args a, int s_lo, int s_hi) {
+    constexpr int LPR = K / 64, RPP = 64 / LPR, ROWB = K / SHV_Q4K_BLOCK * SHV_Q4K_BYTES, NV = K / 4 / 64;
+    constexpr int kMaxSlots = 12;
+    __shared__ __align__(16) float xs[kMaxSlots][lds_padded(K)];
+    __shared__ __align__(16) float xsum[kMaxSlots][K / 32];
+    __shared__ float part[kMaxSlots][kWalkRows];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int t = blockIdx.y, s = s_lo + wave, ns = a.n_used + 1;
+    const int gi = lane % LPR, rsub = lane / LPR, sb = gi >> 2, g = gi & 3;
+    const int passes = a.n_embd / RPP, first = blockIdx.x * passes / gridDim.x, end = (blockIdx.x + 1) * passes / gridDim.x;
+    int32_t e = 0;
+    if (s < a.n_used) e = load_in_turn(a.topk + static_cast<size_t>(t) * a.n_used + s);
+    const float *act = a.act + (static_cast<size_t>(t) * ns + s) * K;
+    float4 av[NV];
+#pragma unroll
+    for (int j = 0; j < NV; j++) av[j] = *reinterpret_cast<const float4 *>(act + 4 * (lane + 64 * j));
+    const char *base = static_cast<const char *>(a.down_sh);
+    if (s < a.n_used) base = static_cast<const char *>(a.down_exps) + static_cast<size_t>(__builtin_amdgcn_readfirstlane(e)) * a.n_embd * ROWB;
+    base += rsub * ROWB + sb * SHV_Q4K_BYTES;
+    const float wt = a.weights[static_cast<size_t>(t) * ns + s];
+    Q4kLane w[D];
+#pragma unroll
+    for (int p = 0; p < D; p++) w[p].load(base + static_cast<size_t>(min(first + p, end - 1)) * (RPP * ROWB), g);
+    // the wave stages its own slot
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const int c = 4 * (lane + 64 * j);
+        *reinterpret_cast<float4 *>(&xs[wave][lds_slot(c)]) = av[j];
+        const float s8 = sum8_all((av[j].x + av[j].y) + (av[j].z + av[j].w));
+        if ((lane & 7) == 0) xsum[wave][c >> 5] = s8;
+    }
+    __builtin_amdgcn_wave_barrier();  // LDS operations of one wave complete in order
+    float xr[64], xs_lo, xs_hi;
+    load_x_slice_presummed(xs[wave], xsum[wave], gi, xr, xs_lo, xs_hi);
+    const NibbleConsts nc = nibble_consts();
+#pragma unroll 1
+    for (int q = first; q < end; q += D) {
+#pragma unroll
+        for (int p = 0; p < D; p++) {
+            const float acc = group_sum<LPR>(w[p].dot(g, nc, xr, xs_lo, xs_hi));
+            // (a run's last pass again past its end, which nobody stores: with a branch here instead 12 rows take 19.2 us)
+            w[p].load(base + static_cast<size_t>(min(q + p + D, end - 1)) * (RPP * ROWB), g);
+            if (group_sum_owner<LPR>(lane) && q + p < end) part[wave][(q + p - first) * RPP + rsub] = wt * acc;
+        }
+    }
+    __syncthreads();
+    for (int r = tid; r < (end - first) * RPP; r += blockDim.x) {
+        float v = 0.f;
+        for (int i = 0; i < s_hi - s_lo; i++) v += part[i][r];  // slot order
+        const int row = first * RPP + r;
+        a.out[static_cast<size_t>(t) * a.out_stride + row] = v + (a.residual ? a.residual[static_cast<size_t>(t) * a.res_stride + row] : 0.f);
+    }
+}
+
 }  // namespace
 
 int shv_launch_moe_router(shv_ctx *ctx, const shv_moe_router_args *pa) {
@@ -1098,15 +1163,20 @@ int shv_launch_moe_down(shv_ctx *ctx, const shv_moe_down_args *pa) {
     switch (a.ffn) {
         case 512: {
             constexpr int RPP = 64 / (512 / 64);
+            // five rows and more, a wave a slot: a block walks a run of rows, as many blocks as compute units (moe_down_walk_kernel)
+            if (a.n_tok >= 5 && a.n_tok <= 48 && a.n_embd % RPP == 0 && shv_aligned16(a.act)) {
+                const int runs = std::min(std::max(ctx->prop.multiProcessorCount / a.n_tok, (a.n_embd + kWalkRows - 1) / kWalkRows), a.n_embd / RPP);
+                if (a.n_tok <= 12) SHV_LAUNCH(ctx, (moe_down_walk_kernel<512, 1>), dim3(runs, a.n_tok), dim3((s_hi - s_lo) * 64), 0, a, s_lo, s_hi);
+                else SHV_LAUNCH(ctx, (moe_down_walk_kernel<512, 2>), dim3(runs, a.n_tok), dim3((s_hi - s_lo) * 64), 0, a, s_lo, s_hi);
+                break;
+            }
             if (a.n_tok >= ctx->moe_tall_min) SHV_LAUNCH(ctx, (moe_down_kernel<512, 12, 8>), dim3((a.n_embd + RPP * 8 - 1) / (RPP * 8), a.n_tok), block, 0, a, s_lo, s_hi);
-            else if (a.n_tok >= 3 && a.n_tok < 8 && a.n_embd % (4 * RPP) == 0 && shv_aligned16(a.act)) SHV_LAUNCH(ctx, (moe_down_slots_kernel<512, 4>),  // three rows and more: four
+            else if (a.n_tok >= 3 && a.n_tok < 5 && a.n_embd % (4 * RPP) == 0 && shv_aligned16(a.act)) SHV_LAUNCH(ctx, (moe_down_slots_kernel<512, 4>),  // three and four rows: four
                 dim3(a.n_embd / (4 * RPP), a.n_tok), dim3((s_hi - s_lo) * 64), 0, a, s_lo, s_hi);  // passes a wave (a 3-row verification pass 2.48 to 2.43 ms; at two rows 2.14 becomes 2.19)
             else if (a.n_tok >= 2 && a.n_tok < 8 && a.n_embd % (2 * RPP) == 0 && shv_aligned16(a.act)) SHV_LAUNCH(ctx, (moe_down_slots_kernel<512, 2>),  // verification passes: one round of blocks
                 dim3(a.n_embd / (2 * RPP), a.n_tok), dim3((s_hi - s_lo) * 64), 0, a, s_lo, s_hi);
             else if (a.n_tok < 8 && a.n_embd % (1 * RPP) == 0 && shv_aligned16(a.act)) SHV_LAUNCH(ctx, (moe_down_slots_kernel<512, 1>),  // the decode step and verification passes
                 dim3(a.n_embd / (1 * RPP), a.n_tok), dim3((s_hi - s_lo) * 64), 0, a, s_lo, s_hi);
-            else if (a.n_tok >= 8 && a.n_tok <= 12 && a.n_embd % (4 * RPP) == 0 && shv_aligned16(a.act)) SHV_LAUNCH(ctx, (moe_down_slots_kernel<512, 4>),  // eight sequences
-                dim3(a.n_embd / (4 * RPP), a.n_tok), dim3((s_hi - s_lo) * 64), 0, a, s_lo, s_hi);                      // decoded together: a wave a slot, one round of blocks (4.32 to 4.25 ms a pass; two passes a wave 4.31, eight 4.48)
             else if (a.n_tok >= 8) SHV_LAUNCH(ctx, (moe_down_kernel<512, 12, 4>),  // eight sequences decoded together: 5.31 to 5.19 ms a pass
                 dim3((a.n_embd + RPP * 4 - 1) / (RPP * 4), a.n_tok), block, 0, a, s_lo, s_hi);
             else SHV_LAUNCH(ctx, (moe_down_kernel<512, 12, 1>), dim3((a.n_embd + RPP - 1) / RPP, a.n_tok), block, 0, a, s_lo, s_hi);

@@ -596,3 +596,39 @@ def test_router_rows_ride_on_a_projection_of_a_few_rows(ctx, T):
     wt = weights.read(np.float32, T * (used + 1)).reshape(T, used + 1)
     assert O.rel_l2(wt[:, :used], want["weights"]) <= 1e-5 and O.rel_l2(wt[:, used], want["sig"]) <= 1e-5
     assert O.rel_l2(out.read(np.float32, T * H).reshape(T, H), want["out"] + h) <= TOL
+
+
+@pytest.mark.parametrize("T,H,U,residual", [(5, 2048, 10, True), (7, 40, 3, False), (8, 1032, 11, True), (12, 2048, 10, True), (13, 2048, 10, False), (17, 8, 1, True),
+                                            (40, 4104, 10, True), (48, 2048, 10, True)])
+def test_down_projection_in_runs_of_rows(T, H, U, residual):
+    """Five to 48 tokens, a block a run of eight rows and more: runs of one pass, of as many as a block holds, uneven ones.  Bit for
+    bit a token's result alone, which up to twelve rows and past them adds the same products in the same order."""
+    c, E, F = A.Context(0), 16, 512
+    rng = np.random.default_rng(T * H)
+    try:
+        wq, ws = (O.quantize_q4k((rng.standard_normal((n * H, F)) * 0.02).astype(np.float32)) for n in (E, 1))
+        topk = np.argsort(rng.random((T, E)), axis=1)[:, :U].astype(np.int32)
+        act, wts, res = (rng.standard_normal(s).astype(np.float32) for s in ((T, U + 1, F), (T, U + 1), (T, H)))
+        dw, ds = c.upload(wq), c.upload(ws)
+
+        def down(rows):
+            out = c.alloc(len(rows) * H * 4)
+            bufs = [c.upload(np.ascontiguousarray(v[rows])) for v in (act, topk, wts, res)]
+            c.dispatch_multi([A.make_op(A.OP_MOE_DOWN, A.MoeDownArgs(bufs[0].ptr, bufs[1].ptr, bufs[2].ptr, dw.ptr, ds.ptr, bufs[3].ptr if residual else None, out.ptr,
+                                                                     len(rows), H, U, F, H, H, 0, 0, E, None, None, 0, 0))])
+            return out.read(np.float32, len(rows) * H).reshape(len(rows), H)
+
+        got = down(np.arange(T))
+        for t in sorted({0, 1, T // 2, T - 1}):
+            assert np.array_equal(got[t].view(np.uint32), down(np.array([t]))[0].view(np.uint32)), t
+        w64, s64 = O.dequant_q4k(wq, F).astype(np.float64).reshape(E, H, F), O.dequant_q4k(ws, F).astype(np.float64)
+        want = res.astype(np.float64) if residual else np.zeros((T, H))
+        size = np.abs(want)
+        for t in range(T):
+            for s in range(U + 1):
+                m, x = (w64[topk[t, s]] if s < U else s64), act[t, s].astype(np.float64) * float(wts[t, s])
+                want[t] += m @ x
+                size[t] += (np.abs(m) + 2 * np.abs(m).max()) @ np.abs(x)
+        assert (np.abs(got - want) <= 2.0 ** -18 * size).all()  # 64 products a chain and its min term, then some twenty sums
+    finally:
+        c.destroy()
