@@ -298,7 +298,7 @@ __global__ __launch_bounds__(64 * W) void gemm_mid_kernel(shv_gemv_q4k_args a, c
 // A fragment of the next tile asked for when this tile's is multiplied: 98.5 to 90.2 us at 4096 rows, 50.4 to 46.7 at 1531; a
 // die's blocks on neighbouring tiles: to 80.7 and 43.3 (150 rows 25.1 to 24.6).
 // A router row's 64 columns asked for by the lane that multiplies them are sixteen bytes of 64 lines a load, all eight waves' more
-// than L1 holds; by four lanes 64 bytes at a time and exchanged through LDS (the whole router op of 513 x 2048, launches overlapping):
+// than L1 holds; by four lanes 64 bytes at a time and exchanged through LDS (513 x 2048, with its staging):
 // 128 rows 18.6 to 13.7 us, 150 19.1 to 14.5, 512 23.3 to 18.9, 1531 32.8 to 29.0, 4096 60.4 to 56.7.
 template <int R>
 __global__ __launch_bounds__(512) void router_rows_kernel(const float *W, const float *extra_row, int n_rows, int K, int n_tok, const char *staged, float *logits,
@@ -402,7 +402,7 @@ __global__ __launch_bounds__(512) void router_rows_kernel(const float *W, const 
 // logit = factor * sum((h * gamma) . w); xn = h * (factor * gamma) for whoever needs the row.  Rows come and are exchanged as above.
 // No chain is longer than 16 products: against float64 the logits' error is 0.9 of the row kernel's below 128 rows (rms 4.4e-7 and
 // 4.9e-7 of logits of 3.7) and 0.63 of the staged form's.  Of the time, 3 us a block are its 256 KB by way of L1; with sixteen bytes
-// of 16 rows a load it took 7.  The whole op, 513 x 2048, before (row kernel to 127 rows, staged from there) and now: 65 rows 15.0
+// of 16 rows a load it took 7.  513 x 2048, before (row kernel to 127 rows, staged from there) and now: 65 rows 15.0
 // and 7.8 us, 100 19.9 and 8.0, 121 22.4 and 8.1, 150 14.5 and 10.4, 256 16.7 and 10.6, 300 17.9 and 16.0, 384 19.2 and 16.7.
 template <int R, int PER_CU>
 __global__ __launch_bounds__(512, 2 * PER_CU) void router_norm_kernel(shv_moe_router_args a, int tiles) {

@@ -320,17 +320,21 @@ __global__ __launch_bounds__(64) void moe_route_kernel(shv_moe_router_args a) {
 // above spends most of its 4 us in dependent instructions (eight exponentials, eight ballots, the
 // candidates' ranks), which eight waves do side by side.  Same rule: probabilities as the
 // reference forms them, the n_used largest in descending order with ties to the lower index,
-// their sum in slot order clamped at 2^-14.  The threshold is the n_used-th largest of the 16
-// half-wave maxima; the few keys at or above it are compacted and ranked by the first wave.
-// Rows with more than 64 candidates (many equal probabilities) take the one-wave road.
+// their sum in slot order clamped at 2^-14.
+// A chain of steps with two block-wide waits.  Behind the first every wave has the 16 half-wave maxima of the logits: their
+// largest, and the n_used-th largest, whose exponential bounds the selected ones from below (exp(l - max) rises with l; what
+// rounding may make of equal probabilities is a few last bits, which the bound leaves room for).  The few at or above it go
+// to a table as they come; behind the second the first wave divides them by the sum and ranks them.  The same bits with waits for
+// the maximum, the sum, the group maxima, the threshold, the counts and the table: router and selection of 12 / 40 / 150 / 1531 rows
+// 11.6 / 13.0 / 16.1 / 37.4 us, so 10.8 / 12.0 / 14.8 / 36.6 (with a wave a row 14.4 / 15.6 / 18.1 / 38.0).
+// Rows with more than 64 candidates (many equal probabilities), with an infinity or a NaN take the one-wave road.
 constexpr int kRouteBlock = 512;
 __global__ __launch_bounds__(kRouteBlock) void moe_route_block_kernel(shv_moe_router_args a) {
     __shared__ __align__(16) float probs[192];  // the one-wave road's scratch
-    __shared__ float s_max[8], s_sum[8];
-    __shared__ uint32_t s_gm[16];
-    __shared__ uint32_t s_thr;
-    __shared__ int s_cnt[8];
-    __shared__ uint32_t cand_p[64];
+    __shared__ __align__(16) float s_gm[16];
+    __shared__ float s_sum[8];
+    __shared__ int s_total;
+    __shared__ float cand_x[64];
     __shared__ int32_t cand_e[64];
     __shared__ int32_t sel_e[kMaxUsed];
     __shared__ float sel_w[kMaxUsed];
@@ -343,76 +347,72 @@ __global__ __launch_bounds__(kRouteBlock) void moe_route_block_kernel(shv_moe_ro
     const float l = has ? lg[e] : -INFINITY;
     // the shared gate's logit is asked for with the rest
     const float lsh = (tid == kRouteBlock - 1 && a.shared_gate) ? lg[a.n_expert] : 0.f;
-    float mx = wave_max_all(l);
-    if (lane == 0) s_max[wave] = mx;
+    float gm = l;
+    gm = fmaxf(gm, dpp_f32<kDppXor1>(gm));
+    gm = fmaxf(gm, dpp_f32<kDppXor2>(gm));
+    gm = fmaxf(gm, dpp_f32<kDppHalfMirror>(gm));
+    gm = fmaxf(gm, dpp_f32<kDppMirror>(gm));
+    gm = fmaxf(gm, dpp_f32<kDppBcast15>(gm));  // the half-wave's, in its second row of lanes
+    if ((lane & 31) == 31) s_gm[tid >> 5] = gm;
+    if (tid == 0) s_total = 0;
     __syncthreads();
+    float mx, thr;
+    {
+        const float mine = s_gm[lane & 15];
+        int rank = 0;
+        mx = mine;
 #pragma unroll
-    for (int w = 0; w < 8; w++) mx = fmaxf(mx, s_max[w]);
+        for (int j4 = 0; j4 < 4; j4++) {
+            const float4 o = *reinterpret_cast<const float4 *>(s_gm + 4 * j4);
+            const float ov[4] = {o.x, o.y, o.z, o.w};
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                rank += (ov[j] > mine || (ov[j] == mine && 4 * j4 + j < (lane & 15))) ? 1 : 0;
+                mx = fmaxf(mx, ov[j]);
+            }
+        }
+        const unsigned long long at = __ballot(rank == a.n_used - 1);
+        thr = at ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine), __ffsll(at) - 1)) : -INFINITY;
+    }
     const float ex = has ? expf(l - mx) : 0.f;
     const float ws = wave_sum_all(ex);
-    if (lane == 0) s_sum[wave] = ws;
-    // half-wave maxima of the unnormalised exponentials give the same threshold as the
-    // probabilities' would (one common positive factor), but the keys compared below are the
-    // probabilities themselves, as the reference's are
-    __syncthreads();
-    float sum = 0.f;
-#pragma unroll
-    for (int w = 0; w < 8; w++) sum += s_sum[w];
-    const float inv = 1.f / sum;
-    const uint32_t kh = has ? __float_as_uint(ex * inv) : 0u;
-    uint32_t gm = kh;
-#pragma unroll
-    for (int off = 1; off < 32; off <<= 1) {
-        const uint32_t o = static_cast<uint32_t>(__shfl_xor(static_cast<int>(gm), off, 64));
-        gm = o > gm ? o : gm;
-    }
-    if ((lane & 31) == 0) s_gm[tid >> 5] = gm;
-    if (tid == 0) s_thr = 0u;
-    __syncthreads();
-    if (tid < 16) {
-        const uint32_t mine = s_gm[tid];
-        int rank = 0;
-#pragma unroll
-        for (int j = 0; j < 16; j++) rank += (s_gm[j] > mine || (s_gm[j] == mine && j < tid)) ? 1 : 0;
-        if (rank == a.n_used - 1) s_thr = mine;
-    }
-    __syncthreads();
-    const uint32_t thr = s_thr;
-    const bool pred = has && kh >= thr;
+    const bool pred = has && ex >= expf(thr - mx) * (1.f - 0x1p-20f);
     const unsigned long long mask = __ballot(pred);
-    if (lane == 0) s_cnt[wave] = __popcll(mask);
-    __syncthreads();
-    int before = 0, total = 0;
-#pragma unroll
-    for (int w = 0; w < 8; w++) {
-        before += w < wave ? s_cnt[w] : 0;
-        total += s_cnt[w];
+    int base = 0;
+    if (lane == 0) {
+        s_sum[wave] = ws;
+        base = atomicAdd(&s_total, __popcll(mask));
     }
-    if (total > 64 || a.n_expert < 64 || a.n_used > 16) {
-        // uniform over the block: many equal probabilities, or a shape the threshold does not cover
-        if (wave == 0) {
-            route_token<8, false>(lg, a.n_expert, a.n_used, topk, wt, probs);
-            if (lane == 0) wt[a.n_used] = a.shared_gate ? sigmoid_exact(lg[a.n_expert]) : 0.f;
-        }
-        return;
-    }
-    if (pred) {
-        const int pos = before + static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(mask >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mask), 0u)));
-        cand_p[pos] = kh;
+    base = __builtin_amdgcn_readfirstlane(base);
+    const int pos = base + static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(mask >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mask), 0u)));
+    if (pred && pos < 64) {
+        cand_x[pos] = ex;
         cand_e[pos] = e;
     }
     if (tid == kRouteBlock - 1) wt[a.n_used] = a.shared_gate ? sigmoid_exact(lsh) : 0.f;
     __syncthreads();
     if (wave != 0) return;
-    // candidates are in expert order; rank of candidate j = how many come before it (as in route_token)
-    const uint32_t my_p = lane < total ? cand_p[lane] : 0u;
+    float sum = 0.f;
+#pragma unroll
+    for (int w = 0; w < 8; w++) sum += s_sum[w];
+    const int total = s_total;
+    if (total > 64 || total < a.n_used || !(sum < INFINITY) || a.n_expert < 64 || a.n_used > 16) {
+        route_token<8, false>(lg, a.n_expert, a.n_used, topk, wt, probs);
+        if (lane == 0) wt[a.n_used] = a.shared_gate ? sigmoid_exact(lg[a.n_expert]) : 0.f;
+        return;
+    }
+    const float inv = 1.f / sum;
+    // rank of a candidate = how many come before it
+    const uint32_t my_p = lane < total ? __float_as_uint(cand_x[lane] * inv) : 0u;
     const int my_e = lane < total ? cand_e[lane] : 0x7FFFFFFF;
     int rank = 0;
-    for (int j = 0; j < total; j++) {
-        const uint32_t pj = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(my_p), j));
-        const int ej = __builtin_amdgcn_readlane(my_e, j);
-        const int bef = __popcll(__ballot(my_p > pj || (my_p == pj && my_e < ej)));
-        rank = lane == j ? bef : rank;
+    for (int j0 = 0; j0 < total; j0 += 4) {
+#pragma unroll
+        for (int j = j0; j < j0 + 4; j++) {  // (past the table: no probability, no expert)
+            const uint32_t pj = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(my_p), j));
+            const int ej = __builtin_amdgcn_readlane(my_e, j);
+            rank += (pj > my_p || (pj == my_p && ej < my_e)) ? 1 : 0;
+        }
     }
     if (lane < total && rank < a.n_used) {
         sel_e[rank] = my_e;

@@ -632,3 +632,38 @@ def test_down_projection_in_runs_of_rows(T, H, U, residual):
         assert (np.abs(got - want) <= 2.0 ** -18 * size).all()  # 64 products a chain and its min term, then some twenty sums
     finally:
         c.destroy()
+
+
+@pytest.mark.parametrize("T,E,used,copies", [(5, 65, 1, 1), (9, 100, 10, 2), (40, 512, 10, 1), (40, 512, 16, 3), (200, 512, 10, 40), (7, 512, 10, 70), (130, 300, 12, 1)])
+def test_selection_from_the_logits_as_they_are(T, E, used, copies):
+    """The selection of a block a token, from the logits the router left: in order, ties (copies of a router row) to the lower index,
+    more of them than the table holds; weights that sum to one; a token whose logits are not finite leaves the others alone.  Weights to
+    a few roundings of an exponential, its sum and a division."""
+    c, H, rng = A.Context(0), 512, np.random.default_rng(T * E + used)
+    try:
+        router = (rng.standard_normal((E, H)) * 0.08).astype(np.float32)
+        best = int(np.argmax(router.sum(axis=1)))
+        router[rng.permutation(E)[:copies]] = router[best]  # as many of the same row, some of them selected where it is
+        h = rng.standard_normal((T, H)).astype(np.float32)
+        h[0] = 1 + np.abs(h[0])
+        h[T - 2, 5] = np.inf
+        xn, logits, topk, wts = c.alloc(T * H * 4), c.alloc(T * (E + 1) * 4), c.alloc(T * used * 4), c.alloc(T * (used + 1) * 4)
+        gate = c.upload((rng.standard_normal(H) * 0.08).astype(np.float32))
+        args = A.MoeRouterArgs(c.upload(h).ptr, c.upload(np.ones(H, np.float32)).ptr, c.upload(router).ptr, gate.ptr, xn.ptr, logits.ptr, topk.ptr, wts.ptr, T, H, E, used, 1e-6, H, 0)
+        c.dispatch_multi([A.make_op(A.OP_MOE_ROUTER, args)])
+        lg, tk = logits.read(np.float32, T * (E + 1)).reshape(T, E + 1), topk.read(np.int32, T * used).reshape(T, used)
+        wt = wts.read(np.float32, T * (used + 1)).reshape(T, used + 1)
+        for t in range(T):
+            if t == T - 2:
+                continue
+            l64 = lg[t].astype(np.float64)
+            want = np.lexsort((np.arange(E), -l64[:E]))[:used]
+            # logits a last bit apart may be one probability, and then go by index
+            assert (np.abs(l64[tk[t]] - l64[want]) <= 4e-7 * np.maximum(1, np.abs(l64[want]))).all() and len(set(tk[t])) == used, t
+            for a, b in zip(tk[t], tk[t][1:]):
+                assert l64[a] > l64[b] or l64[b] - l64[a] <= 4e-7 * max(1, abs(l64[a])) and (lg[t, a] != lg[t, b] or a < b)
+            p = np.exp(l64[tk[t]] - l64[:E].max())
+            assert np.abs(wt[t, :used] - p / p.sum()).max() <= 2e-6
+            assert abs(wt[t, used] - 1 / (1 + np.exp(-l64[E]))) <= 2e-6
+    finally:
+        c.destroy()
