@@ -78,6 +78,48 @@ struct GemvBatch {
     }
 };
 
+// The block's best (value, row) of its lanes' (bv, bi) left for all; the block that arrives last names the best of all.
+__device__ __forceinline__ void finish_amax(const shv_gemv_q4k_args &a, float bv, int bi, float *amax_val, int32_t *amax_idx, int32_t *amax_counter) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = a.n;
+    __shared__ float sv[kWavesPerBlock];
+    __shared__ int si[kWavesPerBlock];
+    __shared__ int is_last;
+    const int nblk = static_cast<int>(gridDim.x);
+    amax_wave(bv, bi);
+    if (lane == 0) { sv[wave] = bv; si[wave] = bi; }
+    __syncthreads();
+    if (tid == 0) {
+#pragma unroll
+        for (int w = 1; w < kWavesPerBlock; w++)
+            if (amax_better(sv[w], si[w], bv, bi)) { bv = sv[w]; bi = si[w]; }
+        store_agent(amax_val + blockIdx.x, bv);
+        store_agent(amax_idx + blockIdx.x, bi);
+    }
+    if (!arrive_last(amax_counter, nblk, &is_last)) return;
+    bv = -INFINITY;
+    bi = n;
+    for (int b = tid; b < nblk; b += kBlock) {
+        const float v = load_agent(amax_val + b);
+        const int i = load_agent(amax_idx + b);
+        if (amax_better(v, i, bv, bi)) { bv = v; bi = i; }
+    }
+    amax_wave(bv, bi);
+    if (lane == 0) { sv[wave] = bv; si[wave] = bi; }
+    __syncthreads();
+    if (tid == 0) {
+#pragma unroll
+        for (int w = 1; w < kWavesPerBlock; w++)
+            if (amax_better(sv[w], si[w], bv, bi)) { bv = sv[w]; bi = si[w]; }
+        if (bi >= n) bi = 0;  // a row of NaN has no element that is `>` -inf: the reference returns 0 there
+        a.amax_best[0] = bi;
+        if (a.amax_ids && a.amax_pos) {
+            const int p = a.amax_pos[0] + (a.amax_advance > 0 ? a.amax_advance : 1);
+            a.amax_ids[p] = bi;
+            a.amax_pos[0] = p;
+        }
+    }
+}
+
 // The grid's waves share the passes round-robin: wave w takes passes w, w + W, w + 2W, ... (W waves
 // in the grid), so at any moment the chip streams one contiguous window of rows and no wave has
 // more than one pass more than another.  U passes are loaded together; n_batches batches a wave.
@@ -248,45 +290,96 @@ __global__ __launch_bounds__(kBlock) void gemv_q4k_kernel(shv_gemv_q4k_args a, i
             B.template compute<AMAX>(a, g, lane, nc, xr, xs_lo, xs_hi, y_off, t0, &bv, &bi);
         }
     }
-    if constexpr (AMAX) {
-        __shared__ float sv[kWavesPerBlock];
-        __shared__ int si[kWavesPerBlock];
-        __shared__ int is_last;
-        const int nblk = static_cast<int>(gridDim.x);
-        amax_wave(bv, bi);
-        if (lane == 0) { sv[wave] = bv; si[wave] = bi; }
-        __syncthreads();
-        if (tid == 0) {
+    if constexpr (AMAX) finish_amax(a, bv, bi, amax_val, amax_idx, amax_counter);
+}
+
+
+// ---- one row against a matrix of many rounds, and its arg-max (the vocabulary projection of a decode step) ----
+// gemv_q4k_kernel's arithmetic, bit for bit, over weights that come by way of LDS: rows are one piece of memory, so a chunk of
+// four is loads of a kilobyte, every line once, straight into the wave's own ring of two, where lanes that fetch header and payload
+// of their group come back to a line eight times; and a lane's registers hold no weights on their way.  Bound by HBM and, near it, by the
+// dot products' instructions.  151936 x 2048, 3 blocks of four waves a compute unit: 43.7 to 39.4 us (of eight waves, a block: 41.2;
+// chunks of eight rows 44.8), 65536 rows 26.0 to 23.5.  Without the arg-max, 3.3 us of that, the two are level (37.8 and 36.2; 17.8
+// and 18.2), and gemv_q4k_kernel is the one that runs.  (A counter an eighth of the blocks shares, with a second level, does not shorten it.)
+typedef const __attribute__((address_space(1))) void *stream_global_t;
+typedef __attribute__((address_space(3))) void *stream_lds_t;
+typedef const __attribute__((address_space(3))) uint32_t __attribute__((ext_vector_type(4))) *stream_quad_t;
+
+__global__ __launch_bounds__(kBlock) void gemv_stream_kernel(shv_gemv_q4k_args a, float *amax_val, int32_t *amax_idx, int32_t *amax_counter) {
+    constexpr int K = 2048, ROWS = 4, LPR = K / 64, RPP = 64 / LPR, ROWB = K / SHV_Q4K_BLOCK * SHV_Q4K_BYTES, CHUNK = ROWS * ROWB, LOADS = (CHUNK + 1023) / 1024;
+    __shared__ __align__(16) char rings[kWavesPerBlock][2 * CHUNK];
+    __shared__ __align__(16) float xs[lds_padded(K)];
+    __shared__ float red[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int gi = lane % LPR, rsub = lane / LPR, sb = gi >> 2, g = gi & 3;
+    const int chunks = (a.n + ROWS - 1) / ROWS, stride = gridDim.x * kWavesPerBlock;
+    char *ring = rings[wave];
+    // a chunk's rows are one piece of memory: 1 KB a load; past the matrix's end its last bytes again
+    const auto ask = [&](int c, char *to) {
+        const char *w = static_cast<const char *>(a.w) + static_cast<size_t>(c) * CHUNK;
+        const int last = (a.n - c * ROWS < ROWS ? a.n - c * ROWS : ROWS) * ROWB - 16;
 #pragma unroll
-            for (int w = 1; w < kWavesPerBlock; w++)
-                if (amax_better(sv[w], si[w], bv, bi)) { bv = sv[w]; bi = si[w]; }
-            store_agent(amax_val + blockIdx.x, bv);
-            store_agent(amax_idx + blockIdx.x, bi);
-        }
-        if (!arrive_last(amax_counter, nblk, &is_last)) return;
-        bv = -INFINITY;
-        bi = n;
-        for (int b = tid; b < nblk; b += kBlock) {
-            const float v = load_agent(amax_val + b);
-            const int i = load_agent(amax_idx + b);
-            if (amax_better(v, i, bv, bi)) { bv = v; bi = i; }
-        }
-        amax_wave(bv, bi);
-        if (lane == 0) { sv[wave] = bv; si[wave] = bi; }
-        __syncthreads();
-        if (tid == 0) {
+        for (int i = 0; i < LOADS; i++)
+            if ((i + 1) * 1024 <= CHUNK || lane < (CHUNK - i * 1024) / 16)
+                __builtin_amdgcn_global_load_lds((stream_global_t)(w + min(i * 1024 + lane * 16, last)), (stream_lds_t)(to + i * 1024), 16, 0, 0);
+    };
+    int c = blockIdx.x * kWavesPerBlock + wave;
+    // the row, as gemv_q4k_kernel stages it; asked for first: loads come back in order
+    {
+        const float *gamma = a.prologue == SHV_PRO_RMSNORM ? a.gamma : a.x;
+        float v[K / kBlock], gm[K / kBlock];
 #pragma unroll
-            for (int w = 1; w < kWavesPerBlock; w++)
-                if (amax_better(sv[w], si[w], bv, bi)) { bv = sv[w]; bi = si[w]; }
-            if (bi >= n) bi = 0;  // a row of NaN has no element that is `>` -inf: the reference returns 0 there
-            a.amax_best[0] = bi;
-            if (a.amax_ids && a.amax_pos) {
-                const int p = a.amax_pos[0] + (a.amax_advance > 0 ? a.amax_advance : 1);
-                a.amax_ids[p] = bi;
-                a.amax_pos[0] = p;
+        for (int i = 0; i < K / kBlock; i++) {
+            v[i] = a.x[tid + i * kBlock];
+            gm[i] = gamma[tid + i * kBlock];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (c < chunks) ask(c, ring);
+        if (c + stride < chunks) ask(c + stride, ring + CHUNK);
+        if (a.prologue == SHV_PRO_RMSNORM) {
+            float ss = 0.f;
+#pragma unroll
+            for (int i = 0; i < K / kBlock; i++) ss = fmaf(v[i], v[i], ss);
+            ss = wave_sum_all(ss);
+            if (lane == 0) red[wave] = ss;
+            __syncthreads();
+            ss = red[0] + red[1] + red[2] + red[3];
+            const float scale = 1.f / sqrtf(ss / static_cast<float>(K) + a.eps);
+#pragma unroll
+            for (int i = 0; i < K / kBlock; i++) v[i] = v[i] * scale * gm[i];
+        }
+#pragma unroll
+        for (int i = 0; i < K / kBlock; i++) xs[lds_slot(tid + i * kBlock)] = v[i];
+    }
+    __syncthreads();
+    float xr[64], xs_lo, xs_hi;
+    load_x_slice(xs, gi, xr, xs_lo, xs_hi);
+    const NibbleConsts nc = nibble_consts();
+    float bv = -INFINITY;
+    int bi = a.n;
+    const int at = rsub * ROWB + sb * SHV_Q4K_BYTES;
+#pragma unroll 1
+    for (int b = 0; c < chunks; c += stride, b ^= 1) {
+        char *slot = ring + b * CHUNK;
+        __builtin_amdgcn_sched_barrier(0);
+        if (c + stride < chunks) __builtin_amdgcn_s_waitcnt(0x0F70 | LOADS);  // all but the next chunk's loads
+        else __builtin_amdgcn_s_waitcnt(0x0F70);
+        __builtin_amdgcn_sched_barrier(0);
+        const auto from = (const __attribute__((address_space(3))) char *)(slot) + at;
+#pragma unroll
+        for (int p = 0; p < ROWS / RPP; p++) {
+            const auto h = *(stream_quad_t)(from + p * RPP * ROWB), q0 = *(stream_quad_t)(from + p * RPP * ROWB + 16 + g * 32), q1 = *(stream_quad_t)(from + p * RPP * ROWB + 32 + g * 32);
+            const float r = group_sum<LPR>(q4k_group_dot(make_uint4(h.x, h.y, h.z, h.w), make_uint4(q0.x, q0.y, q0.z, q0.w), make_uint4(q1.x, q1.y, q1.z, q1.w), g, nc, xr, xs_lo, xs_hi));
+            const int row = c * ROWS + p * RPP + rsub;
+            if (row < a.n && group_sum_owner<LPR>(lane)) {
+                a.y[row] = r;
+                if (amax_better(r, row, bv, bi)) { bv = r; bi = row; }
             }
         }
+        __builtin_amdgcn_sched_barrier(0);  // what has been multiplied has been read
+        if (c + 2 * stride < chunks) ask(c + 2 * stride, slot);
     }
+    finish_amax(a, bv, bi, amax_val, amax_idx, amax_counter);
 }
 
 
@@ -790,6 +883,13 @@ int launch_nt(shv_ctx *ctx, const shv_gemv_q4k_args &a, dim3 grid, dim3 block, s
     }
 }
 
+int launch_stream(shv_ctx *ctx, const shv_gemv_q4k_args &a) {
+    const int blocks = ctx->prop.multiProcessorCount * 3;
+    SHV_REQUIRE(blocks <= shv_ctx::kGemvAmaxBlocks && ctx->gemv_amax_val && ctx->gemv_amax_idx, "gemv_q4k: arg-max over %d blocks", blocks);
+    SHV_LAUNCH(ctx, gemv_stream_kernel, dim3(blocks), dim3(kBlock), 0, a, ctx->gemv_amax_val, ctx->gemv_amax_idx, ctx->counters + shv_ctx::kCounterGemvAmax);
+    return SHV_OK;
+}
+
 template <int K>
 int launch_k(shv_ctx *ctx, const shv_gemv_q4k_args &a) {
     constexpr int RPP = 64 / (K / 64);
@@ -813,6 +913,8 @@ int launch_k(shv_ctx *ctx, const shv_gemv_q4k_args &a) {
     // A matrix of many rounds (the vocabulary projection: 37) is a stream, not a latency: one pass
     // at a time leaves registers for a third wave per SIMD, which hides more of the arithmetic
     // behind the loads (42 -> 36 us for 175 MB).
+    if (K == 2048 && iters >= 8 && a.n_tok == 1 && a.amax_best && !a.residual && !a.y_flat && a.ring_slots == 0 && (a.prologue == SHV_PRO_NONE || a.prologue == SHV_PRO_RMSNORM))
+        return launch_stream(ctx, a);
     if (iters >= 8 && a.n_tok == 1) {
         blocks = static_cast<long long>(ctx->prop.multiProcessorCount) * 3;
         waves = blocks * kWavesPerBlock;

@@ -142,6 +142,33 @@ def test_vocabulary_projection_names_the_next_token_itself(ctx):
         ctx.enqueue(A.OP_GEMV_Q4K, g)
 
 
+@pytest.mark.parametrize("n,prologue", [(28672, A.PRO_RMSNORM), (28673, A.PRO_RMSNORM), (28674, A.PRO_NONE), (36867, A.PRO_NONE), (65536, A.PRO_RMSNORM)])
+def test_a_projection_of_many_rounds_names_its_best(ctx, n, prologue):
+    """The launch that streams its rows in chunks of four, and the one below its line: matrices that end inside a chunk, the best row among
+    the last ones; the plain launch's rows bit for bit and nothing past them."""
+    rng, k = np.random.default_rng(n), 2048
+    f, w = ctx.alloc(n * k * 4), ctx.alloc(n * (k // 256 * 144))
+    ctx.enqueue(A.OP_FILL_NORMAL, A.FillNormalArgs(f.ptr, n * k, n, 0.0, 0.02))
+    ctx.enqueue(A.OP_QUANTIZE_Q4K, A.QuantizeQ4KArgs(f.ptr, w.ptr, n, k))
+    ctx.sync()
+    f.free()
+    rb = k // 256 * 144
+    last = O.dequant_q4k(w.read(np.uint8, rb, (n - 1) * rb).reshape(1, rb), k)[0]
+    gamma = (1 + 0.1 * rng.standard_normal(k)).astype(np.float32)
+    dg, y0, y1, best = ctx.upload(gamma), ctx.alloc(n * 4), ctx.upload(np.full(n + 64, -7.0, np.float32)), ctx.alloc(4)
+    for x in (rng.standard_normal(k).astype(np.float32), (last * 50).astype(np.float32)):
+        dx = ctx.upload(x)
+        ctx.gemv_q4k(w, dx, y0, n, k, prologue=prologue, gamma=dg)
+        g = A.gemv_args(w, dx, y1, n, k, 1, prologue, dg)
+        g.amax_best = best.ptr
+        ctx.enqueue(A.OP_GEMV_Q4K, g)
+        plain, got = y0.read(np.float32, n), y1.read(np.float32, n + 64)
+        assert np.array_equal(plain.view(np.uint32), got[:n].view(np.uint32)) and (got[n:] == -7.0).all()
+        assert best.read(np.int32, 1)[0] == int(np.argmax(plain))
+    assert int(np.argmax(plain)) == n - 1
+    w.free()
+
+
 def test_small_uploads_that_do_not_wait_arrive_in_order(ctx):
     """shv_upload_async: a pass's control words go through pinned staging and the call returns at once.  What a
     later download or op of the context sees is what blocking uploads would have left: several hundred of them in a
