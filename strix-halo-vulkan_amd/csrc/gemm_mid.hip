@@ -286,6 +286,110 @@ __global__ __launch_bounds__(64 * W) void gemm_mid_kernel(shv_gemv_q4k_args a, c
     }
 }
 
+// ------------------------------------------- few rows against a matrix of many rounds ---------
+// The vocabulary projection of five to sixteen rows.  A block of eight waves, two a compute unit, walks groups of 16 weight rows: a
+// group's 18 KB go by way of LDS, the two after it on their way while it is multiplied, and a wave keeps its 256 columns of the one
+// tile of activations in registers.  Sums and their order are gemm_mid_kernel's.
+// Bound by HBM as far as two blocks out of step hide each other's waits (one of 32 rows a group: 52 us).  151936 x 2048, us of 5 / 8 / 9 / 16 rows
+// with the staging launch: gemm_q4k.hip's walk to eight rows and gemm_mid_kernel from nine 74.8 / 73.6 / 64.2 / 66.9, here 46.0 / 45.0 / 45.2 / 47.2, error
+// against float64 0.95 and the same.  A group loaded 64 bytes of sixteen rows at a time, rows' pieces side by side, took 2 us more.
+// Two to four rows gain 7 us alone (52 to 45) and nothing in a pass, gemv_mrows.hip needing no staging launch: they stay there.
+constexpr int kFewRows = 16, kFewSlots = 3, kFewSlot = kFewRows * 8 * SHV_Q4K_BYTES, kFewLoads = kFewSlot / 1024;
+constexpr size_t kFewLds = static_cast<size_t>(kFewSlots) * kFewSlot + 8 * 1024;
+typedef const __attribute__((address_space(1))) void *few_global_t;
+typedef __attribute__((address_space(3))) void *few_lds_t;
+typedef const __attribute__((address_space(3))) char *few_bytes_t;
+typedef const __attribute__((address_space(3))) u32x4_t *few_quad_t;
+
+__global__ __launch_bounds__(512, 4) void gemm_few_kernel(shv_gemv_q4k_args a, const char *staged) {
+    constexpr int W = 8, ROWB = W * SHV_Q4K_BYTES, PIECES = ROWB / 16, NL = (kFewLoads + W - 1) / W;
+    extern __shared__ __align__(16) char smem[];  // the groups' weights, then the waves' sums
+    float *cpart = reinterpret_cast<float *>(smem + kFewSlots * kFewSlot);
+    const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, kb = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const NibbleMasks nc = nibble_masks();
+    const int groups = (a.n + kFewRows - 1) / kFewRows, step = gridDim.x;
+    // a group is one piece of memory, a kilobyte a load, but that a row's pieces of 16 bytes come turned by nine places a row: sixteen
+    // rows' pieces of one number are in different banks
+    int from_row[NL];
+    uint32_t from[NL];
+#pragma unroll
+    for (int i = 0; i < NL; i++) {
+        const int at = (wave + W * i) * 64 + lane, row = at / PIECES;
+        from_row[i] = row;
+        from[i] = row * ROWB + (at % PIECES + 2 * PIECES - 9 * (row % kFewRows)) % PIECES * 16;
+    }
+    const auto ask = [&](int group, char *slot) {
+        const char *w = static_cast<const char *>(a.w) + static_cast<size_t>(group) * kFewSlot;
+        const int last = a.n - 1 - group * kFewRows;  // rows past it are it again: what they give is not stored
+#pragma unroll
+        for (int i = 0; i < NL; i++)
+            if (wave + W * i < kFewLoads)
+                __builtin_amdgcn_global_load_lds((few_global_t)(w + (from[i] - max(from_row[i] - last, 0) * ROWB)), (few_lds_t)(slot + (wave + W * i) * 1024), 16, 0, 0);
+    };
+    const auto piece = [&](int p) { return (n * PIECES + (p + 9 * n) % PIECES) * 16; };
+    const int head_at = piece(9 * wave), q0_at = piece(9 * wave + 1 + 2 * kb), q1_at = piece(9 * wave + 2 + 2 * kb);
+    int group = blockIdx.x;
+    // the pass's rows, then the first groups: loads come back in order
+    half8_t f[8][2];
+    const char *frag = staged + wave * kMidSb + lane * 16;
+#pragma unroll
+    for (int v = 0; v < 8; v++)
+#pragma unroll
+        for (int p = 0; p < 2; p++) f[v][p] = *reinterpret_cast<const half8_t *>(frag + (v * 2 + p) * kMidFrag);
+    const bf16x8_t sx = *reinterpret_cast<const bf16x8_t *>(staged + mid_sums_offset(1, a.k) + wave * kMidSums + lane * 16);
+    // this thread's output: row of a group, and of the pass
+    const int o_row = (tid >> 2) & 15, o_tok = 4 * (tid >> 6 & 3) + (tid & 3);
+    const bool mine = tid < 256 && o_tok < a.n_tok;
+    const size_t to = reinterpret_cast<const size_t *>(staged + mid_rows_offset(1, a.k))[o_tok];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < kFewSlots; k++)
+        if (group + k * step < groups) ask(group + k * step, smem + k * kFewSlot);
+#pragma unroll 1
+    for (int b = 0; group < groups; group += step, b = b + 1 == kFewSlots ? 0 : b + 1) {
+        char *slot = smem + b * kFewSlot;
+        __builtin_amdgcn_sched_barrier(0);
+        // this group has landed: all but what this wave has asked for of the ones after it
+        constexpr int behind = kFewSlots - 1, whole = kFewLoads / W;
+        static_assert(behind * (whole + 1) < 16, "vmcnt");
+        if (group + behind * step >= groups) __builtin_amdgcn_s_waitcnt(0x0F70);
+        else if (wave < kFewLoads % W) __builtin_amdgcn_s_waitcnt(0x0F70 | behind * (whole + 1));
+        else __builtin_amdgcn_s_waitcnt(0x0F70 | behind * whole);
+        lds_barrier();
+        const few_bytes_t rows = (few_bytes_t)(slot);
+        const u32x4_t h = *(few_quad_t)(rows + head_at), q0 = *(few_quad_t)(rows + q0_at), q1 = *(few_quad_t)(rows + q1_at);
+        uint32_t sc, mn;
+        q4k_group_scale_min(make_uint4(h.x, h.y, h.z, h.w), kb, sc, mn);
+        float4_t acc = {0.f, 0.f, 0.f, 0.f}, y;
+#pragma unroll
+        for (int v = 0; v < 8; v++) {
+            const u32x4_t &x = (v & 2) ? q1 : q0;
+            const uint32_t d0 = (v & 1) ? x.z : x.x, d1 = (v & 1) ? x.w : x.y;
+            const half8_t w8 = v < 4 ? weights8<false>(d0, d1, sc & 0xFFu, nc) : weights8<true>(d0, d1, sc >> 8, nc);
+#pragma unroll
+            for (int p = 0; p < 2; p++) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(f[v][p], w8, acc, 0, 0, 0);
+        }
+        const uint32_t am = bf16_pair(mn & 0xFFu, mn >> 8);
+        const u32x4_t m3 = {am, am, am, 0u};  // the same two mins against each part
+        const float4_t cm = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sx, __builtin_bit_cast(bf16x8_t, m3), float4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        const float d = f16_bits_to_f32(h.x), dmin = f16_bits_to_f32(h.x >> 16);
+#pragma unroll
+        for (int j = 0; j < 4; j++) y[j] = fmaf(d, acc[j], -dmin * cm[j]);
+        *reinterpret_cast<float4_t *>(cpart + (wave * 64 + lane) * 4) = y;
+        lds_barrier();
+        const int row = group * kFewRows + o_row;
+        if (mine && row < a.n) {
+            float v = cpart[tid];
+#pragma unroll
+            for (int w = 1; w < W; w++) v += cpart[w * 256 + tid];
+            a.y[to + row] = v + (a.residual ? a.residual[static_cast<size_t>(o_tok) * a.y_stride + row] : 0.f);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (group + kFewSlots * step < groups) ask(group + kFewSlots * step, slot);
+    }
+}
+
 // ------------------------------------------------------------ the router of a long pass -------
 // logits[t][e] = xn[t] . W[e] for float32 rows W (the router's experts and, as one more row, the shared expert's gate)
 // against the staged rows of a pass, in the same way: a block keeps 16 R router rows in registers.  A float32 weight enters
@@ -571,6 +675,24 @@ int launch_stage(shv_ctx *ctx, const shv_gemv_q4k_args &a, int tiles, float *x_o
 // Past 512 gemm_long.hip's blocks read less from L2.
 }  // namespace
 
+// A pass of five to sixteen rows against a matrix of eight groups of rows a block and more (the caller has seen to shv_gemm_q4k_covers).
+bool shv_gemm_few_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a) {
+    return ctx->gemm_stage && a.k == 2048 && a.n_tok >= 5 && a.n_tok <= 16 && !a.fold && !a.amax_best && !a.y_flat && a.n >= 8 * kFewRows * 2 * ctx->prop.multiProcessorCount &&
+           (a.prologue != SHV_PRO_GATED_NORM || 256 % a.head_dim == 0);
+}
+
+int shv_launch_gemm_few(shv_ctx *ctx, const shv_gemv_q4k_args &a) {
+    static std::atomic<bool> raised{false};
+    if (!raised.load(std::memory_order_acquire)) {
+        SHV_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_few_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kFewLds)));
+        raised.store(true, std::memory_order_release);
+    }
+    const int rc = launch_stage(ctx, a, 1, nullptr);
+    if (rc != SHV_OK) return rc;
+    SHV_LAUNCH(ctx, gemm_few_kernel, dim3(2 * ctx->prop.multiProcessorCount), dim3(512), kFewLds, a, static_cast<const char *>(ctx->gemm_stage));
+    return SHV_OK;
+}
+
 bool shv_gemm_mid_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a) {
     if (!ctx->gemm_stage || (a.k != 2048 && a.k != 4096) || a.n_tok < 9 || a.n_tok > 512) return false;
     if (a.n_tok > 48 && a.n_tok <= 64) return false;
@@ -579,6 +701,7 @@ bool shv_gemm_mid_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a) {
 }
 
 int shv_launch_gemm_mid(shv_ctx *ctx, const shv_gemv_q4k_args &a) {
+    if (shv_gemm_few_covers(ctx, a)) return shv_launch_gemm_few(ctx, a);
     const int tiles = (a.n_tok + 15) / 16;
     const int rc = launch_stage(ctx, a, tiles, nullptr);
     if (rc != SHV_OK) return rc;

@@ -469,7 +469,7 @@ bool shv_gemv_mrows_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a) {
     const int sl = a.seq_len > 0 ? a.seq_len : a.n_tok;
     if (a.n_tok % sl != 0) return false;
     // a matrix of many rounds of the chip (the vocabulary projection) is a stream: from five rows on the tiled
-    // kernel, which walks it with every wave resident, is ahead (76 against 110 us at eight rows)
+    // kernels, which walk it with every wave resident, are ahead (45 to 76 against 110 us at eight rows)
     if (a.n_tok >= 5 && (a.n + 15) / 16 >= 8 * ctx->prop.multiProcessorCount) return false;
     return true;
 }

@@ -992,6 +992,8 @@ int shv_launch_gemv_q4k(shv_ctx *ctx, const shv_gemv_q4k_args *pa) {
             default: return shv_set_error(SHV_E_INVALID, "gemv_q4k: k = %d; built for 512, 1024, 2048 and 4096", a.k);
         }
     }
+    // five to eight rows against a matrix of many rounds: a stream (nine and more come to it by way of shv_launch_gemm_mid)
+    if (a.n_tok >= 5 && a.n_tok <= 8 && !ctx->mfma_rows_forced && !ctx->mrows_off && shv_gemm_q4k_covers(a) && shv_gemm_few_covers(ctx, a)) return shv_launch_gemm_few(ctx, a);
     // two to eight rows: every weight formed once for all of them, the products on the matrix cores; 4096 columns
     // wide, up to four rows are quicker side by side in the one-row kernel's shape (6.7 against
     // 8.0 us for three rows of a 2048 x 4096 output projection: a block there stages 16 K columns a row)

@@ -160,6 +160,8 @@ int shv_launch_gemm_mid(shv_ctx *ctx, const shv_gemv_q4k_args &a);
 bool shv_gemm_long_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a);
 int shv_launch_gemm_long(shv_ctx *ctx, const shv_gemv_q4k_args &a);
 int shv_launch_gemm_q4k(shv_ctx *ctx, const shv_gemv_q4k_args &a);
+bool shv_gemm_few_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a);
+int shv_launch_gemm_few(shv_ctx *ctx, const shv_gemv_q4k_args &a);
 bool shv_router_rows_covers(const shv_ctx *ctx, const shv_moe_router_args &a);
 int shv_launch_router_rows(shv_ctx *ctx, const shv_moe_router_args &a);
 int shv_launch_dequant_q4k(shv_ctx *ctx, const shv_dequant_q4k_args *a);

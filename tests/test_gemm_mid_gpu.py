@@ -96,6 +96,38 @@ def test_gates_of_a_pass(rows, k, head_dim, n_seq):
         ctx.destroy()
 
 
+@pytest.mark.parametrize("n,rows", [(65536, 5), (65537, 6), (65551, 8), (65536 + 8191, 9), (70000, 16), (65535, 5), (65536, 4)])
+def test_few_rows_against_a_matrix_of_many_rounds(n, rows):
+    """The walk over groups of sixteen weight rows: the least of them, a last group of one row and of fifteen, blocks with one group more
+    than others, a matrix a row short of it and a pass; a norm folded in, residual rows, and a ring to write that wraps."""
+    k, rng = 2048, np.random.default_rng(n + rows)
+    ctx = A.Context(0)
+    try:
+        part = O.quantize_q4k((rng.standard_normal((4099, k)) * 0.02).astype(np.float32)).reshape(4099, -1)
+        w64 = O.dequant_q4k(part, k).astype(np.float64).reshape(4099, k)
+        of = np.arange(n) % 4099
+        dw = ctx.upload(np.ascontiguousarray(part[of]))
+        x = (rng.standard_normal((rows, k)) * rng.uniform(0.01, 30.0, size=(rows, 1))).astype(np.float32)
+        gamma = (1 + 0.1 * rng.standard_normal(k)).astype(np.float32)
+        x64, res = x.astype(np.float64), rng.standard_normal((rows, n)).astype(np.float32)
+        want = ((x64 / np.sqrt((x64 * x64).mean(axis=1, keepdims=True) + 1e-6) * gamma) @ w64.T)[:, of] + res
+        dy = ctx.upload(np.concatenate([res.ravel(), np.full(64, -7.0, np.float32)]))
+        ctx.gemv_q4k(dw, ctx.upload(x), dy, n, k, n_tok=rows, prologue=A.PRO_RMSNORM, gamma=ctx.upload(gamma), residual=dy)
+        got = dy.read(np.float32, rows * n + 64)
+        assert (got[rows * n:] == -7.0).all()
+        got = got[:rows * n].reshape(rows, n)
+        assert (np.linalg.norm(got - want, axis=1) <= 1e-5 * np.linalg.norm(want, axis=1)).all()
+        assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max()
+        slots, pos = rows + 1, np.array([rows - 1], np.int32)
+        ring = ctx.upload(np.full((slots, n), -7.0, np.float32))
+        ctx.gemv_q4k(dw, ctx.upload(x), ring, n, k, n_tok=rows, pos=ctx.upload(pos), seq_len=rows, ring_slots=slots, ring_stride=n)
+        got, at, want = ring.read(np.float32, slots * n).reshape(slots, n), (pos[0] + np.arange(rows)) % slots, (x64 @ w64.T)[:, of]
+        assert (np.linalg.norm(got[at] - want, axis=1) <= 1e-5 * np.linalg.norm(want, axis=1)).all()
+        assert (np.delete(got, at, axis=0) == -7.0).all()
+    finally:
+        ctx.destroy()
+
+
 @pytest.mark.parametrize("rows,H,E", [(128, 256, 7), (129, 1024, 31), (145, 2304, 64), (2001, 512, 32)])
 def test_router_logits_of_a_long_pass(rows, H, E):
     """Columns of one super-block, of fewer than the block's waves and of more; router rows (the experts and the shared
