@@ -145,6 +145,11 @@ __global__ __launch_bounds__(256) void gemm_mid_stage_kernel(shv_gemv_q4k_args a
         reinterpret_cast<size_t *>(staged + mid_rows_offset(tiles, K))[t] = !on ? 0 : a.ring_slots > 0 && !a.z_ring ? ring_row * a.ring_stride : static_cast<size_t>(t) * a.y_stride;
 }
 
+typedef const __attribute__((address_space(1))) void *mid_global_t;
+typedef __attribute__((address_space(3))) void *mid_lds_t;
+typedef const __attribute__((address_space(3))) char *mid_bytes_t;
+typedef const __attribute__((address_space(3))) u32x4_t *mid_quad_t;
+
 // A barrier behind which the waves' LDS writes are seen; fragments and stores in flight stay in flight.
 __device__ __forceinline__ void lds_barrier() {
     asm volatile("" ::: "memory");
@@ -164,20 +169,19 @@ __global__ __launch_bounds__(64 * W) void gemm_mid_kernel(shv_gemv_q4k_args a, c
     const int row0 = blockIdx.x * (16 * R), tile0 = blockIdx.y * per_chunk;
     const int tile_end = tile0 + per_chunk < tiles ? tile0 + per_chunk : tiles;
     const NibbleMasks nc = nibble_masks();
-    // the wave's weights first: header and this lane's group of every super-block of every row
-    uint4 hdr[S][R], q[S][R][2];
+    // The wave's weights first, its columns of every row one piece of 144 S bytes, by way of a corner of LDS of its own: asked for by the
+    // lanes that form them they are sixteen bytes of 64 lines a load, 64 cycles of the cache's address unit each, and 12 loads for 9 (a
+    // pass of 16 layers, so and now: 9 rows 1352 and 1337 us, 40 rows 2924 and 2882, 150 rows 4918 and 4879, 12 sequences 1620 and 1606).
+    constexpr int PIECES = 9 * S, ASKED = 16 * R * PIECES;
+    char *corner = smem + 2 * W * R * 1024 + wave * (ASKED * 16);
     const char *wbase = static_cast<const char *>(a.w) + static_cast<size_t>(row0) * ROWB + wave * (S * SHV_Q4K_BYTES);
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        const int rr = row0 + 16 * r + n < a.n ? 16 * r + n : a.n - 1 - row0;
-        const char *p = wbase + static_cast<uint32_t>(rr) * ROWB;
-#pragma unroll
-        for (int s = 0; s < S; s++) {
-            hdr[s][r] = load_stream16(p + s * SHV_Q4K_BYTES);
-            q[s][r][0] = load_stream16(p + s * SHV_Q4K_BYTES + 16 + kb * 32);
-            q[s][r][1] = load_stream16(p + s * SHV_Q4K_BYTES + 32 + kb * 32);
-        }
+    for (int i = 0; i < (ASKED + 63) / 64; i++) {
+        const int at = i * 64 + lane, rr = min(at / PIECES, a.n - 1 - row0);
+        if ((i + 1) * 64 <= ASKED || at < ASKED)
+            __builtin_amdgcn_global_load_lds((mid_global_t)(wbase + static_cast<uint32_t>(rr * ROWB + at % PIECES * 16)), (mid_lds_t)(corner + i * 1024), 16, 0, 0);
     }
+    __builtin_amdgcn_sched_barrier(0);
     const char *frag = staged + (static_cast<size_t>(tile0) * SBS + wave * S) * kMidSb + lane * 16;
     const char *sums = staged + mid_sums_offset(tiles, a.k) + (static_cast<size_t>(tile0) * SBS + wave * S) * kMidSums + lane * 16;
     constexpr int D = 4;  // fetches held; eight are no faster
@@ -191,6 +195,10 @@ __global__ __launch_bounds__(64 * W) void gemm_mid_kernel(shv_gemv_q4k_args a, c
     for (int i = 0; i < D - 1; i++) ask(frag, i, f[i]);
 #pragma unroll
     for (int s = 0; s < S; s++) sx[s] = *reinterpret_cast<const bf16x8_t *>(sums + s * kMidSums);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * (D - 1) + S));  // all but the fragments and sums: the weights have landed
+    __builtin_amdgcn_sched_barrier(0);
+    const mid_bytes_t held = (mid_bytes_t)(corner) + n * (PIECES * 16);
     // n * sc of the wave's columns, held for every tile of the chunk
     half8_t wt[S][R][8];
     uint32_t am[S][R];
@@ -199,17 +207,19 @@ __global__ __launch_bounds__(64 * W) void gemm_mid_kernel(shv_gemv_q4k_args a, c
     for (int s = 0; s < S; s++)
 #pragma unroll
         for (int r = 0; r < R; r++) {
+            const mid_bytes_t at = held + r * (16 * PIECES * 16) + s * SHV_Q4K_BYTES;
+            const u32x4_t h = *(mid_quad_t)(at), q0 = *(mid_quad_t)(at + 16 + kb * 32), q1 = *(mid_quad_t)(at + 32 + kb * 32);
             uint32_t sc, mn;
-            q4k_group_scale_min(hdr[s][r], kb, sc, mn);
+            q4k_group_scale_min(make_uint4(h.x, h.y, h.z, h.w), kb, sc, mn);
 #pragma unroll
             for (int v = 0; v < 8; v++) {
-                const uint4 &x = q[s][r][(v >> 1) & 1];
+                const u32x4_t &x = (v & 2) ? q1 : q0;
                 const uint32_t d0 = (v & 1) ? x.z : x.x, d1 = (v & 1) ? x.w : x.y;
                 wt[s][r][v] = v < 4 ? weights8<false>(d0, d1, sc & 0xFFu, nc) : weights8<true>(d0, d1, sc >> 8, nc);
             }
             am[s][r] = bf16_pair(mn & 0xFFu, mn >> 8);
-            d[s][r] = f16_bits_to_f32(hdr[s][r].x);
-            dmin[s][r] = f16_bits_to_f32(hdr[s][r].x >> 16);
+            d[s][r] = f16_bits_to_f32(h.x);
+            dmin[s][r] = f16_bits_to_f32(h.x >> 16);
         }
     constexpr int PER = R * 256 >= 64 * W ? R * 256 / (64 * W) : 1;  // outputs a lane adds up over the waves
     static_assert(PER == 1 || PER == 2 || PER == 4, "a lane's share of a tile");
@@ -296,10 +306,6 @@ __global__ __launch_bounds__(64 * W) void gemm_mid_kernel(shv_gemv_q4k_args a, c
 // Two to four rows gain 7 us alone (52 to 45) and nothing in a pass, gemv_mrows.hip needing no staging launch: they stay there.
 constexpr int kFewRows = 16, kFewSlots = 3, kFewSlot = kFewRows * 8 * SHV_Q4K_BYTES, kFewLoads = kFewSlot / 1024;
 constexpr size_t kFewLds = static_cast<size_t>(kFewSlots) * kFewSlot + 8 * 1024;
-typedef const __attribute__((address_space(1))) void *few_global_t;
-typedef __attribute__((address_space(3))) void *few_lds_t;
-typedef const __attribute__((address_space(3))) char *few_bytes_t;
-typedef const __attribute__((address_space(3))) u32x4_t *few_quad_t;
 
 __global__ __launch_bounds__(512, 4) void gemm_few_kernel(shv_gemv_q4k_args a, const char *staged) {
     constexpr int W = 8, ROWB = W * SHV_Q4K_BYTES, PIECES = ROWB / 16, NL = (kFewLoads + W - 1) / W;
@@ -325,7 +331,7 @@ __global__ __launch_bounds__(512, 4) void gemm_few_kernel(shv_gemv_q4k_args a, c
 #pragma unroll
         for (int i = 0; i < NL; i++)
             if (wave + W * i < kFewLoads)
-                __builtin_amdgcn_global_load_lds((few_global_t)(w + (from[i] - max(from_row[i] - last, 0) * ROWB)), (few_lds_t)(slot + (wave + W * i) * 1024), 16, 0, 0);
+                __builtin_amdgcn_global_load_lds((mid_global_t)(w + (from[i] - max(from_row[i] - last, 0) * ROWB)), (mid_lds_t)(slot + (wave + W * i) * 1024), 16, 0, 0);
     };
     const auto piece = [&](int p) { return (n * PIECES + (p + 9 * n) % PIECES) * 16; };
     const int head_at = piece(9 * wave), q0_at = piece(9 * wave + 1 + 2 * kb), q1_at = piece(9 * wave + 2 + 2 * kb);
@@ -357,8 +363,8 @@ __global__ __launch_bounds__(512, 4) void gemm_few_kernel(shv_gemv_q4k_args a, c
         else if (wave < kFewLoads % W) __builtin_amdgcn_s_waitcnt(0x0F70 | behind * (whole + 1));
         else __builtin_amdgcn_s_waitcnt(0x0F70 | behind * whole);
         lds_barrier();
-        const few_bytes_t rows = (few_bytes_t)(slot);
-        const u32x4_t h = *(few_quad_t)(rows + head_at), q0 = *(few_quad_t)(rows + q0_at), q1 = *(few_quad_t)(rows + q1_at);
+        const mid_bytes_t rows = (mid_bytes_t)(slot);
+        const u32x4_t h = *(mid_quad_t)(rows + head_at), q0 = *(mid_quad_t)(rows + q0_at), q1 = *(mid_quad_t)(rows + q1_at);
         uint32_t sc, mn;
         q4k_group_scale_min(make_uint4(h.x, h.y, h.z, h.w), kb, sc, mn);
         float4_t acc = {0.f, 0.f, 0.f, 0.f}, y;
@@ -630,7 +636,7 @@ int tiles_a_block(const shv_ctx *ctx, int tiles, int blocks) {
 
 template <int R, int S, int W>
 int launch(shv_ctx *ctx, const shv_gemv_q4k_args &a, int tiles) {
-    constexpr size_t lds = static_cast<size_t>(W) * R * 2048;
+    constexpr size_t lds = static_cast<size_t>(W) * R * (2048 + 16 * S * SHV_Q4K_BYTES);  // the waves' sums of two tiles, then their weights
     if (lds > 48 * 1024) {
         static std::atomic<bool> raised{false};
         if (!raised.load(std::memory_order_acquire)) {
