@@ -140,58 +140,55 @@ __global__ __launch_bounds__(256) void embed_kernel(shv_embed_args a) {
         x[c] = ok ? __half2float(__ushort_as_half(row[c])) : __int_as_float(0x7fc00000);
 }
 
-// (value, index) ordered so that the larger value wins and, between equal values, the lower index.
-__device__ __forceinline__ bool better(float v, int i, float bv, int bi) { return v > bv || (v == bv && i < bi); }
-
-__device__ __forceinline__ void wave_best(float &v, int &i) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        const float ov = __shfl_xor(v, off, 64);
-        const int oi = __shfl_xor(i, off, 64);
-        if (better(ov, oi, v, i)) { v = ov; i = oi; }
-    }
-}
-
 // grid: (blocks, n_rows).  Each block scans a contiguous chunk of one row; the last block of the
-// row to arrive reduces the per-block winners.
+// row to arrive reduces the per-block winners.  The rows' arrival counters are lines apart: additions to one line follow one another.
+// us of 1 / 3 / 8 / 12 rows of 151936, a value a load, pairs exchanged by way of LDS and the counters side by side 6.5 / 9.9 / 12.6 / 14.5,
+// now 6.0 / 6.0 / 6.2 / 6.9.
+constexpr int kArgmaxCounterStep = 32;
 __global__ __launch_bounds__(256) void argmax_kernel(shv_argmax_args a, float *pval, int32_t *pidx, int32_t *counters) {
     __shared__ float sv[4];
     __shared__ int si[4];
     __shared__ int is_last;
     const int r = blockIdx.y, nb = gridDim.x;
     const float *lg = a.logits + static_cast<size_t>(r) * a.logits_stride;
-    const int chunk = (a.n + nb - 1) / nb;
-    const int lo = blockIdx.x * chunk, hi = lo + chunk < a.n ? lo + chunk : a.n;
+    const int chunk = ((a.n + nb - 1) / nb + 3) & ~3;
+    const int lo = min(static_cast<int>(blockIdx.x) * chunk, a.n), hi = lo + chunk < a.n ? lo + chunk : a.n;
     // "no candidate" is (-inf, n): any real element beats it, including -inf at a lower index
     float bv = -INFINITY;
     int bi = a.n;
-    for (int i = lo + threadIdx.x; i < hi; i += blockDim.x) {
-        const float v = lg[i];
-        if (better(v, i, bv, bi)) { bv = v; bi = i; }
+    const auto take = [&](float v, int i) {
+        if (amax_better(v, i, bv, bi)) { bv = v; bi = i; }
+    };
+    const int whole = (reinterpret_cast<uintptr_t>(lg) & 15) == 0 ? lo + ((hi - lo) & ~3) : lo;  // rows that do not begin on 16 bytes: one by one
+#pragma unroll 4
+    for (int i = lo + 4 * threadIdx.x; i < whole; i += 4 * 256) {
+        const float4 v = *reinterpret_cast<const float4 *>(lg + i);
+        take(v.x, i), take(v.y, i + 1), take(v.z, i + 2), take(v.w, i + 3);
     }
-    wave_best(bv, bi);
+    for (int i = whole + threadIdx.x; i < hi; i += 256) take(lg[i], i);
+    amax_wave(bv, bi);
     if ((threadIdx.x & 63) == 0) { sv[threadIdx.x >> 6] = bv; si[threadIdx.x >> 6] = bi; }
     __syncthreads();
     if (threadIdx.x == 0) {
         for (int w = 1; w < 4; w++)
-            if (better(sv[w], si[w], bv, bi)) { bv = sv[w]; bi = si[w]; }
+            if (amax_better(sv[w], si[w], bv, bi)) { bv = sv[w]; bi = si[w]; }
         shv::store_agent(pval + r * nb + blockIdx.x, bv);
         shv::store_agent(pidx + r * nb + blockIdx.x, bi);
     }
-    if (!shv::arrive_last(counters + r, nb, &is_last)) return;
+    if (!shv::arrive_last(counters + r * kArgmaxCounterStep, nb, &is_last)) return;
     bv = -INFINITY;
     bi = a.n;
     for (int b = threadIdx.x; b < nb; b += blockDim.x) {
         const float v = shv::load_agent(pval + r * nb + b);
         const int i = shv::load_agent(pidx + r * nb + b);
-        if (better(v, i, bv, bi)) { bv = v; bi = i; }
+        if (amax_better(v, i, bv, bi)) { bv = v; bi = i; }
     }
-    wave_best(bv, bi);
+    amax_wave(bv, bi);
     if ((threadIdx.x & 63) == 0) { sv[threadIdx.x >> 6] = bv; si[threadIdx.x >> 6] = bi; }
     __syncthreads();
     if (threadIdx.x == 0) {
         for (int w = 1; w < 4; w++)
-            if (better(sv[w], si[w], bv, bi)) { bv = sv[w]; bi = si[w]; }
+            if (amax_better(sv[w], si[w], bv, bi)) { bv = sv[w]; bi = si[w]; }
         // a row of NaN (or -inf only at the top) has no element that is `>` -inf: the reference
         // returns 0 there
         if (bi >= a.n) bi = 0;
@@ -225,7 +222,7 @@ __global__ __launch_bounds__(256) void ring_rows_kernel(shv_ring_rows_args a) {
 // allocated: kArgmaxBlocks values, kArgmaxBlocks indices, then kStaticCounters arrival counters.
 // Every GPU holds its own copy until the process ends; in host code the name is only a handle, the
 // device address comes from hipGetSymbolAddress (shv_static_scratch_bind, once per device).
-constexpr int kStaticCounters = 16;
+constexpr int kStaticCounters = 14 * kArgmaxCounterStep;
 constexpr size_t kStaticScratchBytes = shv_ctx::kArgmaxBlocks * (sizeof(float) + sizeof(int32_t)) + kStaticCounters * sizeof(int32_t);
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 
@@ -234,7 +231,8 @@ void *g_scratch_ptr[kMaxDevices] = {};
 std::mutex g_scratch_mutex;  // shv_init may run on several threads at once
 
 __global__ void clear_counters_kernel(int32_t *c, int n) {
-    if (static_cast<int>(threadIdx.x) < n) c[threadIdx.x] = 0;
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) c[i] = 0;
 }
 
 }  // namespace
@@ -304,7 +302,7 @@ int shv_launch_argmax_static(shv_ctx *ctx, const shv_argmax_args *a) {
     int32_t *counters = pidx + shv_ctx::kArgmaxBlocks;
     // the array keeps what the last call left: the arrival counters must start at zero (a fill
     // kernel, not a memset node, so that a caller may record this call into a graph)
-    SHV_LAUNCH(ctx, clear_counters_kernel, dim3(1), dim3(64), 0, counters, kStaticCounters);
+    SHV_LAUNCH(ctx, clear_counters_kernel, dim3((kStaticCounters + 255) / 256), dim3(256), 0, counters, kStaticCounters);
     SHV_LAUNCH(ctx, argmax_kernel, dim3(argmax_blocks(a), a->n_rows), dim3(256), 0, *a, pval, pidx, counters);
     return SHV_OK;
 }

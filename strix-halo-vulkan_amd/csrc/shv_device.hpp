@@ -300,13 +300,29 @@ __device__ __forceinline__ bool arrive_last(int32_t *counter, int expected, int 
 // ---- greedy arg-max: (value, index) pairs ordered so that the larger value wins and, between
 // equal values, the lower index; NaN never wins (Argmax, llm/sample.go:359-367) ------------------
 __device__ __forceinline__ bool amax_better(float v, int i, float bv, int bi) { return v > bv || (v == bv && i < bi); }
+// The wave's best in every lane: its largest value, then the lowest index among the lanes that hold it, each a chain of six DPP steps (pairs
+// by way of LDS, 12 exchanges, are a microsecond a chain longer; a launch has two such chains).  A lane's own value is never NaN.
+template <int CTRL>
+__device__ __forceinline__ int dpp_or_own(int v) { return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xF, 0xF, false); }
 __device__ __forceinline__ void amax_wave(float &v, int &i) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        const float ov = __shfl_xor(v, off, 64);
-        const int oi = __shfl_xor(i, off, 64);
-        if (amax_better(ov, oi, v, i)) { v = ov; i = oi; }
-    }
+    const auto larger = [](float m, int o) { return fmaxf(m, __int_as_float(o)); };
+    float m = v;
+    m = larger(m, dpp_or_own<kDppXor1>(__float_as_int(m)));
+    m = larger(m, dpp_or_own<kDppXor2>(__float_as_int(m)));
+    m = larger(m, dpp_or_own<kDppHalfMirror>(__float_as_int(m)));
+    m = larger(m, dpp_or_own<kDppMirror>(__float_as_int(m)));
+    m = larger(m, dpp_or_own<kDppBcast15>(__float_as_int(m)));
+    m = larger(m, dpp_or_own<kDppBcast31>(__float_as_int(m)));
+    m = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(m), 63));
+    int at = v == m ? i : 0x7FFFFFFF;
+    at = min(at, dpp_or_own<kDppXor1>(at));
+    at = min(at, dpp_or_own<kDppXor2>(at));
+    at = min(at, dpp_or_own<kDppHalfMirror>(at));
+    at = min(at, dpp_or_own<kDppMirror>(at));
+    at = min(at, dpp_or_own<kDppBcast15>(at));
+    at = min(at, dpp_or_own<kDppBcast31>(at));
+    v = m;
+    i = __builtin_amdgcn_readlane(at, 63);
 }
 
 __device__ __forceinline__ float sigmoid_exact(float x) { return 1.f / (1.f + expf(-x)); }

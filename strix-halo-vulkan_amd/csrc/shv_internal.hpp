@@ -101,7 +101,7 @@ struct shv_ctx {
         *e = mark_pool[i + 1];
         return hipSuccess;
     }
-    enum { kCounterRouter = 0, kCounterArgmax = 1, kCounterAttn = 16, kCounterGemvAmax = 15 };
+    enum { kCounterRouter = 0, kCounterArgmax = 64 /* 14 of them, 32 apart */, kCounterGemvAmax = 15 };
     // What the last shv_moe_up on this context left behind for the shv_moe_down that follows it:
     // the pass its per-expert lists in `group` belong to, and whether act holds matrix-core
     // operands instead of floats.  shv_moe_down believes its group_ready / act_packed flags only

@@ -39,6 +39,19 @@ def test_argmax_first_maximum_wins(ctx):
     assert _argmax(ctx, np.full((1, 300), np.nan, np.float32))[0] == 0
 
 
+@pytest.mark.parametrize("rows,n", [(1, 1), (2, 3), (3, 5), (14, 255), (5, 1023), (3, 1024), (7, 4099), (12, 151936), (2, 151937)])
+def test_argmax_of_rows_that_begin_anywhere(ctx, rows, n):
+    """Rows on sixteen bytes and off them, in fours and what is left; equal values in different lanes, waves and blocks, zeros of either
+    sign among them, and maxima at a row's ends."""
+    rng = np.random.default_rng(rows * n)
+    x = rng.integers(-40, 1, size=(rows, n)).astype(np.float32) / 8
+    x[x == 0] = np.where(rng.random((x == 0).sum()) < 0.5, 0.0, -0.0)
+    x[0, n - 1] = 1.0
+    x[-1, :] = -np.inf
+    x[-1, n // 2] = -3.0
+    assert list(_argmax(ctx, x)) == list(np.argmax(x, axis=1))
+
+
 def test_argmax_feeds_the_next_step(ctx):
     logits = np.zeros((1, 5000), np.float32)
     logits[0, 4321] = 1.0
