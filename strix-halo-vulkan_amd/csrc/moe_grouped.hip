@@ -170,6 +170,25 @@ __device__ __forceinline__ void stage_rows(const float *x, int rows, int k, char
     }
 }
 
+// The wave's inclusive sums, lane by lane, and the sums of its halves in their last lanes: DPP steps.  By way of LDS each of
+// eleven exchanges was a trip of its own, and the experts' order took two comparisons a length: a layer's lists and products
+// of 66 rows 168.2 to 167.0 us, of 150 rows 224.3 to 222.7; passes of 65 and 150 rows of 16 layers 3634 to 3609 and 4848 to 4839.
+__device__ __forceinline__ int wave_prefix_sum(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);  // row_shr:1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kDppBcast15, 0xA, 0xF, false);
+    return v + __builtin_amdgcn_update_dpp(0, v, kDppBcast31, 0xC, 0xF, false);
+}
+__device__ __forceinline__ int half_wave_sum(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, kDppXor1, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kDppXor2, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kDppHalfMirror, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kDppMirror, 0xF, 0xF, false);
+    return v + __builtin_amdgcn_update_dpp(0, v, kDppBcast15, 0xA, 0xF, false);
+}
+
 // counts NULL: no launch before; every block counts all pairs itself, those before its own chunk apart.  Blocks past the sixteen,
 // when the launch has them, stage the list kernels' rows x meanwhile.
 __global__ __launch_bounds__(1024) void moe_group_place_kernel(const int32_t *topk, int n_pairs, int chunk, int n_used, int n_expert, const int32_t *counts,
@@ -209,14 +228,10 @@ __global__ __launch_bounds__(1024) void moe_group_place_kernel(const int32_t *to
             before += o < b ? v[o] : 0;
         }
     }
-    int incl = c;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int up = __shfl_up(incl, o, 64);
-        if (lane >= o) incl += up;
-    }
+    const int incl = wave_prefix_sum(c);
     if (lane == 63) s_wsum[wave] = incl;
-    s_len[tid] = tid < n_expert ? c : -1;   // past n_expert: shorter than any list
+    // what orders the experts in one word (a list's length, then the lower index): shapes_covered keeps pairs below 2^19
+    s_len[tid] = tid < n_expert ? (c << 10) | (kMaxExperts - 1 - tid) : -1;  // past n_expert: shorter than any list
     __syncthreads();
     int base = 0;
     for (int w = 0; w < wave; w++) base += s_wsum[w];
@@ -227,7 +242,7 @@ __global__ __launch_bounds__(1024) void moe_group_place_kernel(const int32_t *to
         if (tid == n_expert - 1) group[n_expert] = start + c;
     }
     // An expert's place in the launch: longer lists first, equal lengths by index.  Each block ranks its share of
-    // the experts, 32 threads an expert (each against every 32nd length), instead of one block all of them with a
+    // the experts, 32 threads an expert (each against every 32nd quad of lengths), instead of one block all of them with a
     // thread an expert: E^2 comparisons are most of what one block would spend on a pass's lists.
     {
         const int per = (n_expert + nb - 1) / nb, e0 = b * per;
@@ -235,18 +250,14 @@ __global__ __launch_bounds__(1024) void moe_group_place_kernel(const int32_t *to
         for (int eb = tid >> 5; eb < per; eb += 32) {
             const int e = e0 + eb;
             const bool live = e < n_expert;
-            const int ce = live ? s_len[e] : 0;
+            const int mine = live ? s_len[e] : 0;
             int rank = 0;
-            for (int o = part; o < n_expert; o += 32) {
-                const int co = s_len[o];
-                rank += (co > ce || (co == ce && o < e)) ? 1 : 0;
+            for (int o = 4 * part; o < n_expert; o += 128) {
+                const int4 k = *reinterpret_cast<const int4 *>(s_len + o);
+                rank += (k.x > mine) + (k.y > mine) + (k.z > mine) + (k.w > mine);
             }
-            rank += __shfl_xor(rank, 16, 64);
-            rank += __shfl_xor(rank, 8, 64);
-            rank += __shfl_xor(rank, 4, 64);
-            rank += __shfl_xor(rank, 2, 64);
-            rank += __shfl_xor(rank, 1, 64);
-            if (live && part == 0) group[n_expert + 1 + n_pairs + rank] = e;
+            rank = half_wave_sum(rank);
+            if (live && part == 31) group[n_expert + 1 + n_pairs + rank] = e;
         }
     }
     __syncthreads();
