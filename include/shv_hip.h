@@ -557,8 +557,9 @@ typedef struct {
  * alone (written by the projection before), the conv's history lies in hist, a ring of hist_slots
  * rows ring_stride floats apart.  Rows pos-3 .. pos-1 are taken from hist, and the conv channels
  * (2*hk*d + hv*d floats) of the pass's last three rows are left there for the next pass.
- * n_seq 1, slot NULL, hist_slots >= 3, hist 16-byte aligned; step.ring must have room for three rows
- * more than the pass, which a pass that shv_dn_step takes row by row uses. */
+ * n_seq 1, slot NULL, spec 0 (of a rewound pass hist would hold rows that were not kept),
+ * hist_slots >= 3, hist 16-byte aligned; step.ring must have room for three rows more than the
+ * pass, which a pass that shv_dn_step takes row by row uses. */
 typedef struct {
     shv_dn_step_args step;
     float *hist;

@@ -440,6 +440,8 @@ int shv_launch_dn_pass(shv_ctx *ctx, const shv_dn_pass_args *pa) {
     const shv_dn_step_args &a = pa->step;
     if (int rc = check_step(a)) return rc;
     SHV_REQUIRE(a.n_seq == 1 && !a.slot, "dn_pass: one sequence without a slot table, not %d", a.n_seq);
+    // hist is left with the pass's last three rows: a pass of which only the first k are kept would go on behind another three
+    SHV_REQUIRE(!a.spec, "dn_pass: a rewindable pass keeps its rows in the sequence's own ring (dn_step)");
     SHV_REQUIRE(pa->hist && pa->hist_slots >= a.conv - 1, "dn_pass: a history of %d rows", pa->hist_slots);
     SHV_REQUIRE(shv_aligned16(a.ring) && shv_aligned16(pa->hist) && a.ring_stride % 4 == 0, "dn_pass: rings must be 16-byte aligned, rows a multiple of 4 floats apart");
     if (shv_dn_chunk_covers(a)) return shv_launch_dn_chunk(ctx, a, pa->hist, pa->hist_slots);

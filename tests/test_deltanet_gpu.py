@@ -312,6 +312,11 @@ def test_dn_pass_refuses_what_it_does_not_cover(ctx):
     for n_seq, slot, hist, slots in ((2, None, d.ptr, 3), (1, d.ptr, d.ptr, 3), (1, None, None, 3), (1, None, d.ptr, 2), (1, None, d.ptr + 4, 3)):
         with pytest.raises(shv.pkg.ShvError):
             ctx.enqueue(A.OP_DN_PASS, A.DnPassArgs(step(n_seq, slot), hist, slots))
+    # a rewindable pass, which shv_dn_step takes (three state planes, two rows): the history it would need again is overwritten
+    rewindable = step(1, None)
+    rewindable.seq_len, rewindable.ring_slots, rewindable.n_planes, rewindable.spec = 2, 5, 3, 1
+    with pytest.raises(shv.pkg.ShvError, match="rewindable pass keeps"):
+        ctx.enqueue(A.OP_DN_PASS, A.DnPassArgs(rewindable, d.ptr, 3))
 
 
 def test_dn_step_refuses_unsupported_shapes(ctx):
