@@ -323,7 +323,8 @@ __global__ __launch_bounds__(64) void moe_route_kernel(shv_moe_router_args a) {
 // their sum in slot order clamped at 2^-14.
 // A chain of steps with two block-wide waits.  Behind the first every wave has the 16 half-wave maxima of the logits: their
 // largest, and the n_used-th largest, whose exponential bounds the selected ones from below (exp(l - max) rises with l; what
-// rounding may make of equal probabilities is a few last bits, which the bound leaves room for).  The few at or above it go
+// rounding may make of equal probabilities is a few last bits, or where they are denormal a step of 2^-149 times the sum, at
+// most 512, and the bound leaves room for both).  The few at or above it go
 // to a table as they come; behind the second the first wave divides them by the sum and ranks them.  The same bits with waits for
 // the maximum, the sum, the group maxima, the threshold, the counts and the table: router and selection of 12 / 40 / 150 / 1531 rows
 // 11.6 / 13.0 / 16.1 / 37.4 us, so 10.8 / 12.0 / 14.8 / 36.6 (with a wave a row 14.4 / 15.6 / 18.1 / 38.0).
@@ -376,7 +377,7 @@ __global__ __launch_bounds__(kRouteBlock) void moe_route_block_kernel(shv_moe_ro
     }
     const float ex = has ? expf(l - mx) : 0.f;
     const float ws = wave_sum_all(ex);
-    const bool pred = has && ex >= expf(thr - mx) * (1.f - 0x1p-20f);
+    const bool pred = has && ex >= fmaf(expf(thr - mx), 1.f - 0x1p-20f, -0x1p-139f);
     const unsigned long long mask = __ballot(pred);
     int base = 0;
     if (lane == 0) {

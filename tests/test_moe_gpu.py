@@ -667,3 +667,29 @@ def test_selection_from_the_logits_as_they_are(T, E, used, copies):
             assert abs(wt[t, used] - 1 / (1 + np.exp(-l64[E]))) <= 2e-6
     finally:
         c.destroy()
+
+
+@pytest.mark.parametrize("T", [5, 40])
+def test_selection_where_probabilities_are_denormal(T):
+    """Nine experts share the largest logit and two are e^-98 below, 98 and 101 of float32's smallest steps: a ninth of either is eleven
+    of them (also of either a step or two off), one probability, and the lower index is the tenth.  All eleven in halves of waves of their own."""
+    c, H, E, used = A.Context(0), 512, 512, 10
+    try:
+        logit = np.full(E, -300.0)
+        top = np.arange(2, 11) * 32 + 5
+        logit[top] = 0.0
+        logit[20], logit[40] = (np.log(v) - 149 * np.log(2.0) for v in (98, 101))
+        router = np.zeros((E, H), np.float32)
+        router[:, 0] = logit
+        h, gamma = np.zeros((T, H), np.float32), np.ones(H, np.float32)
+        h[:, 0], gamma[0] = 1.0, np.sqrt(1.0 / H + 1e-6)  # xn: one in the first column
+        logits, topk, wts = c.alloc(T * (E + 1) * 4), c.alloc(T * used * 4), c.alloc(T * (used + 1) * 4)
+        args = A.MoeRouterArgs(c.upload(h).ptr, c.upload(gamma).ptr, c.upload(router).ptr, None, c.alloc(T * H * 4).ptr, logits.ptr, topk.ptr, wts.ptr, T, H, E, used, 1e-6, H, 0)
+        c.dispatch_multi([A.make_op(A.OP_MOE_ROUTER, args)])
+        got = logits.read(np.float32, T * (E + 1)).reshape(T, E + 1)[:, :E].astype(np.float64)
+        assert (np.abs(got[:, [20, 40]] - logit[[20, 40]]) <= 0.01).all()  # a hundredth of a probability: one step
+        assert (topk.read(np.int32, T * used).reshape(T, used) == list(top) + [20]).all()
+        wt = wts.read(np.float32, T * (used + 1)).reshape(T, used + 1)
+        assert np.abs(wt[:, :9] - 1 / 9).max() <= 1e-6 and (wt[:, 9] < 1e-40).all()
+    finally:
+        c.destroy()
