@@ -196,6 +196,7 @@ __global__ __launch_bounds__(64 * W) void gemm_mid_kernel(shv_gemv_q4k_args a, c
 #pragma unroll
     for (int s = 0; s < S; s++) sx[s] = *reinterpret_cast<const bf16x8_t *>(sums + s * kMidSums);
     __builtin_amdgcn_sched_barrier(0);
+    static_assert(2 * (D - 1) + S < 16, "vmcnt");
     __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * (D - 1) + S));  // all but the fragments and sums: the weights have landed
     __builtin_amdgcn_sched_barrier(0);
     const mid_bytes_t held = (mid_bytes_t)(corner) + n * (PIECES * 16);
@@ -670,15 +671,6 @@ int launch_stage(shv_ctx *ctx, const shv_gemv_q4k_args &a, int tiles, float *x_o
     return SHV_OK;
 }
 
-// From nine rows, where the kernels that form every weight once for up to eight of them end, to 512, but for 49 to 64, which
-// keep the kernel of one 64-row group.  That kernel is the slower there (12352 x 2048 of 64 rows 27.7 us, 15.9 here; of 40 rows 24.1
-// and 13.8, of 17 20.6 and 12.4; 2048 x 4096 of 40 rows 17.9 and 11.0) and the less exact (2.1e-6 against 0.4e-6): the line is one of
-// results that stay what they were, since a prompt's whole chunk of 64 rows is one pass whose routing, where a token's tenth expert and
-// its eleventh are level, every token decoded after it carries on (48 layers: the logits after 96 tokens parted by 1e-4 to 2e-3).  It is a
-// line of the results' continuity, of neither speed nor precision: eight layers' logits against the CPU's, median of ten prompts, 56 rows
-// 1.5e-5 there and 1.1e-5 here, 64 rows 1.4e-5 and 1.0e-5 (one of the ten 3.6e-3 there: another expert), where 17 to 48 rows went over
-// from 2.1e-5 to 1.6e-5 at 20 rows, 1.6e-5 to 1.1e-5 at 48.
-// Past 512 gemm_long.hip's blocks read less from L2.
 }  // namespace
 
 // A pass of five to sixteen rows against a matrix of eight groups of rows a block and more (the caller has seen to shv_gemm_q4k_covers).
@@ -699,9 +691,11 @@ int shv_launch_gemm_few(shv_ctx *ctx, const shv_gemv_q4k_args &a) {
     return SHV_OK;
 }
 
+// From nine rows, where the kernels that form every weight once for up to eight of them end, to 512, but for the passes that
+// shv_one_group names.  Past 512 gemm_long.hip's blocks read less from L2.
 bool shv_gemm_mid_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a) {
     if (!ctx->gemm_stage || (a.k != 2048 && a.k != 4096) || a.n_tok < 9 || a.n_tok > 512) return false;
-    if (a.n_tok > 48 && a.n_tok <= 64) return false;
+    if (shv_one_group(a.n_tok)) return false;
     if (a.prologue == SHV_PRO_GATED_NORM && 256 % a.head_dim != 0) return false;
     return mid_bytes((a.n_tok + 15) / 16, a.k) <= static_cast<size_t>(shv_ctx::kGemmStageBytes);
 }
@@ -722,7 +716,7 @@ int shv_launch_gemm_mid(shv_ctx *ctx, const shv_gemv_q4k_args &a) {
 // Which form, of 2048 columns: the float32 blocks while one a compute unit is enough, of 16 experts or of 32 (150 rows of 512 experts,
 // 256 compute units: 11.5 and 10.4 us), and by turns while three are (384 rows 16.7 us, staged 19.2); at 512 rows they lose, 20.3 to 18.9.
 // Below, the row kernel goes through its tokens a few at a time (17 rows 7.8 us to 7.6, 32 10.4 to 7.7, 48 12.5 to 7.8) and is quicker
-// of 16; 49 to 64 rows stay with it as they do with the projections of one 64-row group: a line of the results' continuity.
+// of 16; shv_one_group's passes stay with it.
 namespace {
 
 bool router_aligned(const shv_moe_router_args &a) {
@@ -733,7 +727,7 @@ bool router_aligned(const shv_moe_router_args &a) {
 enum class RouterNorm { none, sixteen, thirty_two, sixteen_by_turns };
 RouterNorm router_norm_form(const shv_ctx *ctx, const shv_moe_router_args &a) {
     const long long cus = ctx->prop.multiProcessorCount, tiles = (a.n_tok + 15) / 16, ones = (a.n_expert + 15) / 16 * tiles, twos = (a.n_expert + 31) / 32 * tiles;
-    if (a.n_embd != 2048 || a.n_tok < 17 || (a.n_tok > 48 && a.n_tok <= 64) || ones > 3 * cus) return RouterNorm::none;
+    if (a.n_embd != 2048 || a.n_tok < 17 || shv_one_group(a.n_tok) || ones > 3 * cus) return RouterNorm::none;
     return ones <= cus ? RouterNorm::sixteen : twos <= cus ? RouterNorm::thirty_two : RouterNorm::sixteen_by_turns;
 }
 

@@ -311,6 +311,7 @@ __global__ __launch_bounds__(kBlock) void gemv_stream_kernel(shv_gemv_q4k_args a
     __shared__ __align__(16) float xs[lds_padded(K)];
     __shared__ float red[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    static_assert(LOADS < 16, "vmcnt");
     const int gi = lane % LPR, rsub = lane / LPR, sb = gi >> 2, g = gi & 3;
     const int chunks = (a.n + ROWS - 1) / ROWS, stride = gridDim.x * kWavesPerBlock;
     char *ring = rings[wave];

@@ -946,8 +946,8 @@ __global__ __launch_bounds__(768) void moe_down_slots_kernel(shv_moe_down_args a
 // Bound by HBM as far as its eleven waves hide their products.  us of 5 / 8 / 9 / 12 rows (10 of 512 experts, 2048 x 512; the same
 // bits): rounds of blocks of four passes 12.4 / 14.0 / 17.6 / 19.4, here 10.6 / 12.9 / 14.4 / 17.4 with one pass ahead (two: 11.2 / 13.0 /
 // 14.6 / 18.2); 13 / 16 / 40 / 48 rows: moe_down_kernel, whose waves walk three slots each, 23.5 / 26.9 / 51.4 / 57.8, here with two
-// ahead 18.8 / 21.1 / 44.7 / 51.5 (one: 18.5 / 22.6 / 45.1), its error against float64 0.95 of that kernel's.  49 to 64 rows, 73 us there and
-// 62 here at 64, stay with it as they do with the projections of one 64-row group.
+// ahead 18.8 / 21.1 / 44.7 / 51.5 (one: 18.5 / 22.6 / 45.1), its error against float64 0.95 of that kernel's.  shv_one_group's passes
+// stay with it.
 // grid: (runs of a token, n_tok), (s_hi - s_lo) * 64 threads; a run is at most kWalkRows rows.
 constexpr int kWalkRows = 512;
 template <int K, int D>

@@ -155,6 +155,13 @@ int shv_launch_gemv_q4k(shv_ctx *ctx, const shv_gemv_q4k_args *a);
 bool shv_gemm_q4k_covers(const shv_gemv_q4k_args &a);
 bool shv_gemv_mrows_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a);
 int shv_launch_gemv_mrows(shv_ctx *ctx, const shv_gemv_q4k_args &a);
+// Passes of 49 to 64 rows, which gemm_q4k.hip takes as one group of 64, keep the row kernel of the router and moe_down_kernel beside it.
+// All are the slower there (12352 x 2048 of 64 rows 27.7 us and 15.9 by gemm_mid.hip, router with selection 18.2 and 11.9, down products
+// 73 and 62), the projections the less exact (2.1e-6 of the result, 0.4e-6).  The line is one of results alone: sums in another order turn
+// near ties between a token's tenth expert and its eleventh, which every token decoded behind the prompt carries on.  Over 54 replies of
+// 96 tokens behind 64-row prompts (48 layers) the last logits part by 1.3e-4 at the median, but three by 2.1e-3, 2.8e-3 and 8.2e-3;
+// with the router's and the down products' kernels alone two of 102 replies and prompts by 2.0e-3 and 2.9e-3 (all with the same tokens).
+inline bool shv_one_group(int n_tok) { return n_tok > 48 && n_tok <= 64; }
 bool shv_gemm_mid_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a);
 int shv_launch_gemm_mid(shv_ctx *ctx, const shv_gemv_q4k_args &a);
 bool shv_gemm_long_covers(const shv_ctx *ctx, const shv_gemv_q4k_args &a);
