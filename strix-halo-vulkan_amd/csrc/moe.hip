@@ -1164,22 +1164,24 @@ int shv_launch_moe_down(shv_ctx *ctx, const shv_moe_down_args *pa) {
     switch (a.ffn) {
         case 512: {
             constexpr int RPP = 64 / (512 / 64);
+            const bool tall = a.n_tok >= ctx->moe_tall_min, wide_act = shv_aligned16(a.act);
             // five rows and more, a wave a slot: a block walks a run of rows, as many blocks as compute units (moe_down_walk_kernel)
-            if (a.n_tok >= 5 && a.n_tok <= 48 && a.n_embd % RPP == 0 && shv_aligned16(a.act)) {
+            if (a.n_tok >= 5 && a.n_tok <= 48 && !(tall && ctx->moe_tall_forced) && a.n_embd % RPP == 0 && wide_act) {
                 const int runs = std::min(std::max(ctx->prop.multiProcessorCount / a.n_tok, (a.n_embd + kWalkRows - 1) / kWalkRows), a.n_embd / RPP);
                 if (a.n_tok <= 12) SHV_LAUNCH(ctx, (moe_down_walk_kernel<512, 1>), dim3(runs, a.n_tok), dim3((s_hi - s_lo) * 64), 0, a, s_lo, s_hi);
                 else SHV_LAUNCH(ctx, (moe_down_walk_kernel<512, 2>), dim3(runs, a.n_tok), dim3((s_hi - s_lo) * 64), 0, a, s_lo, s_hi);
                 break;
             }
-            if (a.n_tok >= ctx->moe_tall_min) SHV_LAUNCH(ctx, (moe_down_kernel<512, 12, 8>), dim3((a.n_embd + RPP * 8 - 1) / (RPP * 8), a.n_tok), block, 0, a, s_lo, s_hi);
-            else if (a.n_tok >= 3 && a.n_tok < 5 && a.n_embd % (4 * RPP) == 0 && shv_aligned16(a.act)) SHV_LAUNCH(ctx, (moe_down_slots_kernel<512, 4>),  // three and four rows: four
-                dim3(a.n_embd / (4 * RPP), a.n_tok), dim3((s_hi - s_lo) * 64), 0, a, s_lo, s_hi);  // passes a wave (a 3-row verification pass 2.48 to 2.43 ms; at two rows 2.14 becomes 2.19)
-            else if (a.n_tok >= 2 && a.n_tok < 8 && a.n_embd % (2 * RPP) == 0 && shv_aligned16(a.act)) SHV_LAUNCH(ctx, (moe_down_slots_kernel<512, 2>),  // verification passes: one round of blocks
-                dim3(a.n_embd / (2 * RPP), a.n_tok), dim3((s_hi - s_lo) * 64), 0, a, s_lo, s_hi);
-            else if (a.n_tok < 8 && a.n_embd % (1 * RPP) == 0 && shv_aligned16(a.act)) SHV_LAUNCH(ctx, (moe_down_slots_kernel<512, 1>),  // the decode step and verification passes
-                dim3(a.n_embd / (1 * RPP), a.n_tok), dim3((s_hi - s_lo) * 64), 0, a, s_lo, s_hi);
-            else if (a.n_tok >= 8) SHV_LAUNCH(ctx, (moe_down_kernel<512, 12, 4>),  // eight sequences decoded together: 5.31 to 5.19 ms a pass
-                dim3((a.n_embd + RPP * 4 - 1) / (RPP * 4), a.n_tok), block, 0, a, s_lo, s_hi);
+            if (tall) SHV_LAUNCH(ctx, (moe_down_kernel<512, 12, 8>), dim3((a.n_embd + RPP * 8 - 1) / (RPP * 8), a.n_tok), block, 0, a, s_lo, s_hi);
+            // one to four rows, a wave a slot and one round of blocks: a 3-row verification pass with two passes a wave 2.48 ms, with four 2.43; of two rows 2.14 and 2.19
+            else if (a.n_tok >= 3 && a.n_tok <= 4 && a.n_embd % (4 * RPP) == 0 && wide_act)
+                SHV_LAUNCH(ctx, (moe_down_slots_kernel<512, 4>), dim3(a.n_embd / (4 * RPP), a.n_tok), dim3((s_hi - s_lo) * 64), 0, a, s_lo, s_hi);
+            else if (a.n_tok >= 2 && a.n_tok <= 4 && a.n_embd % (2 * RPP) == 0 && wide_act)
+                SHV_LAUNCH(ctx, (moe_down_slots_kernel<512, 2>), dim3(a.n_embd / (2 * RPP), a.n_tok), dim3((s_hi - s_lo) * 64), 0, a, s_lo, s_hi);
+            else if (a.n_tok <= 4 && a.n_embd % RPP == 0 && wide_act)
+                SHV_LAUNCH(ctx, (moe_down_slots_kernel<512, 1>), dim3(a.n_embd / RPP, a.n_tok), dim3((s_hi - s_lo) * 64), 0, a, s_lo, s_hi);
+            // rows whose act is off 16 bytes, or a width that is no multiple of eight: 8 / 12 / 15 of them with four passes 13.6 / 17.4 / 21.7 us, with one 15.9 / 20.7 / 24.9
+            else if (a.n_tok >= 8) SHV_LAUNCH(ctx, (moe_down_kernel<512, 12, 4>), dim3((a.n_embd + RPP * 4 - 1) / (RPP * 4), a.n_tok), block, 0, a, s_lo, s_hi);
             else SHV_LAUNCH(ctx, (moe_down_kernel<512, 12, 1>), dim3((a.n_embd + RPP - 1) / RPP, a.n_tok), block, 0, a, s_lo, s_hi);
             break;
         }

@@ -64,7 +64,10 @@ int shv_init(int device, shv_ctx **out) {
     if (const char *e = std::getenv("SHV_MOE_GROUP_BLOCKS")) ctx->moe_group_one_block = std::atoi(e) == 1;
     if (const char *e = std::getenv("SHV_MOE_TALL_MIN")) {
         const int v = std::atoi(e);
-        if (v >= 1) ctx->moe_tall_min = v;
+        if (v >= 1) {
+            ctx->moe_tall_min = v;
+            ctx->moe_tall_forced = true;
+        }
     }
     hipError_t e = hipGetDeviceProperties(&ctx->prop, device);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);

@@ -43,7 +43,10 @@ struct shv_ctx {
     bool moe_group_forced = false;
     bool dn_chunk_no_recs = false;  // SHV_DN_RECS=0: the chunked delta rule forms every chunk's state-independent part inside the walk, whatever the workspace holds
     bool moe_group_one_block = false;  // SHV_MOE_GROUP_BLOCKS=1: the per-expert lists of a long pass by one block in one launch
-    int moe_tall_min = 16;  // tokens from which the MoE kernels' blocks make several passes over their staged rows (SHV_MOE_TALL_MIN)
+    // Tokens from which moe_up_kernel's and moe_down_kernel's blocks make eight passes over the rows they have staged.  Down products
+    // of 512 columns come to that kernel from 49 rows on, or where SHV_MOE_TALL_MIN names the number: then from it on.
+    int moe_tall_min = 16;
+    bool moe_tall_forced = false;
     hipEvent_t ev_begin = nullptr, ev_end = nullptr;
     hipEvent_t stamps[SHV_STAMPS] = {};  // shv_stamp's, made when first used
     // shv_upload_async copies up to kUpSlotBytes into the next slot of a ring of pinned host memory and hands them

@@ -634,6 +634,32 @@ def test_down_projection_in_runs_of_rows(T, H, U, residual):
         c.destroy()
 
 
+def test_tall_blocks_where_they_are_asked_for(monkeypatch):
+    """SHV_MOE_TALL_MIN sends the down products from its number of rows on to the kernel that more than 48 rows take: the same bits a row."""
+    E, H, U, F, T = 8, 264, 4, 512, 49
+    rng = np.random.default_rng(1)
+    wq, ws = (O.quantize_q4k((rng.standard_normal((n * H, F)) * 0.02).astype(np.float32)) for n in (E, 1))
+    topk = np.argsort(rng.random((T, E)), axis=1)[:, :U].astype(np.int32)
+    act, wts = rng.standard_normal((T, U + 1, F)).astype(np.float32), rng.random((T, U + 1)).astype(np.float32)
+
+    def down(rows):
+        c = A.Context(0)
+        try:
+            out = c.alloc(rows * H * 4)
+            bufs = [c.upload(np.ascontiguousarray(v)) for v in (act[:rows], topk[:rows], wts[:rows], wq, ws)]
+            c.dispatch_multi([A.make_op(A.OP_MOE_DOWN, A.MoeDownArgs(*(b.ptr for b in bufs), None, out.ptr, rows, H, U, F, H, H, 0, 0, E, None, None, 0, 0))])
+            return out.read(np.float32, rows * H).reshape(rows, H).view(np.uint32)
+        finally:
+            c.destroy()
+
+    tall = down(T)
+    walk = down(16)
+    monkeypatch.setenv("SHV_MOE_TALL_MIN", "12")
+    assert not np.array_equal(walk, tall[:16])
+    assert np.array_equal(down(12), tall[:12]) and np.array_equal(down(48), tall[:48])
+    assert np.array_equal(down(11), walk[:11])
+
+
 @pytest.mark.parametrize("T,E,used,copies", [(5, 65, 1, 1), (9, 100, 10, 2), (40, 512, 10, 1), (40, 512, 16, 3), (200, 512, 10, 40), (7, 512, 10, 70), (130, 300, 12, 1)])
 def test_selection_from_the_logits_as_they_are(T, E, used, copies):
     """The selection of a block a token, from the logits the router left: in order, ties (copies of a router row) to the lower index,
