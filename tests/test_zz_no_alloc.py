@@ -85,3 +85,25 @@ def test_static_argmax_recorded_into_a_graph_and_replayed(ctx):
             assert got == list(eager.read(np.int32, rows)) == list(np.argmax(logits, axis=1)), rep
     finally:
         rec.destroy()
+
+
+@pytest.mark.parametrize("rows", [8, 9, 14])
+def test_static_argmax_of_as_many_rows_as_it_takes(ctx, rows):
+    """Every row's arrival counter has a line of its own, cleared by a launch of several blocks: eagerly twice in a row and replayed, each
+    time against numpy, rows of several blocks and maxima at their ends."""
+    rng, n = np.random.default_rng(rows), 20011
+    dev, best = ctx.upload(np.zeros((rows, n), np.float32)), ctx.upload(np.full(rows, -7, np.int32))
+    args = A.ArgmaxArgs(dev.ptr, best.ptr, None, None, rows, n, n)
+    rec = ctx.prerecord([A.make_op(A.OP_ARGMAX_STATIC, args)])
+    try:
+        for rep in range(4):
+            logits = rng.standard_normal((rows, n)).astype(np.float32)
+            logits[np.arange(rows), np.where(np.arange(rows) % 2, n - 1 - rep, rep)] = 9.0
+            want, got = _both(ctx, logits)
+            assert got == want == list(np.argmax(logits, axis=1)), rep
+            dev.write(np.roll(logits, 1, axis=0))
+            best.write(np.full(rows, -7, np.int32))
+            rec.submit(1)
+            assert list(best.read(np.int32, rows)) == want[-1:] + want[:-1], rep
+    finally:
+        rec.destroy()
