@@ -192,6 +192,13 @@ def test_router_of_a_lower_pass(rows, E, gate):
         ctx.destroy()
 
 
+@pytest.mark.parametrize("rows", [49, 56, 64])
+def test_passes_of_one_group(rows):
+    """Projections and router on either side of these kernels' gap: the same bounds hold in it."""
+    test_rows_of_a_pass(300, 2048, rows)
+    test_router_of_a_lower_pass(rows, 512, True)
+
+
 @pytest.mark.parametrize("n,k,rows", [(96, 2048, 9), (2048, 4096, 16), (70, 2048, 65), (2048, 4096, 192), (300, 2048, 512)])
 def test_sums_past_binary16(n, k, rows):
     """Every activation is a binary16 number, the sum of a sub-block's 32 is not (65504 is the largest): the min term's sums are

@@ -634,6 +634,31 @@ def test_down_projection_in_runs_of_rows(T, H, U, residual):
         c.destroy()
 
 
+@pytest.mark.parametrize("T", [49, 56, 64])
+def test_down_projection_past_the_runs(T):
+    """The next rows up, slot after slot: as near to float64 as the runs of rows below them."""
+    c, E, F, H, U = A.Context(0), 16, 512, 1032, 10
+    rng = np.random.default_rng(T)
+    try:
+        wq, ws = (O.quantize_q4k((rng.standard_normal((n * H, F)) * 0.02).astype(np.float32)) for n in (E, 1))
+        topk = np.argsort(rng.random((T, E)), axis=1)[:, :U].astype(np.int32)
+        act, wts, res = (rng.standard_normal(s).astype(np.float32) for s in ((T, U + 1, F), (T, U + 1), (T, H)))
+        out = c.alloc(T * H * 4)
+        bufs = [c.upload(v) for v in (act, topk, wts, wq, ws, res)]
+        c.dispatch_multi([A.make_op(A.OP_MOE_DOWN, A.MoeDownArgs(*(b.ptr for b in bufs), out.ptr, T, H, U, F, H, H, 0, 0, E, None, None, 0, 0))])
+        got = out.read(np.float32, T * H).reshape(T, H)
+        w64, s64 = O.dequant_q4k(wq, F).astype(np.float64).reshape(E, H, F), O.dequant_q4k(ws, F).astype(np.float64)
+        want, size = res.astype(np.float64), np.abs(res).astype(np.float64)
+        for t in range(T):
+            for s in range(U + 1):
+                m, x = (w64[topk[t, s]] if s < U else s64), act[t, s].astype(np.float64) * float(wts[t, s])
+                want[t] += m @ x
+                size[t] += (np.abs(m) + 2 * np.abs(m).max()) @ np.abs(x)
+        assert (np.abs(got - want) <= 2.0 ** -18 * size).all()  # 64 products a chain and its min term, then some twenty sums
+    finally:
+        c.destroy()
+
+
 def test_tall_blocks_where_they_are_asked_for(monkeypatch):
     """SHV_MOE_TALL_MIN sends the down products from its number of rows on to the kernel that more than 48 rows take: the same bits a row."""
     E, H, U, F, T = 8, 264, 4, 512, 49
